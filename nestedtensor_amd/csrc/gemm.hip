@@ -15,17 +15,16 @@
 // banks; any other K takes a register-staged loop with padded LDS rows and
 // element-wise tails.
 //
-// Three tile shapes are compiled for problems that fill the chip (256x128,
-// 256x192, 256x256, eight wavefronts each); the launcher picks per problem the
-// one with the least rounds x tile cost over the CUs.  The bigger tiles read less
-// LDS per MFMA and win once the grid is several rounds deep; the smaller ones
-// quantise better on the projection shapes of one attention layer.  A problem
-// with fewer 256x128 tiles than half the CUs (the query and output projections
-// of cross-attention, a few thousand rows) takes 128x64 tiles of four
-// wavefronts, or 128x128 when those would not fit in one round: its duration is
-// one tile's life, and a quarter of a tile on four times as many CUs ends sooner
-// (3200 x 512 x 512: 10.6 -> 6.3 us; the fused in-projection of a layer of a few
-// hundred tokens: 16.0 -> 11.6 us).
+// Two kernels.  phased_kernel, for problems that fill the chip and K of at least two
+// whole K tiles: eight wavefronts in two groups half a phase apart, tile shapes of 128
+// to 320 rows by 128 or 256 columns, one of them picked per problem so that the tiles
+// fill whole rounds of the CUs.  linear_kernel takes everything else: a problem with
+// fewer 256x128 tiles than half the CUs (the query and output projections of
+// cross-attention, a few thousand rows) gets 128x64 tiles of four wavefronts, or 128x128
+// when those would not fit in one round (its duration is one tile's life, and a quarter
+// of a tile on four times as many CUs ends sooner: 3200 x 512 x 512 10.6 -> 6.3 us; the
+// fused in-projection of a layer of a few hundred tokens 16.0 -> 11.6 us), short or
+// ragged K a 256x128 tile.
 //
 // Epilogues:
 //   plain  - C row-major + bias;
@@ -34,6 +33,8 @@
 //            TRANSPOSED into Vt[n - n_split][m] so that the attention kernel
 //            finds V^T tiles key-contiguous.
 #include "nt_common.h"
+
+#include <type_traits>
 
 namespace nt {
 
@@ -93,9 +94,7 @@ struct GemmCfg {
   static constexpr int kPerThread = kPerA + kPerB;
   static constexpr int kBufBytes = (kBM + kBN) * kLdsRow;
   // direct global -> LDS loads: unpadded rows, the K tiles of A and of W in a ring
-  // each, three tiles deep if that fits and two otherwise.  (A third tile for only
-  // one of the operands, which fits beside two whole tiles of the 256x192 shape, was
-  // measured for either operand: no change, the K loop is not waiting for latency.)
+  // each, three tiles deep
   static constexpr int kATileBytes = kBM * BKB_;
   static constexpr int kBTileBytes = kBN * BKB_;
   static constexpr int kLdsBudget = 160 * 1024 - 2048;
@@ -168,8 +167,15 @@ __device__ __forceinline__ u32x4 load_chunk(const T* base, int64_t ld, int64_t r
 // costs the projection GEMMs 10 % (measured)
 enum { kEpiPlain = 0, kEpiQkv = 1, kEpiAct = 2 };
 
-// One BM x BN tile.  VT_OUT marks a V tile of the fused QKV projection, whose
-// result goes transposed into Vt.
+// LDS a wavefront needs to store its accumulators: one 32-row strip.
+template <typename T, int WM, int WN, bool VT_OUT>
+constexpr int strip_bytes() {
+  return 32 * ((VT_OUT ? WM : WN) * 32 * (int)sizeof(T) + 16);
+}
+
+// Epilogue of one wavefront: its (WM * 32) x (WN * 32) accumulators, whose first row
+// is m_wave and whose first column is n0 + n_wave, go to C (or, VT_OUT, transposed to
+// Vt) with the bias added.
 //
 // The accumulators of a 32x32 MFMA block hold, per lane, four runs of four
 // consecutive rows of one column of D.  Both operand fragments have the same
@@ -180,6 +186,114 @@ enum { kEpiPlain = 0, kEpiQkv = 1, kEpiAct = 2 };
 // moves each 32-row strip through a private LDS region of the wavefront, 8 or
 // 16 bytes per lane in, and back out as 16-byte pieces of whole rows, so the
 // global stores are row-contiguous instead of 2 bytes per lane.
+template <typename T, int WM, int WN, bool VT_OUT, bool ACT>
+__device__ __forceinline__ void store_tile(const GemmArgs<T>& a, const acc16 (&acc)[WM][WN], int64_t m_wave,
+                                           int64_t n0, int n_wave, char* strip, const float* lds_bias) {
+  constexpr int kPer = 16 / sizeof(T);
+  const int lane = threadIdx.x & 63;
+  const int l32 = lane & 31;
+  const int g = lane >> 5;
+  constexpr int kStripW = VT_OUT ? WM : WN;                    // 32-wide blocks per strip row
+  constexpr int kStripRow = kStripW * 32 * (int)sizeof(T) + 16;
+  constexpr int kCpr = kStripW * 32 * (int)sizeof(T) / 16;    // 16-byte pieces per strip row
+  typedef T Quad __attribute__((ext_vector_type(4)));
+
+  if (!VT_OUT) {
+    // acc[i][j][e] = C[row, col], row = .. + i*32 + l32, col = .. + j*32 + 8*(e/4) + 4*g + e%4
+    const bool row_vec_ok = (a.ldc * (int64_t)sizeof(T)) % 16 == 0 &&
+                            reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int c0 = j * 32 + 8 * r + 4 * g;
+          const float4 bv = *reinterpret_cast<const float4*>(lds_bias + n_wave + c0);
+          Quad q;
+          if (!ACT) {
+            q[0] = (T)(acc[i][j][4 * r + 0] + bv.x);
+            q[1] = (T)(acc[i][j][4 * r + 1] + bv.y);
+            q[2] = (T)(acc[i][j][4 * r + 2] + bv.z);
+            q[3] = (T)(acc[i][j][4 * r + 3] + bv.w);
+          } else {
+            q[0] = (T)apply_act(acc[i][j][4 * r + 0] + bv.x, a.act);
+            q[1] = (T)apply_act(acc[i][j][4 * r + 1] + bv.y, a.act);
+            q[2] = (T)apply_act(acc[i][j][4 * r + 2] + bv.z, a.act);
+            q[3] = (T)apply_act(acc[i][j][4 * r + 3] + bv.w, a.act);
+          }
+          *reinterpret_cast<Quad*>(strip + l32 * kStripRow + c0 * (int)sizeof(T)) = q;
+        }
+      }
+      __builtin_amdgcn_wave_barrier();   // LDS serves a wavefront's accesses in order
+#pragma unroll
+      for (int it = 0; it < 32 * kCpr / 64; ++it) {
+        const int idx = it * 64 + lane;
+        const int r = idx / kCpr, c = idx % kCpr;
+        const int64_t row = m_wave + i * 32 + r;
+        const int64_t col = n0 + n_wave + c * kPer;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(strip + r * kStripRow + c * 16);
+        if (row < a.M && col < a.N) {
+          T* dst = a.C + row * a.ldc + col;
+          if (row_vec_ok && col + kPer <= a.N) {
+            store16(reinterpret_cast<char*>(dst), v);
+          } else {
+            T tmp[kPer];
+            __builtin_memcpy(tmp, &v, 16);
+#pragma unroll
+            for (int e = 0; e < kPer; ++e)
+              if (col + e < a.N) dst[e] = tmp[e];
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else {
+    // acc[i][j][e] = C[row, col], row = .. + i*32 + 8*(e/4) + 4*g + e%4, col = .. + j*32 + l32
+    const bool row_vec_ok = (a.ldvt * (int64_t)sizeof(T)) % 16 == 0 &&
+                            reinterpret_cast<uintptr_t>(a.Vt) % 16 == 0;
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const float bv = lds_bias[n_wave + j * 32 + l32];
+#pragma unroll
+      for (int i = 0; i < WM; ++i) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          Quad q;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[e] = (T)(acc[i][j][4 * r + e] + bv);
+          *reinterpret_cast<Quad*>(strip + l32 * kStripRow +
+                                   (i * 32 + 8 * r + 4 * g) * (int)sizeof(T)) = q;
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int it = 0; it < 32 * kCpr / 64; ++it) {
+        const int idx = it * 64 + lane;
+        const int r = idx / kCpr, c = idx % kCpr;
+        const int64_t col = n0 + n_wave + j * 32 + r;           // feature
+        const int64_t row = m_wave + c * kPer;          // first token of the piece
+        const u32x4 v = *reinterpret_cast<const u32x4*>(strip + r * kStripRow + c * 16);
+        if (col < a.N && row < a.M) {
+          T* dst = a.Vt + (col - a.n_split) * a.ldvt + row;
+          if (row_vec_ok && row + kPer <= a.M) {
+            store16(reinterpret_cast<char*>(dst), v);
+          } else {
+            T tmp[kPer];
+            __builtin_memcpy(tmp, &v, 16);
+#pragma unroll
+            for (int e = 0; e < kPer; ++e)
+              if (row + e < a.M) dst[e] = tmp[e];
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+
+// One BM x BN tile.  VT_OUT marks a V tile of the fused QKV projection, whose
+// result goes transposed into Vt.
 template <typename T, class Cfg, bool VT_OUT, bool ALIGNED_K, bool ACT = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs<T>& a, int64_t m0, int64_t n0, char* lds) {
   typedef Mma<T> MM;
@@ -425,109 +539,12 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs<T>& a, int64_t m0, int6
     }
   }
 
-  // ---- epilogue ----------------------------------------------------------
-  // (the K loop ended with a barrier and no load into LDS is outstanding: the tile
-  // buffers are free)
-  constexpr int kStripW = VT_OUT ? WM : WN;                    // 32-wide blocks per strip row
-  constexpr int kStripRow = kStripW * 32 * (int)sizeof(T) + 16;
-  constexpr int kCpr = kStripW * 32 * (int)sizeof(T) / 16;    // 16-byte pieces per strip row
-  static_assert((Cfg::kThreads / 64) * 32 * kStripRow <= Cfg::kLdsBytes, "strips must fit");
-  char* strip = lds + wave * (32 * kStripRow);
-  const float* lds_bias = reinterpret_cast<const float*>(lds + Cfg::kLdsBytes);
-  typedef T Quad __attribute__((ext_vector_type(4)));
-
-  if (!VT_OUT) {
-    // acc[i][j][e] = C[row, col], row = .. + i*32 + l32, col = .. + j*32 + 8*(e/4) + 4*g + e%4
-    const bool row_vec_ok = (a.ldc * (int64_t)sizeof(T)) % 16 == 0 &&
-                            reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-#pragma unroll
-      for (int j = 0; j < WN; ++j) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int c0 = j * 32 + 8 * r + 4 * g;
-          const float4 bv = *reinterpret_cast<const float4*>(lds_bias + wn * WN * 32 + c0);
-          Quad q;
-          if (!ACT) {
-            q[0] = (T)(acc[i][j][4 * r + 0] + bv.x);
-            q[1] = (T)(acc[i][j][4 * r + 1] + bv.y);
-            q[2] = (T)(acc[i][j][4 * r + 2] + bv.z);
-            q[3] = (T)(acc[i][j][4 * r + 3] + bv.w);
-          } else {
-            q[0] = (T)apply_act(acc[i][j][4 * r + 0] + bv.x, a.act);
-            q[1] = (T)apply_act(acc[i][j][4 * r + 1] + bv.y, a.act);
-            q[2] = (T)apply_act(acc[i][j][4 * r + 2] + bv.z, a.act);
-            q[3] = (T)apply_act(acc[i][j][4 * r + 3] + bv.w, a.act);
-          }
-          *reinterpret_cast<Quad*>(strip + l32 * kStripRow + c0 * (int)sizeof(T)) = q;
-        }
-      }
-      __builtin_amdgcn_wave_barrier();   // LDS serves a wavefront's accesses in order
-#pragma unroll
-      for (int it = 0; it < 32 * kCpr / 64; ++it) {
-        const int idx = it * 64 + lane;
-        const int r = idx / kCpr, c = idx % kCpr;
-        const int64_t row = m0 + (wm * WM + i) * 32 + r;
-        const int64_t col = n0 + wn * WN * 32 + c * kPer;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(strip + r * kStripRow + c * 16);
-        if (row < a.M && col < a.N) {
-          T* dst = a.C + row * a.ldc + col;
-          if (row_vec_ok && col + kPer <= a.N) {
-            store16(reinterpret_cast<char*>(dst), v);
-          } else {
-            T tmp[kPer];
-            __builtin_memcpy(tmp, &v, 16);
-#pragma unroll
-            for (int e = 0; e < kPer; ++e)
-              if (col + e < a.N) dst[e] = tmp[e];
-          }
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-  } else {
-    // acc[i][j][e] = C[row, col], row = .. + i*32 + 8*(e/4) + 4*g + e%4, col = .. + j*32 + l32
-    const bool row_vec_ok = (a.ldvt * (int64_t)sizeof(T)) % 16 == 0 &&
-                            reinterpret_cast<uintptr_t>(a.Vt) % 16 == 0;
-#pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const float bv = lds_bias[(wn * WN + j) * 32 + l32];
-#pragma unroll
-      for (int i = 0; i < WM; ++i) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          Quad q;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) q[e] = (T)(acc[i][j][4 * r + e] + bv);
-          *reinterpret_cast<Quad*>(strip + l32 * kStripRow +
-                                   (i * 32 + 8 * r + 4 * g) * (int)sizeof(T)) = q;
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int it = 0; it < 32 * kCpr / 64; ++it) {
-        const int idx = it * 64 + lane;
-        const int r = idx / kCpr, c = idx % kCpr;
-        const int64_t col = n0 + (wn * WN + j) * 32 + r;           // feature
-        const int64_t row = m0 + wm * WM * 32 + c * kPer;          // first token of the piece
-        const u32x4 v = *reinterpret_cast<const u32x4*>(strip + r * kStripRow + c * 16);
-        if (col < a.N && row < a.M) {
-          T* dst = a.Vt + (col - a.n_split) * a.ldvt + row;
-          if (row_vec_ok && row + kPer <= a.M) {
-            store16(reinterpret_cast<char*>(dst), v);
-          } else {
-            T tmp[kPer];
-            __builtin_memcpy(tmp, &v, 16);
-#pragma unroll
-            for (int e = 0; e < kPer; ++e)
-              if (row + e < a.M) dst[e] = tmp[e];
-          }
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-  }
+  // the K loop ended with a barrier and no load into LDS is outstanding: the tile
+  // buffers are free
+  static_assert((Cfg::kThreads / 64) * strip_bytes<T, WM, WN, VT_OUT>() <= Cfg::kLdsBytes, "strips must fit");
+  store_tile<T, WM, WN, VT_OUT, ACT>(a, acc, m0 + wm * WM * 32, n0, wn * WN * 32,
+                                     lds + wave * strip_bytes<T, WM, WN, VT_OUT>(),
+                                     reinterpret_cast<const float*>(lds + Cfg::kLdsBytes));
 }
 
 // Workgroup i runs on XCD i % 8 and every XCD has its own L2.  The tile order
@@ -586,21 +603,306 @@ static int launch_cfg(const GemmArgs<T>& a, hipStream_t stream) {
   return launch_kernel<T, Cfg, EPI, false>(a, stream);
 }
 
+// ---- the pipelined tile ---------------------------------------------------------
+//
+// A (64 NI) x (128 NJ) tile of eight wavefronts for problems that fill the chip.  What
+// bounds a tile whose wavefronts all do the same thing at the same time (linear_kernel)
+// is not the matrix pipe: after every barrier all wavefronts first wait for fragments
+// from LDS and only then multiply, and a K tile's loads are waited for in the iteration
+// that issued them.  Here
+//  * the wavefronts form two groups of four, one wavefront of each group per SIMD,
+//    half a phase apart: while one group reads fragments and issues loads (stage M),
+//    the other multiplies (stage C), so a SIMD's matrix pipe always has work;
+//  * a phase is one 64-row block of A (32 rows per group, consecutive from phase to
+//    phase so that a wavefront's rows are one run) against all columns: 4 fragment
+//    reads and 4 NJ matrix instructions per wavefront; the W fragments of a K tile stay
+//    in registers over its NI phases;
+//  * an LDS slot is refilled as soon as its last reader is two phases past it: the load
+//    of a block is issued NI * kBufs - 2 phases before the block is read (2500 to 5000
+//    cycles), and the wait for it counts exactly the loads issued since.
+// Measured (fp16): on operands of zeros a 320 x 256 tile takes 1.12 us per K tile of 64,
+// its 80 matrix instructions per SIMD back to back at 2.3 GHz; on N(0, 1) operands
+// 1.85 us with all CUs at work, where the chip lowers its clock (1.28 PFLOP/s over
+// all CUs; the vendor's 8192^3 product reaches 1.16 to 1.2).  Outside the K loop a launch
+// costs about 3.5 us and 0.9 us per NI * NJ, the burst of stores at 4.7 TB/s.
+// Against linear_kernel: 8040 x 2304 x 768 46.0 -> 32.9 us, 12900 x 3072 x 1024
+// 99.6 -> 80.3, 20000 x 6144 x 2048 501 -> 408, 20500 x 1024 x 512 43.3 -> 30.5,
+// 8040 x 768 x 768 16.5 -> 13.5.  (Whether the four to two loads of a W tile go out one,
+// two or four per phase makes no difference, nor does writing C through or around the
+// L2.)
+template <typename T, int NI_, int NJ_, int BUFS_>
+struct PhasedCfg {
+  static constexpr int kNI = NI_, kNJ = NJ_, kBufs = BUFS_;
+  static constexpr int kThreads = 512;
+  static constexpr int kBM = 64 * NI_, kBN = 128 * NJ_;
+  static constexpr int kABytes = kBM * 128, kBBytes = kBN * 128;   // one K tile: 128 bytes per row
+  static constexpr int kLdsBytes = BUFS_ * (kABytes + kBBytes);
+  static_assert(kLdsBytes + kBN * 4 <= 160 * 1024, "tile buffers must fit the LDS");
+};
+
+// Schedule of the loads.  In phase i of K tile t a wavefront issues one load of A (its
+// eight rows of the block NI * kBufs - 2 phases on) and then some of the Q 64-row parts
+// ("quarters") of a W tile: those of tile T go out in the first phases after the last
+// read of its slot, from phase 2 of tile T - kBufs on.
+template <int NI, int Q>
+struct PhasedSchedule {
+  static constexpr int kPerPhase = (Q + NI - 1) / NI > 2 ? (Q + NI - 1) / NI : 2;
+  static constexpr int window(int i) { return (i + NI - 2) % NI; }       // place of phase i among those NI
+  static constexpr int at_window(int w) {
+    return Q <= kPerPhase * w ? 0 : Q - kPerPhase * w < kPerPhase ? Q - kPerPhase * w : kPerPhase;
+  }
+  static constexpr int quarters(int i) { return at_window(window(i)); }
+  static constexpr int first_quarter(int i) {
+    int q = 0;
+    for (int w = 0; w < window(i); ++w) q += at_window(w);
+    return q;
+  }
+  static constexpr int last_window() { return (Q + kPerPhase - 1) / kPerPhase - 1; }
+  // loads issued before phase i of K tile t (any origin)
+  static constexpr int issued_before(int t, int i) {
+    int n = t * (NI + Q);
+    for (int k = 0; k < i; ++k) n += 1 + quarters(k);
+    return n;
+  }
+  static constexpr int issued_before_phase(int p) {   // p may be negative
+    const int t = (p + 64 * NI) / NI - 64;
+    return issued_before(t, p - t * NI);
+  }
+  // Loads that may be outstanding at the end of stage M of phase i of a K tile with
+  // `left` tiles to go (this one included; the last kBufs tiles issue fewer loads)
+  // such that everything the next phase reads has landed.
+  static constexpr int may_be_outstanding(int bufs, int i, int left) {
+    const int next = i + 1;                           // phase, relative to the tile
+    const int ahead = NI * bufs - 2;
+    int needed = issued_before_phase(next - ahead) + 1;          // A is the first load of its phase
+    if (next == NI) {                                            // a new K tile: its last W quarter
+      const int w = issued_before_phase(NI - NI * bufs + 2 + last_window() + 1);
+      if (w > needed) needed = w;
+    }
+    int issued = issued_before_phase(next);
+    const int final = issued_before_phase((left - bufs) * NI + 2);
+    if (final < issued) issued = final;
+    return issued > needed ? issued - needed : 0;
+  }
+};
+
+template <typename T, class Cfg, bool VT_OUT, bool ACT>
+__device__ __forceinline__ void phased_tile(const GemmArgs<T>& a, int64_t m0, int64_t n0, char* lds) {
+  typedef Mma<T> MM;
+  typedef typename MM::Frag Frag;
+  constexpr int NI = Cfg::kNI, NJ = Cfg::kNJ, kBufs = Cfg::kBufs, kQ = Cfg::kBN / 64;
+  typedef PhasedSchedule<NI, kQ> S;
+  constexpr int kSteps = 128 / (MM::kK * (int)sizeof(T));
+  static_assert(kSteps == 4 && MM::kK * (int)sizeof(T) == 32, "a step is two 16-byte pieces of a row");
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wave >> 2;      // rows group * 32 NI .. of the tile
+  const int wn = wave & 3;          // columns wn * 64 ..
+  const int l32 = lane & 31;
+  const int g = lane >> 5;
+
+  acc16 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+  const int nk = (int)(a.K * (int64_t)sizeof(T) / 128);
+  if (tid < Cfg::kBN) {
+    const int64_t col = n0 + tid;
+    reinterpret_cast<float*>(lds + Cfg::kLdsBytes)[tid] = (a.bias && col < a.N) ? (float)a.bias[col] : 0.0f;
+  }
+
+  // Global addresses: a wavefront loads 8 rows of 128 bytes per instruction, slot p of
+  // row r holding piece p ^ ((r >> 1) & 7) so that fragment reads are conflict-free.
+  // Per-lane 32-bit offsets (rows past the end clamped to the last one: they only feed
+  // accumulators that are not stored) from a scalar base that moves with the K tile.
+  const int r8 = wave * 8 + (lane >> 3);                       // row of the 64-row block
+  const int piece = ((lane & 7) ^ ((r8 >> 1) & 7)) * 16;
+  unsigned a_off[NI], w_off[kQ];
+  const int64_t rows_left = a.M - m0, cols_left = a.N - n0;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    int64_t row = (r8 >> 5) * (32 * NI) + i * 32 + (r8 & 31);
+    row = row < rows_left ? row : rows_left - 1;
+    a_off[i] = (unsigned)(row * a.lda * (int64_t)sizeof(T) + piece);
+  }
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) {
+    int64_t row = q * 64 + r8;
+    row = row < cols_left ? row : cols_left - 1;
+    w_off[q] = (unsigned)(row * a.K * (int64_t)sizeof(T) + piece);
+  }
+  const char* a_base = reinterpret_cast<const char*>(a.A + m0 * a.lda);
+  const char* w_base = reinterpret_cast<const char*>(a.W + n0 * a.K);
+  const unsigned lds_base = (unsigned)reinterpret_cast<uintptr_t>(lds);
+  constexpr unsigned kWRing = kBufs * Cfg::kABytes;
+  const unsigned my_kib = (unsigned)wave * 1024;
+  auto load_lds = [&](const char* base, unsigned off, unsigned dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst)
+                 : "memory");
+  };
+  // the loads of phase i of a K tile: block (i - 2 mod NI) of A and the quarters of W
+  // of K tile `tile`, into its slot
+  auto issue = [&](int i, int tile, int slot) {
+    const int64_t koff = (int64_t)tile * 128;
+    const int blk = (i + NI - 2) % NI;
+    load_lds(a_base + koff, a_off[blk], lds_base + slot * Cfg::kABytes + blk * 8192 + my_kib);
+    const int q0 = S::first_quarter(i);
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      if (q < q0 || q >= q0 + S::quarters(i)) continue;
+      load_lds(w_base + koff, w_off[q], lds_base + kWRing + slot * Cfg::kBBytes + q * 8192 + my_kib);
+    }
+  };
+
+  // fragment addresses: piece 2 s + g of row l32 of a 32-row block
+  const int sw = (l32 >> 1) & 7;
+  int koff[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) koff[s] = ((2 * s + g) ^ sw) * 16;
+  const int a_row = (group * 32 + l32) * 128;
+  const int w_row = (wn * (32 * NJ) + l32) * 128;
+
+  Frag fa[4], fb[NJ][4];
+
+  // Prologue: what the kBufs virtual K tiles before the first would have issued.
+#pragma unroll
+  for (int v = 0; v < kBufs; ++v) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if (v == 0 && i < 2) continue;
+      const int tile = i < 2 ? v - 1 : v;
+      issue(i, tile, tile);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S::may_be_outstanding(kBufs, NI - 1, 64)) : "memory");
+  __syncthreads();
+  if (group == 1) {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+
+  int slot = 0, prev = kBufs - 1;
+  // one K tile; LEFT: tiles to go including this one (any number above kBufs: steady state)
+  auto k_tile = [&](int t, auto left_c) __attribute__((always_inline)) {
+    constexpr int LEFT = decltype(left_c)::value;
+    const char* at = lds + slot * Cfg::kABytes + a_row;
+    const char* wt = lds + kWRing + slot * Cfg::kBBytes + w_row;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      // stage M
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        fa[s] = *reinterpret_cast<const Frag*>(at + i * 8192 + koff[s]);
+        if (i == 0) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) fb[j][s] = *reinterpret_cast<const Frag*>(wt + j * (32 * 128) + koff[s]);
+        }
+      }
+      if (i < 2 ? LEFT >= kBufs : LEFT > kBufs) {
+        if (i < 2) issue(i, t + kBufs - 1, prev);
+        else issue(i, t + kBufs, slot);
+      }
+      if (!(LEFT == 1 && i == NI - 1)) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S::may_be_outstanding(kBufs, i, LEFT)) : "memory");
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      // stage C
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          if (VT_OUT) {
+            acc[i][j] = MM::run(fa[s], fb[j][s], acc[i][j]);
+          } else {
+            acc[i][j] = MM::run(fb[j][s], fa[s], acc[i][j]);
+          }
+        }
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    prev = slot;
+    slot = slot + 1 == kBufs ? 0 : slot + 1;
+  };
+  int t = 0;
+  for (; t < nk - kBufs; ++t) k_tile(t, std::integral_constant<int, 64>());
+  if constexpr (kBufs >= 4) k_tile(t++, std::integral_constant<int, 4>());
+  if constexpr (kBufs >= 3) k_tile(t++, std::integral_constant<int, 3>());
+  k_tile(t++, std::integral_constant<int, 2>());
+  k_tile(t, std::integral_constant<int, 1>());
+  if (group == 0) __builtin_amdgcn_s_barrier();
+  __syncthreads();
+
+  static_assert(8 * strip_bytes<T, NI, NJ, VT_OUT>() <= Cfg::kLdsBytes, "strips must fit");
+  store_tile<T, NI, NJ, VT_OUT, ACT>(a, acc, m0 + group * (32 * NI), n0, wn * (32 * NJ),
+                                    lds + wave * strip_bytes<T, NI, NJ, VT_OUT>(),
+                                    reinterpret_cast<const float*>(lds + Cfg::kLdsBytes));
+}
+
+// Tile order: workgroup i runs on XCD i % 8, and every XCD gets one contiguous run of
+// the tile list (equal lengths up to one tile, so no XCD runs a round more than the
+// others).  The list walks bands of four row tiles, column panel by column panel: the
+// tiles an XCD runs at a time share few rows of A and few panels of W, which its L2
+// serves.
+template <typename T, class Cfg, int EPI>
+__global__ __launch_bounds__(512, 2) void phased_kernel(GemmArgs<T> a) {
+  extern __shared__ __align__(16) char lds[];
+  const int tiles_m = (int)((a.M + Cfg::kBM - 1) / Cfg::kBM);
+  const int tiles_n = (int)((a.N + Cfg::kBN - 1) / Cfg::kBN);
+  const int total = tiles_m * tiles_n;
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int share = total >> 3, more = total & 7;
+  if (local >= share + (xcd < more ? 1 : 0)) return;
+  const int id = xcd * share + (xcd < more ? xcd : more) + local;
+  constexpr int kBand = 4;
+  const int band = id / (kBand * tiles_n);
+  const int in_band = id - band * (kBand * tiles_n);
+  const int rows = tiles_m - band * kBand < kBand ? tiles_m - band * kBand : kBand;
+  const int tn = in_band / rows;
+  const int tm = band * kBand + in_band - tn * rows;
+  const int64_t m0 = (int64_t)tm * Cfg::kBM;
+  const int64_t n0 = (int64_t)tn * Cfg::kBN;
+  if constexpr (EPI == kEpiQkv) {
+    if (n0 >= a.n_split) {
+      phased_tile<T, Cfg, true, false>(a, m0, n0, lds);
+      return;
+    }
+  }
+  phased_tile<T, Cfg, false, EPI == kEpiAct>(a, m0, n0, lds);
+}
+
+template <typename T, class Cfg, int EPI>
+static int launch_phased(const GemmArgs<T>& a, hipStream_t stream) {
+  const int64_t tiles = ((a.M + Cfg::kBM - 1) / Cfg::kBM) * ((a.N + Cfg::kBN - 1) / Cfg::kBN);
+  const int lds_bytes = Cfg::kLdsBytes + Cfg::kBN * (int)sizeof(float);
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(phased_kernel<T, Cfg, EPI>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return fail(NT_ERR_HIP, "linear: %s", hipGetErrorString(e));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((phased_kernel<T, Cfg, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds_bytes, stream,
+                     a);
+  return check_launch("phased_kernel");
+}
+
 // WAVES_M, WAVES_N, WM, WN, K-tile bytes per row
-typedef GemmCfg<4, 2, 2, 2, 128> Cfg128;   // 256 x 128
-typedef GemmCfg<4, 2, 2, 3, 128> Cfg192;   // 256 x 192
-typedef GemmCfg<4, 2, 2, 4, 128> Cfg256;   // 256 x 256
+typedef GemmCfg<4, 2, 2, 2, 128> Cfg128;   // 256 x 128: whatever the pipelined tile does not take
 typedef GemmCfg<2, 2, 2, 1, 128> CfgSmall; // 128 x 64, four wavefronts: problems of fewer 256-row tiles than CUs
 typedef GemmCfg<2, 2, 2, 2, 128> CfgMid;   // 128 x 128, four wavefronts
 
-// Tile shape with the least estimated time.  A tile costs its area divided by the
-// measured steady-state rate of its shape relative to 256x128 (wider wavefront
-// tiles read less LDS and L2 per MFMA).  The number of tiles a CU runs one after
-// the other is taken as the mean of the whole rounds (all tiles start together
-// and take equally long) and of tiles / CUs (a partly filled last round runs
-// faster, it shares the memory path with fewer workgroups); fitted on the
-// projection shapes of the two attention benchmarks and on large square problems.
-static int pick_cfg(int64_t M, int64_t N, int64_t n_split, int* which) {
+static int compute_units(int* n) {
   static int num_cus = 0;
   if (num_cus == 0) {
     int dev = 0;
@@ -611,55 +913,95 @@ static int pick_cfg(int64_t M, int64_t N, int64_t n_split, int* which) {
     }
     num_cus = prop.multiProcessorCount;
   }
-  const int bn[3] = {Cfg128::kBN, Cfg192::kBN, Cfg256::kBN};
-  const double eff[3] = {1.0, 1.08, 1.17};
+  *n = num_cus;
+  return NT_OK;
+}
+
+// Tile shapes of the pipelined kernel.  `alone` and `full`: microseconds per K tile
+// (128 bytes of a row) of a workgroup of 16-bit operands when few CUs and when all CUs
+// are at work; the difference is the clock the chip holds on random operands.
+struct PhasedShape {
+  int ni, nj, bufs;
+  double alone, full;
+};
+static const PhasedShape kPhasedShapes[] = {
+    {2, 2, 3, 0.55, 0.91}, {3, 2, 2, 0.73, 1.31},  {4, 2, 2, 0.90, 1.65}, {5, 2, 2, 1.12, 2.05},
+    {2, 1, 4, 0.37, 0.55}, {3, 1, 3, 0.485, 0.745}, {4, 1, 3, 0.56, 0.94}, {5, 1, 2, 0.70, 1.19}};
+
+// Shape with the least estimated time for M x N with nk K tiles: whole rounds over the
+// CUs at the full rate, a last round at the rate its tiles leave (never below `alone`),
+// 4 us per further round, and the launch and the burst of stores.  The estimate is within
+// 10 % of the measured time on 14 of the 16 projection shapes it was fitted on (512 to
+// 6144 columns, K 512 to 4096, 3 to 24 column panels, one to eight rounds) and ranks the
+// shapes as measured on all of them; the two misses are its own second-best shapes.
+// fp32: 64 cycles of matrix pipe per instruction, no lowered clock.
+static int pick_phased(int64_t M, int64_t N, int64_t n_split, int64_t nk, int elem_bytes, int num_cus) {
   int best = -1;
-  double best_cost = 0.0;
-  for (int c = 0; c < 3; ++c) {
-    if (n_split % bn[c] != 0) continue;          // a tile must not straddle the K | V boundary
-    const int64_t tiles = ((M + 255) / 256) * ((N + bn[c] - 1) / bn[c]);
-    const double whole = (double)((tiles + num_cus - 1) / num_cus);
-    const double fluid = (double)tiles / num_cus;
-    const double cost = 0.5 * (whole + fluid) * bn[c] / eff[c];
-    if (best < 0 || cost < best_cost) {
+  double best_us = 0.0;
+  for (int c = 0; c < (int)(sizeof(kPhasedShapes) / sizeof(kPhasedShapes[0])); ++c) {
+    const PhasedShape& s = kPhasedShapes[c];
+    const int64_t bm = 64 * s.ni, bn = 128 * s.nj;
+    // a tile must not straddle the K | V boundary, and the prologue fills its whole ring
+    if (n_split % bn != 0 || nk < s.bufs) continue;
+    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const int64_t whole = tiles / num_cus, rest = tiles % num_cus;
+    const double alone = elem_bytes == 4 ? 0.853 * s.ni * s.nj : s.alone;
+    const double full = elem_bytes == 4 ? alone : s.full;
+    double last = full * (double)rest / num_cus;
+    if (rest > 0 && last < alone) last = alone;
+    const double us = nk * (whole * full + last) + 4.0 * (double)(whole + (rest > 0) - 1) +
+                      3.5 + 0.9 * s.ni * s.nj * (elem_bytes / 2);
+    if (best < 0 || us < best_us) {
       best = c;
-      best_cost = cost;
+      best_us = us;
     }
   }
-  if (best < 0) {
-    return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of a column tile",
-                (long long)n_split);
-  }
-  // Fewer 256 x 128 tiles than half the CUs: the launch is one tile's life on a
-  // fraction of the chip, and a quarter-size tile on four times as many CUs is shorter.
-  if (((M + 255) / 256) * ((N + 127) / 128) * 2 <= num_cus) {
-    const int small = ((M + 127) / 128) * ((N + 63) / 64) <= num_cus ? 3 : 4;
-    const int64_t small_bn = small == 3 ? CfgSmall::kBN : CfgMid::kBN;
-    if (n_split % small_bn == 0) best = small;   // (a tile must not straddle the K | V boundary)
-  }
-  *which = best;
-  return NT_OK;
+  return best;
 }
 
 template <typename T, int EPI>
 static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
-  int which = 0;
-  // the fp32 path exists for parity checks; it is compiled for one shape only
-  if constexpr (sizeof(T) == 4) {
-    if (EPI == kEpiQkv && a.n_split % Cfg128::kBN != 0) {
-      return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of the column tile",
-                  (long long)a.n_split);
+  const int64_t n_split = EPI == kEpiQkv ? a.n_split : 0;
+  int num_cus = 0;
+  const int rc = compute_units(&num_cus);
+  if (rc != NT_OK) return rc;
+  // Fewer 256 x 128 tiles than half the CUs: the launch is one tile's life on a fraction
+  // of the chip, and a quarter-size tile on four times as many CUs is shorter
+  // (3200 x 512 x 512: 6.2 us, against 6.8 with the smallest pipelined tile).
+  if constexpr (sizeof(T) == 2) {
+    if (((a.M + 255) / 256) * ((a.N + 127) / 128) * 2 <= num_cus) {
+      const bool small = ((a.M + 127) / 128) * ((a.N + 63) / 64) <= num_cus;
+      if (small && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
+      if (!small && n_split % CfgMid::kBN == 0) return launch_cfg<T, CfgMid, EPI>(a, stream);
     }
-    return launch_cfg<T, Cfg128, EPI>(a, stream);
-  } else {
-    const int rc = pick_cfg(a.M, a.N, EPI == kEpiQkv ? a.n_split : 0, &which);
-    if (rc != NT_OK) return rc;
-    if (which == 3) return launch_cfg<T, CfgSmall, EPI>(a, stream);
-    if (which == 4) return launch_cfg<T, CfgMid, EPI>(a, stream);
-    if (which == 1) return launch_cfg<T, Cfg192, EPI>(a, stream);
-    if (which == 2) return launch_cfg<T, Cfg256, EPI>(a, stream);
-    return launch_cfg<T, Cfg128, EPI>(a, stream);
   }
+  // The pipelined tile needs whole K tiles, at least two of them, and 32-bit offsets
+  // inside a tile.  (fp32: row-major results only, the transposed strips
+  // would not fit its LDS.)
+  constexpr int64_t kMaxSpan = (int64_t(1) << 32) - 1;
+  const int64_t row_bytes = a.K * (int64_t)sizeof(T);
+  if constexpr (sizeof(T) == 2 || EPI != kEpiQkv) {
+    if (row_bytes % 128 == 0 && row_bytes >= 2 * 128 && a.lda * (int64_t)sizeof(T) * 320 < kMaxSpan &&
+        row_bytes * 256 < kMaxSpan && (a.M / 64 + 1) * (a.N / 64 + 1) < (int64_t(1) << 30)) {
+      switch (pick_phased(a.M, a.N, n_split, row_bytes / 128, (int)sizeof(T), num_cus)) {
+        case 0: return launch_phased<T, PhasedCfg<T, 2, 2, 3>, EPI>(a, stream);
+        case 1: return launch_phased<T, PhasedCfg<T, 3, 2, 2>, EPI>(a, stream);
+        case 2: return launch_phased<T, PhasedCfg<T, 4, 2, 2>, EPI>(a, stream);
+        case 3: return launch_phased<T, PhasedCfg<T, 5, 2, 2>, EPI>(a, stream);
+        case 4: return launch_phased<T, PhasedCfg<T, 2, 1, 4>, EPI>(a, stream);
+        case 5: return launch_phased<T, PhasedCfg<T, 3, 1, 3>, EPI>(a, stream);
+        case 6: return launch_phased<T, PhasedCfg<T, 4, 1, 3>, EPI>(a, stream);
+        case 7: return launch_phased<T, PhasedCfg<T, 5, 1, 2>, EPI>(a, stream);
+      }
+    }
+  }
+  if constexpr (sizeof(T) == 2) {
+    if (n_split % Cfg128::kBN != 0 && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
+  }
+  if (n_split % Cfg128::kBN != 0) {
+    return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of a column tile", (long long)n_split);
+  }
+  return launch_cfg<T, Cfg128, EPI>(a, stream);
 }
 
 template <typename T>
