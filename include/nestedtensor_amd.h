@@ -311,6 +311,20 @@ int nt_varlen_attention_vt(const void* q, int64_t ldq, const void* k, int64_t ld
                            int64_t n_work, int64_t num_heads, int64_t head_dim,
                            int64_t total_kv_tokens, float scale, int dtype, void* stream);
 
+/* The work list nt_varlen_attention_vt and nt_varlen_attention_scheduled take, from
+ * the query and key lengths of the B sequences (HOST int64 arrays; k_lens NULL: each
+ * sequence attends to itself): one item per q_tile query rows of every sequence,
+ * longest key sequences first, ties in their order.  nt_attention_schedule_items
+ * counts the items (minus an NT_ERR_* code on error); nt_attention_schedule writes
+ * them to `schedule` (device, int32[8 n_items]) with launches that carry the lengths
+ * in their arguments, so nothing is copied and `stream` is not waited for.  It
+ * returns NT_ERR_UNSUPPORTED when there are more than 2^31 - 1 query or key tokens.
+ * The counterpart of the per-call metadata the reference builds on the host
+ * (nestedtensor/csrc/cuda/mha.cpp:35-57). */
+int64_t nt_attention_schedule_items(const int64_t* q_lens, int64_t B, int64_t q_tile);
+int nt_attention_schedule(const int64_t* q_lens, const int64_t* k_lens, int64_t B, int64_t q_tile,
+                          int32_t* schedule, int64_t n_items, void* stream);
+
 /* The same attention from a PLAN instead of a work list (head_dim 64, f16 / bf16):
  * persistent workgroups, one per compute unit, twelve wavefronts each, that bring a
  * sequence's K and V^T tiles into LDS with direct global -> LDS loads, 256 keys per

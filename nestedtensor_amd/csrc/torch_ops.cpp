@@ -974,6 +974,31 @@ Tensor attention_plan(const Tensor& q_lens, const Tensor& k_lens, int64_t num_he
   return plan.to(device);
 }
 
+// Work list of the attention kernels (nt_attention_schedule) on `device` for nested
+// sizes whose first column holds the lengths (host int64 [B, D]).
+Tensor attention_schedule(const Tensor& q_sizes, const Tensor& k_sizes, int64_t q_tile, c10::Device device) {
+  TORCH_CHECK(q_sizes.device().is_cpu() && k_sizes.device().is_cpu() && q_sizes.scalar_type() == at::kLong &&
+                  k_sizes.scalar_type() == at::kLong && q_sizes.dim() == 2 && k_sizes.dim() == 2 &&
+                  q_sizes.size(0) == k_sizes.size(0) && q_sizes.size(1) > 0 && k_sizes.size(1) > 0,
+              "attention_schedule: the nested sizes must be host int64 [B, D] tables of one B");
+  TORCH_CHECK(device.is_cuda(), "attention_schedule: the work list is for a GPU");
+  const int64_t B = q_sizes.size(0);
+  std::vector<int64_t> lens(static_cast<size_t>(2 * B));
+  const int64_t *q = q_sizes.const_data_ptr<int64_t>(), *k = k_sizes.const_data_ptr<int64_t>();
+  for (int64_t b = 0; b < B; ++b) {
+    lens[b] = q[b * q_sizes.stride(0)];
+    lens[B + b] = k[b * k_sizes.stride(0)];
+  }
+  const int64_t n = nt_attention_schedule_items(lens.data(), B, q_tile);
+  TORCH_CHECK(n >= 0, "attention_schedule: ", nt_last_error());
+  c10::hip::HIPGuard guard(device.index());
+  Tensor out = at::empty({n, 8}, at::TensorOptions().dtype(at::kInt).device(device));
+  const int rc = nt_attention_schedule(lens.data(), lens.data() + B, B, q_tile, n > 0 ? out.data_ptr<int32_t>() : nullptr, n,
+                                       stream_of(out));
+  TORCH_CHECK(rc == NT_OK, nt_last_error());
+  return out;
+}
+
 // Self-attention layer on the packed token buffer x [T, E] (min_mha, mha.cpp:18-69;
 // bt_min_mha, cuda/mha.cpp:22-107, passes no out bias): fused QKV projection with V
 // written transposed, attention over each sequence's own keys, output projection.
@@ -1434,6 +1459,7 @@ TORCH_LIBRARY(nestedtensor, m) {
   m.def("softmax_rows(Tensor x, Tensor offsets, Tensor row_offsets, int total_rows, bool log) -> Tensor");
   m.def("activation_packed(Tensor x, int act) -> Tensor");
   m.def("linear_packed(Tensor x, Tensor weight, Tensor? bias, int act) -> Tensor");
+  m.def("attention_schedule(Tensor q_sizes, Tensor k_sizes, int q_tile, Device device) -> Tensor");
   m.def("attention_plan(Tensor q_lens, Tensor k_lens, int num_heads, int head_dim, Device device) -> Tensor");
   m.def("mha_self_packed(Tensor x, Tensor schedule, int num_heads, int head_dim, Tensor in_proj_weight, "
         "Tensor? in_proj_bias, float scaling, Tensor out_proj_weight, Tensor? out_proj_bias) -> Tensor");
@@ -1473,6 +1499,7 @@ TORCH_LIBRARY_IMPL(nestedtensor, CUDA, m) {
 // element) for any device and raises for host tensors otherwise.
 TORCH_LIBRARY_IMPL(nestedtensor, CompositeExplicitAutograd, m) {
   m.impl("merge_tensor_mask", merge_tensor_mask);
+  m.impl("attention_schedule", attention_schedule);
   m.impl("attention_plan", attention_plan);   // host lengths in, device plan out
   m.impl("nt_from_tensor_mask", nt_from_tensor_mask_op);
   m.impl("from_tensor_mask_lowered", from_tensor_mask_lowered);

@@ -152,8 +152,8 @@ class NestedTensorImpl:
         return self._last_dim_rows
 
     def attention_schedule(self, kv=None, q_tile=128):
-        """Work list of the attention kernel, built from the host copies of the
-        nested sizes and cached on the device: int32 [n_work, 8] rows {first query
+        """Work list of the attention kernel (nt_attention_schedule), built from the
+        host copies of the nested sizes and cached on the device: int32 [n_work, 8] rows {first query
         token, query length, first query row of the tile, 0, first key token, key
         length, 0, 0}, one per q_tile query rows of every sequence, longest key
         sequences first (they take the most key tiles, so they should start
@@ -164,21 +164,7 @@ class NestedTensorImpl:
         cached = self._attn_schedule
         if cached is not None and cached[0] is kv.sizes:
             return cached[1]
-        q_lens, k_lens = self.sizes[:, 0], kv.sizes[:, 0]
-        if int(q_lens.sum()) > 0x7fffffff or int(k_lens.sum()) > 0x7fffffff:
-            raise RuntimeError("attention: %d query and %d key tokens; the work list holds token indices "
-                               "as int32" % (int(q_lens.sum()), int(k_lens.sum())))
-        q_starts = torch.cumsum(q_lens, 0) - q_lens
-        k_starts = torch.cumsum(k_lens, 0) - k_lens
-        order = torch.argsort(k_lens, descending=True, stable=True)
-        ntile = (q_lens[order] + q_tile - 1) // q_tile
-        seq = order[torch.repeat_interleave(torch.arange(order.numel()), ntile)]
-        first = torch.cumsum(ntile, 0) - ntile
-        rank = torch.repeat_interleave(torch.arange(order.numel()), ntile)
-        q0 = (torch.arange(int(ntile.sum())) - first[rank]) * q_tile
-        zero = torch.zeros_like(q0)
-        items = torch.stack([q_starts[seq], q_lens[seq], q0, zero, k_starts[seq], k_lens[seq], zero, zero], 1)
-        sched = items.to(torch.int32).contiguous().to(self.buffer.device)
+        sched = _attention_schedule(self.sizes, kv.sizes, q_tile, self.buffer.device)
         self._attn_schedule = (kv.sizes, sched)      # holds kv.sizes, so the identity test stays valid
         return sched
 
@@ -225,6 +211,7 @@ class NestedTensorImpl:
         return out
 
 
+_attention_schedule = _C.ops.attention_schedule.default
 _offsets_from_sizes = _C.ops.offsets_from_sizes.default
 
 
