@@ -151,6 +151,14 @@ int nt_pack_table(const int64_t* table_host, int64_t B, int64_t D, void* packed,
  * (nestedtensor/csrc/masking.cpp:471-472, 578-579). */
 int nt_upload_table(const int64_t* table_host, int64_t n, int64_t* table_dev, void* stream);
 
+/* A host nested size to device memory as sizes[B, D] together with the element
+ * offsets[B + 1] scanned from it, carried (as int32) by the arguments of up to four
+ * one-workgroup launches: no copy, nothing waits.  nt_upload_sizes_supported says
+ * whether a nested size fits (896 extents per launch, none above INT32_MAX, B and D
+ * at least 1); the upload refuses one that does not. */
+int nt_upload_sizes_supported(const int64_t* sizes_host, int64_t B, int64_t D);
+int nt_upload_sizes(const int64_t* sizes_host, int64_t B, int64_t D, int64_t* sizes, int64_t* offsets, void* stream);
+
 /* ---- mask -> nested size, compaction ----------------------------------- */
 
 /* Row statistics of a byte mask viewed as [R, M] (nonzero = true):

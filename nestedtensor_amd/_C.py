@@ -46,6 +46,8 @@ SIGNATURES = {
     "nt_pack_table_max_entries": (_i64, []),
     "nt_pack_table": (_int, [_c_void_p, _i64, _i64, _c_void_p, _c_void_p, _int, _c_void_p]),
     "nt_upload_table": (_int, [_c_void_p, _i64, _c_void_p, _c_void_p]),
+    "nt_upload_sizes_supported": (_int, [_c_void_p, _i64, _i64]),
+    "nt_upload_sizes": (_int, [_c_void_p, _i64, _i64, _c_void_p, _c_void_p, _c_void_p]),
     "nt_mask_row_counts": (_int, [_c_void_p, _i64, _i64, _c_void_p, _c_void_p, _c_void_p]),
     "nt_leading_boxes_max_dims": (_i64, []),
     "nt_leading_boxes": (_int, [_c_void_p, _c_void_p, _i64, _i64, _c_void_p, _i64, _c_void_p, _c_void_p, ctypes.c_uint32,

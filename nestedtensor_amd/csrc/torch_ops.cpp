@@ -126,6 +126,45 @@ Tensor offsets_from_sizes(const Tensor& sizes_dev) {
   return offsets;
 }
 
+// (sizes[B, D], offsets[B + 1]) on `device` from the host's sizes, without a wait where
+// the table fits a few launches' arguments (nt_upload_sizes); a larger one, or one with
+// extents beyond int32, takes a copy and the device scan.
+std::tuple<Tensor, Tensor> upload_sizes(const Tensor& sizes_in, c10::Device device) {
+  TORCH_CHECK(sizes_in.device().is_cpu() && sizes_in.scalar_type() == at::kLong && sizes_in.dim() == 2,
+              "upload_sizes: the nested size must be a host int64 [B, D] table");
+  TORCH_CHECK(device.is_cuda(), "nestedtensor_amd: device metadata is for a GPU");
+  const Tensor sizes = sizes_in.contiguous();
+  const int64_t B = sizes.size(0), D = sizes.size(1);
+  const int64_t* h = sizes.const_data_ptr<int64_t>();
+  if (!nt_upload_sizes_supported(h, B, D)) {
+    const Tensor sizes_dev = sizes.to(device);
+    return std::make_tuple(sizes_dev, offsets_from_sizes(sizes_dev));
+  }
+  c10::hip::HIPGuard guard(device.index());
+  const Tensor meta = at::empty({B * D + B + 1}, at::TensorOptions().dtype(at::kLong).device(device));
+  int64_t* p = meta.data_ptr<int64_t>();
+  check(nt_upload_sizes(h, B, D, p, p + B * D, stream_of(meta)));
+  return std::make_tuple(meta.narrow(0, 0, B * D).view({B, D}), meta.narrow(0, B * D, B + 1));
+}
+
+// A host int64 table of any shape on `device`: in the arguments of a few launches
+// (nt_upload_table), or by a copy that waits where it is larger than that.
+Tensor upload_table(const Tensor& table_in, c10::Device device) {
+  TORCH_CHECK(table_in.device().is_cpu() && table_in.scalar_type() == at::kLong,
+              "upload_table: the table must be a host int64 tensor");
+  TORCH_CHECK(device.is_cuda(), "nestedtensor_amd: device metadata is for a GPU");
+  const Tensor table = table_in.contiguous();
+  const int64_t n = table.numel(), per_launch = nt_pack_table_max_entries();
+  if (n > 4 * per_launch) return table.to(device);
+  c10::hip::HIPGuard guard(device.index());
+  Tensor out = at::empty(table.sizes(), table.options().device(device));
+  const int64_t* h = table.const_data_ptr<int64_t>();
+  for (int64_t done = 0; done < n; done += per_launch) {
+    check(nt_upload_table(h + done, std::min(per_launch, n - done), out.data_ptr<int64_t>() + done, stream_of(out)));
+  }
+  return out;
+}
+
 // ---- packed <-> padded --------------------------------------------------------
 
 struct PadArgs {
@@ -1459,6 +1498,8 @@ TORCH_LIBRARY(nestedtensor, m) {
   m.def("softmax_rows(Tensor x, Tensor offsets, Tensor row_offsets, int total_rows, bool log) -> Tensor");
   m.def("activation_packed(Tensor x, int act) -> Tensor");
   m.def("linear_packed(Tensor x, Tensor weight, Tensor? bias, int act) -> Tensor");
+  m.def("upload_sizes(Tensor sizes, Device device) -> (Tensor, Tensor)");
+  m.def("upload_table(Tensor table, Device device) -> Tensor");
   m.def("attention_schedule(Tensor q_sizes, Tensor k_sizes, int q_tile, Device device) -> Tensor");
   m.def("attention_plan(Tensor q_lens, Tensor k_lens, int num_heads, int head_dim, Device device) -> Tensor");
   m.def("mha_self_packed(Tensor x, Tensor schedule, int num_heads, int head_dim, Tensor in_proj_weight, "
@@ -1499,6 +1540,8 @@ TORCH_LIBRARY_IMPL(nestedtensor, CUDA, m) {
 // element) for any device and raises for host tensors otherwise.
 TORCH_LIBRARY_IMPL(nestedtensor, CompositeExplicitAutograd, m) {
   m.impl("merge_tensor_mask", merge_tensor_mask);
+  m.impl("upload_sizes", upload_sizes);
+  m.impl("upload_table", upload_table);
   m.impl("attention_schedule", attention_schedule);
   m.impl("attention_plan", attention_plan);   // host lengths in, device plan out
   m.impl("nt_from_tensor_mask", nt_from_tensor_mask_op);

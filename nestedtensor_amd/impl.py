@@ -25,8 +25,7 @@ from . import _C
 
 class NestedTensorImpl:
     __slots__ = ("buffer", "sizes", "_opt_sizes", "_sizes_dev", "_offsets_dev",
-                 "_row_offsets_dev", "_max_sizes", "_attn_schedule", "_attn_plan", "_last_dim_rows", "_has_empty", "_transpose_meta",
-                 "channels_last")
+                 "_meta_stream", "_max_sizes", "_attn_schedule", "_attn_plan", "_has_empty", "_kept", "channels_last")
 
     def __init__(self, buffer, sizes, channels_last=False):
         """buffer: 1-D contiguous tensor; sizes: CPU int64 [B, D], or 0-d for an
@@ -45,13 +44,12 @@ class NestedTensorImpl:
         self._opt_sizes = None
         self._sizes_dev = None
         self._offsets_dev = None
-        self._row_offsets_dev = None
+        self._meta_stream = None
         self._max_sizes = None
         self._attn_schedule = None
         self._attn_plan = None
-        self._last_dim_rows = None
         self._has_empty = None
-        self._transpose_meta = None
+        self._kept = None
 
     # ---- host metadata ----------------------------------------------------
     @property
@@ -120,36 +118,61 @@ class NestedTensorImpl:
         return out
 
     # ---- device metadata ---------------------------------------------------
+    def _ready(self, table):
+        return table is not None and (self._meta_stream is None or
+                                      usable_on(self._meta_stream, current_stream_id(self.buffer.device)))
+
+    def _size_tables(self):
+        """(sizes, offsets) on the device, written by one launch (nt_upload_sizes) on first
+        use.  A conversion that has them in hand with its buffer sets them instead, with
+        _meta_stream None: they are ordered like the buffer itself."""
+        _C.require_device(self.buffer, "device metadata")
+        if self.sizes.dim() != 2:
+            return self.sizes.to(self.buffer.device), None
+        tables = _upload_sizes(self.sizes, self.buffer.device)
+        if not torch.cuda.is_current_stream_capturing():
+            self._sizes_dev, self._offsets_dev = tables
+            self._meta_stream = current_stream_id(self.buffer.device)
+        return tables
+
     def sizes_dev(self):
-        if self._sizes_dev is None:
-            _C.require_device(self.buffer, "device metadata")
-            self._sizes_dev = self.sizes.contiguous().to(self.buffer.device)
-        return self._sizes_dev
+        """int64 [B, D] mirror of the nested size."""
+        return self._sizes_dev if self._ready(self._sizes_dev) else self._size_tables()[0]
 
     def offsets_dev(self):
-        """int64 [B + 1] element offsets, built on the device by the prefix scan."""
-        if self._offsets_dev is None:
-            self._offsets_dev = device_offsets(self.sizes_dev(), self.B, self.D)
-        return self._offsets_dev
+        """int64 [B + 1] element offsets, scanned on the device."""
+        return self._offsets_dev if self._ready(self._offsets_dev) else self._size_tables()[1]
+
+    def kept(self, name, build):
+        """What build() returns, kept under `name` with this nested size for later calls on
+        the same device and stream.  For device metadata that kernels wrote: work on
+        another stream gets its own (see usable_on)."""
+        device = self.buffer.device
+        stream = current_stream_id(device)
+        if self._kept is None:
+            self._kept = {}
+        entry = self._kept.get(name)
+        if entry is None or entry[0] != device or not usable_on(entry[1], stream):
+            entry = (device, stream, build())
+            if not torch.cuda.is_current_stream_capturing():
+                self._kept[name] = entry
+        return entry[2]
 
     def row_offsets_dev(self):
         """int64 [B + 1] offsets counted in rows of the first constituent dim
         (token offsets for a [B, L_i, E] nested tensor)."""
-        if self._row_offsets_dev is None:
-            first = self.sizes_dev()[:, :1].contiguous()
-            self._row_offsets_dev = device_offsets(first, self.B, 1)
-        return self._row_offsets_dev
+        _C.require_device(self.buffer, "device metadata")
+        return self.kept("rows", lambda: _upload_sizes(self.sizes[:, :1], self.buffer.device)[1])
 
     def last_dim_rows(self):
         """(row_offsets, total_rows): int64 [B + 1] on the device, the number of
         rows along the last dim (product of all other constituent dims) of the
         constituents before b, and their total."""
-        if self._last_dim_rows is None:
+        def build():
             rows = self.sizes[:, :-1].prod(1)
-            row_offsets = torch.zeros(self.B + 1, dtype=torch.int64)
-            row_offsets[1:] = torch.cumsum(rows, 0)
-            self._last_dim_rows = (row_offsets.to(self.buffer.device), int(row_offsets[-1]))
-        return self._last_dim_rows
+            return _upload_sizes(rows.reshape(-1, 1), self.buffer.device)[1], int(rows.sum())
+        _C.require_device(self.buffer, "device metadata")
+        return self.kept("last_dim_rows", build)
 
     def attention_schedule(self, kv=None, q_tile=128):
         """Work list of the attention kernel (nt_attention_schedule), built from the
@@ -162,10 +185,12 @@ class NestedTensorImpl:
         if kv is None or kv.sizes is self.sizes:
             kv = self
         cached = self._attn_schedule
-        if cached is not None and cached[0] is kv.sizes:
+        stream = current_stream_id(self.buffer.device)
+        if cached is not None and cached[0] is kv.sizes and usable_on(cached[2], stream):
             return cached[1]
         sched = _attention_schedule(self.sizes, kv.sizes, q_tile, self.buffer.device)
-        self._attn_schedule = (kv.sizes, sched)      # holds kv.sizes, so the identity test stays valid
+        if not torch.cuda.is_current_stream_capturing():
+            self._attn_schedule = (kv.sizes, sched, stream)      # holds kv.sizes, so the identity test stays valid
         return sched
 
     def attention_plan(self, num_heads, head_dim, kv=None):
@@ -188,6 +213,7 @@ class NestedTensorImpl:
         that a conversion has already built for this nested size."""
         if sizes_dev.device == self.buffer.device and tuple(sizes_dev.shape) == tuple(self.sizes.shape):
             self._sizes_dev = sizes_dev
+            self._meta_stream = None
             if offsets_dev.numel() == self.B + 1:
                 self._offsets_dev = offsets_dev
 
@@ -203,15 +229,30 @@ class NestedTensorImpl:
         if buffer.device == self.buffer.device:
             out._sizes_dev = self._sizes_dev
             out._offsets_dev = self._offsets_dev
-            out._row_offsets_dev = self._row_offsets_dev
+            out._meta_stream = self._meta_stream
             out._attn_schedule = self._attn_schedule
             out._attn_plan = self._attn_plan
-            out._last_dim_rows = self._last_dim_rows
-            out._transpose_meta = self._transpose_meta
+            if self._kept is None:
+                self._kept = {}
+            out._kept = self._kept
         return out
 
 
+def current_stream_id(device):
+    """Identity of torch's current stream on `device` (0: the default stream)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def usable_on(made_on, stream):
+    """Whether metadata that a kernel wrote on stream `made_on` may be read by work on
+    `stream`.  On another stream nothing orders the reader behind the writer, and the
+    block could be handed out again while the reader still runs, so such a caller writes
+    its own copy (a launch).  A capture keeps what its eager warm-up has made."""
+    return made_on == stream or torch.cuda.is_current_stream_capturing()
+
+
 _attention_schedule = _C.ops.attention_schedule.default
+_upload_sizes = _C.ops.upload_sizes.default
 _offsets_from_sizes = _C.ops.offsets_from_sizes.default
 
 

@@ -21,6 +21,7 @@ from .impl import NestedTensorImpl
 # The schemas (same names and argument order as the reference) and the lowered
 # operators that do the work live in the C++ extension csrc/torch_ops.cpp
 # (TORCH_LIBRARY(nestedtensor, ...)), loaded by _C.  Overloads are resolved once.
+_upload_table = _C.ops.upload_table.default
 _add_padding = _C.ops.add_padding.default
 _add_padding_mask = _C.ops.add_padding_mask.default
 _remove_padding = _C.ops.remove_padding.default
@@ -695,22 +696,17 @@ def _conv1x1_row_major(impl, w2d):
         return None
     tn = int(_C.lib.nt_conv1x1_tile_pixels())
     B = impl.B
-    if impl._transpose_meta is None:
-        impl._transpose_meta = {}
-    key = ("conv1x1", tn)
-    cached = impl._transpose_meta.get(key)
-    if cached is not None and cached[0].device == buf.device:
-        meta_dev, total_tiles = cached
-    else:
+
+    def tables():
         pix = impl.sizes[:, 1] * impl.sizes[:, 2]
         meta = torch.zeros((2, B + 1), dtype=torch.int64)
         meta[0, 1:] = torch.cumsum(pix, 0)
         # a tile is one 128-byte line of every output row; the rows' lines start up to
         # tn - 1 pixels before a multiple of tn, hence one tile more than ceil(P / tn)
         meta[1, 1:] = torch.cumsum(torch.where(pix > 0, (pix + tn - 1) // tn + 1, pix), 0)
-        total_tiles = int(meta[1, B])
-        meta_dev = meta.to(buf.device)
-        impl._transpose_meta[key] = (meta_dev, total_tiles)
+        return _upload_table(meta, buf.device), int(meta[1, B])
+
+    meta_dev, total_tiles = impl.kept(("conv1x1", tn), tables)
     w2d = w2d.contiguous()
     sizes = impl.sizes.clone()
     sizes[:, 0] = c_out
@@ -980,12 +976,8 @@ def _transpose_constituents(impl, rows, cols, new_sizes, which):
     _C.require_device(buf, "transpose")
     B = impl.B
     which = (which, buf.element_size())       # the tile shape depends on the element size
-    if impl._transpose_meta is None:
-        impl._transpose_meta = {}
-    cached = impl._transpose_meta.get(which)
-    if cached is not None and cached[0].device == buf.device:
-        meta_dev, total_tiles, tr, tc = cached
-    else:
+
+    def tables():
         tr, tc = _transpose_tile(int(rows.max()) if B else 0, int(cols.max()) if B else 0, buf.element_size())
         if (tr, tc) == (64, 64) and buf.element_size() == 2 and bool((rows % 64 != 0).any()):
             # output rows that do not begin on 128-byte lines: the kernel that gives every
@@ -998,9 +990,9 @@ def _transpose_constituents(impl, rows, cols, new_sizes, which):
         meta = torch.zeros((3, B + 1), dtype=torch.int64)
         meta[0, :B], meta[1, :B] = rows, cols
         meta[2, 1:] = torch.cumsum(tiles, 0)
-        total_tiles = int(meta[2, B])
-        meta_dev = meta.to(buf.device)
-        impl._transpose_meta[which] = (meta_dev, total_tiles, tr, tc)
+        return _upload_table(meta, buf.device), int(meta[2, B]), tr, tc
+
+    meta_dev, total_tiles, tr, tc = impl.kept(which, tables)
     out = torch.empty_like(buf)
     if total_tiles:
         with _C.on_device(buf.device):
@@ -1015,7 +1007,8 @@ def _transpose_constituents(impl, rows, cols, new_sizes, which):
                     _C.ptr(meta_dev[1]), _C.ptr(meta_dev[2]), B, total_tiles, tr, tc, buf.element_size(),
                     _C.current_stream(buf.device)))
     res = NestedTensorImpl(out, new_sizes)
-    res._offsets_dev = impl._offsets_dev      # the constituents keep their extents
+    # the constituents keep their extents
+    res._offsets_dev, res._meta_stream = impl._offsets_dev, impl._meta_stream
     return res
 
 
@@ -1068,7 +1061,7 @@ def contiguous(impl, memory_format=torch.contiguous_format):
             return impl
         s = impl.sizes
         as_nhwc = NestedTensorImpl(impl.buffer, torch.stack([s[:, 1], s[:, 2], s[:, 0]], 1).contiguous())
-        as_nhwc._offsets_dev = impl._offsets_dev
+        as_nhwc._offsets_dev, as_nhwc._meta_stream = impl._offsets_dev, impl._meta_stream
         out = transpose_nhwc_nchw(as_nhwc)
         return impl.with_buffer(out.buffer, channels_last=False)
     if memory_format == torch.channels_last:

@@ -34,3 +34,17 @@ def test_schedule_rejects_token_indices_beyond_int32():
     sizes = torch.tensor([[1 << 30, 64], [1 << 30, 64]])
     with pytest.raises(RuntimeError, match="the work list holds token indices as int32"):
         _C.ops.attention_schedule.default(sizes, sizes, 1 << 20, DEV)
+
+
+def test_schedule_is_kept_per_stream():
+    # a work list that a kernel on one stream wrote is not handed to work on another
+    import nestedtensor_amd as nt
+    impl = nt.nested_tensor([torch.randn(n, 64) for n in (5, 130)], device=DEV, dtype=torch.float16)._impl
+    first = impl.attention_schedule()
+    assert impl.attention_schedule() is first
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        other = impl.attention_schedule()
+    torch.cuda.synchronize()
+    assert other.data_ptr() != first.data_ptr() and torch.equal(other, first)
