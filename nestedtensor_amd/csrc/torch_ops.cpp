@@ -126,6 +126,51 @@ Tensor offsets_from_sizes(const Tensor& sizes_dev) {
   return offsets;
 }
 
+// What the operators ask of a nested size, in one pass over the host's int64 [B, D] table:
+// per dim the extent every constituent has (-1: they differ), the largest and the smallest,
+// and the elements in all.  As small tensor operations each of these questions costs 5 to
+// 20 us, more than launching the kernel it is asked for.
+std::tuple<std::vector<int64_t>, std::vector<int64_t>, std::vector<int64_t>, int64_t> size_summary(const Tensor& sizes_in) {
+  TORCH_CHECK(sizes_in.device().is_cpu() && sizes_in.scalar_type() == at::kLong && sizes_in.dim() == 2 &&
+                  sizes_in.numel() > 0,
+              "size_summary: the nested size must be a non-empty host int64 [B, D] table");
+  const Tensor sizes = sizes_in.contiguous();
+  const int64_t B = sizes.size(0), D = sizes.size(1);
+  const int64_t* s = sizes.const_data_ptr<int64_t>();
+  std::vector<int64_t> regular(s, s + D), largest(s, s + D), smallest(s, s + D);
+  int64_t numel = 0;
+  for (int64_t b = 0; b < B; ++b) {
+    int64_t prod = 1;
+    for (int64_t k = 0; k < D; ++k) {
+      const int64_t v = s[b * D + k];
+      prod *= v;
+      if (v != s[k]) regular[k] = -1;
+      largest[k] = std::max(largest[k], v);
+      smallest[k] = std::min(smallest[k], v);
+    }
+    numel += prod;
+  }
+  return std::make_tuple(std::move(regular), std::move(largest), std::move(smallest), numel);
+}
+
+// The nested size of an operator's result: `sizes` with its last extent set to `last`, or
+// with `last` as one more extent.
+Tensor sizes_with_last(const Tensor& sizes_in, int64_t last, bool append) {
+  TORCH_CHECK(sizes_in.device().is_cpu() && sizes_in.scalar_type() == at::kLong && sizes_in.dim() == 2 &&
+                  (append || sizes_in.size(1) > 0),
+              "sizes_with_last: the nested size must be a host int64 [B, D] table");
+  const Tensor sizes = sizes_in.contiguous();
+  const int64_t B = sizes.size(0), D = sizes.size(1), E = D + (append ? 1 : 0);
+  Tensor out = at::empty({B, E}, at::kLong);
+  const int64_t* s = sizes.const_data_ptr<int64_t>();
+  int64_t* o = out.data_ptr<int64_t>();
+  for (int64_t b = 0; b < B; ++b) {
+    for (int64_t k = 0; k < D; ++k) o[b * E + k] = s[b * D + k];
+    o[b * E + E - 1] = last;
+  }
+  return out;
+}
+
 // (sizes[B, D], offsets[B + 1]) on `device` from the host's sizes, without a wait where
 // the table fits a few launches' arguments (nt_upload_sizes); a larger one, or one with
 // extents beyond int32, takes a copy and the device scan.
@@ -1498,6 +1543,8 @@ TORCH_LIBRARY(nestedtensor, m) {
   m.def("softmax_rows(Tensor x, Tensor offsets, Tensor row_offsets, int total_rows, bool log) -> Tensor");
   m.def("activation_packed(Tensor x, int act) -> Tensor");
   m.def("linear_packed(Tensor x, Tensor weight, Tensor? bias, int act) -> Tensor");
+  m.def("size_summary(Tensor sizes) -> (int[], int[], int[], int)");
+  m.def("sizes_with_last(Tensor sizes, int last, bool append) -> Tensor");
   m.def("upload_sizes(Tensor sizes, Device device) -> (Tensor, Tensor)");
   m.def("upload_table(Tensor table, Device device) -> Tensor");
   m.def("attention_schedule(Tensor q_sizes, Tensor k_sizes, int q_tile, Device device) -> Tensor");
@@ -1540,6 +1587,8 @@ TORCH_LIBRARY_IMPL(nestedtensor, CUDA, m) {
 // element) for any device and raises for host tensors otherwise.
 TORCH_LIBRARY_IMPL(nestedtensor, CompositeExplicitAutograd, m) {
   m.impl("merge_tensor_mask", merge_tensor_mask);
+  m.impl("size_summary", size_summary);
+  m.impl("sizes_with_last", sizes_with_last);
   m.impl("upload_sizes", upload_sizes);
   m.impl("upload_table", upload_table);
   m.impl("attention_schedule", attention_schedule);

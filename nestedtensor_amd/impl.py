@@ -25,7 +25,7 @@ from . import _C
 
 class NestedTensorImpl:
     __slots__ = ("buffer", "sizes", "_opt_sizes", "_sizes_dev", "_offsets_dev",
-                 "_meta_stream", "_max_sizes", "_attn_schedule", "_attn_plan", "_has_empty", "_kept", "channels_last")
+                 "_meta_stream", "_summary", "_attn_schedule", "_attn_plan", "_kept", "channels_last")
 
     def __init__(self, buffer, sizes, channels_last=False):
         """buffer: 1-D contiguous tensor; sizes: CPU int64 [B, D], or 0-d for an
@@ -45,10 +45,9 @@ class NestedTensorImpl:
         self._sizes_dev = None
         self._offsets_dev = None
         self._meta_stream = None
-        self._max_sizes = None
+        self._summary = None
         self._attn_schedule = None
         self._attn_plan = None
-        self._has_empty = None
         self._kept = None
 
     # ---- host metadata ----------------------------------------------------
@@ -67,37 +66,37 @@ class NestedTensorImpl:
     def nested_dim(self):
         return 1
 
+    def _summarize(self):
+        """(regular extents with -1 where they differ, largest, smallest, numel) of a nested
+        size with at least one extent, taken once (the nested size never changes)."""
+        if self._summary is None:
+            self._summary = _size_summary(self.sizes)
+        return self._summary
+
     def numel(self):
         # EfficientSizeNode::numel (EfficientSizeNode.h:113-131)
         if self.sizes.dim() == 0 or self.sizes.numel() == 0:
             return 0
-        return int(self.sizes.prod(1).sum())
+        return self._summarize()[3]
 
     def opt_sizes(self):
         # construct_efficient_size (EfficientSizeNode.h:27-49)
         if self._opt_sizes is None:
             res = [self.B]
-            if self.sizes.dim() > 0 and self.B > 0:
-                first = self.sizes[0]
-                same = (self.sizes == first).all(0)
-                for j in range(self.D):
-                    res.append(int(first[j]) if bool(same[j]) else None)
+            if self.B > 0 and self.D > 0:
+                res += [None if v < 0 else v for v in self._summarize()[0]]
             self._opt_sizes = res
         return list(self._opt_sizes)
 
     def max_sizes(self):
         # get_max_size_from_efficient_size (masking.cpp:83-103)
-        if self._max_sizes is None:
-            if self.B > 0 and self.D > 0:
-                self._max_sizes = [int(v) for v in self.sizes.max(0).values]
-            else:
-                self._max_sizes = []
-        return list(self._max_sizes)
+        return list(self._summarize()[1]) if self.B > 0 and self.D > 0 else []
+
+    def min_sizes(self):
+        return list(self._summarize()[2]) if self.B > 0 and self.D > 0 else []
 
     def has_empty_constituent(self):
-        if self._has_empty is None:
-            self._has_empty = self.B > 0 and self.D > 0 and bool((self.sizes == 0).any())
-        return self._has_empty
+        return self.B > 0 and self.D > 0 and min(self._summarize()[2]) == 0
 
     def shapes(self):
         return [tuple(int(v) for v in row) for row in self.sizes] if self.sizes.dim() > 0 else []
@@ -224,8 +223,7 @@ class NestedTensorImpl:
         out = NestedTensorImpl(buffer, self.sizes,
                                self.channels_last if channels_last is None else channels_last)
         out._opt_sizes = self._opt_sizes
-        out._max_sizes = self._max_sizes
-        out._has_empty = self._has_empty
+        out._summary = self._summary
         if buffer.device == self.buffer.device:
             out._sizes_dev = self._sizes_dev
             out._offsets_dev = self._offsets_dev
@@ -252,6 +250,7 @@ def usable_on(made_on, stream):
 
 
 _attention_schedule = _C.ops.attention_schedule.default
+_size_summary = _C.ops.size_summary.default
 _upload_sizes = _C.ops.upload_sizes.default
 _offsets_from_sizes = _C.ops.offsets_from_sizes.default
 

@@ -63,11 +63,12 @@ def nested_tensor_impl(data, dtype, device, requires_grad, pin_memory, channels_
         raise TypeError("nested_tensor(): argument 'data' must be a sequence of Tensors, not %s"
                         % type(data).__name__)
     tensors = list(data)
-    for t in tensors:
-        if isinstance(t, nested.NestedTensor):
-            raise RuntimeError("Currently do not support NestedTensor entries.")
-        if not torch.is_tensor(t):
-            raise RuntimeError("Currently only supporting a sequence of Tensors.")
+    if set(map(type, tensors)) != {torch.Tensor}:
+        for t in tensors:
+            if isinstance(t, nested.NestedTensor):
+                raise RuntimeError("Currently do not support NestedTensor entries.")
+            if not torch.is_tensor(t):
+                raise RuntimeError("Currently only supporting a sequence of Tensors.")
     device = torch.device(device)
     if len(tensors) == 0:
         # Packed.h:77-79: at::ones({0}); EfficientSizeNode.h:10-12: 0-d sizes

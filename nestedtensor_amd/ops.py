@@ -21,6 +21,7 @@ from .impl import NestedTensorImpl
 # The schemas (same names and argument order as the reference) and the lowered
 # operators that do the work live in the C++ extension csrc/torch_ops.cpp
 # (TORCH_LIBRARY(nestedtensor, ...)), loaded by _C.  Overloads are resolved once.
+_sizes_with_last = _C.ops.sizes_with_last.default
 _upload_table = _C.ops.upload_table.default
 _add_padding = _C.ops.add_padding.default
 _add_padding_mask = _C.ops.add_padding_mask.default
@@ -346,9 +347,7 @@ def linear_nt(impl, weight, bias=None, activation=None):
     if impl.dim() != 3 or opt[2] is None:
         raise NotImplementedError("linear on a NestedTensor needs dim 3 and a regular last dim.")
     out = linear(impl.buffer.reshape(-1, opt[2]), weight, bias, activation)
-    sizes = impl.sizes.clone()
-    sizes[:, 1] = weight.size(0)
-    return NestedTensorImpl(out.reshape(-1), sizes)
+    return NestedTensorImpl(out.reshape(-1), _sizes_with_last(impl.sizes, weight.size(0), False))
 
 
 def activation(impl, kind):
@@ -383,6 +382,10 @@ def _attention_work(query, key, num_heads, head_dim):
     return query.attention_schedule(kv=key)
 
 
+def _same_sizes(a, b):
+    return a.sizes is b.sizes or torch.equal(a.sizes, b.sizes)
+
+
 def _check_mha_inputs(query, key, value):
     if query.dim() != 3:
         raise RuntimeError("query needs to be 3 dim.")
@@ -409,7 +412,7 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
         raise RuntimeError("key and value must have the embedding dimension of query.")
     if key.B != query.B or value.B != query.B:
         raise RuntimeError("query, key and value must hold the same number of sequences.")
-    if not torch.equal(key.sizes, value.sizes):
+    if not _same_sizes(key, value):
         raise RuntimeError("key and value must have the same nested size.")
     _C.require_device(query.buffer, "multi-head attention")
     dtype = query.buffer.dtype
@@ -419,8 +422,7 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
     xq = query.buffer.reshape(-1, E)
     same = (key is query or key.buffer.data_ptr() == query.buffer.data_ptr()) and \
         (value is query or value.buffer.data_ptr() == query.buffer.data_ptr()) and \
-        torch.equal(key.sizes, query.sizes)
-    max_q = int(query.sizes[:, 0].max()) if query.B > 0 else 0
+        _same_sizes(key, query)
     mfma_path = head_dim in (32, 64, 128) and dtype in (torch.float16, torch.bfloat16)
     fused = same and mfma_path and (2 * E) % 128 == 0
     if in_proj_bias is not None:
@@ -437,7 +439,7 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
                                float(scaling), out_proj_weight, out_proj_bias)
         return query.with_buffer(out.reshape(-1))
     xk, xv = key.buffer.reshape(-1, E), value.buffer.reshape(-1, E)
-    if mfma_path and bool((key.sizes[:, 0] > 0).all()):
+    if mfma_path and (key.B == 0 or key.min_sizes()[0] > 0):
         # cross-attention (or an embedding size the fused projection does not tile),
         # head_dim 32 / 64 / 128: three projections (the value one written
         # transposed), then the same attention kernel with one key sequence per
@@ -452,7 +454,8 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
     sched = None
     if dtype == torch.float32 and head_dim in (32, 64, 128):
         sched = query.attention_schedule(kv=None if same else key)
-    out = _mha_rowmajor_packed(xq, xk, xv, same, sched, query.row_offsets_dev(), key.row_offsets_dev(), max_q,
+    out = _mha_rowmajor_packed(xq, xk, xv, same, sched, query.row_offsets_dev(), key.row_offsets_dev(),
+                               query.max_sizes()[0] if query.B > 0 else 0,
                                num_heads, head_dim, W, in_proj_bias, float(scaling), out_proj_weight,
                                out_proj_bias)
     return query.with_buffer(out.reshape(-1))
@@ -511,7 +514,7 @@ def layer_norm(impl, normalized_shape, weight=None, bias=None, eps=1e-5, residua
                                "on the input's device" % n)
     res_buf = None
     if residual is not None:
-        if not torch.equal(residual.sizes, impl.sizes) or residual.buffer.dtype != buf.dtype:
+        if not _same_sizes(residual, impl) or residual.buffer.dtype != buf.dtype:
             raise RuntimeError("layer_norm: the residual must have the nested size and dtype of the input")
         res_buf = residual.buffer
     if n == 0 or buf.numel() == 0:
@@ -528,7 +531,7 @@ def add(impl, other, alpha=1):
     buf = impl.buffer
     _C.require_device(buf, "add")
     if isinstance(other, NestedTensorImpl):
-        if other.sizes.shape != impl.sizes.shape or not torch.equal(other.sizes, impl.sizes):
+        if not _same_sizes(other, impl):
             raise NotImplementedError("add of nested tensors of different nested size is not on the packed path.")
         if not (impl.channels_last and other.channels_last):
             # two channels-last operands add buffer to buffer and stay channels-last
@@ -864,7 +867,7 @@ def embedding(weight, indices, padding_idx=None, max_norm=None, norm_type=2.0,
     if indices.sizes.dim() == 0:
         sizes = indices.sizes
     else:
-        sizes = torch.cat([indices.sizes, torch.full((indices.B, 1), E, dtype=torch.int64)], 1)
+        sizes = _sizes_with_last(indices.sizes, E, True)
     return NestedTensorImpl(out, sizes)
 
 
