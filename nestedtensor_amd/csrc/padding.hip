@@ -470,9 +470,8 @@ __global__ __launch_bounds__(256) void row_batch_kernel(RowParams p) {
 // of one index of the first) share their entry of the size table and their
 // offset, so a lane group that walks `rows_per_group` consecutive rows decodes
 // once (two divisions, one round trip to the tables) and then only adds strides;
-// the rows are moved two at a time.  With one row per workgroup the decode was
-// most of a workgroup's life: 4.4 TB/s on 16 fp32 images [3, H, W] against
-// 5.9 TB/s this way.
+// the rows are moved two at a time.  For masks of less than 1 MiB and what plane_kernel
+// cannot index.
 template <int EB, int MODE, int kT>
 __global__ __launch_bounds__(256) void row_group_kernel(RowParams p, int rows_per_group) {
   constexpr int kGroups = 256 / kT;
@@ -545,6 +544,139 @@ __global__ __launch_bounds__(256) void row_group_kernel(RowParams p, int rows_pe
       }
     }
     move_rows<EB, MODE, kT, 2>(r, on, p, tid);
+  }
+}
+
+// q = x / d and r = x % d by a multiplication: m = 0xffffffff / d, and the high word of x m
+// is q or q - 1 (x below 2^31, d at least 1).
+__device__ __forceinline__ void div_by(unsigned x, unsigned d, unsigned m, unsigned& q, unsigned& r) {
+  q = __umulhi(x, m);
+  r = x - q * d;
+  if (r >= d) {
+    ++q;
+    r -= d;
+  }
+}
+
+struct PlaneGeometry {
+  unsigned M0, M1, row;        // rows of a padded constituent as [M0][M1] (M0 = 1 for two ragged dims), elements of a row
+  unsigned m_M1, m_row;        // 0xffffffff / M1, 0xffffffff / row
+  unsigned inner;
+  int64_t B;
+};
+
+// Constituents with two or three ragged dims, pad and un-pad: grid.y walks the constituents
+// and the lanes take 16-byte chunks of the destination's constituent as it lies in memory,
+// whatever rows they cover.  What bounds the row-by-row kernels here is not HBM: a packed
+// row begins anywhere inside a 16-byte chunk, so every row has up to 32 bytes of element
+// stores at its ends and half-written lines, and every row costs a decode.  Flat, all
+// stores but the constituent's first and last are whole aligned chunks, the table is read
+// once per workgroup, and a chunk finds its row with two multiplications; only chunks that
+// meet the end of a row are put together element by element (their loads are independent).
+// U chunks per lane are loaded before the first is stored.
+// Pad / un-pad, us (TB/s): 16 fp32 images [3, 480..1024, 480..1024] 48.6 / 41.2 -> 42.2 / 36.2
+// (7.2 / 6.3), in fp16 45.9 / 36.7 -> 25.3 / 20.0, 16 fp64 [3, 301..1000, ..] 124 / 112 ->
+// 75.6 / 57.4, 6 fp32 [3, 900..2000, ..] 90.1 / 81.2 -> 53.7 / 46.1; 4 images of 20 to 40
+// pixels 5.8 / 11.6 -> 5.8 / 9.5, so there is no size below which rows are better.
+template <int EB, int MODE, int U>
+__global__ __launch_bounds__(256) void plane_kernel(RowParams p, PlaneGeometry g) {
+  typedef typename ElemT<EB>::type T;
+  constexpr unsigned kPer = 16 / EB;
+  const int64_t b = (int64_t)blockIdx.y + (int64_t)blockIdx.z * 65535;
+  if (b >= g.B) return;
+  const int64_t* sz = p.sizes + b * p.D;
+  const bool three = p.nrag > 2;
+  const unsigned s0 = three ? (unsigned)sz[0] : 1u;
+  const unsigned s1 = (unsigned)sz[three ? 1 : 0];
+  const unsigned len = (unsigned)sz[three ? 2 : 1] * g.inner;       // elements of a packed row
+  const T* src = reinterpret_cast<const T*>(p.src);
+  T* dst = reinterpret_cast<T*>(p.dst);
+  unsigned total, d_row, d_M1, m_row, m_M1;                          // of the destination
+  if (MODE == kPad) {
+    total = g.M0 * g.M1 * g.row;
+    d_row = g.row;
+    d_M1 = g.M1;
+    m_row = g.m_row;
+    m_M1 = g.m_M1;
+    dst += b * (int64_t)total;
+    src += p.offsets[b];
+  } else {
+    total = s0 * s1 * len;
+    if (total == 0) return;
+    d_row = len;
+    d_M1 = s1;
+    m_row = 0xffffffffu / len;
+    m_M1 = 0xffffffffu / s1;
+    src += b * ((int64_t)g.M0 * g.M1 * g.row);
+    dst += p.offsets[b];
+  }
+  // elements before the first and behind the last whole chunk
+  unsigned head = (unsigned)((0 - (uintptr_t)dst) & 15) / EB;
+  if (head > total) head = total;
+  const unsigned chunks = (total - head) / kPer;
+  T pad;
+  __builtin_memcpy(&pad, &p.pad, EB);
+
+  // the source element behind destination (i0, i1, col); false: padding
+  auto locate = [&](unsigned i0, unsigned i1, unsigned col, unsigned& at) {
+    if (MODE == kPad) {
+      at = (i0 * s1 + i1) * len + col;
+      return i0 < s0 && i1 < s1 && col < len;
+    }
+    at = (i0 * g.M1 + i1) * g.row + col;
+    return true;
+  };
+  auto element = [&](unsigned i0, unsigned i1, unsigned col) {
+    unsigned at;
+    return locate(i0, i1, col, at) ? src[at] : pad;
+  };
+  auto decode = [&](unsigned e, unsigned& i0, unsigned& i1, unsigned& col) {
+    unsigned row;
+    div_by(e, d_row, m_row, row, col);
+    div_by(row, d_M1, m_M1, i0, i1);
+  };
+
+  u32x4 v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const unsigned c = (blockIdx.x * U + u) * 256 + threadIdx.x;
+    if (c >= chunks) continue;
+    unsigned i0, i1, col, at;
+    decode(head + c * kPer, i0, i1, col);
+    const bool data = locate(i0, i1, col, at);
+    if (data && col + kPer <= len) {
+      v[u] = load16_unaligned(reinterpret_cast<const char*>(src + at));
+    } else if (MODE == kPad && !data && col + kPer <= g.row) {
+      v[u] = p.pad;
+    } else {
+      T e[kPer];
+#pragma unroll
+      for (unsigned k = 0; k < kPer; ++k) {
+        e[k] = element(i0, i1, col);
+        if (++col == d_row) {
+          col = 0;
+          if (++i1 == d_M1) {
+            i1 = 0;
+            ++i0;
+          }
+        }
+      }
+      __builtin_memcpy(&v[u], e, 16);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const unsigned c = (blockIdx.x * U + u) * 256 + threadIdx.x;
+    if (c < chunks) store16_stream(reinterpret_cast<char*>(dst + head + (size_t)c * kPer), v[u]);
+  }
+  if (blockIdx.x == 0) {
+    const unsigned tail = head + chunks * kPer, edges = head + (total - tail);
+    if (threadIdx.x < edges) {
+      const unsigned e = threadIdx.x < head ? threadIdx.x : tail + (threadIdx.x - head);
+      unsigned i0, i1, col;
+      decode(e, i0, i1, col);
+      dst[e] = element(i0, i1, col);
+    }
   }
 }
 
@@ -728,11 +860,52 @@ static int launch_batch(int eb, const RowParams& p, hipStream_t stream) {
   return check_launch("row_group_kernel");
 }
 
+// plane_kernel where its 32-bit indexes hold (a padded constituent of less than 2^31
+// elements; larger ones take the row kernels); *done says whether it ran.
+template <int MODE>
+static int try_planes(int eb, const RowParams& p, hipStream_t stream, bool* done) {
+  *done = false;
+  const int64_t M0 = p.nrag == 2 ? 1 : p.M0, M1 = p.nrag == 2 ? p.M0 : p.M1, Mlast = p.nrag == 2 ? p.M1 : p.M2;
+  constexpr int64_t kLimit = ((int64_t)1 << 31) - 16;
+  if (p.nrag < 2 || M0 < 1 || M1 < 1 || Mlast < 1 || p.inner < 1) return NT_OK;
+  if (M0 > kLimit || M1 > kLimit / M0 || Mlast > kLimit / (M0 * M1) || p.inner > kLimit / (M0 * M1 * Mlast)) return NT_OK;
+  if ((eb != 1 && eb != 2 && eb != 4 && eb != 8) ||
+      (reinterpret_cast<uintptr_t>(p.dst) | reinterpret_cast<uintptr_t>(p.src)) % eb != 0) {
+    return NT_OK;
+  }
+  constexpr int U = MODE == kPad ? 1 : 2;     // chunks per lane; the other way round and 4 are 5 to 15 % slower on images
+  const int64_t per_wg = 256 * U * (16 / eb), elems = M0 * M1 * Mlast * p.inner;
+  PlaneGeometry g;
+  g.M0 = (unsigned)M0;
+  g.M1 = (unsigned)M1;
+  g.row = (unsigned)(Mlast * p.inner);
+  g.m_M1 = 0xffffffffu / g.M1;
+  g.m_row = 0xffffffffu / g.row;
+  g.inner = (unsigned)p.inner;
+  g.B = p.nrows / (M0 * M1);
+  const dim3 grid((unsigned)((elems + per_wg - 1) / per_wg), (unsigned)(g.B < 65535 ? g.B : 65535),
+                  (unsigned)((g.B + 65534) / 65535));
+  if (grid.z > 65535) return NT_OK;
+  switch (eb) {
+    case 1: hipLaunchKernelGGL((plane_kernel<1, MODE, U>), grid, dim3(256), 0, stream, p, g); break;
+    case 2: hipLaunchKernelGGL((plane_kernel<2, MODE, U>), grid, dim3(256), 0, stream, p, g); break;
+    case 4: hipLaunchKernelGGL((plane_kernel<4, MODE, U>), grid, dim3(256), 0, stream, p, g); break;
+    default: hipLaunchKernelGGL((plane_kernel<8, MODE, U>), grid, dim3(256), 0, stream, p, g); break;
+  }
+  *done = true;
+  return check_launch("plane_kernel");
+}
+
 template <int MODE>
 static int launch_rows(int eb, const RowParams& p, int64_t max_row_bytes, hipStream_t stream) {
   if (p.nrows == 0 || max_row_bytes == 0) return NT_OK;
   if (p.nrows > 0x7fffffffLL) {
     return fail(NT_ERR_UNSUPPORTED, "row count %lld exceeds the grid limit", (long long)p.nrows);
+  }
+  if constexpr (MODE == kPad || MODE == kUnpad) {
+    bool done = false;
+    const int rc = try_planes<MODE>(eb, p, stream, &done);
+    if (rc != NT_OK || done) return rc;
   }
   if (MODE != kPack && p.nrows >= 4096) {
     // many short rows: several rows per lane group, all of their chunks in flight

@@ -1,0 +1,55 @@
+"""Pad and un-pad of constituents with two and three ragged dims by flat 16-byte chunks, bit for
+bit against slicing: rows shorter than a chunk, rows of one element, chunks over several rows,
+constituents that begin anywhere inside a chunk, empty ones, and guards behind both buffers."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+SHAPES = {
+    "images": [(3, 17, 33), (3, 40, 5), (3, 1, 64), (3, 64, 1)],
+    "three": [(1, 1, 1), (2, 5, 3), (4, 1, 7), (3, 9, 2)],
+    "empty": [(2, 3, 5), (0, 4, 6), (3, 0, 9), (1, 7, 0)],
+    "inner": [(5, 9, 3), (11, 2, 3), (1, 31, 3)],          # two ragged dims, a regular last one
+    "flat": [(7, 300), (50, 1), (3, 65)],                  # two ragged dims
+    "wide": [(2, 3000), (5, 1111)],
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.float16, torch.float32, torch.float64])
+@pytest.mark.parametrize("name", sorted(SHAPES))
+@pytest.mark.parametrize("wider", [0, 3])
+def test_planes(name, dtype, wider):
+    from nestedtensor_amd import _C
+    eb = torch.empty(0, dtype=dtype).element_size()
+    shapes = SHAPES[name]
+    D = len(shapes[0])
+    nrag = 2 if name == "inner" or D == 2 else 3
+    ext = [max(s[k] for s in shapes) + (wider if k < nrag else 0) for k in range(D)]
+    parts = [(torch.rand(s) * 200 + 1).to(dtype) for s in shapes]
+    sizes = torch.tensor(shapes)
+    sizes_dev, offsets = _C.ops.upload_sizes.default(sizes, DEV)
+    total = int(offsets[-1])
+    flat = torch.cat([t.reshape(-1) for t in parts])
+    # both buffers at the start of an allocation and one element into it, a guard behind them
+    for shift in (0, 1):
+        packed = torch.full((total + shift + 40,), 99, dtype=dtype, device=DEV)
+        packed[shift:shift + total] = flat.to(DEV)
+        expect = torch.full([len(shapes)] + ext, 7, dtype=dtype)
+        for b, t in enumerate(parts):
+            expect[(b,) + tuple(slice(0, n) for n in t.shape)] = t
+        n = expect.numel()
+        padded = torch.full((n + shift + 40,), 99, dtype=dtype, device=DEV)
+        seven = torch.tensor([7], dtype=dtype).view(torch.uint8)
+        bits = int.from_bytes(bytes(seven.tolist()), "little")
+        stream = _C.current_stream(DEV)
+        _C.check(_C.lib.nt_add_padding(_C.ptr(packed[shift:]), _C.ptr(padded[shift:]), _C.ptr(offsets), _C.ptr(sizes_dev),
+                                       len(shapes), D, nrag, _C.i64_array(ext), eb, bits, stream))
+        assert torch.equal(padded[shift:shift + n].cpu(), expect.reshape(-1))
+        assert bool((padded[:shift] == 99).all()) and bool((padded[shift + n:] == 99).all())
+        back = torch.full((total + shift + 40,), 99, dtype=dtype, device=DEV)
+        _C.check(_C.lib.nt_remove_padding(_C.ptr(padded[shift:]), _C.ptr(back[shift:]), _C.ptr(offsets), _C.ptr(sizes_dev),
+                                          len(shapes), D, nrag, _C.i64_array(ext), eb, stream))
+        assert torch.equal(back[shift:shift + total].cpu(), flat)
+        assert bool((back[:shift] == 99).all()) and bool((back[shift + total:] == 99).all())
