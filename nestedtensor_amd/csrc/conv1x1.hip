@@ -35,6 +35,14 @@
 // of the wavefront then writes eight whole lines; only a row's first and last
 // line are partial.
 //
+// (3) With two wavefronts per SIMD the instructions of a tile count.  Nearly all tiles lie
+// inside their image with their whole window, and those load and store without a look at
+// the bounds; an output row's position moves on by one addition, and the half-dword
+// shift of a window is the variable count of v_alignbit.  Stores go past the L2, which
+// a result of this size does not fit.  64 -> 256 channels on 589 481 pixels (377 MB)
+// 131.5 -> 100.4 us, 32 -> 128 on 1.35 M (431 MB) 119.5 -> 86 us, a copy of the same bytes
+// taking 71 and 80 us; the stores alone are a third of it.
+//
 // Persistent workgroups (the weight is loaded into LDS once each) of WAVES
 // wavefronts, and every wavefront works on tiles of its own with its own X tile
 // and strip: no workgroup barrier after the weight is in place, the next tile's
@@ -42,6 +50,7 @@
 // stored, and the wavefronts of a compute unit drift apart so that their loads,
 // products and stores overlap.
 #include "attn_common.h"
+#include <type_traits>
 
 namespace nt {
 
@@ -109,23 +118,36 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
     }
     k64 = (id - t_lo) * kConvTile;
   };
+  // all 128 pixels of the tile's window lie inside the image
+  auto interior = [&](int64_t k, int64_t pixels) { return k >= kConvTile && k + kConvTile <= pixels; };
   auto fetch = [&]() {
     const int64_t first = k64 - kConvTile + chunk * 8;      // first pixel of this piece, may lie outside [0, P)
-    const T* xb = x + pix0 * c_in + first;
+    const char* p = reinterpret_cast<const char*>(x + pix0 * c_in + first + row0 * P);
+    const int64_t step = 8 * P;                             // bytes from one row of four to the next
+    if (interior(k64, P)) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        if (4 * i < c_in) stage[i] = load16_unaligned(p);
+        p += step;
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const T* p = xb + (int64_t)(row0 + 4 * i) * P;
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (row0 + 4 * i >= c_in) {
+      if (4 * i >= c_in) {
       } else if (first >= 0 && first + 8 <= P) {
-        v = load16_unaligned(reinterpret_cast<const char*>(p));
+        v = load16_unaligned(p);
       } else if (first + 8 > 0 && first < P) {
         T e[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) e[j] = (first + j >= 0 && first + j < P) ? p[j] : (T)0.0f;
+        for (int j = 0; j < 8; ++j) {
+          e[j] = (first + j >= 0 && first + j < P) ? reinterpret_cast<const T*>(p)[j] : (T)0.0f;
+        }
         __builtin_memcpy(&v, e, 16);
       }
       stage[i] = v;
+      p += step;
     }
   };
   if (tile < total_tiles) {
@@ -140,7 +162,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
     // registers -> this wavefront's X tile
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      if (row0 + 4 * i < c_in) {
+      if (4 * i < c_in) {
         uint32_t* d = Xl + (row0 + 4 * i) * S + chunk * 4;
         d[0] = stage[i].x;
         d[1] = stage[i].y;
@@ -176,6 +198,11 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
     }
     __builtin_amdgcn_wave_barrier();                          // the X tile is dead from here on
     const int64_t y_img = cur_pix0 * c_out;                  // first element of the image in y
+    const bool whole = interior(cur_k64, cur_P);
+    // first element of the output row a lane is at: r0, then every eighth row
+    const int r0 = l >> 3, j8 = 8 * (l & 7);
+    int64_t row_start = y_img + r0 * cur_P;
+    T* const y_tile = y + cur_k64 + j8;
     for (int ob = 0; ob < nob; ++ob) {
       acc16 acc[kPB];
 #pragma unroll
@@ -205,39 +232,40 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
         }
       __builtin_amdgcn_wave_barrier();
       // every row takes the 64 pixels of its own line k out of the strip
+auto rows = [&](auto whole_c) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole_c)::value;
 #pragma unroll
-      for (int ps = 0; ps < 4; ++ps) {
-        const int r = ps * 8 + (l >> 3), j = l & 7;
-        const int64_t row_start = y_img + (int64_t)(ob * 32 + r) * cur_P;     // element index in y
-        const int ph = (int)(row_start & 63);
-        const int col = kConvTile - ph + 8 * j;                              // first strip element of the piece
-        const uint32_t* src = strip + r * SSD + (col >> 1);
-        uint32_t d[5];
+        for (int ps = 0; ps < 4; ++ps) {
+          const int ph = (int)row_start & 63;
+          const int col = kConvTile - ph + j8;                                 // first strip element of the piece
+          const uint32_t* src = strip + (r0 + 8 * ps) * SSD + (col >> 1);
+          uint32_t d[5];
 #pragma unroll
-        for (int i = 0; i < 5; ++i) d[i] = src[i];
-        u32x4 v;
-        if (col & 1) {
-          v.x = __builtin_amdgcn_alignbit(d[1], d[0], 16);
-          v.y = __builtin_amdgcn_alignbit(d[2], d[1], 16);
-          v.z = __builtin_amdgcn_alignbit(d[3], d[2], 16);
-          v.w = __builtin_amdgcn_alignbit(d[4], d[3], 16);
-        } else {
-          v.x = d[0];
-          v.y = d[1];
-          v.z = d[2];
-          v.w = d[3];
+          for (int i = 0; i < 5; ++i) d[i] = src[i];
+          const uint32_t odd = (uint32_t)(col & 1) * 16;
+          u32x4 v;
+          v.x = __builtin_amdgcn_alignbit(d[1], d[0], odd);
+          v.y = __builtin_amdgcn_alignbit(d[2], d[1], odd);
+          v.z = __builtin_amdgcn_alignbit(d[3], d[2], odd);
+          v.w = __builtin_amdgcn_alignbit(d[4], d[3], odd);
+          T* qd = y_tile + (row_start - ph);                                 // 16-byte aligned by construction
+          const int64_t pixel = cur_k64 - ph + j8;                             // first pixel of the piece
+          if (WHOLE || (pixel >= 0 && pixel + 8 <= cur_P)) {
+            store16_stream(reinterpret_cast<char*>(qd), v);
+          } else if (pixel + 8 > 0 && pixel < cur_P) {
+            T e[8];
+            __builtin_memcpy(e, &v, 16);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              if (pixel + i >= 0 && pixel + i < cur_P) qd[i] = e[i];
+          }
+          row_start += 8 * cur_P;
         }
-        const int64_t pixel = cur_k64 - ph + 8 * j;                          // first pixel of the piece
-        T* qd = y + row_start + pixel;
-        if (pixel >= 0 && pixel + 8 <= cur_P) {
-          *reinterpret_cast<u32x4*>(qd) = v;                                 // 16-byte aligned by construction
-        } else if (pixel + 8 > 0 && pixel < cur_P) {
-          T e[8];
-          __builtin_memcpy(e, &v, 16);
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (pixel + i >= 0 && pixel + i < cur_P) qd[i] = e[i];
-        }
+      };
+      if (whole) {
+        rows(std::true_type());
+      } else {
+        rows(std::false_type());
       }
       __builtin_amdgcn_wave_barrier();
     }
