@@ -975,6 +975,14 @@ static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
       if (!small && n_split % CfgMid::kBN == 0) return launch_cfg<T, CfgMid, EPI>(a, stream);
     }
   }
+  // At most 64 columns: such a product reads A once and is bound by that, half of a
+  // 128-column tile would be padding, and three workgroups of this tile share a CU where the
+  // larger ones have it to themselves while they fill and drain (589481 x 64 x 256
+  // 95.8 -> 77.5 us = 4.9 TB/s, 300000 x 32 x 64 33.2 -> 22.6, 100000 x 32 x 256 18.1 -> 13.4;
+  // with 128 columns it loses: 300000 x 128 x 128 32.4 -> 49.2).
+  if constexpr (sizeof(T) == 2) {
+    if (a.N <= CfgSmall::kBN && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
+  }
   // The pipelined tile needs whole K tiles, at least two of them, and 32-bit offsets
   // inside a tile.  (fp32: row-major results only, the transposed strips
   // would not fit its LDS.)

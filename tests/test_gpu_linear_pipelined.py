@@ -74,3 +74,11 @@ def test_linear_qkv_pipelined_shapes(M, E, dtype):
     assert bool(((qk.double() - ref[:, :2 * E]).abs() <= bound[:, :2 * E]).all())
     assert bool(((vt[:, :M].double() - ref[:, 2 * E:].t()).abs() <= bound[:, 2 * E:].t()).all())
     assert bool((vt[:, M:] == 7.0).all())          # nothing is written past the last token
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(40001, 64, 128), (40001, 65, 128), (33000, 33, 64), (70003, 8, 72), (16385, 64, 8)])
+def test_linear_few_columns(M, N, K, dtype):
+    from nestedtensor_amd import ops
+    x, w, b, ref, bound = _case(M, N, K, dtype)
+    assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
