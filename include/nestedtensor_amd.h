@@ -441,6 +441,13 @@ int nt_mul_packed(const void* a, const void* b, double scale, void* out, int64_t
 int nt_gather_rows(const void* src, int64_t src_rows, int64_t row_bytes, const int64_t* index,
                    void* dst, int64_t n_rows, int32_t* oob_count, void* stream);
 
+/* Number of the n indices (1 <= n <= nt_count_outside_max()) outside [0, rows), rows at
+ * least 1, stored to *word (device-visible host memory, 8-byte aligned) as
+ * count | (uint64_t)stamp << 32 in one store: a host that polls the word for its stamp
+ * has the count. */
+int64_t nt_count_outside_max(void);
+int nt_count_outside(const int64_t* index, int64_t n, int64_t rows, uint64_t* word, uint32_t stamp, void* stream);
+
 /* Row order of torch.nn.utils.rnn.PackedSequence for the sequences of a nested
  * tensor [B, L_i, *]: index_out[step_starts[t] + rank[b]] = offsets[b] + t for
  * every token t of every sequence b.  offsets int64[B + 1] are token offsets,

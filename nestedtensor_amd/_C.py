@@ -88,6 +88,8 @@ SIGNATURES = {
     "nt_activation_packed": (_int, [_c_void_p, _c_void_p, _i64, _int, _int, _c_void_p]),
     "nt_mul_packed": (_int, [_c_void_p, _c_void_p, _f64, _c_void_p, _i64, _i64, _int, _c_void_p]),
     "nt_gather_rows": (_int, [_c_void_p, _i64, _i64, _c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p]),
+    "nt_count_outside_max": (_i64, []),
+    "nt_count_outside": (_int, [_c_void_p, _i64, _i64, _c_void_p, ctypes.c_uint32, _c_void_p]),
     "nt_packed_sequence_index": (_int, [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _c_void_p, _c_void_p]),
     "nt_ragged_arange": (_int, [_c_void_p, _i64, _i64, _c_void_p, _c_void_p]),
     "nt_transpose_ragged": (_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64,

@@ -44,6 +44,36 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(
   }
 }
 
+// How many of up to kCountMax indices lie outside [0, rows), for a host that waits for the
+// answer: one workgroup, and the count leaves with the caller's stamp in one 8-byte
+// store to host memory, which needs no copy and no completion word behind it.
+constexpr int64_t kCountMax = 32768;
+constexpr int kCountThreads = 1024, kCountBatch = 8;
+__global__ __launch_bounds__(kCountThreads) void count_outside_kernel(const int64_t* __restrict__ index, int n,
+                                                                      int64_t rows, uint64_t* word, uint32_t stamp) {
+  __shared__ int s_wave[kCountThreads / kWave];
+  int count = 0;
+  for (int base = 0; base < n; base += kCountThreads * kCountBatch) {
+    int64_t v[kCountBatch];
+#pragma unroll
+    for (int k = 0; k < kCountBatch; ++k) {
+      const int i = base + k * kCountThreads + (int)threadIdx.x;
+      v[k] = i < n ? index[i] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kCountBatch; ++k) count += (uint64_t)v[k] >= (uint64_t)rows ? 1 : 0;
+  }
+  count = wave_reduce_sum(count);
+  if ((threadIdx.x & (kWave - 1)) == 0) s_wave[threadIdx.x / kWave] = count;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int total = 0;
+    for (int w = 0; w < kCountThreads / kWave; ++w) total += s_wave[w];
+    __hip_atomic_store(word, (uint64_t)(uint32_t)total | ((uint64_t)stamp << 32), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // Time-major order of a PackedSequence: token t of the sequence at sorted
 // position r goes to row step_starts[t] + r.  index_out[that row] = source row.
 __global__ __launch_bounds__(256) void packed_sequence_index_kernel(
@@ -246,6 +276,20 @@ extern "C" int nt_gather_rows(const void* src, int64_t src_rows, int64_t row_byt
     default: launch_gather<1>(src, src_rows, row_bytes, index, dst, n_rows, oob_count, s); break;
   }
   return check_launch("gather_rows_kernel");
+}
+
+extern "C" int64_t nt_count_outside_max(void) { return kCountMax; }
+
+extern "C" int nt_count_outside(const int64_t* index, int64_t n, int64_t rows, uint64_t* word, uint32_t stamp,
+                                void* stream) {
+  // rows of at least 1: the padding of the last batch of indices counts as index 0
+  if (n < 1 || rows < 1 || !index || !word) return fail(NT_ERR_INVALID_ARGUMENT, "count_outside: bad arguments");
+  if (n > kCountMax) {
+    return fail(NT_ERR_UNSUPPORTED, "count_outside: %lld indices, at most %lld", (long long)n, (long long)kCountMax);
+  }
+  hipLaunchKernelGGL(count_outside_kernel, dim3(1), dim3(kCountThreads), 0, (hipStream_t)stream, index, (int)n, rows,
+                     word, stamp);
+  return check_launch("count_outside_kernel");
 }
 
 extern "C" int nt_packed_sequence_index(const int64_t* offsets, const int64_t* rank,

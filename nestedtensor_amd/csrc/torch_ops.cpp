@@ -1252,6 +1252,50 @@ Tensor embedding_packed(const Tensor& weight_in, const Tensor& indices, const c1
   return out;
 }
 
+// embedding_packed for a caller that must know before it returns whether an index was out
+// of range: (result, their number, or -1 where `mirror` holds the counter as this call has
+// left it).  The count of a batch of ordinary size is a launch
+// of its own in front of the gather, so the host has it while the rows are still being
+// gathered; behind the gather it came with a copy and a wait for the whole stream, and the
+// launches that follow began that much later (an encoder layer from 8040 token ids
+// 305 -> 268 us).
+std::tuple<Tensor, int64_t> embedding_checked(const Tensor& weight_in, const Tensor& indices, const Tensor& counter,
+                                              const Tensor& mirror) {
+  require_device(indices, "embedding");
+  const int64_t T = indices.numel();
+  static const int64_t kCountMax = nt_count_outside_max();
+  const bool early = T > 0 && T <= kCountMax && weight_in.dim() == 2 && weight_in.numel() > 0 &&
+                     indices.scalar_type() == at::kLong && weight_in.device() == indices.device();
+  if (!early) {
+    Tensor out = embedding_packed(weight_in, indices, counter, mirror);
+    C10_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream_of(indices))));
+    return std::make_tuple(out, static_cast<int64_t>(-1));
+  }
+  static thread_local Tensor word_t;
+  static thread_local uint32_t stamp = 0;
+  if (!word_t.defined()) word_t = at::zeros({8}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  if (++stamp == 0) ++stamp;
+  uint64_t* word = reinterpret_cast<uint64_t*>(word_t.data_ptr());
+  const Tensor idx = indices.contiguous();
+  c10::hip::HIPGuard guard(indices.device().index());
+  void* stream = stream_of(indices);
+  check(nt_count_outside(idx.const_data_ptr<int64_t>(), T, weight_in.size(0), word, stamp, stream));
+  Tensor out = embedding_packed(weight_in, idx, c10::nullopt, c10::nullopt);
+  const auto t0 = std::chrono::steady_clock::now();
+  uint64_t seen;
+  for (int spin = 0; static_cast<uint32_t>((seen = __atomic_load_n(word, __ATOMIC_ACQUIRE)) >> 32) != stamp; ++spin) {
+    __builtin_ia32_pause();
+    if ((spin & 255) == 255 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(500)) {
+      // the stream has much to do before this call: hand the wait to the runtime
+      C10_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+      seen = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+      TORCH_CHECK(static_cast<uint32_t>(seen >> 32) == stamp, "embedding: the device did not deliver the index check");
+      break;
+    }
+  }
+  return std::make_tuple(out, static_cast<int64_t>(static_cast<uint32_t>(seen)));
+}
+
 // _nn_functional_embedding_bag (nested/nested.py:43-118): the bags are the
 // constituents, `offsets` the nested tensor's device offsets.  mode: 0 sum, 1 mean, 2 max.
 Tensor embedding_bag_packed(const Tensor& weight_in, const Tensor& indices, const Tensor& offsets, int64_t mode,
@@ -1533,6 +1577,7 @@ TORCH_LIBRARY(nestedtensor, m) {
   m.def("build_mask(Tensor sizes, int[] extents) -> Tensor");
   m.def("from_tensor_mask_lowered(Tensor tensor, Tensor mask, int nested_dim) -> (Tensor, Tensor, Tensor, Tensor)");
   m.def("from_padded_value_lowered(Tensor tensor, float padding, int nested_dim) -> (Tensor, Tensor, Tensor, Tensor)");
+  m.def("embedding_checked(Tensor weight, Tensor indices, Tensor counter, Tensor mirror) -> (Tensor, int)");
   m.def("embedding_packed(Tensor weight, Tensor indices, Tensor? counter, Tensor? mirror) -> Tensor");
   m.def("embedding_bag_packed(Tensor weight, Tensor indices, Tensor offsets, int mode, Tensor? counter, "
         "Tensor? mirror) -> Tensor");
@@ -1577,6 +1622,7 @@ TORCH_LIBRARY_IMPL(nestedtensor, CUDA, m) {
   m.impl("binary_packed", binary_packed);
   m.impl("softmax_rows", softmax_rows);
   m.impl("activation_packed", activation_packed);
+  m.impl("embedding_checked", embedding_checked);
   m.impl("embedding_packed", embedding_packed);
   m.impl("embedding_bag_packed", embedding_bag_packed);
   m.impl("packed_sequence_lowered", packed_sequence_lowered);

@@ -35,6 +35,7 @@ _layer_norm_packed = _C.ops.layer_norm_packed.default
 _binary_packed = _C.ops.binary_packed.default
 _softmax_rows = _C.ops.softmax_rows.default
 _activation_packed = _C.ops.activation_packed.default
+_embedding_checked = _C.ops.embedding_checked.default
 _embedding_packed = _C.ops.embedding_packed.default
 _embedding_bag_packed = _C.ops.embedding_bag_packed.default
 _packed_sequence_lowered = _C.ops.packed_sequence_lowered.default
@@ -860,9 +861,14 @@ def embedding(weight, indices, padding_idx=None, max_norm=None, norm_type=2.0,
     slot = _oob_begin(weight.device, "embedding")
     if slot is None:
         out = _embedding_packed(weight, idx, None, None)
+    elif _index_check_mode == "immediate" and not torch.cuda.is_current_stream_capturing():
+        out, outside = _embedding_checked(weight, idx, slot[0], slot[1])
+        if outside < 0:
+            _report_index_errors(slot, "embedding")
+        elif outside:
+            raise IndexError("embedding: %d index value(s) out of range" % outside)
     else:
         out = _embedding_packed(weight, idx, slot[0], slot[1])
-        _oob_end(slot, "embedding")
     out = out.reshape(-1)
     if indices.sizes.dim() == 0:
         sizes = indices.sizes

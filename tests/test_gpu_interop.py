@@ -359,3 +359,17 @@ def test_transpose_ragged_strips(dtype, narrow):
         assert torch.equal(fwd._impl.buffer.cpu(), exp.buffer)
         back = nt.transpose_nhwc_nchw(fwd)
         assert torch.equal(back._impl.buffer, a._impl.buffer)
+
+
+@pytest.mark.parametrize("n", [1, 1023, 8192, 8193, 32768, 32769])
+def test_embedding_counts_out_of_range_indices_before_it_returns(n):
+    # up to 32768 indices by a launch of its own, in batches of 8192; more behind the gather
+    w = torch.randn(50, 8, device=DEV)
+    ids = torch.randint(0, 50, (n,), generator=torch.Generator().manual_seed(n))
+    good = torch.nn.functional.embedding(nt.nested_tensor([ids.to(DEV)], dtype=torch.int64, device=DEV), w)
+    assert torch.equal(good.unbind()[0], w[ids.to(DEV)])
+    bad = ids.clone()
+    bad[0], bad[n // 2], bad[-1] = -1, 1 << 40, 50
+    with pytest.raises(IndexError, match="%d index value" % len({0, n // 2, n - 1})):
+        torch.nn.functional.embedding(nt.nested_tensor([bad.to(DEV)], dtype=torch.int64, device=DEV), w)
+    torch.nn.functional.embedding(nt.nested_tensor([ids.to(DEV)], dtype=torch.int64, device=DEV), w)
