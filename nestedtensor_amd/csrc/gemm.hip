@@ -123,14 +123,6 @@ struct GemmArgs {
   int act;          // row-major tiles: 0 none, 1 relu, 2 gelu (erf) applied to A W^T + bias
 };
 
-// The activation of a feed-forward layer, applied in fp32 before the one rounding
-// of the epilogue (wavefront-uniform switch; `act` is a kernel argument).
-__device__ __forceinline__ float apply_act(float v, int act) {
-  if (act == 1) return fmaxf(v, 0.0f);
-  if (act == 2) return gelu_erf(v);
-  return v;
-}
-
 // 16-byte piece of a row at element k.
 // ALIGNED_K (K is a multiple of the K tile): branch-free and mask-free.
 // Out-of-range rows are clamped to the last row -- they only feed accumulators
@@ -206,23 +198,28 @@ __device__ __forceinline__ void store_tile(const GemmArgs<T>& a, const acc16 (&a
     for (int i = 0; i < WM; ++i) {
 #pragma unroll
       for (int j = 0; j < WN; ++j) {
+        auto block = [&](auto act) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int c0 = j * 32 + 8 * r + 4 * g;
-          const float4 bv = *reinterpret_cast<const float4*>(lds_bias + n_wave + c0);
-          Quad q;
-          if (!ACT) {
-            q[0] = (T)(acc[i][j][4 * r + 0] + bv.x);
-            q[1] = (T)(acc[i][j][4 * r + 1] + bv.y);
-            q[2] = (T)(acc[i][j][4 * r + 2] + bv.z);
-            q[3] = (T)(acc[i][j][4 * r + 3] + bv.w);
-          } else {
-            q[0] = (T)apply_act(acc[i][j][4 * r + 0] + bv.x, a.act);
-            q[1] = (T)apply_act(acc[i][j][4 * r + 1] + bv.y, a.act);
-            q[2] = (T)apply_act(acc[i][j][4 * r + 2] + bv.z, a.act);
-            q[3] = (T)apply_act(acc[i][j][4 * r + 3] + bv.w, a.act);
+          for (int r = 0; r < 4; ++r) {
+            const int c0 = j * 32 + 8 * r + 4 * g;
+            const float4 bv = *reinterpret_cast<const float4*>(lds_bias + n_wave + c0);
+            Quad q;
+            q[0] = (T)act(acc[i][j][4 * r + 0] + bv.x);
+            q[1] = (T)act(acc[i][j][4 * r + 1] + bv.y);
+            q[2] = (T)act(acc[i][j][4 * r + 2] + bv.z);
+            q[3] = (T)act(acc[i][j][4 * r + 3] + bv.w);
+            *reinterpret_cast<Quad*>(strip + l32 * kStripRow + c0 * (int)sizeof(T)) = q;
           }
-          *reinterpret_cast<Quad*>(strip + l32 * kStripRow + c0 * (int)sizeof(T)) = q;
+        };
+        // The activation of a feed-forward layer, in fp32 before the one rounding.  The
+        // choice (a kernel argument) is made once per 32 x 32 block: made per element it
+        // kept the sixteen chains of a lane apart, and nothing else runs beside them.
+        if (ACT && a.act == 2) {
+          block([](float v) { return gelu_erf(v); });
+        } else if (ACT && a.act == 1) {
+          block([](float v) { return fmaxf(v, 0.0f); });
+        } else {
+          block([](float v) { return v; });
         }
       }
       __builtin_amdgcn_wave_barrier();   // LDS serves a wavefront's accesses in order

@@ -48,21 +48,27 @@ __device__ __forceinline__ void store16_stream(char* p, u32x4 v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
-// gelu(x) = x/2 (1 + erf(x / sqrt 2)) with erf from Abramowitz & Stegun 7.1.26
-// (absolute error below 1.5e-7, i.e. below fp32 rounding of the result for |x| of
-// order 1): one reciprocal, one 2^x and nine multiply-adds instead of the ~40
-// instructions of erff, which made a fused epilogue slower than a second pass.
+// gelu(x) = x Phi(x), Phi the normal distribution function, from its tail: Phi(-|x|) is
+// 2^Q(|x|) with Q a polynomial of degree 8 fitted to log2 Phi(-u) on [0, 5] (least
+// squares reweighted towards the smallest largest error of Phi).  Q falls without end past 5, so the tail
+// goes to 0 by itself.  In a projection's epilogue nothing hides these instructions: eight
+// multiply-adds and one 2^x, against a reciprocal, a 2^x and fourteen others of the erf of
+// Abramowitz & Stegun 7.1.26 that was here.  Against 64 bits the largest error over
+// [-12, 12] is 3.8e-7 (4.7e-7 before), its root mean square 4.0e-8 (6.3e-8), and between
+// -5.5 and -2, where 1 + erf cancels, 1.6e-3 of the result (0.57).
 __device__ __forceinline__ float gelu_erf(float x) {
-  const float z = fabsf(x) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * z);
-  float p = 1.061405429f;
-  p = fmaf(p, t, -1.453152027f);
-  p = fmaf(p, t, 1.421413741f);
-  p = fmaf(p, t, -0.284496736f);
-  p = fmaf(p, t, 0.254829592f);
-  const float e = __builtin_amdgcn_exp2f(-z * z * 1.4426950408889634f);
-  const float erf_abs = 1.0f - p * t * e;
-  return 0.5f * x * (1.0f + copysignf(erf_abs, x));
+  const float u = fabsf(x);
+  float q = -1.1560465309e-06f;
+  q = fmaf(q, u, 1.9096820324e-05f);
+  q = fmaf(q, u, -9.0532266768e-05f);
+  q = fmaf(q, u, -3.6171370631e-04f);
+  q = fmaf(q, u, 7.3426929303e-03f);
+  q = fmaf(q, u, -5.2675705403e-02f);
+  q = fmaf(q, u, -4.5915418863e-01f);
+  q = fmaf(q, u, -1.1511111259f);
+  q = fmaf(q, u, -9.9999988079e-01f);
+  const float tail = __builtin_amdgcn_exp2f(q);
+  return x * (x >= 0.0f ? 1.0f - tail : tail);
 }
 
 // b with offsets[b] <= i < offsets[b + 1] (offsets non-decreasing, offsets[B] > i)
