@@ -110,7 +110,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
   int64_t P = 0, k64 = 0, img = 0, pix0 = 0, t_lo = 0, t_hi = 0;
   auto locate = [&](int64_t id) {
     if (id >= t_hi) {
-      img = find_segment(tile_offsets, B, id);
+      img = find_segment_uniform(tile_offsets, B, id);
       t_lo = tile_offsets[img];
       t_hi = tile_offsets[img + 1];
       pix0 = pix_offsets[img];

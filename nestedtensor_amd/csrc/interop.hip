@@ -472,12 +472,13 @@ __global__ __launch_bounds__(256) void transpose_u16_kernel(
     const int64_t per_xcd = gridDim.x / 8;
     if (id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
   }
-  const int64_t b = find_segment(tile_offsets, B, id);
+  const int64_t b = find_segment_uniform(tile_offsets, B, id);
   const int64_t R = rows[b], C = cols[b];
-  const int64_t tiles_c = (C + TC - 1) / TC;
-  const int64_t local = id - tile_offsets[b];
-  const int64_t r0 = (local / tiles_c) * TR;
-  const int64_t c0 = (local % tiles_c) * TC;
+  const unsigned tiles_c = (unsigned)((C + TC - 1) / TC);
+  const unsigned local = (unsigned)(id - tile_offsets[b]);      // a launch has less than 2^31 tiles
+  const unsigned line = local / tiles_c;
+  const int64_t r0 = (int64_t)line * TR;
+  const int64_t c0 = (int64_t)(local - line * tiles_c) * TC;
   const uint16_t* src = in + offsets[b];
   uint16_t* dst = out + offsets[b];
   {
@@ -566,12 +567,13 @@ __global__ __launch_bounds__(256) void transpose_u16_lines_kernel(
     const int64_t per_xcd = gridDim.x / 8;
     if (id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
   }
-  const int64_t b = find_segment(tile_offsets, B, id);
+  const int64_t b = find_segment_uniform(tile_offsets, B, id);
   const int64_t R = rows[b], C = cols[b];
-  const int64_t tiles_c = (C + 63) / 64;
-  const int64_t local = id - tile_offsets[b];
-  const int64_t k64 = (local / tiles_c) * 64;      // 64 k
-  const int64_t c0 = (local % tiles_c) * 64;
+  const unsigned tiles_c = (unsigned)((C + 63) / 64);
+  const unsigned local = (unsigned)(id - tile_offsets[b]);      // a launch has less than 2^31 tiles
+  const unsigned line = local / tiles_c;
+  const int64_t k64 = (int64_t)line * 64;
+  const int64_t c0 = (int64_t)(local - line * tiles_c) * 64;
   const uint16_t* src = in + offsets[b];
   uint16_t* dst = out + offsets[b];
   {

@@ -85,6 +85,21 @@ __device__ __forceinline__ int64_t find_segment(const int64_t* offsets, int64_t 
   return lo;
 }
 
+// find_segment for an i that a whole wavefront shares: its lanes look at 64 entries at a
+// time, one round trip to memory for up to 64 segments and two for up to 4096.
+__device__ __forceinline__ int64_t find_segment_uniform(const int64_t* offsets, int64_t B, int64_t i) {
+  const int64_t lane = threadIdx.x & (kWave - 1);
+  int64_t lo = 0, n = B;      // answer in [lo, lo + n)
+  for (;;) {
+    const int64_t step = (n + kWave - 1) / kWave;
+    const int64_t at = lane * step;
+    const int64_t below = __popcll(__ballot(at < n && offsets[lo + (at < n ? at : 0)] <= i)) - 1;
+    lo += below * step;
+    if (step == 1) return lo;
+    n = n - below * step < step ? n - below * step : step;
+  }
+}
+
 // Reductions over the 64 lanes of a wavefront on the vector ALU's data-parallel
 // primitives: four shifted adds within each row of 16 lanes, then the row totals
 // are passed on to rows 1 and 3 and to rows 2 and 3 (row_bcast:15, row_bcast:31);
