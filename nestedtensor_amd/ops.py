@@ -996,9 +996,11 @@ def _transpose_constituents(impl, rows, cols, new_sizes, which):
                                 torch.zeros_like(rows))
         else:
             tiles = ((rows + tr - 1) // tr) * ((cols + tc - 1) // tc)
-        meta = torch.zeros((3, B + 1), dtype=torch.int64)
+        # one table, one launch: rows, cols, first tile and first element of every constituent
+        meta = torch.zeros((4, B + 1), dtype=torch.int64)
         meta[0, :B], meta[1, :B] = rows, cols
         meta[2, 1:] = torch.cumsum(tiles, 0)
+        meta[3, 1:] = torch.cumsum(rows * cols, 0)
         return _upload_table(meta, buf.device), int(meta[2, B]), tr, tc
 
     meta_dev, total_tiles, tr, tc = impl.kept(which, tables)
@@ -1007,12 +1009,12 @@ def _transpose_constituents(impl, rows, cols, new_sizes, which):
         with _C.on_device(buf.device):
             if tr == 0:
                 _C.check(_C.lib.nt_transpose_ragged_lines(
-                    _C.ptr(buf), _C.ptr(out), _C.ptr(impl.offsets_dev()), _C.ptr(meta_dev[0]),
+                    _C.ptr(buf), _C.ptr(out), _C.ptr(meta_dev[3]), _C.ptr(meta_dev[0]),
                     _C.ptr(meta_dev[1]), _C.ptr(meta_dev[2]), B, total_tiles, buf.element_size(),
                     _C.current_stream(buf.device)))
             else:
                 _C.check(_C.lib.nt_transpose_ragged(
-                    _C.ptr(buf), _C.ptr(out), _C.ptr(impl.offsets_dev()), _C.ptr(meta_dev[0]),
+                    _C.ptr(buf), _C.ptr(out), _C.ptr(meta_dev[3]), _C.ptr(meta_dev[0]),
                     _C.ptr(meta_dev[1]), _C.ptr(meta_dev[2]), B, total_tiles, tr, tc, buf.element_size(),
                     _C.current_stream(buf.device)))
     res = NestedTensorImpl(out, new_sizes)
