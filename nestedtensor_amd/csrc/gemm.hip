@@ -895,7 +895,9 @@ static int launch_phased(const GemmArgs<T>& a, hipStream_t stream) {
 }
 
 // WAVES_M, WAVES_N, WM, WN, K-tile bytes per row
-typedef GemmCfg<4, 2, 2, 2, 128> Cfg128;   // 256 x 128: whatever the pipelined tile does not take
+typedef GemmCfg<4, 2, 2, 2, 128> Cfg128;   // 256 x 128: whatever the pipelined tile does not take,
+typedef GemmCfg<4, 2, 2, 3, 128> Cfg192;   // and in 16 bit 256 x 192
+typedef GemmCfg<4, 2, 2, 4, 128> Cfg256;   // and 256 x 256
 typedef GemmCfg<2, 2, 2, 1, 128> CfgSmall; // 128 x 64, four wavefronts: problems of fewer 256-row tiles than CUs
 typedef GemmCfg<2, 2, 2, 2, 128> CfgMid;   // 128 x 128, four wavefronts
 
@@ -1001,7 +1003,27 @@ static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
     }
   }
   if constexpr (sizeof(T) == 2) {
-    if (n_split % Cfg128::kBN != 0 && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
+    // K is no whole number of K tiles.  Estimated time: tile area over the measured rate of
+    // its shape (wider tiles read less LDS and L2 per product), times the mean of the whole
+    // rounds and of tiles / CUs.  Never the 256 x 128 tile alone: an attention layer of 15 heads
+    // of 32 on 35548 tokens (its projections have K = 480) took 285 us with it, 262 like this.
+    const int bn[3] = {Cfg128::kBN, Cfg192::kBN, Cfg256::kBN};
+    const double rate[3] = {1.0, 1.08, 1.17};
+    int best = -1;
+    double best_cost = 0.0;
+    for (int c = 0; c < 3; ++c) {
+      if (n_split % bn[c] != 0) continue;          // a tile must not straddle the K | V boundary
+      const int64_t tiles = ((a.M + 255) / 256) * ((a.N + bn[c] - 1) / bn[c]);
+      const double rounds = 0.5 * ((double)((tiles + num_cus - 1) / num_cus) + (double)tiles / num_cus);
+      const double cost = rounds * bn[c] / rate[c];
+      if (best < 0 || cost < best_cost) {
+        best = c;
+        best_cost = cost;
+      }
+    }
+    if (best == 1) return launch_cfg<T, Cfg192, EPI>(a, stream);
+    if (best == 2) return launch_cfg<T, Cfg256, EPI>(a, stream);
+    if (best < 0 && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
   }
   if (n_split % Cfg128::kBN != 0) {
     return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of a column tile", (long long)n_split);

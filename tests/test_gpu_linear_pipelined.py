@@ -82,3 +82,16 @@ def test_linear_few_columns(M, N, K, dtype):
     from nestedtensor_amd import ops
     x, w, b, ref, bound = _case(M, N, K, dtype)
     assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [
+    (33000, 200, 72),     # K of no whole tile: 256 x 256
+    (20000, 190, 488),    # 256 x 192
+    (33000, 480, 480),
+    (9000, 300, 104),     # 256 x 128
+])
+def test_linear_ragged_depth(M, N, K, dtype):
+    from nestedtensor_amd import ops
+    x, w, b, ref, bound = _case(M, N, K, dtype)
+    assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
