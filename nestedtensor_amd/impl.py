@@ -24,8 +24,8 @@ from . import _C
 
 
 class NestedTensorImpl:
-    __slots__ = ("buffer", "sizes", "_opt_sizes", "_sizes_dev", "_offsets_dev",
-                 "_meta_stream", "_summary", "_attn_schedule", "_attn_plan", "_kept", "channels_last")
+    __slots__ = ("buffer", "sizes", "_opt_sizes", "_tables", "_summary", "_attn_schedule", "_attn_plan", "_kept",
+                 "channels_last")
 
     def __init__(self, buffer, sizes, channels_last=False):
         """buffer: 1-D contiguous tensor; sizes: CPU int64 [B, D], or 0-d for an
@@ -42,9 +42,7 @@ class NestedTensorImpl:
         self.buffer = buffer
         self.sizes = sizes
         self._opt_sizes = None
-        self._sizes_dev = None
-        self._offsets_dev = None
-        self._meta_stream = None
+        self._tables = None
         self._summary = None
         self._attn_schedule = None
         self._attn_plan = None
@@ -117,30 +115,38 @@ class NestedTensorImpl:
         return out
 
     # ---- device metadata ---------------------------------------------------
-    def _ready(self, table):
-        return table is not None and (self._meta_stream is None or
-                                      usable_on(self._meta_stream, current_stream_id(self.buffer.device)))
-
-    def _size_tables(self):
-        """(sizes, offsets) on the device, written by one launch (nt_upload_sizes) on first
-        use.  A conversion that has them in hand with its buffer sets them instead, with
-        _meta_stream None: they are ordered like the buffer itself."""
+    def _table(self, which):
+        """Entry `which` of _tables = (stream, sizes, offsets): the stream that wrote the two
+        device tables (None: they are ordered like the buffer itself, any stream may read
+        them) and the tables, either None where only the other is known.  The three are
+        one attribute, assigned and read once: another thread sees all of them or none."""
+        tables = self._tables
+        if tables is not None and tables[which] is not None and (
+                tables[0] is None or usable_on(tables[0], current_stream_id(self.buffer.device))):
+            return tables[which]
         _C.require_device(self.buffer, "device metadata")
         if self.sizes.dim() != 2:
-            return self.sizes.to(self.buffer.device), None
-        tables = _upload_sizes(self.sizes, self.buffer.device)
+            return (None, self.sizes.to(self.buffer.device), None)[which]
+        # written by one launch (nt_upload_sizes) on first use
+        stream = current_stream_id(self.buffer.device)
+        tables = (stream,) + tuple(_upload_sizes(self.sizes, self.buffer.device))
         if not torch.cuda.is_current_stream_capturing():
-            self._sizes_dev, self._offsets_dev = tables
-            self._meta_stream = current_stream_id(self.buffer.device)
-        return tables
+            self._tables = tables
+        return tables[which]
 
     def sizes_dev(self):
         """int64 [B, D] mirror of the nested size."""
-        return self._sizes_dev if self._ready(self._sizes_dev) else self._size_tables()[0]
+        return self._table(1)
 
     def offsets_dev(self):
         """int64 [B + 1] element offsets, scanned on the device."""
-        return self._offsets_dev if self._ready(self._offsets_dev) else self._size_tables()[1]
+        return self._table(2)
+
+    def share_offsets(self, other):
+        """Take over the device offsets of `other`, whose constituents hold as many elements."""
+        tables = other._tables
+        if tables is not None:
+            self._tables = (tables[0], None, tables[2])
 
     def kept(self, name, build):
         """What build() returns, kept under `name` with this nested size for later calls on
@@ -211,10 +217,7 @@ class NestedTensorImpl:
         """Take over device copies of the nested size and of the element offsets
         that a conversion has already built for this nested size."""
         if sizes_dev.device == self.buffer.device and tuple(sizes_dev.shape) == tuple(self.sizes.shape):
-            self._sizes_dev = sizes_dev
-            self._meta_stream = None
-            if offsets_dev.numel() == self.B + 1:
-                self._offsets_dev = offsets_dev
+            self._tables = (None, sizes_dev, offsets_dev if offsets_dev.numel() == self.B + 1 else None)
 
     def with_buffer(self, buffer, channels_last=None):
         """Same nested size over another buffer (in the same layout unless
@@ -225,9 +228,7 @@ class NestedTensorImpl:
         out._opt_sizes = self._opt_sizes
         out._summary = self._summary
         if buffer.device == self.buffer.device:
-            out._sizes_dev = self._sizes_dev
-            out._offsets_dev = self._offsets_dev
-            out._meta_stream = self._meta_stream
+            out._tables = self._tables
             out._attn_schedule = self._attn_schedule
             out._attn_plan = self._attn_plan
             if self._kept is None:

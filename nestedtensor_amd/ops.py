@@ -1018,8 +1018,7 @@ def _transpose_constituents(impl, rows, cols, new_sizes, which):
                     _C.ptr(meta_dev[1]), _C.ptr(meta_dev[2]), B, total_tiles, tr, tc, buf.element_size(),
                     _C.current_stream(buf.device)))
     res = NestedTensorImpl(out, new_sizes)
-    # the constituents keep their extents
-    res._offsets_dev, res._meta_stream = impl._offsets_dev, impl._meta_stream
+    res.share_offsets(impl)       # the constituents keep their extents
     return res
 
 
@@ -1072,7 +1071,7 @@ def contiguous(impl, memory_format=torch.contiguous_format):
             return impl
         s = impl.sizes
         as_nhwc = NestedTensorImpl(impl.buffer, torch.stack([s[:, 1], s[:, 2], s[:, 0]], 1).contiguous())
-        as_nhwc._offsets_dev, as_nhwc._meta_stream = impl._offsets_dev, impl._meta_stream
+        as_nhwc.share_offsets(impl)
         out = transpose_nhwc_nchw(as_nhwc)
         return impl.with_buffer(out.buffer, channels_last=False)
     if memory_format == torch.channels_last:
