@@ -5,9 +5,9 @@ Counterpart of the reference's NestedTensorImpl / EfficientSizeNode
 nestedtensor/csrc/storage/EfficientSizeNode.h:53-138): one contiguous 1-D
 buffer, a host int64 table ``sizes[B, D]`` and the per-dimension "regular or
 not" summary ``opt_sizes``.  What is new here is the device side of the
-metadata: ``sizes`` mirrored in HBM and int64 element ``offsets[B + 1]`` built
-by the device prefix scan (nt_offsets_from_sizes), both cached on the impl and
-created on first use on the buffer's stream.  Only nested_dim 1 exists
+metadata: ``sizes`` mirrored in HBM and int64 element ``offsets[B + 1]``, written
+by one launch (nt_upload_sizes) on first use and kept on the impl for the stream
+that asked.  Only nested_dim 1 exists
 (EfficientSizeNode.h:86-88).
 
 Two storage layouts exist, as in the reference (Packed.h:100-163): every
@@ -24,8 +24,7 @@ from . import _C
 
 
 class NestedTensorImpl:
-    __slots__ = ("buffer", "sizes", "_opt_sizes", "_tables", "_summary", "_attn_schedule", "_attn_plan", "_kept",
-                 "channels_last")
+    __slots__ = ("buffer", "sizes", "_opt_sizes", "_given", "_summary", "_attn_plan", "_kept", "channels_last")
 
     def __init__(self, buffer, sizes, channels_last=False):
         """buffer: 1-D contiguous tensor; sizes: CPU int64 [B, D], or 0-d for an
@@ -42,11 +41,10 @@ class NestedTensorImpl:
         self.buffer = buffer
         self.sizes = sizes
         self._opt_sizes = None
-        self._tables = None
+        self._given = None
         self._summary = None
-        self._attn_schedule = None
         self._attn_plan = None
-        self._kept = None
+        self._kept = {}
 
     # ---- host metadata ----------------------------------------------------
     @property
@@ -115,53 +113,48 @@ class NestedTensorImpl:
         return out
 
     # ---- device metadata ---------------------------------------------------
-    def _table(self, which):
-        """Entry `which` of _tables = (stream, sizes, offsets): the stream that wrote the two
-        device tables (None: they are ordered like the buffer itself, any stream may read
-        them) and the tables, either None where only the other is known.  The three are
-        one attribute, assigned and read once: another thread sees all of them or none."""
-        tables = self._tables
-        if tables is not None and tables[which] is not None and (
-                tables[0] is None or usable_on(tables[0], current_stream_id(self.buffer.device))):
-            return tables[which]
+    def kept(self, name, build, keys=None):
+        """What build() returns, kept under `name` with this nested size for later calls.
+
+        One entry per stream that asked, and none is replaced or dropped while the nested
+        size lives.  Per stream, because nothing orders work on one stream behind the
+        kernel that wrote another's table.  For good, because a captured graph reads the
+        table it was given on every replay, whatever other streams do in between.  A
+        capture takes what eager calls on its stream have made, or else on any stream;
+        what it has to write itself is part of the graph and not kept.
+
+        keys: the other nested size that the table depends on.  Only the last one's table
+        is kept per stream (with that nested size itself, so the identity test stays valid)."""
+        device = self.buffer.device
+        key = (name, device.index, current_stream_id(device))
+        entry = self._kept.get(key)
+        if entry is not None and entry[0] is keys:
+            return entry[1]
+        if torch.cuda.is_current_stream_capturing():
+            made = [e[1] for k, e in list(self._kept.items()) if k[:2] == key[:2] and e[0] is keys]
+            return made[0] if made else build()
+        entry = (keys, build())
+        if keys is not None:
+            self._kept[key] = entry
+            return entry[1]
+        return self._kept.setdefault(key, entry)[1]      # the first of two threads on one stream wins
+
+    def _size_tables(self):
+        """(sizes, offsets) on the device, written by one launch (nt_upload_sizes) on first use."""
         _C.require_device(self.buffer, "device metadata")
         if self.sizes.dim() != 2:
-            return (None, self.sizes.to(self.buffer.device), None)[which]
-        # written by one launch (nt_upload_sizes) on first use
-        stream = current_stream_id(self.buffer.device)
-        tables = (stream,) + tuple(_upload_sizes(self.sizes, self.buffer.device))
-        if not torch.cuda.is_current_stream_capturing():
-            self._tables = tables
-        return tables[which]
+            return self.sizes.to(self.buffer.device), None
+        return self.kept("sizes", lambda: _upload_sizes(self.sizes, self.buffer.device))
 
     def sizes_dev(self):
         """int64 [B, D] mirror of the nested size."""
-        return self._table(1)
+        given = self._given
+        return given[0] if given is not None and given[0] is not None else self._size_tables()[0]
 
     def offsets_dev(self):
         """int64 [B + 1] element offsets, scanned on the device."""
-        return self._table(2)
-
-    def share_offsets(self, other):
-        """Take over the device offsets of `other`, whose constituents hold as many elements."""
-        tables = other._tables
-        if tables is not None:
-            self._tables = (tables[0], None, tables[2])
-
-    def kept(self, name, build):
-        """What build() returns, kept under `name` with this nested size for later calls on
-        the same device and stream.  For device metadata that kernels wrote: work on
-        another stream gets its own (see usable_on)."""
-        device = self.buffer.device
-        stream = current_stream_id(device)
-        if self._kept is None:
-            self._kept = {}
-        entry = self._kept.get(name)
-        if entry is None or entry[0] != device or not usable_on(entry[1], stream):
-            entry = (device, stream, build())
-            if not torch.cuda.is_current_stream_capturing():
-                self._kept[name] = entry
-        return entry[2]
+        given = self._given
+        return given[1] if given is not None and given[1] is not None else self._size_tables()[1]
 
     def row_offsets_dev(self):
         """int64 [B + 1] offsets counted in rows of the first constituent dim
@@ -181,22 +174,22 @@ class NestedTensorImpl:
 
     def attention_schedule(self, kv=None, q_tile=128):
         """Work list of the attention kernel (nt_attention_schedule), built from the
-        host copies of the nested sizes and cached on the device: int32 [n_work, 8] rows {first query
-        token, query length, first query row of the tile, 0, first key token, key
-        length, 0, 0}, one per q_tile query rows of every sequence, longest key
+        host copies of the nested sizes and kept per stream (see kept): int32 [n_work, 8]
+        rows {first query token, query length, first query row of the tile, 0, first key
+        token, key length, 0, 0}, one per q_tile query rows of every sequence, longest key
         sequences first (they take the most key tiles, so they should start
         first).  Tiles that do not exist are never listed, hence never launched.
         kv: the nested tensor of the keys (None: self-attention)."""
         if kv is None or kv.sizes is self.sizes:
             kv = self
-        cached = self._attn_schedule
-        stream = current_stream_id(self.buffer.device)
-        if cached is not None and cached[0] is kv.sizes and usable_on(cached[2], stream):
-            return cached[1]
-        sched = _attention_schedule(self.sizes, kv.sizes, q_tile, self.buffer.device)
-        if not torch.cuda.is_current_stream_capturing():
-            self._attn_schedule = (kv.sizes, sched, stream)      # holds kv.sizes, so the identity test stays valid
-        return sched
+        def build():
+            return _attention_schedule(self.sizes, kv.sizes, q_tile, self.buffer.device)
+        return self.kept("work list", build) if kv is self else self.kept("work list of keys", build, kv.sizes)
+
+    @property
+    def _attn_schedule(self):
+        """The work lists written for this nested size, None before the first."""
+        return [e[1] for k, e in list(self._kept.items()) if k[0] in ("work list", "work list of keys")] or None
 
     def attention_plan(self, num_heads, head_dim, kv=None):
         """Plan of the planned attention kernel (nt_attention_plan) for this nested
@@ -215,9 +208,16 @@ class NestedTensorImpl:
 
     def adopt_device_metadata(self, sizes_dev, offsets_dev):
         """Take over device copies of the nested size and of the element offsets
-        that a conversion has already built for this nested size."""
+        that a conversion has already built for this nested size.  They are ordered like
+        the buffer that was written with them, so every stream may read them."""
         if sizes_dev.device == self.buffer.device and tuple(sizes_dev.shape) == tuple(self.sizes.shape):
-            self._tables = (None, sizes_dev, offsets_dev if offsets_dev.numel() == self.B + 1 else None)
+            self._given = (sizes_dev, offsets_dev if offsets_dev.numel() == self.B + 1 else None)
+
+    def share_offsets(self, other):
+        """Take over the offsets that a conversion has built for `other`, whose
+        constituents hold as many elements."""
+        if other._given is not None:
+            self._given = (None, other._given[1])
 
     def with_buffer(self, buffer, channels_last=None):
         """Same nested size over another buffer (in the same layout unless
@@ -228,11 +228,8 @@ class NestedTensorImpl:
         out._opt_sizes = self._opt_sizes
         out._summary = self._summary
         if buffer.device == self.buffer.device:
-            out._tables = self._tables
-            out._attn_schedule = self._attn_schedule
+            out._given = self._given
             out._attn_plan = self._attn_plan
-            if self._kept is None:
-                self._kept = {}
             out._kept = self._kept
         return out
 
@@ -240,14 +237,6 @@ class NestedTensorImpl:
 def current_stream_id(device):
     """Identity of torch's current stream on `device` (0: the default stream)."""
     return torch._C._cuda_getCurrentRawStream(device.index)
-
-
-def usable_on(made_on, stream):
-    """Whether metadata that a kernel wrote on stream `made_on` may be read by work on
-    `stream`.  On another stream nothing orders the reader behind the writer, and the
-    block could be handed out again while the reader still runs, so such a caller writes
-    its own copy (a launch).  A capture keeps what its eager warm-up has made."""
-    return made_on == stream or torch.cuda.is_current_stream_capturing()
 
 
 _attention_schedule = _C.ops.attention_schedule.default

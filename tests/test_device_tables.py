@@ -1,6 +1,7 @@
 """Who may read which device table of a nested size, and for how long: launches, streams and
 captures are stubbed, so everything here runs on the host."""
 import sys
+import weakref
 
 import pytest
 import torch
@@ -19,6 +20,7 @@ class Device:
         monkeypatch.setattr(impl_module._C, "require_device", lambda *a: None)
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: self.capturing)
         monkeypatch.setattr(impl_module, "_upload_sizes", lambda sizes, device: (self._table(), self._table()))
+        monkeypatch.setattr(impl_module, "_attention_schedule", lambda *a: self._table())
 
     def _table(self):
         self.launches += 1
@@ -74,3 +76,59 @@ def test_tables_of_a_conversion_serve_every_stream(device):
         assert made.sizes_dev() is sizes and made.offsets_dev() is offsets
         assert same.sizes_dev() is sizes and same.offsets_dev() is offsets
     assert device.launches == 0
+
+
+TABLES = {
+    "sizes": NestedTensorImpl.sizes_dev,
+    "offsets": NestedTensorImpl.offsets_dev,
+    "row offsets": NestedTensorImpl.row_offsets_dev,
+    "last dim rows": lambda t: t.last_dim_rows()[0],
+    "work list": NestedTensorImpl.attention_schedule,
+}
+
+
+@pytest.mark.parametrize("name", sorted(TABLES))
+def test_captured_table_outlives_calls_on_other_streams(device, name):
+    table, a = TABLES[name], nested()
+    shared = a.with_buffer(a.buffer + 1)
+    table(a)                                             # warm-up on the default stream and on the side stream
+    device.stream = 2
+    table(a)
+    device.capturing = True
+    captured = weakref.ref(table(a))
+    also = weakref.ref(table(shared))
+    device.capturing = False
+    memory = nested((4, 4))
+    for device.stream in (1, 3, 1, 2):
+        table(a)
+        table(shared)
+        a.attention_schedule(kv=memory)
+    assert captured() is not None and writer(captured()) == 2
+    assert also() is not None and writer(also()) == 2
+    device.capturing, device.stream = True, 2
+    assert table(a) is captured()
+
+
+@pytest.mark.parametrize("name", sorted(TABLES))
+def test_streams_in_turn_write_a_table_once_each(device, name):
+    table, a = TABLES[name], nested()
+    mine = {}
+    for device.stream in (1, 2):
+        mine[device.stream] = table(a)
+        assert writer(mine[device.stream]) == device.stream
+    launches = device.launches
+    for device.stream in (1, 2, 1, 2, 2, 1):
+        assert table(a) is mine[device.stream]
+    assert device.launches == launches
+
+
+@pytest.mark.parametrize("name", sorted(TABLES))
+def test_capture_takes_what_eager_calls_have_made(device, name):
+    table, a = TABLES[name], nested()
+    device.capturing = True
+    own = table(a)                                       # nothing made yet: the graph writes its own ..
+    device.capturing = False
+    first = table(a)
+    assert first is not own                              # .. which eager calls do not see
+    device.stream, device.capturing = 2, True
+    assert table(a) is first
