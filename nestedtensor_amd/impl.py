@@ -124,20 +124,27 @@ class NestedTensorImpl:
         what it has to write itself is part of the graph and not kept.
 
         keys: the other nested size that the table depends on.  Only the last one's table
-        is kept per stream (with that nested size itself, so the identity test stays valid)."""
+        is kept per stream (with that nested size itself, so the identity test stays valid),
+        and what a capture was given."""
         device = self.buffer.device
         key = (name, device.index, current_stream_id(device))
         entry = self._kept.get(key)
         if entry is not None and entry[0] is keys:
-            return entry[1]
+            return entry[1] if keys is None else self._given_out(entry[1])
         if torch.cuda.is_current_stream_capturing():
             made = [e[1] for k, e in list(self._kept.items()) if k[:2] == key[:2] and e[0] is keys]
-            return made[0] if made else build()
+            return self._given_out(made[0]) if made else build()
         entry = (keys, build())
         if keys is not None:
             self._kept[key] = entry
             return entry[1]
         return self._kept.setdefault(key, entry)[1]      # the first of two threads on one stream wins
+
+    def _given_out(self, table):
+        """`table`, kept with this nested size from now on if a capture is under way."""
+        if torch.cuda.is_current_stream_capturing():
+            self._kept["captured", id(table)] = (None, table)
+        return table
 
     def _size_tables(self):
         """(sizes, offsets) on the device, written by one launch (nt_upload_sizes) on first use."""
@@ -200,9 +207,9 @@ class NestedTensorImpl:
             kv = self
         cached = self._attn_plan
         if cached is not None and cached[0] is kv.sizes and cached[1] == (num_heads, head_dim):
-            return cached[2]
-        plan = _C.ops.attention_plan.default(self.sizes[:, 0].contiguous(), kv.sizes[:, 0].contiguous(),
-                                             num_heads, head_dim, self.buffer.device)
+            return self._given_out(cached[2])
+        plan = _attention_plan(self.sizes[:, 0].contiguous(), kv.sizes[:, 0].contiguous(), num_heads, head_dim,
+                               self.buffer.device)
         self._attn_plan = (kv.sizes, (num_heads, head_dim), plan)
         return plan
 
@@ -239,6 +246,7 @@ def current_stream_id(device):
     return torch._C._cuda_getCurrentRawStream(device.index)
 
 
+_attention_plan = _C.ops.attention_plan.default
 _attention_schedule = _C.ops.attention_schedule.default
 _size_summary = _C.ops.size_summary.default
 _upload_sizes = _C.ops.upload_sizes.default

@@ -21,6 +21,7 @@ class Device:
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: self.capturing)
         monkeypatch.setattr(impl_module, "_upload_sizes", lambda sizes, device: (self._table(), self._table()))
         monkeypatch.setattr(impl_module, "_attention_schedule", lambda *a: self._table())
+        monkeypatch.setattr(impl_module, "_attention_plan", lambda *a: self._table())
 
     def _table(self):
         self.launches += 1
@@ -132,3 +133,17 @@ def test_capture_takes_what_eager_calls_have_made(device, name):
     assert first is not own                              # .. which eager calls do not see
     device.stream, device.capturing = 2, True
     assert table(a) is first
+
+
+@pytest.mark.parametrize("table", [lambda q, kv: q.attention_schedule(kv=kv), lambda q, kv: q.attention_plan(8, 64, kv=kv)],
+                         ids=["work list", "plan"])
+def test_captured_table_outlives_calls_with_other_keys(device, table):
+    queries, memory, other = nested(), nested((7, 1)), nested((2, 2))
+    table(queries, memory)
+    device.capturing = True
+    captured = weakref.ref(table(queries, memory))
+    device.capturing = False
+    assert captured() is table(queries, memory)
+    kept = [weakref.ref(table(queries, keys)) for keys in (other, memory, other)]
+    assert captured() is not None
+    assert kept[0]() is None and kept[1]() is None          # only the last one is kept otherwise
