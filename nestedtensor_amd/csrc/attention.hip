@@ -23,6 +23,7 @@
 #include "attn_common.h"
 
 #include <algorithm>
+#include <new>
 #include <vector>
 
 namespace nt {
@@ -1061,8 +1062,8 @@ extern "C" int64_t nt_attention_schedule_items(const int64_t* q_lens, int64_t B,
   return n;
 }
 
-extern "C" int nt_attention_schedule(const int64_t* q_lens, const int64_t* k_lens, int64_t B, int64_t q_tile,
-                                     int32_t* schedule, int64_t n_items, void* stream) {
+static int launch_schedule(const int64_t* q_lens, const int64_t* k_lens, int64_t B, int64_t q_tile, int32_t* schedule,
+                           int64_t n_items, hipStream_t stream) {
   const int64_t expect = nt_attention_schedule_items(q_lens, B, q_tile);
   if (expect < 0) return NT_ERR_INVALID_ARGUMENT;
   if (expect != n_items || (n_items > 0 && !schedule) || q_tile > 0x7fffffff) {
@@ -1101,10 +1102,19 @@ extern "C" int nt_attention_schedule(const int64_t* q_lens, const int64_t* k_len
       c.s[i].first = (int)first;
       first += (c.s[i].q_len + q_tile - 1) / q_tile;
     }
-    hipLaunchKernelGGL(nt::attention_schedule_kernel, dim3((c.n + 3) / 4), dim3(256), 0, (hipStream_t)stream, c,
+    hipLaunchKernelGGL(nt::attention_schedule_kernel, dim3((c.n + 3) / 4), dim3(256), 0, stream, c,
                        reinterpret_cast<int4*>(schedule));
   }
   return check_launch("attention_schedule_kernel");
+}
+
+extern "C" int nt_attention_schedule(const int64_t* q_lens, const int64_t* k_lens, int64_t B, int64_t q_tile,
+                                     int32_t* schedule, int64_t n_items, void* stream) {
+  try {
+    return launch_schedule(q_lens, k_lens, B, q_tile, schedule, n_items, (hipStream_t)stream);
+  } catch (const std::bad_alloc&) {
+    return fail(NT_ERR_UNSUPPORTED, "attention_schedule: no host memory for %lld sequences", (long long)B);
+  }
 }
 
 extern "C" int nt_varlen_attention_vt(const void* q, int64_t ldq, const void* k, int64_t ldk,
