@@ -83,6 +83,7 @@ int nt_offsets_from_sizes_noalloc(const int64_t* sizes, int64_t B, int64_t D, in
  * with padded of shape [B, padded_sizes_host[0..D)] (the batch maxima).
  * `n_ragged` (1..3) leading constituent dims may differ between constituents;
  * the trailing D - n_ragged dims must equal padded_sizes_host[k] for every b.
+ * A leading extent above the padded one is cut off.
  * `elem_bytes` in {1, 2, 4, 8}; `pad_bits` is the padding value already
  * converted to the element type, in the low elem_bytes bytes.
  * Replaces add_padding_kernelLauncher<T> (nestedtensor/csrc/cuda/padding.h:12-23,
@@ -106,8 +107,9 @@ int nt_add_padding_mask(const void* packed, void* padded, uint8_t* mask, const i
                         const int64_t* padded_sizes_host, int elem_bytes, uint64_t pad_bits,
                         void* stream);
 
-/* packed[offsets[b] + lin(i)] = padded[b, i] for i inside sizes[b]: the
- * length-based inverse of nt_add_padding.  Replaces
+/* packed[offsets[b] + lin(i)] = padded[b, i] for i inside sizes[b], none of
+ * which may exceed padded_sizes_host: the length-based inverse of
+ * nt_add_padding.  Replaces
  * remove_padding_kernelLauncher<T> (nestedtensor/csrc/cuda/padding.h:36-45,
  * kernels padding.cu:286-394) as called by from_padded_tensor
  * (nestedtensor/csrc/masking.cpp:459-509). */

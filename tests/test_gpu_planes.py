@@ -53,3 +53,48 @@ def test_planes(name, dtype, wider):
                                           len(shapes), D, nrag, _C.i64_array(ext), eb, stream))
         assert torch.equal(back[shift:shift + total].cpu(), flat)
         assert bool((back[:shift] == 99).all()) and bool((back[shift + total:] == 99).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.float16, torch.float32, torch.float64])
+@pytest.mark.parametrize("name,cut", [("images", (2, 9, 12)), ("three", (2, 4, 3)), ("inner", (4, 6, 3)), ("flat", (7, 70)),
+                                      ("flat", (20, 299)), ("wide", (3, 1200))])
+def test_planes_cut_off(name, cut, dtype):
+    # padded extents below a constituent's: pad cuts off, row by row, whatever chunk the row ends in
+    from nestedtensor_amd import _C
+    eb = torch.empty(0, dtype=dtype).element_size()
+    shapes = SHAPES[name]
+    nrag = 2 if name == "inner" or len(cut) == 2 else 3
+    parts = [(torch.rand(s) * 200 + 1).to(dtype) for s in shapes]
+    sizes_dev, offsets = _C.ops.upload_sizes.default(torch.tensor(shapes), DEV)
+    packed = torch.cat([t.reshape(-1) for t in parts]).to(DEV)
+    expect = torch.full((len(shapes),) + cut, 7, dtype=dtype)
+    for b, t in enumerate(parts):
+        inside = tuple(slice(0, min(n, m)) for n, m in zip(t.shape, cut))
+        expect[(b,) + inside] = t[inside]
+    padded = torch.full((expect.numel() + 40,), 99, dtype=dtype, device=DEV)
+    seven = torch.tensor([7], dtype=dtype).view(torch.uint8)
+    _C.check(_C.lib.nt_add_padding(_C.ptr(packed), _C.ptr(padded), _C.ptr(offsets), _C.ptr(sizes_dev), len(shapes), len(cut),
+                                   nrag, _C.i64_array(cut), eb, int.from_bytes(bytes(seven.tolist()), "little"),
+                                   _C.current_stream(DEV)))
+    assert torch.equal(padded[:expect.numel()].cpu(), expect.reshape(-1))
+    assert bool((padded[expect.numel():] == 99).all())
+    # un-pad of that has no result, but writes nothing outside the packed buffer
+    back = torch.full((packed.numel() + 40,), 99, dtype=dtype, device=DEV)
+    _C.check(_C.lib.nt_remove_padding(_C.ptr(padded), _C.ptr(back), _C.ptr(offsets), _C.ptr(sizes_dev), len(shapes), len(cut),
+                                      nrag, _C.i64_array(cut), eb, _C.current_stream(DEV)))
+    assert bool((back[packed.numel():] == 99).all())
+
+
+def test_planes_cut_off_a_constituent_past_32_bits():
+    from nestedtensor_amd import _C
+    shapes, cut = [(70000, 70000), (3, 60)], (70, 50)
+    sizes_dev, offsets = _C.ops.upload_sizes.default(torch.tensor(shapes), DEV)
+    packed = torch.empty(int(offsets[-1]), dtype=torch.uint8, device=DEV)
+    parts = [packed[:70000 * 70000].view(70000, 70000), packed[70000 * 70000:].view(3, 60)]
+    parts[0][:71] = torch.randint(1, 99, (71, 70000), dtype=torch.uint8, device=DEV)
+    parts[1].copy_(torch.randint(1, 99, (3, 60), dtype=torch.uint8, device=DEV))
+    padded = torch.full((2, 70, 50), 99, dtype=torch.uint8, device=DEV)
+    _C.check(_C.lib.nt_add_padding(_C.ptr(packed), _C.ptr(padded), _C.ptr(offsets), _C.ptr(sizes_dev), 2, 2, 2,
+                                   _C.i64_array(cut), 1, 7, _C.current_stream(DEV)))
+    assert torch.equal(padded[0], parts[0][:70, :50])
+    assert torch.equal(padded[1, :3], parts[1][:, :50]) and bool((padded[1, 3:] == 7).all())
