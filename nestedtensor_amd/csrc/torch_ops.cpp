@@ -1307,7 +1307,15 @@ std::tuple<Tensor, int64_t> embedding_checked(const Tensor& weight_in, const Ten
   c10::hip::HIPGuard guard(indices.device().index());
   void* stream = stream_of(indices);
   check(nt_count_outside(idx.const_data_ptr<int64_t>(), T, weight_in.size(0), word, stamp, stream));
-  Tensor out = embedding_packed(weight_in, idx, c10::nullopt, c10::nullopt);
+  Tensor out;
+  try {
+    out = embedding_packed(weight_in, idx, c10::nullopt, c10::nullopt);
+  } catch (...) {
+    // The count is still on its way to the word: it must not arrive over the next call's
+    // from another stream, or after the word has gone with its thread.
+    (void)hipStreamSynchronize(static_cast<hipStream_t>(stream));
+    throw;
+  }
   const auto t0 = std::chrono::steady_clock::now();
   uint64_t seen;
   for (int spin = 0; static_cast<uint32_t>((seen = __atomic_load_n(word, __ATOMIC_ACQUIRE)) >> 32) != stamp; ++spin) {

@@ -373,3 +373,22 @@ def test_embedding_counts_out_of_range_indices_before_it_returns(n):
     with pytest.raises(IndexError, match="%d index value" % len({0, n // 2, n - 1})):
         torch.nn.functional.embedding(nt.nested_tensor([bad.to(DEV)], dtype=torch.int64, device=DEV), w)
     torch.nn.functional.embedding(nt.nested_tensor([ids.to(DEV)], dtype=torch.int64, device=DEV), w)
+
+
+def test_embedding_that_fails_leaves_no_count_on_its_way():
+    # a table of 2^42 elements by strides of zero: its rows cannot be laid out for the gather
+    w = torch.zeros(1, 1, device=DEV).expand(1 << 20, 1 << 22)
+    ids = nt.nested_tensor([torch.zeros(5, dtype=torch.int64, device=DEV)], dtype=torch.int64, device=DEV)
+    a = torch.randn(4096, 4096, device=DEV)
+    side = torch.cuda.Stream()
+    torch.mm(a, a)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(40):                      # some tens of milliseconds in front of the count
+            torch.mm(a, a)
+        with pytest.raises(RuntimeError):
+            torch.nn.functional.embedding(ids, w)
+        assert side.query()
+    torch.cuda.synchronize()
+    good = torch.nn.functional.embedding(ids, torch.ones(3, 8, device=DEV))
+    assert bool((good._impl.buffer == 1).all())
