@@ -23,8 +23,8 @@
 // cross-attention, a few thousand rows) gets 128x64 tiles of four wavefronts, or 128x128
 // when those would not fit in one round (its duration is one tile's life, and a quarter
 // of a tile on four times as many CUs ends sooner: 3200 x 512 x 512 10.6 -> 6.3 us; the
-// fused in-projection of a layer of a few hundred tokens 16.0 -> 11.6 us), short or
-// ragged K a 256x128 tile.
+// fused in-projection of a layer of a few hundred tokens 16.0 -> 11.6 us), at most 64
+// columns 128x64 tiles, short or ragged K tiles of 256 rows by 128, 192 or 256 columns.
 //
 // Epilogues:
 //   plain  - C row-major + bias;
@@ -696,7 +696,7 @@ __device__ __forceinline__ void phased_tile(const GemmArgs<T>& a, int64_t m0, in
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave >> 2;      // rows group * 32 NI .. of the tile
-  const int wn = wave & 3;          // columns wn * 64 ..
+  const int wn = wave & 3;          // columns wn * 32 NJ ..
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
@@ -958,52 +958,42 @@ static int pick_phased(int64_t M, int64_t N, int64_t n_split, int64_t nk, int el
   return best;
 }
 
-template <typename T, int EPI>
-static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
-  const int64_t n_split = EPI == kEpiQkv ? a.n_split : 0;
-  int num_cus = 0;
-  const int rc = compute_units(&num_cus);
-  if (rc != NT_OK) return rc;
+// What a problem runs on: a shape of linear_kernel or, kTilePhased + c, kPhasedShapes[c].
+enum { kTile256x128, kTile256x192, kTile256x256, kTile128x64, kTile128x128, kTilePhased };
+
+// The tile of M x N x K; row-major A has lda elements per row, columns from n_split on go
+// transposed into Vt (n_split = 0: to either side of no boundary).  qkv: there are such
+// columns.  -1: a tile would straddle the boundary.
+static int choose_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_split, bool qkv, int elem_bytes,
+                       int num_cus) {
+  const bool half = elem_bytes == 2;
   // Fewer 256 x 128 tiles than half the CUs: the launch is one tile's life on a fraction
   // of the chip, and a quarter-size tile on four times as many CUs is shorter
   // (3200 x 512 x 512: 6.2 us, against 6.8 with the smallest pipelined tile).
-  if constexpr (sizeof(T) == 2) {
-    if (((a.M + 255) / 256) * ((a.N + 127) / 128) * 2 <= num_cus) {
-      const bool small = ((a.M + 127) / 128) * ((a.N + 63) / 64) <= num_cus;
-      if (small && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
-      if (!small && n_split % CfgMid::kBN == 0) return launch_cfg<T, CfgMid, EPI>(a, stream);
-    }
+  if (half && ((M + 255) / 256) * ((N + 127) / 128) * 2 <= num_cus) {
+    const bool small = ((M + 127) / 128) * ((N + 63) / 64) <= num_cus;
+    if (small && n_split % CfgSmall::kBN == 0) return kTile128x64;
+    if (!small && n_split % CfgMid::kBN == 0) return kTile128x128;
   }
   // At most 64 columns: such a product reads A once and is bound by that, half of a
   // 128-column tile would be padding, and three workgroups of this tile share a CU where the
   // larger ones have it to themselves while they fill and drain (589481 x 64 x 256
   // 95.8 -> 77.5 us = 4.9 TB/s, 300000 x 32 x 64 33.2 -> 22.6, 100000 x 32 x 256 18.1 -> 13.4;
   // with 128 columns it loses: 300000 x 128 x 128 32.4 -> 49.2).
-  if constexpr (sizeof(T) == 2) {
-    if (a.N <= CfgSmall::kBN && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
-  }
+  if (half && N <= CfgSmall::kBN && n_split % CfgSmall::kBN == 0) return kTile128x64;
   // The pipelined tile needs whole K tiles, at least two of them, and 32-bit offsets
   // inside a tile.  (fp32: row-major results only, the transposed strips
   // would not fit its LDS.)
   constexpr int64_t kMaxSpan = (int64_t(1) << 32) - 1;
-  const int64_t row_bytes = a.K * (int64_t)sizeof(T);
-  if constexpr (sizeof(T) == 2 || EPI != kEpiQkv) {
-    if (row_bytes % 128 == 0 && row_bytes >= 2 * 128 && a.lda * (int64_t)sizeof(T) * 320 < kMaxSpan &&
-        row_bytes * 256 < kMaxSpan && (a.M / 64 + 1) * (a.N / 64 + 1) < (int64_t(1) << 30)) {
-      switch (pick_phased(a.M, a.N, n_split, row_bytes / 128, (int)sizeof(T), num_cus)) {
-        case 0: return launch_phased<T, PhasedCfg<T, 2, 2, 3>, EPI>(a, stream);
-        case 1: return launch_phased<T, PhasedCfg<T, 3, 2, 2>, EPI>(a, stream);
-        case 2: return launch_phased<T, PhasedCfg<T, 4, 2, 2>, EPI>(a, stream);
-        case 3: return launch_phased<T, PhasedCfg<T, 5, 2, 2>, EPI>(a, stream);
-        case 4: return launch_phased<T, PhasedCfg<T, 2, 1, 4>, EPI>(a, stream);
-        case 5: return launch_phased<T, PhasedCfg<T, 3, 1, 3>, EPI>(a, stream);
-        case 6: return launch_phased<T, PhasedCfg<T, 4, 1, 3>, EPI>(a, stream);
-        case 7: return launch_phased<T, PhasedCfg<T, 5, 1, 2>, EPI>(a, stream);
-      }
-    }
+  const int64_t row_bytes = K * elem_bytes;
+  if ((half || !qkv) && row_bytes % 128 == 0 && row_bytes >= 2 * 128 && lda * elem_bytes * 320 < kMaxSpan &&
+      row_bytes * 256 < kMaxSpan && (M / 64 + 1) * (N / 64 + 1) < (int64_t(1) << 30)) {
+    const int c = pick_phased(M, N, n_split, row_bytes / 128, elem_bytes, num_cus);
+    if (c >= 0) return kTilePhased + c;
   }
-  if constexpr (sizeof(T) == 2) {
-    // K is no whole number of K tiles.  Estimated time: tile area over the measured rate of
+  if (half) {
+    // What is left: K of no whole number of K tiles or of one, rows of A or W too long for
+    // 32-bit offsets.  Estimated time: tile area over the measured rate of
     // its shape (wider tiles read less LDS and L2 per product), times the mean of the whole
     // rounds and of tiles / CUs.  Never the 256 x 128 tile alone: an attention layer of 15 heads
     // of 32 on 35548 tokens (its projections have K = 480) took 285 us with it, 262 like this.
@@ -1013,7 +1003,7 @@ static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
     double best_cost = 0.0;
     for (int c = 0; c < 3; ++c) {
       if (n_split % bn[c] != 0) continue;          // a tile must not straddle the K | V boundary
-      const int64_t tiles = ((a.M + 255) / 256) * ((a.N + bn[c] - 1) / bn[c]);
+      const int64_t tiles = ((M + 255) / 256) * ((N + bn[c] - 1) / bn[c]);
       const double rounds = 0.5 * ((double)((tiles + num_cus - 1) / num_cus) + (double)tiles / num_cus);
       const double cost = rounds * bn[c] / rate[c];
       if (best < 0 || cost < best_cost) {
@@ -1021,11 +1011,40 @@ static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
         best_cost = cost;
       }
     }
-    if (best == 1) return launch_cfg<T, Cfg192, EPI>(a, stream);
-    if (best == 2) return launch_cfg<T, Cfg256, EPI>(a, stream);
-    if (best < 0 && n_split % CfgSmall::kBN == 0) return launch_cfg<T, CfgSmall, EPI>(a, stream);
+    if (best >= 0) return kTile256x128 + best;
+    if (n_split % CfgSmall::kBN == 0) return kTile128x64;
   }
-  if (n_split % Cfg128::kBN != 0) {
+  return n_split % Cfg128::kBN == 0 ? kTile256x128 : -1;
+}
+
+template <typename T, int EPI>
+static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
+  const int64_t n_split = EPI == kEpiQkv ? a.n_split : 0;
+  int num_cus = 0;
+  const int rc = compute_units(&num_cus);
+  if (rc != NT_OK) return rc;
+  const int tile = choose_tile(a.M, a.N, a.K, a.lda, n_split, EPI == kEpiQkv, (int)sizeof(T), num_cus);
+  if constexpr (sizeof(T) == 2 || EPI != kEpiQkv) {
+    switch (tile) {
+      case kTilePhased + 0: return launch_phased<T, PhasedCfg<T, 2, 2, 3>, EPI>(a, stream);
+      case kTilePhased + 1: return launch_phased<T, PhasedCfg<T, 3, 2, 2>, EPI>(a, stream);
+      case kTilePhased + 2: return launch_phased<T, PhasedCfg<T, 4, 2, 2>, EPI>(a, stream);
+      case kTilePhased + 3: return launch_phased<T, PhasedCfg<T, 5, 2, 2>, EPI>(a, stream);
+      case kTilePhased + 4: return launch_phased<T, PhasedCfg<T, 2, 1, 4>, EPI>(a, stream);
+      case kTilePhased + 5: return launch_phased<T, PhasedCfg<T, 3, 1, 3>, EPI>(a, stream);
+      case kTilePhased + 6: return launch_phased<T, PhasedCfg<T, 4, 1, 3>, EPI>(a, stream);
+      case kTilePhased + 7: return launch_phased<T, PhasedCfg<T, 5, 1, 2>, EPI>(a, stream);
+    }
+  }
+  if constexpr (sizeof(T) == 2) {
+    switch (tile) {
+      case kTile256x192: return launch_cfg<T, Cfg192, EPI>(a, stream);
+      case kTile256x256: return launch_cfg<T, Cfg256, EPI>(a, stream);
+      case kTile128x64: return launch_cfg<T, CfgSmall, EPI>(a, stream);
+      case kTile128x128: return launch_cfg<T, CfgMid, EPI>(a, stream);
+    }
+  }
+  if (tile != kTile256x128) {
     return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of a column tile", (long long)n_split);
   }
   return launch_cfg<T, Cfg128, EPI>(a, stream);
@@ -1094,6 +1113,26 @@ extern "C" int nt_linear_act(const void* A, int64_t lda, const void* W, const vo
     default: return fail(NT_ERR_INVALID_ARGUMENT, "linear: unknown dtype %d", dtype);
   }
 #undef NT_LIN_CASE
+}
+
+extern "C" int nt_linear_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_split, int dtype, int num_cus,
+                              int* tile) {
+  if (M < 1 || N < 1 || K < 0 || lda < K || n_split > N || num_cus < 0 || !tile ||
+      (dtype != NT_F32 && dtype != NT_F16 && dtype != NT_BF16)) {
+    return fail(NT_ERR_INVALID_ARGUMENT, "linear_tile: bad arguments");
+  }
+  if (num_cus == 0) {
+    const int rc = compute_units(&num_cus);
+    if (rc != NT_OK) return rc;
+  }
+  const bool qkv = n_split >= 0;
+  const int c = choose_tile(M, N, K, lda, qkv ? n_split : 0, qkv, dtype == NT_F32 ? 4 : 2, num_cus);
+  if (c < 0) return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of a column tile", (long long)n_split);
+  static const int kShapes[kTilePhased][2] = {{256, 128}, {256, 192}, {256, 256}, {128, 64}, {128, 128}};
+  tile[0] = c >= kTilePhased ? 64 * kPhasedShapes[c - kTilePhased].ni : kShapes[c][0];
+  tile[1] = c >= kTilePhased ? 128 * kPhasedShapes[c - kTilePhased].nj : kShapes[c][1];
+  tile[2] = c >= kTilePhased ? kPhasedShapes[c - kTilePhased].bufs : 0;
+  return NT_OK;
 }
 
 extern "C" int nt_linear(const void* A, int64_t lda, const void* W, const void* bias, void* C,

@@ -1,5 +1,7 @@
 """The pipelined projection kernel: every tile shape its launcher can pick, with row and
 column remainders and with fewer, as many and more K tiles than its LDS ring holds."""
+import ctypes
+
 import pytest
 import torch
 
@@ -15,6 +17,14 @@ def _bound(x, w, ref, dtype):
     return (x.abs() @ w.abs().t()) * (x.size(1) * 2.0 ** -24) + ref.abs() * unit + 1e-6
 
 
+def _tile(M, N, K, dtype, n_split=-1):
+    """(rows, columns, K tiles in flight; 0: not the pipelined kernel) that the launcher picks."""
+    from nestedtensor_amd import _C
+    tile = (ctypes.c_int * 3)()
+    _C.check(_C.lib.nt_linear_tile(M, N, K, K, n_split, _C.dtype_code(dtype), 0, tile))
+    return tuple(tile)
+
+
 def _case(M, N, K, dtype):
     g = torch.Generator("cuda").manual_seed(M + 3 * N + 7 * K)
     x = torch.randn(M, K, device=DEV, generator=g).to(dtype)
@@ -24,47 +34,52 @@ def _case(M, N, K, dtype):
     return x, w, b, ref, _bound(x.double(), w.double(), ref, dtype)
 
 
-@pytest.mark.parametrize("dtype,M,N,K", [
-    (torch.float16, 6430, 520, 256),    # 128 x 128, ring of four, as many K tiles
-    (torch.bfloat16, 6430, 520, 448),   # ... seven K tiles
-    (torch.float16, 6536, 520, 192),    # 192 x 128, ring of three
-    (torch.bfloat16, 6536, 520, 320),
-    (torch.float16, 9822, 520, 192),    # 256 x 128, ring of three
-    (torch.float16, 9822, 520, 320),
-    (torch.float16, 7172, 1100, 192),   # 320 x 128, ring of two
-    (torch.bfloat16, 6430, 520, 128),   # ... two K tiles
-    (torch.float16, 8073, 768, 192),    # 128 x 256, ring of three
-    (torch.float16, 8073, 768, 448),
-    (torch.bfloat16, 8974, 1100, 128),  # 192 x 256, ring of two
-    (torch.float16, 8974, 1100, 320),
-    (torch.float16, 9822, 1100, 128),   # 256 x 256
-    (torch.bfloat16, 9822, 1100, 448),
-    (torch.float16, 7172, 2304, 128),   # 320 x 256
-    (torch.bfloat16, 7172, 2304, 256),
-    (torch.float32, 300, 520, 160),     # fp32: 128 x 128
-    (torch.float32, 6001, 768, 128),    # 192 x 128
+@pytest.mark.parametrize("dtype,M,N,K,tile", [
+    (torch.float16, 6430, 520, 256, (128, 128, 4)),     # as many K tiles as the ring holds
+    (torch.bfloat16, 6430, 520, 448, (128, 128, 4)),    # seven K tiles
+    (torch.float16, 6536, 520, 192, (192, 128, 3)),
+    (torch.bfloat16, 6536, 520, 320, (192, 128, 3)),
+    (torch.float16, 9822, 520, 192, (256, 128, 3)),
+    (torch.float16, 9822, 520, 320, (256, 128, 3)),
+    (torch.float16, 7172, 1100, 192, (320, 128, 2)),
+    (torch.bfloat16, 6430, 520, 128, (320, 128, 2)),
+    (torch.float16, 8073, 768, 192, (128, 256, 3)),
+    (torch.float16, 8073, 768, 448, (128, 256, 3)),
+    (torch.bfloat16, 8974, 1100, 128, (192, 256, 2)),
+    (torch.float16, 8974, 1100, 320, (192, 256, 2)),
+    (torch.float16, 9822, 1100, 128, (256, 256, 2)),
+    (torch.bfloat16, 9822, 1100, 448, (256, 256, 2)),
+    (torch.float16, 7172, 2304, 128, (320, 256, 2)),
+    (torch.bfloat16, 7172, 2304, 256, (320, 256, 2)),
+    (torch.float32, 300, 520, 160, (128, 128, 4)),
+    (torch.float32, 6001, 768, 128, (192, 128, 3)),
 ])
-def test_linear_pipelined_shapes(dtype, M, N, K):
+def test_linear_pipelined_shapes(dtype, M, N, K, tile):
     from nestedtensor_amd import ops
+    assert _tile(M, N, K, dtype) == tile
     x, w, b, ref, bound = _case(M, N, K, dtype)
     assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
     relu = ops.linear(x, w, b, "relu").double()
     assert bool(((relu - ref.clamp_min(0)).abs() <= bound).all())
+    # the slope of gelu is at most 1.13, its error 4e-7 in fp32 before the one rounding
+    gelu = 0.5 * ref * torch.special.erfc(-ref * 0.5 ** 0.5)
+    assert bool(((ops.linear(x, w, b, "gelu").double() - gelu).abs() <= 1.13 * bound + 4e-7).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("M,E", [
-    (10781, 128),   # 320 x 128 tiles, two K tiles
-    (5423, 256),    # 192 x 128
-    (2561, 512),    # 128 x 128
-    (8073, 512),    # 256 x 256
-    (4045, 512),    # 128 x 256
-    (5479, 512),    # 192 x 256
-    (3305, 640),    # 256 x 128, a boundary between K and V at a multiple of 128
-    (10779, 512),   # 320 x 256
+@pytest.mark.parametrize("M,E,tile", [
+    (10781, 128, (320, 128, 2)),
+    (5423, 256, (192, 128, 3)),
+    (2561, 512, (128, 128, 4)),
+    (8073, 512, (256, 256, 2)),
+    (4045, 512, (128, 256, 3)),
+    (5479, 512, (192, 256, 2)),
+    (3305, 640, (256, 128, 3)),     # a boundary between K and V at a multiple of 128
+    (10779, 512, (320, 256, 2)),
 ])
-def test_linear_qkv_pipelined_shapes(M, E, dtype):
+def test_linear_qkv_pipelined_shapes(M, E, tile, dtype):
     from nestedtensor_amd import _C
+    assert _tile(M, 3 * E, E, dtype, 2 * E) == tile
     x, w, b, ref, bound = _case(M, 3 * E, E, dtype)
     ld = (M + 72 + 7) // 8 * 8
     qk = torch.empty(M, 2 * E, dtype=dtype, device=DEV)
@@ -77,21 +92,25 @@ def test_linear_qkv_pipelined_shapes(M, E, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("M,N,K", [(40001, 64, 128), (40001, 65, 128), (33000, 33, 64), (70003, 8, 72), (16385, 64, 8)])
-def test_linear_few_columns(M, N, K, dtype):
+@pytest.mark.parametrize("M,N,K,tile", [
+    (40001, 64, 128, (128, 64, 0)), (40001, 65, 128, (320, 128, 2)), (33000, 33, 64, (128, 64, 0)),
+    (70003, 8, 72, (128, 64, 0)), (16385, 64, 8, (128, 64, 0))])
+def test_linear_few_columns(M, N, K, tile, dtype):
     from nestedtensor_amd import ops
+    assert _tile(M, N, K, dtype) == tile
     x, w, b, ref, bound = _case(M, N, K, dtype)
     assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("M,N,K", [
-    (33000, 200, 72),     # K of no whole tile: 256 x 256
-    (20000, 190, 488),    # 256 x 192
-    (33000, 480, 480),
-    (9000, 300, 104),     # 256 x 128
+@pytest.mark.parametrize("M,N,K,tile", [
+    (33000, 200, 72, (256, 256, 0)),     # K of no whole tile
+    (33000, 480, 480, (256, 192, 0)),
+    (20000, 190, 488, (256, 128, 0)),
+    (9000, 300, 104, (128, 128, 0)),
 ])
-def test_linear_ragged_depth(M, N, K, dtype):
+def test_linear_ragged_depth(M, N, K, tile, dtype):
     from nestedtensor_amd import ops
+    assert _tile(M, N, K, dtype) == tile
     x, w, b, ref, bound = _case(M, N, K, dtype)
     assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
