@@ -44,7 +44,11 @@ __device__ __forceinline__ void piece_values(u32x4 raw, u32x4 raw_res, bool has_
 // WAVES wavefronts (1: four rows per workgroup, 4: the workgroup shares one row and
 // combines its partial sums through LDS); every lane keeps P pieces in registers,
 // so a row has at most 64 * WAVES * P pieces.
-template <typename T, int P, int WAVES>
+// AFFINE: there is a gain or a shift.  Without either a kernel of its own: told apart by the
+// pointers alone, the arithmetic on both is done and thrown away and their registers are
+// held (us: bf16 937500 x 32 281 -> 212, 117187 x 256 37.6 -> 29.5, 3000 x 4096 9.1 -> 7.2,
+// fp16 39062 x 768 20.9 -> 18.4, 57692 x 520 29.0 -> 21.0).
+template <typename T, int P, int WAVES, bool AFFINE>
 __global__ __launch_bounds__(kWave * kNormRowsPerBlock) void layer_norm_rows_kernel(
     const T* __restrict__ x, const T* __restrict__ residual, const T* __restrict__ gamma,
     const T* __restrict__ beta, T* __restrict__ out, int64_t rows, int n, float eps) {
@@ -82,8 +86,8 @@ __global__ __launch_bounds__(kWave * kNormRowsPerBlock) void layer_norm_rows_ker
   for (int p = 0; p < P; ++p) {
     const int c = t + p * kTeam;
     if (c < pieces) {
-      if (kEarly && gamma) raw_gamma[p] = load16_unaligned(reinterpret_cast<const char*>(gamma + c * kPer));
-      if (kEarly && beta) raw_beta[p] = load16_unaligned(reinterpret_cast<const char*>(beta + c * kPer));
+      if (AFFINE && kEarly && gamma) raw_gamma[p] = load16_unaligned(reinterpret_cast<const char*>(gamma + c * kPer));
+      if (AFFINE && kEarly && beta) raw_beta[p] = load16_unaligned(reinterpret_cast<const char*>(beta + c * kPer));
       const u32x4 raw = *reinterpret_cast<const u32x4*>(xr + c * 16);
       u32x4 raw_res = raw;
       if (has_res) raw_res = *reinterpret_cast<const u32x4*>(rr + c * 16);
@@ -113,17 +117,19 @@ __global__ __launch_bounds__(kWave * kNormRowsPerBlock) void layer_norm_rows_ker
   for (int p = 0; p < P; ++p) {
     const int c = t + p * kTeam;
     if (c < pieces) {
-      if (!kEarly && gamma) raw_gamma[p] = load16_unaligned(reinterpret_cast<const char*>(gamma + c * kPer));
-      if (!kEarly && beta) raw_beta[p] = load16_unaligned(reinterpret_cast<const char*>(beta + c * kPer));
+      if (AFFINE && !kEarly && gamma) raw_gamma[p] = load16_unaligned(reinterpret_cast<const char*>(gamma + c * kPer));
+      if (AFFINE && !kEarly && beta) raw_beta[p] = load16_unaligned(reinterpret_cast<const char*>(beta + c * kPer));
       T g[kPer], b[kPer];
-      __builtin_memcpy(g, &raw_gamma[p], 16);
-      __builtin_memcpy(b, &raw_beta[p], 16);
+      if (AFFINE) {
+        __builtin_memcpy(g, &raw_gamma[p], 16);
+        __builtin_memcpy(b, &raw_beta[p], 16);
+      }
       T y[kPer];
 #pragma unroll
       for (int j = 0; j < kPer; ++j) {
         float v = (f[p][j] - mean) * rstd;
-        if (gamma) v = v * (float)g[j];
-        if (beta) v = v + (float)b[j];
+        if (AFFINE && gamma) v = v * (float)g[j];
+        if (AFFINE && beta) v = v + (float)b[j];
         y[j] = (T)v;
       }
       u32x4 o;
@@ -172,9 +178,9 @@ static int launch_layer_norm_vec(const void* x, const void* residual, const void
   constexpr int kRows = kNormRowsPerBlock / WAVES;
   const int64_t blocks = (rows + kRows - 1) / kRows;
   if (blocks > 0x7fffffffLL) return fail(NT_ERR_UNSUPPORTED, "layer_norm: too many rows");
-  hipLaunchKernelGGL((layer_norm_rows_kernel<T, P, WAVES>), dim3((unsigned)blocks),
-                     dim3(kWave * kNormRowsPerBlock), 0, stream, static_cast<const T*>(x),
-                     static_cast<const T*>(residual), static_cast<const T*>(gamma),
+  auto* const kernel = gamma || beta ? layer_norm_rows_kernel<T, P, WAVES, true> : layer_norm_rows_kernel<T, P, WAVES, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kWave * kNormRowsPerBlock), 0, stream,
+                     static_cast<const T*>(x), static_cast<const T*>(residual), static_cast<const T*>(gamma),
                      static_cast<const T*>(beta), static_cast<T*>(out), rows, (int)n, (float)eps);
   return check_launch("layer_norm_rows_kernel");
 }

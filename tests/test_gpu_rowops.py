@@ -60,6 +60,17 @@ def test_layer_norm_no_affine_and_4d():
     _close(got._impl.buffer, exp.buffer, torch.float32)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("pieces", [1, 64, 65, 128, 129, 256, 257, 512, 513, 1024])
+def test_layer_norm_without_gain_and_shift_equals_one_and_zero(pieces, dtype):
+    # the two have kernels of their own; x * 1 + 0 changes nothing
+    n = pieces * 16 // torch.empty(0, dtype=dtype).element_size()
+    a = nt.nested_tensor(_tensors([(5, n), (1, n), (13, n)], dtype, pieces), device=DEV, dtype=dtype)
+    one, zero = torch.ones(n, device=DEV, dtype=dtype), torch.zeros(n, device=DEV, dtype=dtype)
+    plain = torch.nn.functional.layer_norm(a, (n,))
+    assert torch.equal(plain._impl.buffer, torch.nn.functional.layer_norm(a, (n,), one, zero)._impl.buffer)
+
+
 def test_layer_norm_errors():
     a = nt.nested_tensor([torch.randn(3, 4), torch.randn(2, 5)], device=DEV)
     with pytest.raises(RuntimeError, match="Cannot normalize across irregular dimension 2"):
