@@ -988,6 +988,10 @@ static int choose_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_s
   const int64_t row_bytes = K * elem_bytes;
   if ((half || !qkv) && row_bytes % 128 == 0 && row_bytes >= 2 * 128 && lda * elem_bytes * 320 < kMaxSpan &&
       row_bytes * 256 < kMaxSpan && (M / 64 + 1) * (N / 64 + 1) < (int64_t(1) << 30)) {
+    // fp32, two K tiles and one round of 256 x 128 tiles: linear_kernel fills sooner (9000 x 128 x 64
+    // 13.5 us against 15.5, 53000 x 64 x 64 14.3 against 16.6; in two rounds it loses, 20000 x
+    // 512 x 64 28.7 against 19.6).
+    if (!half && row_bytes == 256 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus) return kTile256x128;
     const int c = pick_phased(M, N, n_split, row_bytes / 128, elem_bytes, num_cus);
     if (c >= 0) return kTilePhased + c;
   }

@@ -53,6 +53,8 @@ def _case(M, N, K, dtype):
     (torch.bfloat16, 7172, 2304, 256, (320, 256, 2)),
     (torch.float32, 300, 520, 160, (128, 128, 4)),
     (torch.float32, 6001, 768, 128, (192, 128, 3)),
+    (torch.float32, 6001, 768, 64, (256, 128, 0)),      # two K tiles and one round of tiles
+    (torch.float32, 20000, 520, 64, (256, 256, 2)),
 ])
 def test_linear_pipelined_shapes(dtype, M, N, K, tile):
     from nestedtensor_amd import ops
