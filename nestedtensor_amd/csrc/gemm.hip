@@ -980,7 +980,9 @@ static int choose_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_s
   // larger ones have it to themselves while they fill and drain (589481 x 64 x 256
   // 95.8 -> 77.5 us = 4.9 TB/s, 300000 x 32 x 64 33.2 -> 22.6, 100000 x 32 x 256 18.1 -> 13.4;
   // with 128 columns it loses: 300000 x 128 x 128 32.4 -> 49.2).
-  if (half && N <= CfgSmall::kBN && n_split % CfgSmall::kBN == 0) return kTile128x64;
+  // Deep whole K tiles keep the CU busy by themselves (70000 x 64 x 3072: 97 us, 84 with 320 x 128;
+  // 40000 x 64 x 8192: 173, 142 with 192 x 128; 33000 x 64 x 2048: 27.7, 28.6 with 256 x 128).
+  if (half && N <= CfgSmall::kBN && n_split % CfgSmall::kBN == 0 && (K <= 2048 || K % 64 != 0)) return kTile128x64;
   // The pipelined tile needs whole K tiles, at least two of them, and 32-bit offsets
   // inside a tile.  (fp32: row-major results only, the transposed strips
   // would not fit its LDS.)

@@ -96,7 +96,8 @@ def test_linear_qkv_pipelined_shapes(M, E, tile, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,tile", [
     (40001, 64, 128, (128, 64, 0)), (40001, 65, 128, (320, 128, 2)), (33000, 33, 64, (128, 64, 0)),
-    (70003, 8, 72, (128, 64, 0)), (16385, 64, 8, (128, 64, 0))])
+    (70003, 8, 72, (128, 64, 0)), (16385, 64, 8, (128, 64, 0)),
+    (33001, 64, 2048, (128, 64, 0)), (33001, 64, 2112, (192, 128, 3)), (33001, 64, 2056, (128, 64, 0))])
 def test_linear_few_columns(M, N, K, tile, dtype):
     from nestedtensor_amd import ops
     assert _tile(M, N, K, dtype) == tile
