@@ -61,7 +61,7 @@ SIGNATURES = {
     "nt_exclusive_scan_i32": (_int, [_c_void_p, _i64, _c_void_p, _c_void_p, _size_t, _c_void_p]),
     "nt_linear": (_int, [_c_void_p, _i64, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i64,
                          _int, _c_void_p]),
-    "nt_linear_tile": (_int, [_i64, _i64, _i64, _i64, _i64, _int, _int, _c_void_p]),
+    "nt_linear_tile": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _c_void_p]),
     "nt_linear_act": (_int, [_c_void_p, _i64, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i64,
                              _int, _int, _c_void_p]),
     "nt_linear_qkv": (_int, [_c_void_p, _i64, _c_void_p, _c_void_p, _c_void_p, _i64, _c_void_p, _i64, _i64,

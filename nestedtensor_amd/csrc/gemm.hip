@@ -916,40 +916,59 @@ static int compute_units(int* n) {
   return NT_OK;
 }
 
-// Tile shapes of the pipelined kernel.  `alone` and `full`: microseconds per K tile
-// (128 bytes of a row) of a workgroup of 16-bit operands when few CUs and when all CUs
-// are at work; the difference is the clock the chip holds on random operands.
+// What a problem of 16-bit operands takes on a tile shape, in microseconds: `alone` and
+// `full` per K tile (128 bytes of a row) of a workgroup when few CUs and when all CUs are at
+// work (the difference is the clock the chip holds on random operands), `first` for the fill
+// and the burst of stores of one round over the CUs and `round` for those of a further one,
+// `pieces` for a round of stores to rows that are no whole 16-byte pieces.  Fitted on the
+// shape that is fastest of all in 903 problems (72 to 8192 columns, K 128 to 4096, 2500 to
+// 200000 rows) and not on single times: what it picks takes 1.010 times the fastest shape's
+// time on average, 1.07 at the 95th percentile.  Without the shapes of linear_kernel, with 4 us for any
+// further round and aligned rows throughout it was 1.030 and 1.17, and one problem in five
+// (two to six K tiles, or rows that end inside a piece) lost 3 to 40 % against linear_kernel.
+struct TileCost {
+  double alone, full, first, round, pieces;
+};
 struct PhasedShape {
   int ni, nj, bufs;
-  double alone, full;
+  TileCost cost;
 };
 static const PhasedShape kPhasedShapes[] = {
-    {2, 2, 3, 0.55, 0.91}, {3, 2, 2, 0.73, 1.31},  {4, 2, 2, 0.90, 1.65}, {5, 2, 2, 1.12, 2.05},
-    {2, 1, 4, 0.37, 0.55}, {3, 1, 3, 0.485, 0.745}, {4, 1, 3, 0.56, 0.94}, {5, 1, 2, 0.70, 1.19}};
+    {2, 2, 3, {0.602, 0.956, 3.46, 3.89, 2.47}},
+    {3, 2, 2, {1.1, 1.23, 4.06, 7.84, 3.37}},
+    {4, 2, 2, {1.1, 1.63, 5.17, 8.88, 11.8}},
+    {5, 2, 2, {1.6, 1.95, 9.4, 9.5, 7.15}},
+    {2, 1, 4, {0.25, 0.522, 1, 2.87, 8.7}},
+    {3, 1, 3, {0.35, 0.756, 2.01, 5.04, 4.29}},
+    {4, 1, 3, {0.735, 0.987, 3.51, 4.38, 6.58}},
+    {5, 1, 2, {0.9, 1.17, 3.94, 5.97, 8.67}}};
+constexpr int kPhasedCount = (int)(sizeof(kPhasedShapes) / sizeof(kPhasedShapes[0]));
+// linear_kernel's tiles of 256 rows by 128, 192 and 256 columns
+static const TileCost kLinearCosts[] = {
+    {0.406, 1.1, 0.741, 6.47, 3.54},
+    {0.669, 1.9, 2, 6.09, 7.69},
+    {1.83, 2, 2, 9.84, 13.3}};
 
-// Shape with the least estimated time for M x N with nk K tiles: whole rounds over the
-// CUs at the full rate, a last round at the rate its tiles leave (never below `alone`),
-// 4 us per further round, and the launch and the burst of stores.  The estimate is within
-// 10 % of the measured time on 14 of the 16 projection shapes it was fitted on (512 to
-// 6144 columns, K 512 to 4096, 3 to 24 column panels, one to eight rounds) and ranks the
-// shapes as measured on all of them; the two misses are its own second-best shapes.
-// fp32: 64 cycles of matrix pipe per instruction, no lowered clock.
-static int pick_phased(int64_t M, int64_t N, int64_t n_split, int64_t nk, int elem_bytes, int num_cus) {
+static double tile_time(const TileCost& c, double launch, int64_t tiles, int64_t nk, bool pieces, int num_cus) {
+  const int64_t whole = tiles / num_cus, rest = tiles % num_cus;
+  double last = c.full * (double)rest / num_cus;
+  if (rest > 0 && last < c.alone) last = c.alone;
+  const double us = launch + nk * (whole * c.full + last) + c.first + c.round * (double)(whole + (rest > 0) - 1);
+  return us + (pieces ? c.pieces * (whole > 0 ? (double)tiles / num_cus : 1.0) : 0.0);
+}
+
+// Pipelined shape with the least estimated time for M x N with nk K tiles of fp32: 64
+// cycles of matrix pipe per instruction, no lowered clock.
+static int pick_phased_f32(int64_t M, int64_t N, int64_t nk, int num_cus) {
   int best = -1;
   double best_us = 0.0;
-  for (int c = 0; c < (int)(sizeof(kPhasedShapes) / sizeof(kPhasedShapes[0])); ++c) {
+  for (int c = 0; c < kPhasedCount; ++c) {
     const PhasedShape& s = kPhasedShapes[c];
-    const int64_t bm = 64 * s.ni, bn = 128 * s.nj;
-    // a tile must not straddle the K | V boundary, and the prologue fills its whole ring
-    if (n_split % bn != 0 || nk < s.bufs) continue;
-    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-    const int64_t whole = tiles / num_cus, rest = tiles % num_cus;
-    const double alone = elem_bytes == 4 ? 0.853 * s.ni * s.nj : s.alone;
-    const double full = elem_bytes == 4 ? alone : s.full;
-    double last = full * (double)rest / num_cus;
-    if (rest > 0 && last < alone) last = alone;
-    const double us = nk * (whole * full + last) + 4.0 * (double)(whole + (rest > 0) - 1) +
-                      3.5 + 0.9 * s.ni * s.nj * (elem_bytes / 2);
+    if (nk < s.bufs) continue;                       // the prologue fills the whole ring
+    const int64_t tiles = ((M + 64 * s.ni - 1) / (64 * s.ni)) * ((N + 128 * s.nj - 1) / (128 * s.nj));
+    const double area = s.ni * s.nj;
+    const TileCost cost = {0.853 * area, 0.853 * area, 1.8 * area, 4.0, 0.0};
+    const double us = tile_time(cost, 3.5, tiles, nk, false, num_cus);
     if (best < 0 || us < best_us) {
       best = c;
       best_us = us;
@@ -963,9 +982,10 @@ enum { kTile256x128, kTile256x192, kTile256x256, kTile128x64, kTile128x128, kTil
 
 // The tile of M x N x K; row-major A has lda elements per row, columns from n_split on go
 // transposed into Vt (n_split = 0: to either side of no boundary).  qkv: there are such
-// columns.  -1: a tile would straddle the boundary.
-static int choose_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_split, bool qkv, int elem_bytes,
-                       int num_cus) {
+// columns.  pieces: the rows of the result end inside a 16-byte piece.  -1: a tile would
+// straddle the boundary.
+static int choose_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_split, bool qkv, bool pieces,
+                       int elem_bytes, int num_cus) {
   const bool half = elem_bytes == 2;
   // Fewer 256 x 128 tiles than half the CUs: the launch is one tile's life on a fraction
   // of the chip, and a quarter-size tile on four times as many CUs is shorter
@@ -990,12 +1010,33 @@ static int choose_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_s
   const int64_t row_bytes = K * elem_bytes;
   if ((half || !qkv) && row_bytes % 128 == 0 && row_bytes >= 2 * 128 && lda * elem_bytes * 320 < kMaxSpan &&
       row_bytes * 256 < kMaxSpan && (M / 64 + 1) * (N / 64 + 1) < (int64_t(1) << 30)) {
-    // fp32, two K tiles and one round of 256 x 128 tiles: linear_kernel fills sooner (9000 x 128 x 64
-    // 13.5 us against 15.5, 53000 x 64 x 64 14.3 against 16.6; in two rounds it loses, 20000 x
-    // 512 x 64 28.7 against 19.6).
-    if (!half && row_bytes == 256 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus) return kTile256x128;
-    const int c = pick_phased(M, N, n_split, row_bytes / 128, elem_bytes, num_cus);
-    if (c >= 0) return kTilePhased + c;
+    const int64_t nk = row_bytes / 128;
+    if (!half) {
+      // Two K tiles and one round of 256 x 128 tiles: linear_kernel fills sooner (9000 x 128 x 64
+      // 13.5 us against 15.5, 53000 x 64 x 64 14.3 against 16.6; in two rounds it loses, 20000 x
+      // 512 x 64 28.7 against 19.6).
+      if (nk == 2 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus) return kTile256x128;
+      const int c = pick_phased_f32(M, N, nk, num_cus);
+      if (c >= 0) return kTilePhased + c;
+    } else {
+      int best = -1;
+      double best_us = 0.0;
+      for (int c = 0; c < 3 + kPhasedCount; ++c) {
+        const bool phased = c >= 3;
+        const PhasedShape& s = kPhasedShapes[phased ? c - 3 : 0];
+        const int64_t bm = phased ? 64 * s.ni : 256, bn = phased ? 128 * s.nj : 128 + 64 * c;
+        // a tile must not straddle the K | V boundary, and the prologue fills the whole ring
+        if (n_split % bn != 0 || (phased && nk < s.bufs)) continue;
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        const double us = phased ? tile_time(s.cost, 2.59, tiles, nk, pieces, num_cus)
+                                 : tile_time(kLinearCosts[c], 4.7, tiles, nk, pieces, num_cus);
+        if (best < 0 || us < best_us) {
+          best = phased ? kTilePhased + c - 3 : kTile256x128 + c;
+          best_us = us;
+        }
+      }
+      if (best >= 0) return best;
+    }
   }
   if (half) {
     // What is left: K of no whole number of K tiles or of one, rows of A or W too long for
@@ -1029,7 +1070,8 @@ static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
   int num_cus = 0;
   const int rc = compute_units(&num_cus);
   if (rc != NT_OK) return rc;
-  const int tile = choose_tile(a.M, a.N, a.K, a.lda, n_split, EPI == kEpiQkv, (int)sizeof(T), num_cus);
+  const bool pieces = ((EPI == kEpiQkv && n_split == 0 ? a.ldvt : a.ldc) * (int64_t)sizeof(T)) % 16 != 0;
+  const int tile = choose_tile(a.M, a.N, a.K, a.lda, n_split, EPI == kEpiQkv, pieces, (int)sizeof(T), num_cus);
   if constexpr (sizeof(T) == 2 || EPI != kEpiQkv) {
     switch (tile) {
       case kTilePhased + 0: return launch_phased<T, PhasedCfg<T, 2, 2, 3>, EPI>(a, stream);
@@ -1121,9 +1163,9 @@ extern "C" int nt_linear_act(const void* A, int64_t lda, const void* W, const vo
 #undef NT_LIN_CASE
 }
 
-extern "C" int nt_linear_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_split, int dtype, int num_cus,
-                              int* tile) {
-  if (M < 1 || N < 1 || K < 0 || lda < K || n_split > N || num_cus < 0 || !tile ||
+extern "C" int nt_linear_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldc, int64_t n_split, int dtype,
+                              int num_cus, int* tile) {
+  if (M < 1 || N < 1 || K < 0 || lda < K || ldc < 1 || n_split > N || num_cus < 0 || !tile ||
       (dtype != NT_F32 && dtype != NT_F16 && dtype != NT_BF16)) {
     return fail(NT_ERR_INVALID_ARGUMENT, "linear_tile: bad arguments");
   }
@@ -1132,7 +1174,8 @@ extern "C" int nt_linear_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int6
     if (rc != NT_OK) return rc;
   }
   const bool qkv = n_split >= 0;
-  const int c = choose_tile(M, N, K, lda, qkv ? n_split : 0, qkv, dtype == NT_F32 ? 4 : 2, num_cus);
+  const int elem_bytes = dtype == NT_F32 ? 4 : 2;
+  const int c = choose_tile(M, N, K, lda, qkv ? n_split : 0, qkv, ldc * elem_bytes % 16 != 0, elem_bytes, num_cus);
   if (c < 0) return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of a column tile", (long long)n_split);
   static const int kShapes[kTilePhased][2] = {{256, 128}, {256, 192}, {256, 256}, {128, 64}, {128, 128}};
   tile[0] = c >= kTilePhased ? 64 * kPhasedShapes[c - kTilePhased].ni : kShapes[c][0];

@@ -21,7 +21,7 @@ def _tile(M, N, K, dtype, n_split=-1):
     """(rows, columns, K tiles in flight; 0: not the pipelined kernel) that the launcher picks."""
     from nestedtensor_amd import _C
     tile = (ctypes.c_int * 3)()
-    _C.check(_C.lib.nt_linear_tile(M, N, K, K, n_split, _C.dtype_code(dtype), 0, tile))
+    _C.check(_C.lib.nt_linear_tile(M, N, K, K, N if n_split < 0 else n_split, n_split, _C.dtype_code(dtype), 0, tile))
     return tuple(tile)
 
 
@@ -35,22 +35,25 @@ def _case(M, N, K, dtype):
 
 
 @pytest.mark.parametrize("dtype,M,N,K,tile", [
-    (torch.float16, 6430, 520, 256, (128, 128, 4)),     # as many K tiles as the ring holds
-    (torch.bfloat16, 6430, 520, 448, (128, 128, 4)),    # seven K tiles
-    (torch.float16, 6536, 520, 192, (192, 128, 3)),
-    (torch.bfloat16, 6536, 520, 320, (192, 128, 3)),
-    (torch.float16, 9822, 520, 192, (256, 128, 3)),
-    (torch.float16, 9822, 520, 320, (256, 128, 3)),
-    (torch.float16, 7172, 1100, 192, (320, 128, 2)),
-    (torch.bfloat16, 6430, 520, 128, (320, 128, 2)),
-    (torch.float16, 8073, 768, 192, (128, 256, 3)),
-    (torch.float16, 8073, 768, 448, (128, 256, 3)),
-    (torch.bfloat16, 8974, 1100, 128, (192, 256, 2)),
-    (torch.float16, 8974, 1100, 320, (192, 256, 2)),
-    (torch.float16, 9822, 1100, 128, (256, 256, 2)),
-    (torch.bfloat16, 9822, 1100, 448, (256, 256, 2)),
-    (torch.float16, 7172, 2304, 128, (320, 256, 2)),
-    (torch.bfloat16, 7172, 2304, 256, (320, 256, 2)),
+    (torch.float16, 10843, 264, 256, (128, 128, 4)),    # as many K tiles as the ring holds
+    (torch.bfloat16, 10843, 264, 448, (128, 128, 4)),   # seven K tiles
+    (torch.float16, 10843, 264, 192, (192, 128, 3)),
+    (torch.bfloat16, 10940, 264, 320, (192, 128, 3)),
+    (torch.float16, 32938, 264, 192, (256, 128, 3)),
+    (torch.bfloat16, 18980, 264, 448, (256, 128, 3)),
+    (torch.float16, 21971, 264, 128, (320, 128, 2)),
+    (torch.bfloat16, 21971, 264, 192, (320, 128, 2)),
+    (torch.float16, 3665, 1100, 192, (128, 256, 3)),
+    (torch.bfloat16, 3859, 1100, 448, (128, 256, 3)),
+    (torch.float16, 7254, 1100, 128, (192, 256, 2)),
+    (torch.bfloat16, 7254, 1100, 320, (192, 256, 2)),
+    (torch.float16, 6963, 1544, 128, (256, 256, 2)),
+    (torch.bfloat16, 27953, 264, 448, (256, 256, 2)),
+    (torch.float16, 32938, 264, 128, (320, 256, 2)),
+    (torch.bfloat16, 26956, 520, 192, (320, 256, 2)),
+    (torch.float16, 10754, 300, 128, (256, 128, 0)),    # rows that end inside a 16-byte piece
+    (torch.bfloat16, 24962, 300, 128, (256, 192, 0)),
+    (torch.float16, 52878, 200, 128, (256, 256, 0)),    # few columns, two K tiles
     (torch.float32, 300, 520, 160, (128, 128, 4)),
     (torch.float32, 6001, 768, 128, (192, 128, 3)),
     (torch.float32, 6001, 768, 64, (256, 128, 0)),      # two K tiles and one round of tiles
@@ -70,14 +73,15 @@ def test_linear_pipelined_shapes(dtype, M, N, K, tile):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,E,tile", [
-    (10781, 128, (320, 128, 2)),
-    (5423, 256, (192, 128, 3)),
-    (2561, 512, (128, 128, 4)),
-    (8073, 512, (256, 256, 2)),
-    (4045, 512, (128, 256, 3)),
-    (5479, 512, (192, 256, 2)),
-    (3305, 640, (256, 128, 3)),     # a boundary between K and V at a multiple of 128
-    (10779, 512, (320, 256, 2)),
+    (4121, 640, (320, 128, 2)),
+    (2690, 512, (192, 128, 3)),
+    (2054, 640, (128, 128, 4)),
+    (9845, 384, (256, 256, 2)),
+    (4068, 512, (128, 256, 3)),
+    (5128, 640, (192, 256, 2)),
+    (3273, 640, (256, 128, 3)),
+    (8202, 640, (320, 256, 2)),
+    (10799, 128, (256, 128, 0)),    # two K tiles, a boundary between K and V at a multiple of 128
 ])
 def test_linear_qkv_pipelined_shapes(M, E, tile, dtype):
     from nestedtensor_amd import _C
@@ -95,7 +99,7 @@ def test_linear_qkv_pipelined_shapes(M, E, tile, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,tile", [
-    (40001, 64, 128, (128, 64, 0)), (40001, 65, 128, (320, 128, 2)), (33000, 33, 64, (128, 64, 0)),
+    (40001, 64, 128, (128, 64, 0)), (40001, 65, 128, (256, 128, 0)), (33000, 33, 64, (128, 64, 0)),
     (70003, 8, 72, (128, 64, 0)), (16385, 64, 8, (128, 64, 0)),
     (33001, 64, 2048, (128, 64, 0)), (33001, 64, 2112, (192, 128, 3)), (33001, 64, 2056, (128, 64, 0))])
 def test_linear_few_columns(M, N, K, tile, dtype):
