@@ -470,8 +470,8 @@ __global__ __launch_bounds__(256) void row_batch_kernel(RowParams p) {
 // of one index of the first) share their entry of the size table and their
 // offset, so a lane group that walks `rows_per_group` consecutive rows decodes
 // once (two divisions, one round trip to the tables) and then only adds strides;
-// the rows are moved two at a time.  For masks of less than 1 MiB and what plane_kernel
-// cannot index.
+// the rows are moved two at a time.  For masks of less than 1 MiB, many constituents of a
+// few short rows and what plane_kernel cannot index.
 template <int EB, int MODE, int kT>
 __global__ __launch_bounds__(256) void row_group_kernel(RowParams p, int rows_per_group) {
   constexpr int kGroups = 256 / kT;
@@ -577,7 +577,8 @@ struct PlaneGeometry {
 // Pad / un-pad, us (TB/s): 16 fp32 images [3, 480..1024, 480..1024] 48.6 / 41.2 -> 42.2 / 36.2
 // (7.2 / 6.3), in fp16 45.9 / 36.7 -> 25.3 / 20.0, 16 fp64 [3, 301..1000, ..] 124 / 112 ->
 // 75.6 / 57.4, 6 fp32 [3, 900..2000, ..] 90.1 / 81.2 -> 53.7 / 46.1; 4 images of 20 to 40
-// pixels 5.8 / 11.6 -> 5.8 / 9.5, so there is no size below which rows are better.
+// pixels 5.8 / 11.6 -> 5.8 / 9.5.  What it does not do well are many constituents of a few
+// short rows (few_short_rows).
 template <int EB, int MODE, int U>
 __global__ __launch_bounds__(256) void plane_kernel(RowParams p, PlaneGeometry g) {
   typedef typename ElemT<EB>::type T;
@@ -887,6 +888,21 @@ static int launch_batch(int eb, const RowParams& p, hipStream_t stream) {
   return check_launch("row_group_kernel");
 }
 
+// Many constituents of a few short rows each: a workgroup of plane_kernel per constituent is
+// mostly idle lanes and costs 0.65 ns (pad) and 0.9 ns (un-pad) whatever it moves, where
+// row_group_kernel gives a wavefront four rows and costs 0.15 to 0.2 ns per row.  100 000
+// constituents, us, rows / flat: un-pad of 1, 2, 3, 5, 6, 8 rows of 8 fp32 20 / 88, 32 / 89,
+// 45 / 89, 75 / 90, 94 / 90, 124 / 90; pad of one row of 8, 200 fp32 23 / 60, 35 / 62, of two of
+// 8, 64 38 / 60, 50 / 62 (30 000 of two of 200: 20 / 20), of three of 16, 64 57 / 61, 70 / 62, of four
+// of 2 57 / 69.  With fewer constituents pad gains nothing (8000: 6 to 9 / 6 to 7), un-pad does
+// down to a few thousand rows (8000 constituents of one to five: 6 to 9 / 8 to 9).
+template <int MODE>
+static bool few_short_rows(const RowParams& p, int64_t rows, int64_t row_bytes) {
+  const int64_t B = p.nrows / rows;
+  if (MODE == kUnpad) return rows <= 5 && row_bytes <= 1024 && p.nrows >= 4096;
+  return rows <= 5 && row_bytes <= (1024 >> (2 * (rows - 1))) && B >= 16384;
+}
+
 // plane_kernel where its 32-bit indexes hold (a padded constituent of less than 2^31
 // elements; larger ones take the row kernels); *done says whether it ran.
 template <int MODE>
@@ -900,6 +916,7 @@ static int try_planes(int eb, const RowParams& p, hipStream_t stream, bool* done
       (reinterpret_cast<uintptr_t>(p.dst) | reinterpret_cast<uintptr_t>(p.src)) % eb != 0) {
     return NT_OK;
   }
+  if (few_short_rows<MODE>(p, M0 * M1, Mlast * p.inner * eb)) return NT_OK;
   constexpr int U = MODE == kPad ? 1 : 2;     // chunks per lane; the other way round and 4 are 5 to 15 % slower on images
   const int64_t per_wg = 256 * U * (16 / eb), elems = M0 * M1 * Mlast * p.inner;
   PlaneGeometry g;

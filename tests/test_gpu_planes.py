@@ -98,3 +98,34 @@ def test_planes_cut_off_a_constituent_past_32_bits():
                                    _C.i64_array(cut), 1, 7, _C.current_stream(DEV)))
     assert torch.equal(padded[0], parts[0][:70, :50])
     assert torch.equal(padded[1, :3], parts[1][:, :50]) and bool((padded[1, 3:] == 7).all())
+
+
+# few short rows of many constituents go row by row: un-pad up to five rows of 1 KiB from 4096
+# rows on, pad one, two, three .. rows of 1 KiB, 256, 64 .. bytes from 16384 constituents on
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.float16, torch.float64])
+@pytest.mark.parametrize("B,rows,row_bytes", [
+    (4095, 1, 1024), (4096, 1, 1024), (820, 5, 1024), (820, 5, 1040), (700, 6, 48), (1024, 4, 8),
+    (16383, 2, 256), (16384, 2, 256), (16384, 2, 272), (16384, 3, 64), (16384, 3, 72), (16384, 1, 1032), (20000, 4, 16)])
+@pytest.mark.parametrize("three", [False, True])
+def test_many_constituents_of_few_short_rows(B, rows, row_bytes, dtype, three):
+    from nestedtensor_amd import _C
+    eb = torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator().manual_seed(B + rows)
+    ext = [rows, row_bytes // eb]
+    sizes = torch.stack([torch.randint(0, n + 1, (B,), generator=g) for n in ext], 1)
+    sizes[0], sizes[-1] = torch.tensor(ext), torch.tensor(ext)
+    if three:
+        ext, sizes = [1] + ext, torch.cat([torch.ones(B, 1, dtype=torch.int64), sizes], 1)
+    sizes_dev, offsets = _C.ops.upload_sizes.default(sizes, DEV)
+    total = int(offsets[-1])
+    packed = torch.randint(1, 100, (total,), generator=g).to(dtype).to(DEV)
+    i = torch.arange(rows, device=DEV).view(1, -1, 1)
+    j = torch.arange(row_bytes // eb, device=DEV).view(1, 1, -1)
+    s0, s1 = (sizes_dev[:, k].view(-1, 1, 1) for k in (-2, -1))
+    inside = (i < s0) & (j < s1)
+    expect = torch.full(inside.shape, 7, dtype=dtype, device=DEV)
+    expect[inside] = packed[(offsets[:-1].view(-1, 1, 1) + i * s1 + j)[inside]]
+    n_ragged = len(ext)
+    padded = torch.ops.nestedtensor.add_padding(packed, sizes_dev, offsets, ext, n_ragged, 7.0)
+    assert torch.equal(padded.view(expect.shape), expect)
+    assert torch.equal(torch.ops.nestedtensor.remove_padding(padded, sizes_dev, offsets, total, n_ragged), packed)
