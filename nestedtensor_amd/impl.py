@@ -84,15 +84,25 @@ class NestedTensorImpl:
             self._opt_sizes = res
         return list(self._opt_sizes)
 
+    def _extents(self, which):
+        """The regular (0), largest (1) or smallest (2) extents, [] where there are none.  Asked
+        on every call of most operators, so the summary is looked at before the table is."""
+        summary = self._summary
+        if summary is None:
+            if self.B == 0 or self.D == 0:
+                return []
+            summary = self._summarize()
+        return list(summary[which])
+
     def max_sizes(self):
         # get_max_size_from_efficient_size (masking.cpp:83-103)
-        return list(self._summarize()[1]) if self.B > 0 and self.D > 0 else []
+        return self._extents(1)
 
     def min_sizes(self):
-        return list(self._summarize()[2]) if self.B > 0 and self.D > 0 else []
+        return self._extents(2)
 
     def has_empty_constituent(self):
-        return self.B > 0 and self.D > 0 and min(self._summarize()[2]) == 0
+        return 0 in self._extents(2)
 
     def shapes(self):
         return [tuple(int(v) for v in row) for row in self.sizes] if self.sizes.dim() > 0 else []

@@ -708,17 +708,17 @@ def _conv1x1_row_major(impl, w2d):
         # a tile is one 128-byte line of every output row; the rows' lines start up to
         # tn - 1 pixels before a multiple of tn, hence one tile more than ceil(P / tn)
         meta[1, 1:] = torch.cumsum(torch.where(pix > 0, (pix + tn - 1) // tn + 1, pix), 0)
-        return _upload_table(meta, buf.device), int(meta[1, B])
+        return _upload_table(meta, buf.device).unbind(0), int(meta[1, B])
 
-    meta_dev, total_tiles = impl.kept(("conv1x1", tn), tables)
+    (pixels_dev, tiles_dev), total_tiles = impl.kept(("conv1x1", tn), tables)
     w2d = w2d.contiguous()
     sizes = impl.sizes.clone()
     sizes[:, 0] = c_out
     out = torch.empty(int(sizes.prod(1).sum()), dtype=buf.dtype, device=buf.device)
     if total_tiles:
         with _C.on_device(buf.device):
-            _C.check(_C.lib.nt_conv1x1_nchw(_C.ptr(buf), _C.ptr(w2d), _C.ptr(out), _C.ptr(meta_dev[0]),
-                                            _C.ptr(meta_dev[1]), B, total_tiles, c_in, c_out,
+            _C.check(_C.lib.nt_conv1x1_nchw(_C.ptr(buf), _C.ptr(w2d), _C.ptr(out), _C.ptr(pixels_dev),
+                                            _C.ptr(tiles_dev), B, total_tiles, c_in, c_out,
                                             _C.dtype_code(buf.dtype), _C.current_stream(buf.device)))
     return NestedTensorImpl(out, sizes)
 
@@ -1001,21 +1001,21 @@ def _transpose_constituents(impl, rows, cols, new_sizes, which):
         meta[0, :B], meta[1, :B] = rows, cols
         meta[2, 1:] = torch.cumsum(tiles, 0)
         meta[3, 1:] = torch.cumsum(rows * cols, 0)
-        return _upload_table(meta, buf.device), int(meta[2, B]), tr, tc
+        return _upload_table(meta, buf.device).unbind(0), int(meta[2, B]), tr, tc
 
-    meta_dev, total_tiles, tr, tc = impl.kept(which, tables)
+    (rows_dev, cols_dev, tiles_dev, offsets_dev), total_tiles, tr, tc = impl.kept(which, tables)
     out = torch.empty_like(buf)
     if total_tiles:
         with _C.on_device(buf.device):
             if tr == 0:
                 _C.check(_C.lib.nt_transpose_ragged_lines(
-                    _C.ptr(buf), _C.ptr(out), _C.ptr(meta_dev[3]), _C.ptr(meta_dev[0]),
-                    _C.ptr(meta_dev[1]), _C.ptr(meta_dev[2]), B, total_tiles, buf.element_size(),
+                    _C.ptr(buf), _C.ptr(out), _C.ptr(offsets_dev), _C.ptr(rows_dev),
+                    _C.ptr(cols_dev), _C.ptr(tiles_dev), B, total_tiles, buf.element_size(),
                     _C.current_stream(buf.device)))
             else:
                 _C.check(_C.lib.nt_transpose_ragged(
-                    _C.ptr(buf), _C.ptr(out), _C.ptr(meta_dev[3]), _C.ptr(meta_dev[0]),
-                    _C.ptr(meta_dev[1]), _C.ptr(meta_dev[2]), B, total_tiles, tr, tc, buf.element_size(),
+                    _C.ptr(buf), _C.ptr(out), _C.ptr(offsets_dev), _C.ptr(rows_dev),
+                    _C.ptr(cols_dev), _C.ptr(tiles_dev), B, total_tiles, tr, tc, buf.element_size(),
                     _C.current_stream(buf.device)))
     res = NestedTensorImpl(out, new_sizes)
     res.share_offsets(impl)       # the constituents keep their extents
