@@ -137,12 +137,14 @@ class NestedTensorImpl:
         is kept per stream (with that nested size itself, so the identity test stays valid),
         and what a capture was given."""
         device = self.buffer.device
-        key = (name, device.index, current_stream_id(device))
+        if device.index is None:                                 # a host tensor
+            _C.require_device(self.buffer, "device metadata")
+        key = (name, current_stream_id(device))                  # _kept is for one device (with_buffer)
         entry = self._kept.get(key)
         if entry is not None and entry[0] is keys:
             return entry[1] if keys is None else self._given_out(entry[1])
         if torch.cuda.is_current_stream_capturing():
-            made = [e[1] for k, e in list(self._kept.items()) if k[:2] == key[:2] and e[0] is keys]
+            made = [e[1] for k, e in list(self._kept.items()) if k[0] == name and e[0] is keys]
             return self._given_out(made[0]) if made else build()
         entry = (keys, build())
         if keys is not None:
@@ -156,27 +158,30 @@ class NestedTensorImpl:
             self._kept["captured", id(table)] = (None, table)
         return table
 
-    def _size_tables(self):
-        """(sizes, offsets) on the device, written by one launch (nt_upload_sizes) on first use."""
-        _C.require_device(self.buffer, "device metadata")
+    def device_tables(self):
+        """(int64 [B, D] mirror of the nested size, int64 [B + 1] element offsets) on the device."""
+        given = self._given
+        if given is not None and given[0] is not None and given[1] is not None:
+            return given
+        return self.kept("sizes", self._write_tables)
+
+    def _write_tables(self):
+        # one launch (nt_upload_sizes) on first use
         if self.sizes.dim() != 2:
             return self.sizes.to(self.buffer.device), None
-        return self.kept("sizes", lambda: _upload_sizes(self.sizes, self.buffer.device))
+        return _upload_sizes(self.sizes, self.buffer.device)
 
     def sizes_dev(self):
-        """int64 [B, D] mirror of the nested size."""
         given = self._given
-        return given[0] if given is not None and given[0] is not None else self._size_tables()[0]
+        return given[0] if given is not None and given[0] is not None else self.kept("sizes", self._write_tables)[0]
 
     def offsets_dev(self):
-        """int64 [B + 1] element offsets, scanned on the device."""
         given = self._given
-        return given[1] if given is not None and given[1] is not None else self._size_tables()[1]
+        return given[1] if given is not None and given[1] is not None else self.kept("sizes", self._write_tables)[1]
 
     def row_offsets_dev(self):
         """int64 [B + 1] offsets counted in rows of the first constituent dim
         (token offsets for a [B, L_i, E] nested tensor)."""
-        _C.require_device(self.buffer, "device metadata")
         return self.kept("rows", lambda: _upload_sizes(self.sizes[:, :1], self.buffer.device)[1])
 
     def last_dim_rows(self):
@@ -186,7 +191,6 @@ class NestedTensorImpl:
         def build():
             rows = self.sizes[:, :-1].prod(1)
             return _upload_sizes(rows.reshape(-1, 1), self.buffer.device)[1], int(rows.sum())
-        _C.require_device(self.buffer, "device metadata")
         return self.kept("last_dim_rows", build)
 
     def attention_schedule(self, kv=None, q_tile=128):
@@ -198,10 +202,9 @@ class NestedTensorImpl:
         first).  Tiles that do not exist are never listed, hence never launched.
         kv: the nested tensor of the keys (None: self-attention)."""
         if kv is None or kv.sizes is self.sizes:
-            kv = self
-        def build():
-            return _attention_schedule(self.sizes, kv.sizes, q_tile, self.buffer.device)
-        return self.kept("work list", build) if kv is self else self.kept("work list of keys", build, kv.sizes)
+            return self.kept("work list", lambda: _attention_schedule(self.sizes, self.sizes, q_tile, self.buffer.device))
+        return self.kept("work list of keys",
+                         lambda: _attention_schedule(self.sizes, kv.sizes, q_tile, self.buffer.device), kv.sizes)
 
     @property
     def _attn_schedule(self):

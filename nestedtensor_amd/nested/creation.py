@@ -80,7 +80,7 @@ def nested_tensor_impl(data, dtype, device, requires_grad, pin_memory, channels_
         # buffer by one operator of the extension (one launch, one metadata upload)
         buffer, sizes, sizes_dev, offsets = _pack_device(tensors)
         impl = NestedTensorImpl(buffer, sizes)
-        impl.adopt_device_metadata(sizes_dev, offsets)
+        impl._given = sizes_dev, offsets      # (what adopt_device_metadata checks holds here)
         if buffer.dtype != dtype or buffer.device != device:
             impl = impl.with_buffer(buffer.to(device, dtype))
         return impl

@@ -123,9 +123,8 @@ def add_padding(impl, padding, with_mask=False, shape=None):
         raise RuntimeError("to_padded_tensor supports at most 3 irregular dimensions.")
     _elem_bytes(impl.buffer.dtype)
     if with_mask:
-        return _add_padding_mask(impl.buffer, impl.sizes_dev(), impl.offsets_dev(), max_size, nrag,
-                                 float(padding))
-    return _add_padding(impl.buffer, impl.sizes_dev(), impl.offsets_dev(), max_size, nrag, float(padding))
+        return _add_padding_mask(impl.buffer, *impl.device_tables(), max_size, nrag, float(padding))
+    return _add_padding(impl.buffer, *impl.device_tables(), max_size, nrag, float(padding))
 
 
 def pad_nt(impl, shape):
@@ -313,7 +312,7 @@ def from_padded_tensor(padded, target):
         return target.with_buffer(torch.empty(0, dtype=padded.dtype, device=padded.device))
     if target.buffer.device != padded.device:
         target = target.with_buffer(torch.empty(0, dtype=padded.dtype, device=padded.device))
-    out = _remove_padding(padded, target.sizes_dev(), target.offsets_dev(), total, nrag)
+    out = _remove_padding(padded, *target.device_tables(), total, nrag)
     return target.with_buffer(out)
 
 
