@@ -52,3 +52,40 @@ def test_tables_are_kept_per_stream():
     for a, b in zip(first, second):
         assert a.data_ptr() != b.data_ptr() and torch.equal(a, b)
     assert second[2].tolist() == [0, 3, 3, 10]
+
+
+def test_graph_replays_between_calls_on_other_streams():
+    # the graph reads the tables and the work list that it was captured with, whatever runs on
+    # another stream and is allocated on its own in between
+    import nestedtensor_amd as nt
+    g = torch.Generator().manual_seed(7)
+    rows = nt.nested_tensor([torch.randn(n, 64, generator=g) for n in (5, 130, 64, 1)], device=DEV, dtype=torch.float16)
+    maps = nt.nested_tensor([torch.randn(16, h, w, generator=g) for h, w in ((9, 17), (4, 30))], device=DEV, dtype=torch.float16)
+    weights = [(torch.randn(s, generator=g) * 0.1).half().to(DEV) for s in ((192, 64), (192,), (64, 64), (64,), (32, 16, 1, 1))]
+
+    def work():
+        y = torch.ops.nestedtensor.min_mha(1, 64, 0.0, False, rows, rows, rows, *weights[:2], 0.125, *weights[2:4])
+        z = torch.conv2d(maps, weights[4]).contiguous(memory_format=torch.channels_last)
+        return y._impl.buffer, rows.to_padded_tensor(0), z._impl.buffer, maps.to_padded_tensor(0)
+
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    work()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        work()
+        with torch.cuda.graph(graph, stream=side):
+            outs = work()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        expect = work()
+        with torch.cuda.stream(side):
+            junk = [torch.full((n,), -1, dtype=torch.int64, device=DEV) for n in (8, 16, 40, 64, 200, 600) for _ in range(20)]
+        torch.cuda.synchronize()
+        for t in (rows, maps):
+            t._impl.buffer.add_(0.5)
+        graph.replay()
+        torch.cuda.synchronize()
+        expect = work()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, expect))
+        del junk
