@@ -39,9 +39,10 @@
 // inside their image with their whole window, and those load and store without a look at
 // the bounds; an output row's position moves on by one addition, and the half-dword
 // shift of a window is the variable count of v_alignbit.  Stores go past the L2, which
-// a result of this size does not fit.  64 -> 256 channels on 589 481 pixels (377 MB)
-// 131.5 -> 100.4 us, 32 -> 128 on 1.35 M (431 MB) 119.5 -> 86 us, a copy of the same bytes
-// taking 71 and 80 us; the stores alone are a third of it.
+// a result of this size does not fit.  On input that no cache holds 64 -> 256 channels on
+// 591 264 pixels (378 MB) 129.9 -> 111.0 us = 3.4 TB/s, 32 -> 128 on 1.4 M (448 MB) 118.5 -> 101.7,
+// 128 -> 64 on 128 437 (49 MB) 45.8 -> 40.7; on input that lies in the memory-side cache 128.5 ->
+// 102.2, 119.4 -> 81.9 and 42.8 -> 38.6.
 //
 // Persistent workgroups (the weight is loaded into LDS once each) of WAVES
 // wavefronts, and every wavefront works on tiles of its own with its own X tile
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
         }
       __builtin_amdgcn_wave_barrier();
       // every row takes the 64 pixels of its own line k out of the strip
-auto rows = [&](auto whole_c) __attribute__((always_inline)) {
+      auto rows = [&](auto whole_c) __attribute__((always_inline)) {
         constexpr bool WHOLE = decltype(whole_c)::value;
 #pragma unroll
         for (int ps = 0; ps < 4; ++ps) {

@@ -15,16 +15,17 @@
 // banks; any other K takes a register-staged loop with padded LDS rows and
 // element-wise tails.
 //
-// Two kernels.  phased_kernel, for problems that fill the chip and K of at least two
-// whole K tiles: eight wavefronts in two groups half a phase apart, tile shapes of 128
-// to 320 rows by 128 or 256 columns, one of them picked per problem so that the tiles
-// fill whole rounds of the CUs.  linear_kernel takes everything else: a problem with
-// fewer 256x128 tiles than half the CUs (the query and output projections of
-// cross-attention, a few thousand rows) gets 128x64 tiles of four wavefronts, or 128x128
-// when those would not fit in one round (its duration is one tile's life, and a quarter
-// of a tile on four times as many CUs ends sooner: 3200 x 512 x 512 10.6 -> 6.3 us; the
-// fused in-projection of a layer of a few hundred tokens 16.0 -> 11.6 us), at most 64
-// columns 128x64 tiles, short or ragged K tiles of 256 rows by 128, 192 or 256 columns.
+// Two kernels.  phased_kernel, for problems that fill the chip and K of at least two whole
+// K tiles: eight wavefronts in two groups half a phase apart, tile shapes of 128 to 320 rows
+// by 128 or 256 columns.  linear_kernel, whose wavefronts all do the same thing at the same
+// time: a problem with fewer 256x128 tiles than half the CUs (the query and output
+// projections of cross-attention, a few thousand rows) gets 128x64 tiles of four wavefronts,
+// or 128x128 when those would not fit in one round (its duration is one tile's life, and a
+// quarter of a tile on four times as many CUs ends sooner: 3200 x 512 x 512 10.6 -> 6.3 us;
+// the fused in-projection of a layer of a few hundred tokens 16.0 -> 11.6 us), at most 64
+// columns 128x64 tiles, ragged K tiles of 256 rows by 128, 192 or 256 columns, and those
+// also where few K tiles or rows that end inside a 16-byte piece leave phased_kernel
+// nothing to gain (choose_tile).
 //
 // Epilogues:
 //   plain  - C row-major + bias;
@@ -923,8 +924,8 @@ static int compute_units(int* n) {
 // `pieces` for a round of stores to rows that are no whole 16-byte pieces.  Fitted on the
 // shape that is fastest of all in 903 problems (72 to 8192 columns, K 128 to 4096, 2500 to
 // 200000 rows) and not on single times: what it picks takes 1.010 times the fastest shape's
-// time on average, 1.07 at the 95th percentile.  Without the shapes of linear_kernel, with 4 us for any
-// further round and aligned rows throughout it was 1.030 and 1.17, and one problem in five
+// time on average, 1.06 at the 95th percentile.  Without the shapes of linear_kernel, with 4 us
+// for any further round and whole pieces throughout it was 1.031 and 1.16, and one problem in five
 // (two to six K tiles, or rows that end inside a piece) lost 3 to 40 % against linear_kernel.
 struct TileCost {
   double alone, full, first, round, pieces;
