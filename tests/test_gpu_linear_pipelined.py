@@ -58,10 +58,17 @@ def _case(M, N, K, dtype):
     (torch.float32, 6001, 768, 128, (192, 128, 3)),
     (torch.float32, 6001, 768, 64, (256, 128, 0)),      # two K tiles and one round of tiles
     (torch.float32, 20000, 520, 64, (256, 256, 2)),
+    # remainders and depths on whatever is picked
+    (torch.float16, 6430, 520, 256, None), (torch.bfloat16, 6430, 520, 448, None), (torch.float16, 6536, 520, 192, None),
+    (torch.bfloat16, 6536, 520, 320, None), (torch.float16, 9822, 520, 192, None), (torch.float16, 9822, 520, 320, None),
+    (torch.float16, 7172, 1100, 192, None), (torch.bfloat16, 6430, 520, 128, None), (torch.float16, 8073, 768, 192, None),
+    (torch.float16, 8073, 768, 448, None), (torch.bfloat16, 8974, 1100, 128, None), (torch.float16, 8974, 1100, 320, None),
+    (torch.float16, 9822, 1100, 128, None), (torch.bfloat16, 9822, 1100, 448, None), (torch.float16, 7172, 2304, 128, None),
+    (torch.bfloat16, 7172, 2304, 256, None),
 ])
 def test_linear_pipelined_shapes(dtype, M, N, K, tile):
     from nestedtensor_amd import ops
-    assert _tile(M, N, K, dtype) == tile
+    assert tile is None or _tile(M, N, K, dtype) == tile
     x, w, b, ref, bound = _case(M, N, K, dtype)
     assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
     relu = ops.linear(x, w, b, "relu").double()
@@ -82,10 +89,12 @@ def test_linear_pipelined_shapes(dtype, M, N, K, tile):
     (3273, 640, (256, 128, 3)),
     (8202, 640, (320, 256, 2)),
     (10799, 128, (256, 128, 0)),    # two K tiles, a boundary between K and V at a multiple of 128
+    (10781, 128, None), (5423, 256, None), (2561, 512, None), (8073, 512, None), (4045, 512, None), (5479, 512, None),
+    (3305, 640, None), (10779, 512, None),
 ])
 def test_linear_qkv_pipelined_shapes(M, E, tile, dtype):
     from nestedtensor_amd import _C
-    assert _tile(M, 3 * E, E, dtype, 2 * E) == tile
+    assert tile is None or _tile(M, 3 * E, E, dtype, 2 * E) == tile
     x, w, b, ref, bound = _case(M, 3 * E, E, dtype)
     ld = (M + 72 + 7) // 8 * 8
     qk = torch.empty(M, 2 * E, dtype=dtype, device=DEV)
