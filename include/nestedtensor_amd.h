@@ -241,7 +241,8 @@ int nt_linear(const void* A, int64_t lda, const void* W, const void* bias, void*
 
 /* The tile that nt_linear and its variants run a problem on, for num_cus compute units
  * (0: those of the current device): tile[0] rows by tile[1] columns, tile[2] K tiles of 128
- * bytes in flight (0: not the pipelined kernel).  n_split: the first column that is
+ * bytes in flight (0: not the pipelined kernel; -1: fp32 operands split into three bf16
+ * parts for the bf16 matrix instruction).  n_split: the first column that is
  * written transposed, -1 where there is none; ldc: the row stride of the result (of the
  * transposed one for n_split 0). */
 int nt_linear_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldc, int64_t n_split, int dtype,

@@ -15,7 +15,8 @@
 // banks; any other K takes a register-staged loop with padded LDS rows and
 // element-wise tails.
 //
-// Two kernels.  phased_kernel, for problems that fill the chip and K of at least two whole
+// Three kernels.  split_kernel, fp32 of at least 192 k: operands split into three bf16 parts
+// for the bf16 instruction.  phased_kernel, for problems that fill the chip and K of at least two whole
 // K tiles: eight wavefronts in two groups half a phase apart, tile shapes of 128 to 320 rows
 // by 128 or 256 columns.  linear_kernel, whose wavefronts all do the same thing at the same
 // time: a problem with fewer 256x128 tiles than half the CUs (the query and output
@@ -851,16 +852,15 @@ __device__ __forceinline__ void phased_tile(const GemmArgs<T>& a, int64_t m0, in
 // the tile list (equal lengths up to one tile, so no XCD runs a round more than the
 // others).  The list walks bands of four row tiles, column panel by column panel: the
 // tiles an XCD runs at a time share few rows of A and few panels of W, which its L2
-// serves.
-template <typename T, class Cfg, int EPI>
-__global__ __launch_bounds__(512, 2) void phased_kernel(GemmArgs<T> a) {
-  extern __shared__ __align__(16) char lds[];
-  const int tiles_m = (int)((a.M + Cfg::kBM - 1) / Cfg::kBM);
-  const int tiles_n = (int)((a.N + Cfg::kBN - 1) / Cfg::kBN);
+// serves.  False: the workgroup has no tile.
+template <int BM, int BN>
+__device__ __forceinline__ bool tile_of_workgroup(int64_t M, int64_t N, int64_t* m0, int64_t* n0) {
+  const int tiles_m = (int)((M + BM - 1) / BM);
+  const int tiles_n = (int)((N + BN - 1) / BN);
   const int total = tiles_m * tiles_n;
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
   const int share = total >> 3, more = total & 7;
-  if (local >= share + (xcd < more ? 1 : 0)) return;
+  if (local >= share + (xcd < more ? 1 : 0)) return false;
   const int id = xcd * share + (xcd < more ? xcd : more) + local;
   constexpr int kBand = 4;
   const int band = id / (kBand * tiles_n);
@@ -868,8 +868,16 @@ __global__ __launch_bounds__(512, 2) void phased_kernel(GemmArgs<T> a) {
   const int rows = tiles_m - band * kBand < kBand ? tiles_m - band * kBand : kBand;
   const int tn = in_band / rows;
   const int tm = band * kBand + in_band - tn * rows;
-  const int64_t m0 = (int64_t)tm * Cfg::kBM;
-  const int64_t n0 = (int64_t)tn * Cfg::kBN;
+  *m0 = (int64_t)tm * BM;
+  *n0 = (int64_t)tn * BN;
+  return true;
+}
+
+template <typename T, class Cfg, int EPI>
+__global__ __launch_bounds__(512, 2) void phased_kernel(GemmArgs<T> a) {
+  extern __shared__ __align__(16) char lds[];
+  int64_t m0, n0;
+  if (!tile_of_workgroup<Cfg::kBM, Cfg::kBN>(a.M, a.N, &m0, &n0)) return;
   if constexpr (EPI == kEpiQkv) {
     if (n0 >= a.n_split) {
       phased_tile<T, Cfg, true, false>(a, m0, n0, lds);
@@ -893,6 +901,332 @@ static int launch_phased(const GemmArgs<T>& a, hipStream_t stream) {
   hipLaunchKernelGGL((phased_kernel<T, Cfg, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds_bytes, stream,
                      a);
   return check_launch("phased_kernel");
+}
+
+// ---- fp32 products on the bf16 matrix instruction ---------------------------------
+//
+// The fp32 matrix instruction does a sixteenth of the bf16 one's work per cycle, and a
+// product of fp32 operands is bound by it (phased_kernel reached 0.8 of its rate).  An fp32
+// number is the sum of three bf16 ones (24 significant bits in three of 8, each the rounded
+// rest of the one before: exact), so a product of two is nine bf16 products, of which the
+// six largest are kept: what is left out is below 2^-25 of |x| |w|, half the rounding of one
+// fp32 product.  (Splitting by rounding and rest is Dekker's; products of bf16 numbers are exact
+// in the fp32 accumulators.)  The error against 64 bits is smaller than the fp32
+// instruction's, which rounds more partial sums: 2.1e-7 against 2.5e-7 of the 2-norm at K 768,
+// 2.7e-7 against 3.1e-7 at 1024, 7.8e-8 against 9.2e-8 at 256.
+//
+// The operands are split on the way from global memory to LDS, once per tile: a step of 16
+// k of all its rows is fetched into registers kDepth steps ahead, split between the matrix
+// instructions of the step before its own and written to the other of two tile buffers.
+// Bound by the matrix pipe at the clock that random operands leave (8040 x 2304 x 768 on
+// zeros 111 us, on N(0, 1) operands 137 to 160); before, on the fp32 instruction: 260.
+// 8040 x 768 x 768 76-84 -> 52-56, 20000 x 3072 x 1024 900 -> 545, 2000 x 1536 x 512 39.5 -> 24,
+// 300 x 768 x 256 19.4 -> 8.9, and 0.49 of the time over 174 products of K 192 to 2048 (0.74 at most).
+template <int GM_, int GN_, int NI_, int NJ_, int DEPTH_>
+struct SplitCfg {
+  static constexpr int kGM = GM_, kGN = GN_, kNI = NI_, kNJ = NJ_;   // wavefronts, 32 x 32 blocks of each
+  static constexpr int kDepth = DEPTH_;                              // steps fetched ahead of the one written to LDS
+  static_assert(GM_ * GN_ == 8, "eight wavefronts");
+  static constexpr int kBM = GM_ * NI_ * 32, kBN = GN_ * NJ_ * 32;
+  static constexpr int kBlocks = (kBM + kBN) / 32;
+  static constexpr int kBufBytes = kBlocks * 3 * 1024;               // 16 k of all rows, three parts
+  static constexpr int kLdsBytes = 2 * kBufBytes;
+  static_assert(8 * strip_bytes<float, NI_, NJ_, false>() <= kLdsBytes, "strips must fit");
+  static_assert(kLdsBytes + kBN * 4 + 16 <= 160 * 1024, "tile buffers must fit the LDS");
+};
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// 32-row blocks of A and W lie in LDS as three parts of 1 KiB, a part as the 16-byte pieces
+// (k 0..3 and 8..11, or, half 1, the others) of the 32 rows one after the other.  In the
+// second half rows trade places by eights, so that sixteen consecutive lanes fall into
+// distinct banks both as a fragment's rows (reads) and as two pieces of eight rows (writes).
+// The order of the 16 k is the same for A and W, which is all that the product asks for.
+__device__ __forceinline__ int split_slot(int half, int row) { return half * 512 + ((row ^ (half << 3)) << 4); }
+
+// One thread's part of a K step: FLOATS (8, 4 or 2) consecutive values of a row of A or W,
+// or with 8 two runs of four eight apart, their three parts written to LDS FLOATS * 2 bytes
+// each.
+template <int FLOATS, int DEPTH>
+struct SplitPiece {
+  const char* base;      // of A or W at the first row of the tile, the same in a wavefront
+  unsigned off;          // of the row and the thread's place in it, in bytes
+  unsigned dst;          // in a tile buffer
+  uint32_t raw[DEPTH][FLOATS];
+
+  __device__ __forceinline__ void place(const GemmArgs<float>& a, int64_t m0, int64_t n0, int a_blocks, int block,
+                                        int row_in_block, int piece) {
+    const bool is_a = block < a_blocks;
+    int64_t row = (is_a ? block : block - a_blocks) * 32 + row_in_block;
+    const int64_t left = is_a ? a.M - m0 : a.N - n0;
+    row = row < left ? row : left - 1;               // only feeds accumulators that are not stored
+    base = reinterpret_cast<const char*>(is_a ? a.A + m0 * a.lda : a.W + n0 * a.K);
+    off = (unsigned)(row * (is_a ? a.lda : a.K) * 4) + piece * (FLOATS == 8 ? 16 : FLOATS * 4);
+    // the four k that the piece begins with or lies in, for 8 floats: 0..3 or 4..7
+    const int four = FLOATS == 2 ? piece >> 1 : piece;
+    dst = block * 3072 + split_slot(four & 1, row_in_block) + (four >> 1) * 8 + (FLOATS == 2 ? (piece & 1) * 4 : 0);
+  }
+  __device__ __forceinline__ void fetch(int step, int slot) {
+    const char* src = base + (int64_t)step * 64;
+    __builtin_memcpy(raw[slot], src + off, FLOATS < 8 ? FLOATS * 4 : 16);
+    if constexpr (FLOATS == 8) __builtin_memcpy(raw[slot] + 4, src + off + 32, 16);
+  }
+  __device__ __forceinline__ void put(char* buf, int slot, u16x2& smallest) const {
+    uint32_t part[3][FLOATS / 2];
+#pragma unroll
+    for (int e = 0; e < FLOATS / 2; ++e) {
+      float x = __builtin_bit_cast(float, raw[slot][2 * e]);
+      float y = __builtin_bit_cast(float, raw[slot][2 * e + 1]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const f32x2 v = {x, y};
+        const uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+        if (p < 2) {
+          x -= __builtin_bit_cast(float, pair << 16);
+          y -= __builtin_bit_cast(float, pair & 0xffff0000u);
+        }
+        if (p == 0) {
+          const u16x2 magnitude = __builtin_bit_cast(u16x2, pair) * (uint16_t)2 - (uint16_t)1;   // of a zero: largest
+          smallest = __builtin_elementwise_min(smallest, magnitude);
+        }
+        part[p][e] = pair;
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      __builtin_memcpy(__builtin_assume_aligned(buf + dst + p * 1024, FLOATS * 2), part[p], FLOATS * 2);
+  }
+};
+
+template <class Cfg, bool ACT>
+__device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0, int64_t n0, char* lds) {
+  constexpr int NI = Cfg::kNI, NJ = Cfg::kNJ, kDepth = Cfg::kDepth;
+  constexpr int kUnits = Cfg::kBlocks / 8, kTail4 = Cfg::kBlocks & 4, kTail2 = Cfg::kBlocks & 2;
+  static_assert(Cfg::kBlocks % 2 == 0, "blocks are dealt to the wavefronts whole, by halves and by quarters");
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / Cfg::kGN, wn = wave % Cfg::kGN;
+  const int l32 = lane & 31;
+  const int g = lane >> 5;
+
+  acc16 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+  float* lds_bias = reinterpret_cast<float*>(lds + Cfg::kLdsBytes);
+  int* lds_tiny = reinterpret_cast<int*>(lds_bias + Cfg::kBN);
+  if (tid < Cfg::kBN) {
+    const int64_t col = n0 + tid;
+    lds_bias[tid] = (a.bias && col < a.N) ? a.bias[col] : 0.0f;
+  }
+  if (tid == 0) *lds_tiny = 0;
+
+  const int n_steps = (int)(a.K / 16);
+  constexpr int kABlocks = Cfg::kBM / 32;
+  SplitPiece<8, kDepth> unit[kUnits > 0 ? kUnits : 1];
+  SplitPiece<4, kDepth> half;
+  SplitPiece<2, kDepth> quarter;
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u)
+    unit[u].place(a, m0, n0, kABlocks, wave + 8 * u, lane >> 1, lane & 1);
+  if (kTail4)
+    half.place(a, m0, n0, kABlocks, 8 * kUnits + (wave >> 1), (wave & 1) * 16 + (lane >> 2), lane & 3);
+  if (kTail2)
+    quarter.place(a, m0, n0, kABlocks, 8 * kUnits + kTail4 + (wave >> 2), (wave & 3) * 8 + (lane >> 3), lane & 7);
+  u16x2 smallest = {0xffff, 0xffff};
+
+  constexpr int kPuts = kUnits + (kTail4 ? 1 : 0) + (kTail2 ? 1 : 0);
+  auto fetch = [&](int u, int step, int slot) __attribute__((always_inline)) {
+    step = step < n_steps ? step : n_steps - 1;          // past the end: not used
+    if (u < kUnits) unit[u < kUnits ? u : 0].fetch(step, slot);
+    else if (u == kUnits && kTail4) half.fetch(step, slot);
+    else quarter.fetch(step, slot);
+  };
+  auto put = [&](int u, char* buf, int slot) __attribute__((always_inline)) {
+    if (u < kUnits) unit[u < kUnits ? u : 0].put(buf, slot, smallest);
+    else if (u == kUnits && kTail4) half.put(buf, slot, smallest);
+    else quarter.put(buf, slot, smallest);
+  };
+  auto publish = [] __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // the pieces of step s wait in slot s % kDepth
+#pragma unroll
+  for (int d = 0; d < kDepth; ++d)
+#pragma unroll
+    for (int u = 0; u < kPuts; ++u) fetch(u, d, d);
+#pragma unroll
+  for (int u = 0; u < kPuts; ++u) {
+    put(u, lds, 0);
+    fetch(u, kDepth, 0);
+  }
+  publish();
+
+  const char* a_lds = lds + wm * NI * 3072 + split_slot(g, l32);
+  const char* w_lds = lds + (kABlocks + wn * NJ) * 3072 + split_slot(g, l32);
+  bf16x8 fa[2][3], fb[NJ][3];
+  auto read_a = [&](bf16x8 (&f)[3], int buf, int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) f[p] = *reinterpret_cast<const bf16x8*>(a_lds + buf + i * 3072 + p * 1024);
+  };
+  read_a(fa[0], 0, 0);
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) fb[j][p] = *reinterpret_cast<const bf16x8*>(w_lds + j * 3072 + p * 1024);
+
+  int cur = 0;
+  auto one_step = [&](int step, int slot) __attribute__((always_inline)) {   // slot: that of the next step
+    const int other = Cfg::kBufBytes - cur;
+    bf16x8 fb_next[NJ][3];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      // the splits of the next step, dealt out over the blocks in front of the last
+      constexpr int kSlots = NI > 1 ? NI - 1 : 1;
+#pragma unroll
+      for (int u = 0; u < kPuts; ++u)
+        if (u * kSlots / kPuts == i) {
+          put(u, lds + other, slot);
+          fetch(u, step + 1 + kDepth, slot);
+        }
+      if (i + 1 < NI) {
+        read_a(fa[(i + 1) & 1], cur, i + 1);
+      } else {
+        // Every fragment of this step is read and every piece of the next written: the one
+        // barrier of a step, with a block's products left to cover the first reads behind it.
+        publish();
+        read_a(fa[(i + 1) & 1], other, 0);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            fb_next[j][p] = *reinterpret_cast<const bf16x8*>(w_lds + other + j * 3072 + p * 1024);
+      }
+      // smallest products first
+      constexpr int kPa[6] = {0, 1, 2, 1, 0, 0}, kPw[6] = {2, 1, 0, 0, 1, 0};
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          acc[i][j] = Mma<__bf16>::run(fb[j][kPw[p]], fa[i & 1][kPa[p]], acc[i][j]);
+      if (i + 1 < NI) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // the next block's reads first
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) fb[j][p] = fb_next[j][p];
+    if (NI & 1) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) fa[0][p] = fa[1][p];
+    }
+    cur = other;
+  };
+  int step = 0;
+  for (; step + kDepth <= n_steps; step += kDepth) {
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) one_step(step + d, (d + 1) % kDepth);
+  }
+#pragma unroll
+  for (int d = 0; d + 1 < kDepth; ++d)
+    if (step + d < n_steps) one_step(step + d, (d + 1) % kDepth);
+
+  // A magnitude below 2^-100 other than zero: its third part may be lost below the smallest
+  // bf16 number.  A result that is no finite number: an infinity or NaN went in (their rests
+  // are NaN), a first part rounded up to infinity, or the sum overflowed.  Both are computed
+  // again by the fp32 instruction.
+  constexpr uint16_t kTiny = 2 * (27 << 7) - 1;
+  if (smallest[0] < kTiny || smallest[1] < kTiny) *lds_tiny = 1;
+  float probe = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) probe = fmaf(acc[i][j][e], 0.0f, probe);
+  __syncthreads();
+  char* strip = lds + wave * strip_bytes<float, NI, NJ, false>();
+  if (*lds_tiny == 0 && __ballot(probe != probe) == 0) {
+    store_tile<float, NI, NJ, false, ACT>(a, acc, m0 + wm * (32 * NI), n0, wn * (32 * NJ), strip, lds_bias);
+    return;
+  }
+#pragma unroll 1
+  for (int i = 0; i < NI; ++i) {
+    acc16 row[1][NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) row[0][j][e] = 0.0f;
+    const int64_t m = m0 + (wm * NI + i) * 32 + l32;
+    const float* ap = a.A + (m < a.M ? m : a.M - 1) * a.lda + g * 4;
+    const float* wp[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int64_t n = n0 + (wn * NJ + j) * 32 + l32;
+      wp[j] = a.W + (n < a.N ? n : a.N - 1) * a.K + g * 4;
+    }
+    f32x4 xa[2], xw[NJ][2];
+    auto load = [&](int64_t k) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        xa[h] = __builtin_bit_cast(f32x4, load16_unaligned(reinterpret_cast<const char*>(ap + k + 8 * h)));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          xw[j][h] = __builtin_bit_cast(f32x4, load16_unaligned(reinterpret_cast<const char*>(wp[j] + k + 8 * h)));
+      }
+    };
+    load(0);
+#pragma unroll 1
+    for (int64_t k = 0; k < a.K; k += 16) {
+      f32x4 ya[2], yw[NJ][2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        ya[h] = xa[h];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) yw[j][h] = xw[j][h];
+      }
+      load(k + 16 < a.K ? k + 16 : 0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) row[0][j] = Mma<float>::run(yw[j][h], ya[h], row[0][j]);
+    }
+    store_tile<float, 1, NJ, false, ACT>(a, row, m0 + (wm * NI + i) * 32, n0, wn * (32 * NJ), strip, lds_bias);
+  }
+}
+
+template <class Cfg, int EPI>
+__global__ __launch_bounds__(512, 2) void split_kernel(GemmArgs<float> a) {
+  extern __shared__ __align__(16) char lds[];
+  int64_t m0, n0;
+  if (!tile_of_workgroup<Cfg::kBM, Cfg::kBN>(a.M, a.N, &m0, &n0)) return;
+  split_tile<Cfg, EPI == kEpiAct>(a, m0, n0, lds);
+}
+
+template <class Cfg, int EPI>
+static int launch_split(const GemmArgs<float>& a, hipStream_t stream) {
+  const int64_t tiles = ((a.M + Cfg::kBM - 1) / Cfg::kBM) * ((a.N + Cfg::kBN - 1) / Cfg::kBN);
+  const int lds_bytes = Cfg::kLdsBytes + Cfg::kBN * (int)sizeof(float) + 16;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_kernel<Cfg, EPI>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return fail(NT_ERR_HIP, "linear: %s", hipGetErrorString(e));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((split_kernel<Cfg, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds_bytes, stream, a);
+  return check_launch("split_kernel");
 }
 
 // WAVES_M, WAVES_N, WM, WN, K-tile bytes per row
@@ -978,8 +1312,41 @@ static int pick_phased_f32(int64_t M, int64_t N, int64_t nk, int num_cus) {
   return best;
 }
 
-// What a problem runs on: a shape of linear_kernel or, kTilePhased + c, kPhasedShapes[c].
-enum { kTile256x128, kTile256x192, kTile256x256, kTile128x64, kTile128x128, kTilePhased };
+// Tiles of split_kernel and what one takes, in microseconds per 16 k; fitted like the above on
+// 174 products (16 to 60000 rows, K 192 to 2048): what it picks takes 1.002 times the fastest
+// shape's time on average, 1.03 at most.
+struct SplitShape {
+  int bm, bn;
+  TileCost cost;
+};
+static const SplitShape kSplitShapes[] = {
+    {320, 256, {2.167, 2.421, 15.83, 1.72, 0.0}},
+    {256, 256, {1.58, 1.951, 17.17, 7.19, 0.0}},
+    {192, 128, {0.752, 0.842, 5.86, 2.52, 0.0}},
+    {128, 128, {0.552, 0.623, 4.1, 2.25, 0.0}},
+    {64, 128, {0.451, 0.368, 1.33, 1.33, 0.0}},
+    {128, 64, {0.306, 0.361, 4.55, 0.974, 0.0}}};
+constexpr int kSplitCount = (int)(sizeof(kSplitShapes) / sizeof(kSplitShapes[0]));
+
+static int pick_split(int64_t M, int64_t N, int64_t K, int num_cus) {
+  int best = 0;
+  double best_us = 0.0;
+  for (int c = 0; c < kSplitCount; ++c) {
+    const SplitShape& s = kSplitShapes[c];
+    const int64_t tiles = ((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+    const double us = tile_time(s.cost, 0.0, tiles, K / 16, false, num_cus);
+    if (c == 0 || us < best_us) {
+      best = c;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// What a problem runs on: a shape of linear_kernel or, kTilePhased + c, kPhasedShapes[c] or,
+// kTileSplit + c, kSplitShapes[c].
+enum { kTile256x128, kTile256x192, kTile256x256, kTile128x64, kTile128x128, kTilePhased,
+       kTileSplit = kTilePhased + kPhasedCount };
 
 // The tile of M x N x K; row-major A has lda elements per row, columns from n_split on go
 // transposed into Vt (n_split = 0: to either side of no boundary).  qkv: there are such
@@ -1009,6 +1376,12 @@ static int choose_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t n_s
   // would not fit its LDS.)
   constexpr int64_t kMaxSpan = (int64_t(1) << 32) - 1;
   const int64_t row_bytes = K * elem_bytes;
+  // fp32 goes to the bf16 instruction in whole steps of 16 k.  Products of less than 192 k, of
+  // which the store of the result is the larger part, stay on the fp32 instruction.
+  if (!half && !qkv && K % 16 == 0 && K >= 192 && lda * elem_bytes * 320 < kMaxSpan && row_bytes * 256 < kMaxSpan &&
+      (M / 64 + 1) * (N / 64 + 1) < (int64_t(1) << 30)) {
+    return kTileSplit + pick_split(M, N, K, num_cus);
+  }
   if ((half || !qkv) && row_bytes % 128 == 0 && row_bytes >= 2 * 128 && lda * elem_bytes * 320 < kMaxSpan &&
       row_bytes * 256 < kMaxSpan && (M / 64 + 1) * (N / 64 + 1) < (int64_t(1) << 30)) {
     const int64_t nk = row_bytes / 128;
@@ -1083,6 +1456,16 @@ static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
       case kTilePhased + 5: return launch_phased<T, PhasedCfg<T, 3, 1, 3>, EPI>(a, stream);
       case kTilePhased + 6: return launch_phased<T, PhasedCfg<T, 4, 1, 3>, EPI>(a, stream);
       case kTilePhased + 7: return launch_phased<T, PhasedCfg<T, 5, 1, 2>, EPI>(a, stream);
+    }
+  }
+  if constexpr (sizeof(T) == 4 && EPI != kEpiQkv) {
+    switch (tile) {
+      case kTileSplit + 0: return launch_split<SplitCfg<2, 4, 5, 2, 1>, EPI>(a, stream);
+      case kTileSplit + 1: return launch_split<SplitCfg<2, 4, 4, 2, 1>, EPI>(a, stream);
+      case kTileSplit + 2: return launch_split<SplitCfg<2, 4, 3, 1, 2>, EPI>(a, stream);
+      case kTileSplit + 3: return launch_split<SplitCfg<2, 4, 2, 1, 4>, EPI>(a, stream);
+      case kTileSplit + 4: return launch_split<SplitCfg<2, 4, 1, 1, 2>, EPI>(a, stream);
+      case kTileSplit + 5: return launch_split<SplitCfg<4, 2, 1, 1, 2>, EPI>(a, stream);
     }
   }
   if constexpr (sizeof(T) == 2) {
@@ -1178,6 +1561,12 @@ extern "C" int nt_linear_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int6
   const int elem_bytes = dtype == NT_F32 ? 4 : 2;
   const int c = choose_tile(M, N, K, lda, qkv ? n_split : 0, qkv, ldc * elem_bytes % 16 != 0, elem_bytes, num_cus);
   if (c < 0) return fail(NT_ERR_UNSUPPORTED, "linear: QKV split %lld is not a multiple of a column tile", (long long)n_split);
+  if (c >= kTileSplit) {
+    tile[0] = kSplitShapes[c - kTileSplit].bm;
+    tile[1] = kSplitShapes[c - kTileSplit].bn;
+    tile[2] = -1;
+    return NT_OK;
+  }
   static const int kShapes[kTilePhased][2] = {{256, 128}, {256, 192}, {256, 256}, {128, 64}, {128, 128}};
   tile[0] = c >= kTilePhased ? 64 * kPhasedShapes[c - kTilePhased].ni : kShapes[c][0];
   tile[1] = c >= kTilePhased ? 128 * kPhasedShapes[c - kTilePhased].nj : kShapes[c][1];

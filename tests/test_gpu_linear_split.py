@@ -1,0 +1,116 @@
+"""fp32 projections on the bf16 matrix instruction: every tile shape with row, column and
+step remainders, operand rows that lie anywhere, and what the split cannot carry
+(infinities, NaN, magnitudes next to the largest and the smallest fp32 numbers)."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+
+
+def _tile(M, N, K):
+    from nestedtensor_amd import _C
+    tile = (ctypes.c_int * 3)()
+    _C.check(_C.lib.nt_linear_tile(M, N, K, K, N, -1, _C.dtype_code(torch.float32), 0, tile))
+    return tuple(tile)
+
+
+def _case(M, N, K, seed=0):
+    g = torch.Generator("cuda").manual_seed(M + 3 * N + 7 * K + seed)
+    x = torch.randn(M, K, device=DEV, generator=g)
+    w = torch.randn(N, K, device=DEV, generator=g) * 0.25
+    b = torch.randn(N, device=DEV, generator=g)
+    return x, w, b
+
+
+def _bound(x, w, ref):
+    # six products per k; were the sums of an instruction rounded after every four k, 1.5 K
+    # roundings of partial sums below sum |x||w|; half a rounding per k for the products left
+    # out; the bias and the store
+    return (x.double().abs() @ w.double().abs().t()) * (2 * x.size(1) * 2.0 ** -24) + ref.abs() * 2.0 ** -24 + 1e-30
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (1, 1, 192, (64, 128, -1)), (3, 130, 192, (64, 128, -1)), (64, 129, 208, (64, 128, -1)),
+    (1000, 300, 224, (64, 128, -1)), (500, 2050, 2064, (128, 64, -1)), (60001, 33, 192, (128, 64, -1)),
+    (2000, 1536, 512, (128, 128, -1)), (2001, 1537, 528, (128, 128, -1)), (129, 12000, 208, (128, 128, -1)),
+    (8040, 768, 768, (192, 128, -1)), (20001, 1026, 208, (192, 128, -1)), (16001, 1025, 1040, (192, 128, -1)),
+    (16001, 1024, 208, (256, 256, -1)), (16001, 1022, 240, (256, 256, -1)),
+    (8040, 2304, 768, (320, 256, -1)), (8167, 2300, 304, (320, 256, -1)),
+])
+def test_linear_split_shapes(M, N, K, tile):
+    from nestedtensor_amd import ops
+    assert _tile(M, N, K)[2] == -1 and (tile is None or _tile(M, N, K) == tile)
+    x, w, b = _case(M, N, K)
+    ref = x.double() @ w.double().t() + b.double()
+    bound = _bound(x, w, ref)
+    assert bool(((ops.linear(x, w, b).double() - ref).abs() <= bound).all())
+    assert bool(((ops.linear(x, w, b, "relu").double() - ref.clamp_min(0)).abs() <= bound).all())
+    gelu = 0.5 * ref * torch.special.erfc(-ref * 0.5 ** 0.5)
+    assert bool(((ops.linear(x, w, b, "gelu").double() - gelu).abs() <= 1.13 * bound + 4e-7).all())
+
+
+def test_linear_split_is_chosen_by_depth():
+    assert _tile(8040, 768, 192)[2] == -1 and _tile(8040, 768, 176)[2] != -1 and _tile(8040, 768, 200)[2] != -1
+
+
+@pytest.mark.parametrize("M,N,K,lda,shift", [(300, 200, 192, 201, 1), (700, 64, 208, 1000, 3), (129, 333, 256, 257, 0)])
+def test_linear_split_unaligned_rows(M, N, K, lda, shift):
+    from nestedtensor_amd import _C
+    x, w, b = _case(M, N, K)
+    held = torch.full((M * lda + 4,), float("nan"), device=DEV)
+    rows = held[shift:shift + M * lda].view(M, lda)
+    rows[:, :K] = x
+    out = torch.full((M, N + 3), 7.0, device=DEV)
+    _C.check(_C.lib.nt_linear(_C.ptr(rows), lda, _C.ptr(w), _C.ptr(b), _C.ptr(out), N + 3, M, N, K,
+                              _C.dtype_code(torch.float32), _C.current_stream(DEV)))
+    ref = x.double() @ w.double().t() + b.double()
+    assert bool(((out[:, :N].double() - ref).abs() <= _bound(x, w, ref)).all())
+    assert bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 7, 192), (300, 200, 256), (2001, 1537, 224), (8040, 2304, 208)])
+def test_linear_split_special_values(M, N, K):
+    from nestedtensor_amd import ops
+    inf, big = float("inf"), torch.finfo(torch.float32).max
+    x, w, b = _case(M, N, K)
+    for i, v in enumerate((inf, -inf, float("nan"), big, -big)):
+        x[(3 * i) % M, (5 * i) % K] = v
+    w[N - 1, 3] = inf
+    w[N // 2, :] = 0.0                                   # infinity times zero
+    ref = x.double() @ w.double().t() + b.double()
+    y = ops.linear(x, w, b)
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    over = ref.abs() > big                               # infinities and what 32 bits cannot hold
+    near = over & (ref.abs() < 2.0 * big)                # a partial sum may or may not have overflowed
+    assert torch.equal(y[over & ~near], ref[over & ~near].float())
+    fine = ~over & ~torch.isnan(ref) & (ref.abs() < 0.5 * big)
+    bound = _bound(torch.nan_to_num(x, 0.0, 0.0, 0.0), torch.nan_to_num(w, 0.0, 0.0, 0.0), ref)
+    assert bool(((y.double() - ref).abs()[fine] <= bound[fine]).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 7, 192), (300, 200, 256), (2001, 1537, 224)])
+def test_linear_split_small_magnitudes(M, N, K):
+    """The third part of a number below 2^-110 lies below the smallest bf16 number."""
+    from nestedtensor_amd import ops
+    x, w, _ = _case(M, N, K)
+    for ex, ew in ((-118, 100), (90, -120), (-60, -40), (-100, 0)):
+        xs, ws = torch.ldexp(x, torch.tensor(ex, device=DEV)), torch.ldexp(w, torch.tensor(ew, device=DEV))
+        ref = xs.double() @ ws.double().t()
+        assert bool(((ops.linear(xs, ws, None).double() - ref).abs() <= _bound(xs, ws, ref)).all()), (ex, ew)
+
+
+@pytest.mark.parametrize("M,N,K", [(4000, 512, 256), (4000, 768, 768), (2000, 1024, 1024)])
+def test_linear_split_precision(M, N, K):
+    """No further from 64 bits than a chain of fp32 multiply-adds, one rounding per k."""
+    from nestedtensor_amd import ops
+    x, w, b = _case(M, N, K)
+    ref = x.double() @ w.double().t() + b.double()
+    acc = torch.zeros(M, N, device=DEV)
+    for k in range(K):
+        acc = (acc.double() + x[:, k:k + 1].double() * w[:, k].double()).float()
+    chain = ((acc + b).double() - ref).norm()
+    assert (ops.linear(x, w, b).double() - ref).norm() <= chain
