@@ -16,8 +16,8 @@
 // the softmax row reductions are in-lane plus one cross-half shuffle, and the
 // score accumulators are, as they stand, the B-operand of the second product.
 //
-// fp32 with head_dim 32 / 64 / 128 has a kernel of its own on the fp32 matrix
-// instruction (further down).  Any other head_dim takes the generic kernel (one
+// fp32 with head_dim 32 / 64 / 128 has a kernel of its own on the bf16 matrix instruction
+// (operands in three parts, further down).  Any other head_dim takes the generic kernel (one
 // wavefront per query row, fp32 FMA); it is the parity path for shapes the MFMA
 // kernels do not cover, not a performance path.
 #include "attn_common.h"
@@ -830,39 +830,319 @@ __device__ __forceinline__ void attention_f32_tile(
   }
 }
 
+// The same tile on the bf16 matrix instruction (v_mfma_f32_32x32x16_bf16): Q, K, V and P are
+// split into three bf16 parts each and the six largest of the nine products kept, an
+// error below half a rounding of one fp32 product; scores, softmax and sums stay fp32.
+// The fp32 instruction does a sixteenth of the work per cycle and was what bounded the tile.
+//
+// A K tile of 32 keys is split on its way into LDS, one 16-byte piece (8 k) per part:
+//  * K: 8 head dims of a key, the keys of a piece number one after the other, their
+//    order XOR-ed with the piece so that writes (a key's pieces) and reads (a piece's
+//    keys) of sixteen lanes fall into distinct banks;
+//  * V: transposed by the loads themselves, a lane fetching eight keys of its head dim
+//    (whole rows over the lanes): the keys that the score accumulators 8 s .. 8 s + 7 of a
+//    lane half hold, which makes those accumulators, split, the other operand.
+// The next tile but one is in flight in registers, the next one is split between the matrix
+// instructions of the current one.  Wavefronts without a query row only fetch.
+// Bound by matrix and vector instructions, which share a SIMD badly: 48 matrix and some 300
+// vector instructions per tile of head_dim 64, of which the splits of P, K and V are 200
+// (measured apart, a SIMD keeps its matrix pipe full beside four vector instructions per
+// matrix instruction of each of two wavefronts; each further one costs its own time).
+// Against attention_f32_tile: 32 sequences of 32 to 512, 12 heads of 64: 126 -> 82 us; 8 of
+// 256 to 2048, 8 heads of 64: 239 -> 148; 8 heads of 32: 52 -> 38; 16 of 64 to 1024, 16 heads of
+// 128: 556 -> 456 (one wavefront per SIMD: its Q parts alone take 96 registers); 64 of 10 to 200,
+// 8 heads of 128: 79 -> 77.  Error against 64 bits 0.78 to 0.85 of what it was.
+template <int HD>
+struct SplitAttention {
+  static constexpr int kKT = 32;
+  static constexpr int kKPart = kKT * HD * 2, kBuf = 6 * kKPart;   // three parts of K, three of V
+  static constexpr int kLdsBytes = 2 * kBuf;
+  static_assert(kLdsBytes >= 2 * 32 * (2 * HD + 12) * (int)sizeof(float), "attention_f32_tile runs in the same LDS");
+};
+
+template <int HD>
+__device__ __forceinline__ void attention_split_tile(
+    const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
+    const float* __restrict__ Vp, int64_t ldv, float* __restrict__ O, int64_t ldo,
+    const int64_t q_begin, const int64_t Lq, const int64_t q0, const int64_t kv_begin, const int64_t Lk,
+    const int h, float scale_log2e, char* lds) {
+  typedef SplitAttention<HD> S;
+  constexpr int kKT = S::kKT, kPart = S::kKPart;
+  constexpr int kT = HD / 16;                      // steps of the first product
+  constexpr int kJ = HD / 32;                      // 32-row blocks of the second
+  constexpr int kPer = HD >= 64 ? HD / 64 : 1;     // pieces of K and of V per thread (32: of one of them)
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  const bool fetches_k = HD >= 64 || wave < 2, fetches_v = HD >= 64 || wave >= 2;
+  SmallestBf16 smallest;
+
+  auto split8 = [&](const float (&x)[8], u32x4 (&part)[3]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t a, b, c;
+      split_bf16_pair(x[2 * e], x[2 * e + 1], a, b, c);
+      part[0][e] = a;
+      part[1][e] = b;
+      part[2][e] = c;
+    }
+  };
+
+  // this lane's query row, prescaled: dims 16 t + 8 half .. of step t
+  const int64_t qrow = q0 + wave * 32 + col;
+  const bool q_ok = qrow < Lq;
+  const bool active = q0 + wave * 32 < Lq;         // uniform
+  bf16x8 qf[kT][3];
+  {
+    const float* qp = Q + (q_begin + (q_ok ? qrow : q0)) * ldq + (int64_t)h * HD + 8 * half;
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+      float x[8];
+      __builtin_memcpy(x, __builtin_assume_aligned(qp + 16 * t, 16), 32);
+      u32x4 part[3];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = q_ok ? x[e] * scale_log2e : 0.0f;
+      split8(x, part);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) qf[t][p] = __builtin_bit_cast(bf16x8, part[p]);
+    }
+  }
+
+  // Rows past the last key are read as the last one: their scores are replaced and their
+  // probabilities zero (a zero times an infinity sends the tile to the fp32 instruction).
+  const char* kbase = reinterpret_cast<const char*>(Kp + kv_begin * ldk + (int64_t)h * HD);
+  const char* vbase = reinterpret_cast<const char*>(Vp + kv_begin * ldv + (int64_t)h * HD);
+  const int64_t kld = ldk * 4, vld = ldv * 4;
+  float kraw[kPer][8], vraw[kPer][8];
+  constexpr int kKeyPieces = HD / 8;
+  auto gload = [&](int64_t t) __attribute__((always_inline)) {
+    const int64_t rest = Lk - t * kKT;
+    const int last = rest < kKT ? (int)rest - 1 : kKT - 1;
+    const char* kt = kbase + t * kKT * kld;
+    const char* vt = vbase + t * kKT * vld;
+    if (fetches_k) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int c = tid + 256 * i;
+        const int key = c / kKeyPieces, piece = c % kKeyPieces;
+        const int64_t row = key < last ? key : last;
+        __builtin_memcpy(kraw[i], __builtin_assume_aligned(kt + row * kld + piece * 32, 16), 32);
+      }
+    }
+    if (fetches_v) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int sg = HD >= 64 ? (wave + 4 * i) * 64 / HD : 2 * (wave - 2) + half;   // uniform from 64 on
+        const int d = HD >= 64 ? ((wave + 4 * i) * 64 + lane) % HD : col;
+        const int first = (sg >> 1) * 16 + (sg & 1) * 4;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = first + (e & 3) + (e >> 2) * 8;
+          const char* row = vt + (key < last ? key : last) * vld;      // uniform from 64 on
+          vraw[i][e] = *reinterpret_cast<const float*>(row + (unsigned)(d * 4));
+        }
+      }
+    }
+  };
+  auto put = [&](char* buf) __attribute__((always_inline)) {
+    if (fetches_k) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int c = tid + 256 * i;
+        const int key = c / kKeyPieces, piece = c % kKeyPieces;
+        u32x4 part[3];
+        split8(kraw[i], part);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
+        char* dst = buf + (piece * 32 + (key ^ (piece * (128 / HD) & 15))) * 16;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dst + p * kPart) = part[p];
+      }
+    }
+    if (fetches_v) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        u32x4 part[3];
+        split8(vraw[i], part);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
+        // piece (sg, d): sg * HD + d counts the threads
+        char* dst = buf + 3 * kPart + (HD >= 64 ? tid + 256 * i : tid - 128) * 16;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dst + p * kPart) = part[p];
+      }
+    }
+  };
+
+  acc16 o[kJ];
+#pragma unroll
+  for (int j = 0; j < kJ; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[j][i] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;       // l_run: this lane half's keys only
+  constexpr int kPa[6] = {0, 1, 2, 1, 0, 0}, kPb[6] = {2, 1, 0, 0, 1, 0};   // smallest products first
+
+  const int64_t n_tiles = (Lk + kKT - 1) / kKT;
+  if (n_tiles > 0) {
+    gload(0);
+    put(lds);
+    gload(n_tiles > 1 ? 1 : 0);
+  }
+  __syncthreads();
+  for (int64_t t = 0; t < n_tiles; ++t) {
+    const char* cur = lds + (t & 1) * S::kBuf;
+    char* next = lds + ((t + 1) & 1) * S::kBuf;
+    const int64_t ahead = t + 2 < n_tiles ? t + 2 : n_tiles - 1;     // past the end: not used
+    if (!active) {
+      put(next);
+      gload(ahead);
+    } else {
+      acc16 s;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+      for (int tt = 0; tt < kT; ++tt) {
+        const int piece = 2 * tt + half;
+        const char* kp = cur + (piece * 32 + (col ^ (piece * (128 / HD) & 15))) * 16;
+        bf16x8 kf[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) kf[p] = *reinterpret_cast<const bf16x8*>(kp + p * kPart);
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kPa[p]], qf[tt][kPb[p]], s, 0, 0, 0);
+      }
+      put(next);
+      gload(ahead);
+      // accumulator i: key 8 (i / 4) + 4 half + i % 4 of the tile, query col
+      const int64_t left = Lk - t * kKT;
+      if (left < kKT) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          if (8 * (i / 4) + 4 * half + (i % 4) >= left) s[i] = -INFINITY;
+        }
+      }
+      float m_tile = s[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) m_tile = fmaxf(m_tile, s[i]);
+      m_tile = max_across_halves(m_tile);                      // finite: the tile holds a valid key
+      const float m_new = fmaxf(m_run, m_tile);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      float l_tile = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[i] = __builtin_amdgcn_exp2f(s[i] - m_new);
+        l_tile += s[i];
+      }
+      l_run = l_run * alpha + l_tile;
+      if (__ballot(alpha != 1.0f) != 0) {
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[j][i] *= alpha;
+        }
+      }
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = s[8 * st + e];
+        u32x4 part[3];
+        split8(x, part);
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) {
+          const char* vp = cur + 3 * kPart + ((2 * st + half) * HD + 32 * j + col) * 16;
+          bf16x8 vf[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) vf[p] = *reinterpret_cast<const bf16x8*>(vp + p * kPart);
+#pragma unroll
+          for (int p = 0; p < 6; ++p)
+            o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[kPa[p]], __builtin_bit_cast(bf16x8, part[kPb[p]]), o[j],
+                                                           0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();
+  }
+
+  const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  // No finite result: an infinity or NaN went in or came out of a product or a split.  Those
+  // tiles, and the ones with magnitudes that the split cannot carry, run on the fp32
+  // instruction instead.
+  float probe = l_tot * 0.0f;
+#pragma unroll
+  for (int j = 0; j < kJ; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) probe = fmaf(o[j][i], 0.0f, probe);
+  if (__syncthreads_or(smallest.tiny() || probe != probe)) {
+    attention_f32_tile<HD>(Q, ldq, Kp, ldk, Vp, ldv, O, ldo, q_begin, Lq, q0, kv_begin, Lk, h, scale_log2e,
+                           reinterpret_cast<float*>(lds));
+    return;
+  }
+  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;     // no keys: zeros
+  if (q_ok) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    // accumulator i of block j: head dim 32 j + 8 (i / 4) + 4 half + i % 4
+    float* op = O + (q_begin + qrow) * ldo + (int64_t)h * HD + 4 * half;
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 v = {o[j][4 * g] * inv, o[j][4 * g + 1] * inv, o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv};
+        *reinterpret_cast<f32x4*>(op + 32 * j + 8 * g) = v;
+      }
+    }
+  }
+}
+
 // Workgroup = (128 query rows, head, sequence) on a padded grid: tiles past a
 // sequence's last query row leave at once.
 template <int HD>
-__global__ __launch_bounds__(256) void varlen_attention_f32_kernel(
+__global__ __launch_bounds__(256, HD < 128 ? 2 : 1) void varlen_attention_f32_kernel(
     const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
     const float* __restrict__ Vp, int64_t ldv, float* __restrict__ O, int64_t ldo,
     const int64_t* __restrict__ q_offsets, const int64_t* __restrict__ kv_offsets,
     float scale_log2e) {
-  __shared__ __align__(16) float lds[2 * 32 * (2 * HD + 12)];
+  extern __shared__ __align__(16) char lds[];
   const int b = blockIdx.z, h = blockIdx.y;
   const int64_t q_begin = q_offsets[b];
   const int64_t Lq = q_offsets[b + 1] - q_begin;
   const int64_t q0 = (int64_t)blockIdx.x * 128;
   if (q0 >= Lq) return;                        // uniform
   const int64_t kv_begin = kv_offsets[b];
-  attention_f32_tile<HD>(Q, ldq, Kp, ldk, Vp, ldv, O, ldo, q_begin, Lq, q0, kv_begin,
-                         kv_offsets[b + 1] - kv_begin, h, scale_log2e, lds);
+  attention_split_tile<HD>(Q, ldq, Kp, ldk, Vp, ldv, O, ldo, q_begin, Lq, q0, kv_begin,
+                           kv_offsets[b + 1] - kv_begin, h, scale_log2e, lds);
 }
 
 // The same tiles from a work list (the items of nt_varlen_attention_vt): only
 // tiles that exist are launched, longest key sequences first, head fastest.
 template <int HD>
-__global__ __launch_bounds__(256) void varlen_attention_f32_sched_kernel(
+__global__ __launch_bounds__(256, HD < 128 ? 2 : 1) void varlen_attention_f32_sched_kernel(
     const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
     const float* __restrict__ Vp, int64_t ldv, float* __restrict__ O, int64_t ldo,
     const int4* __restrict__ schedule, unsigned num_heads, float scale_log2e) {
-  __shared__ __align__(16) float lds[2 * 32 * (2 * HD + 12)];
+  extern __shared__ __align__(16) char lds[];
   const int h = (int)(blockIdx.x % num_heads);
   const int4 item = schedule[2 * (blockIdx.x / num_heads)];
   const int4 item_kv = schedule[2 * (blockIdx.x / num_heads) + 1];
   if (item.y <= 0 || item.z >= item.y) return;   // uniform: no query rows in this tile
-  attention_f32_tile<HD>(Q, ldq, Kp, ldk, Vp, ldv, O, ldo, item.x, item.y, item.z, item_kv.x,
-                         item_kv.y > 0 ? item_kv.y : 0, h, scale_log2e, lds);
+  attention_split_tile<HD>(Q, ldq, Kp, ldk, Vp, ldv, O, ldo, item.x, item.y, item.z, item_kv.x,
+                           item_kv.y > 0 ? item_kv.y : 0, h, scale_log2e, lds);
+}
+
+// Dynamic LDS beyond 48 KiB has to be asked for, once per kernel.
+template <auto KERNEL>
+static int allow_lds(int bytes) {
+  static bool done = false;
+  if (!done && bytes > 48 * 1024) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       bytes);
+    if (e != hipSuccess) return fail(NT_ERR_HIP, "attention: %s", hipGetErrorString(e));
+    done = true;
+  }
+  return NT_OK;
 }
 
 template <int HD>
@@ -870,7 +1150,9 @@ static int launch_f32(const void* q, int64_t ldq, const void* k, int64_t ldk, co
                       int64_t ldv, void* out, int64_t ldo, const int64_t* qo, const int64_t* kvo,
                       int64_t B, int64_t H, int64_t max_q, float scale, hipStream_t s) {
   dim3 grid((unsigned)((max_q + 127) / 128), (unsigned)H, (unsigned)B);
-  hipLaunchKernelGGL((varlen_attention_f32_kernel<HD>), grid, dim3(256), 0, s,
+  const int rc = allow_lds<varlen_attention_f32_kernel<HD>>(SplitAttention<HD>::kLdsBytes);
+  if (rc != NT_OK) return rc;
+  hipLaunchKernelGGL((varlen_attention_f32_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kLdsBytes, s,
                      static_cast<const float*>(q), ldq, static_cast<const float*>(k), ldk,
                      static_cast<const float*>(v), ldv, static_cast<float*>(out), ldo, qo, kvo,
                      scale * 1.4426950408889634f);
@@ -978,13 +1260,16 @@ static void launch_vt(dim3 grid, hipStream_t s, const void* q, int64_t ldq, cons
 }
 
 template <int HD>
-static void launch_f32_sched(dim3 grid, hipStream_t s, const void* q, int64_t ldq, const void* k, int64_t ldk,
+static int launch_f32_sched(dim3 grid, hipStream_t s, const void* q, int64_t ldq, const void* k, int64_t ldk,
                              const void* v, int64_t ldv, void* out, int64_t ldo, const int4* sched,
                              unsigned num_heads, float scale_log2e) {
-  hipLaunchKernelGGL((varlen_attention_f32_sched_kernel<HD>), grid, dim3(256), 0, s,
+  const int rc = allow_lds<varlen_attention_f32_sched_kernel<HD>>(SplitAttention<HD>::kLdsBytes);
+  if (rc != NT_OK) return rc;
+  hipLaunchKernelGGL((varlen_attention_f32_sched_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kLdsBytes, s,
                      static_cast<const float*>(q), ldq, static_cast<const float*>(k), ldk,
                      static_cast<const float*>(v), ldv, static_cast<float*>(out), ldo, sched, num_heads,
                      scale_log2e);
+  return check_launch("varlen_attention_f32_sched_kernel");
 }
 
 extern "C" int nt_varlen_attention_scheduled(const void* q, int64_t ldq, const void* k, int64_t ldk,
@@ -1015,10 +1300,9 @@ extern "C" int nt_varlen_attention_scheduled(const void* q, int64_t ldq, const v
   hipStream_t s = (hipStream_t)stream;
   const int4* sched = reinterpret_cast<const int4*>(schedule);
   const unsigned nh = (unsigned)num_heads;
-  if (head_dim == 32) launch_f32_sched<32>(grid, s, q, ldq, k, ldk, v, ldv, out, ldo, sched, nh, scale_log2e);
-  else if (head_dim == 64) launch_f32_sched<64>(grid, s, q, ldq, k, ldk, v, ldv, out, ldo, sched, nh, scale_log2e);
-  else launch_f32_sched<128>(grid, s, q, ldq, k, ldk, v, ldv, out, ldo, sched, nh, scale_log2e);
-  return check_launch("varlen_attention_f32_sched_kernel");
+  if (head_dim == 32) return launch_f32_sched<32>(grid, s, q, ldq, k, ldk, v, ldv, out, ldo, sched, nh, scale_log2e);
+  if (head_dim == 64) return launch_f32_sched<64>(grid, s, q, ldq, k, ldk, v, ldv, out, ldo, sched, nh, scale_log2e);
+  return launch_f32_sched<128>(grid, s, q, ldq, k, ldk, v, ldv, out, ldo, sched, nh, scale_log2e);
 }
 
 // ---- the work list -----------------------------------------------------------------

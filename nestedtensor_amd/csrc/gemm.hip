@@ -935,11 +935,6 @@ struct SplitCfg {
   static_assert(kLdsBytes + kBN * 4 + 16 <= 160 * 1024, "tile buffers must fit the LDS");
 };
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-
 // 32-row blocks of A and W lie in LDS as three parts of 1 KiB, a part as the 16-byte pieces
 // (k 0..3 and 8..11, or, half 1, the others) of the 32 rows one after the other.  In the
 // second half rows trade places by eights, so that sixteen consecutive lanes fall into
@@ -974,26 +969,13 @@ struct SplitPiece {
     __builtin_memcpy(raw[slot], src + off, FLOATS < 8 ? FLOATS * 4 : 16);
     if constexpr (FLOATS == 8) __builtin_memcpy(raw[slot] + 4, src + off + 32, 16);
   }
-  __device__ __forceinline__ void put(char* buf, int slot, u16x2& smallest) const {
+  __device__ __forceinline__ void put(char* buf, int slot, SmallestBf16& smallest) const {
     uint32_t part[3][FLOATS / 2];
 #pragma unroll
     for (int e = 0; e < FLOATS / 2; ++e) {
-      float x = __builtin_bit_cast(float, raw[slot][2 * e]);
-      float y = __builtin_bit_cast(float, raw[slot][2 * e + 1]);
-#pragma unroll
-      for (int p = 0; p < 3; ++p) {
-        const f32x2 v = {x, y};
-        const uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-        if (p < 2) {
-          x -= __builtin_bit_cast(float, pair << 16);
-          y -= __builtin_bit_cast(float, pair & 0xffff0000u);
-        }
-        if (p == 0) {
-          const u16x2 magnitude = __builtin_bit_cast(u16x2, pair) * (uint16_t)2 - (uint16_t)1;   // of a zero: largest
-          smallest = __builtin_elementwise_min(smallest, magnitude);
-        }
-        part[p][e] = pair;
-      }
+      split_bf16_pair(__builtin_bit_cast(float, raw[slot][2 * e]), __builtin_bit_cast(float, raw[slot][2 * e + 1]),
+                      part[0][e], part[1][e], part[2][e]);
+      smallest.add(part[0][e]);
     }
 #pragma unroll
     for (int p = 0; p < 3; ++p)
@@ -1041,7 +1023,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
     half.place(a, m0, n0, kABlocks, 8 * kUnits + (wave >> 1), (wave & 1) * 16 + (lane >> 2), lane & 3);
   if (kTail2)
     quarter.place(a, m0, n0, kABlocks, 8 * kUnits + kTail4 + (wave >> 2), (wave & 3) * 8 + (lane >> 3), lane & 7);
-  u16x2 smallest = {0xffff, 0xffff};
+  SmallestBf16 smallest;
 
   constexpr int kPuts = kUnits + (kTail4 ? 1 : 0) + (kTail2 ? 1 : 0);
   auto fetch = [&](int u, int step, int slot) __attribute__((always_inline)) {
@@ -1146,8 +1128,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
   // bf16 number.  A result that is no finite number: an infinity or NaN went in (their rests
   // are NaN), a first part rounded up to infinity, or the sum overflowed.  Both are computed
   // again by the fp32 instruction.
-  constexpr uint16_t kTiny = 2 * (27 << 7) - 1;
-  if (smallest[0] < kTiny || smallest[1] < kTiny) *lds_tiny = 1;
+  if (smallest.tiny()) *lds_tiny = 1;
   float probe = 0.0f;
 #pragma unroll
   for (int i = 0; i < NI; ++i)

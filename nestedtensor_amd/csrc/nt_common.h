@@ -48,6 +48,39 @@ __device__ __forceinline__ void store16_stream(char* p, u32x4 v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
+// Two fp32 numbers as three packed pairs of bf16 each, every one the rounded rest of the one
+// before: x is the exact sum of its parts unless it lies below 2^-110 (the third part may
+// fall below the smallest bf16 number), is no finite number or next to the largest
+// (NaN among the parts).
+__device__ __forceinline__ void split_bf16_pair(float x, float y, uint32_t& first, uint32_t& second, uint32_t& third) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  auto round_pair = [&] { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, bf16x2)); };
+  auto take_rest = [&](uint32_t pair) {
+    x -= __builtin_bit_cast(float, pair << 16);
+    y -= __builtin_bit_cast(float, pair & 0xffff0000u);
+  };
+  first = round_pair();
+  take_rest(first);
+  second = round_pair();
+  take_rest(second);
+  third = round_pair();
+}
+
+// The smallest magnitudes, other than zero, of the first parts of a number of pairs.
+struct SmallestBf16 {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 bits = {0xffff, 0xffff};       // twice the magnitude's bits less one: of a zero the largest
+  __device__ __forceinline__ void add(uint32_t first) {
+    bits = __builtin_elementwise_min(bits, (u16x2)(__builtin_bit_cast(u16x2, first) * (uint16_t)2 - (uint16_t)1));
+  }
+  // one of them below 2^-100
+  __device__ __forceinline__ bool tiny() const {
+    constexpr uint16_t kTiny = 2 * (27 << 7) - 1;
+    return bits[0] < kTiny || bits[1] < kTiny;
+  }
+};
+
 // gelu(x) = x Phi(x), Phi the normal distribution function, from its tail: Phi(-|x|) is
 // 2^Q(|x|) with Q a polynomial of degree 8 fitted to log2 Phi(-u) on [0, 5] (least
 // squares reweighted towards the smallest largest error of Phi).  Q falls without end past 5, so the tail
