@@ -44,6 +44,8 @@
 // 128 -> 64 on 128 437 (49 MB) 45.8 -> 40.7; on input that lies in the memory-side cache 128.5 ->
 // 102.2, 119.4 -> 81.9 and 42.8 -> 38.6.
 //
+// Large results only; the others take conv1x1_direct_kernel.
+//
 // Persistent workgroups (the weight is loaded into LDS once each) of WAVES
 // wavefronts, and every wavefront works on tiles of its own with its own X tile
 // and strip: no workgroup barrier after the weight is in place, the next tile's
@@ -57,6 +59,17 @@ namespace nt {
 
 constexpr int kConvTile = 64;                 // pixels of a row that one tile writes
 constexpr int kConvMaxIn = 128, kConvMaxOut = 512;
+
+// The weight into LDS, rows of `ld` elements.
+template <typename T, int THREADS>
+__device__ __forceinline__ void load_weight(const T* __restrict__ w, T* lds, int ld, int c_in, int c_out) {
+  const int per_row = c_in / 8;
+  for (int i = threadIdx.x; i < c_out * per_row; i += THREADS) {
+    const int row = i / per_row, ch = i - row * per_row;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(w + (size_t)row * c_in + ch * 8);
+    *reinterpret_cast<u32x4*>(lds + (size_t)row * ld + ch * 8) = v;
+  }
+}
 
 template <typename T, int WAVES, int LOADS>
 __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __restrict__ x, const T* __restrict__ w,
@@ -85,15 +98,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
   uint32_t* Xl = reinterpret_cast<uint32_t*>(mine);
   uint32_t* strip = reinterpret_cast<uint32_t*>(mine);
 
-  // the weight, once
-  {
-    const int per_row = c_in / 8;
-    for (int i = t; i < c_out * per_row; i += 64 * WAVES) {
-      const int row = i / per_row, ch = i - row * per_row;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(w + (size_t)row * c_in + ch * 8);
-      *reinterpret_cast<u32x4*>(Wl + (size_t)row * SW + ch * 8) = v;
-    }
-  }
+  load_weight<T, 64 * WAVES>(w, Wl, SW, c_in, c_out);     // once
   __syncthreads();
   // tiles of this wavefront: first, first + G * WAVES, ... with G workgroups; the
   // workgroups of one XCD (ids congruent modulo 8) take a contiguous run
@@ -274,6 +279,138 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
   }
 }
 
+// The same product without LDS for pixels and results.  A wavefront takes a window of 64
+// pixels; lane n holds pixels 2 n and 2 n + 1, one dword of every channel row straight from
+// global memory, and v_perm makes an operand of the even and one of the odd pixels of it.  With
+// the weight as the A operand a lane ends up with runs of four output channels of its pixels,
+// so the even and the odd accumulator of a channel are one dword of the result: 128 contiguous
+// bytes of a row per store and lane half.  Nothing is transposed, no window is
+// multiplied twice, and CG wavefronts share a window, a CG-th of the output channels each, so
+// that a small batch still spreads over the chip (us, in the cache / not):
+//   64 -> 256 on 2 600, 29 000, 127 000 pixels    27 -> 9, 30 -> 11, 41 / 42 -> 27 / 29
+//   64 -> 64  on 2 800, 32 000, 128 000           15 -> 9, 16 -> 9, 18 / 21 -> 14 / 17
+//   32 -> 128 on 3 400, 31 000, 122 000           14 -> 8, 16 -> 9, 16 / 17 -> 14 / 15
+//   128 -> 256 on 35 000, 110 000, 517 000        66 -> 20, 89 -> 27 / 32, 268 / 270 -> 138 / 145
+//   128 -> 64  on 95 000, 549 000                 36 -> 15 / 16, 93 / 99 -> 53 / 66
+// A row's 128 bytes are no whole line, and the parts of a line come from two wavefronts: they
+// meet in the L2 as long as the result is not much larger than that.  Beyond 64 MiB the
+// whole lines of conv1x1_nchw_kernel win (64 -> 256 on 552 000 pixels 84 / 93 against 127 / 168,
+// 64 -> 64 on 559 000 43 / 49 against 39 / 57, 96 -> 256 on 443 000 121 / 127 against 130 / 142), but not
+// where its tiles leave the LDS no room for enough wavefronts (96 -> 64 on 524 000 147 / 208
+// against 45 / 56, 128 channels above).
+template <typename T, int KS, int CG>
+__global__ __launch_bounds__(512, 2) void conv1x1_direct_kernel(const T* __restrict__ x, const T* __restrict__ w,
+                                                                T* __restrict__ y, const int64_t* __restrict__ pix_offsets,
+                                                                const int64_t* __restrict__ tile_offsets, int64_t B,
+                                                                int64_t total_tiles, int c_in, int c_out) {
+  typedef AttnT<T> AT;
+  typedef typename AT::Frag Frag;
+  typedef uint32_t Pair __attribute__((aligned(2)));       // two pixels of a row, wherever it begins
+  constexpr int WAVES = 8;
+  extern __shared__ __align__(16) char lds[];
+  const int SW = c_in + 8;                      // elements per row of the weight in LDS
+  const int t = threadIdx.x, l = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int n = l & 31, g = l >> 5;
+  T* Wl = reinterpret_cast<T*>(lds);
+  load_weight<T, 64 * WAVES>(w, Wl, SW, c_in, c_out);
+  __syncthreads();
+
+  const int nob = c_out / 32, cg = wave % CG;
+  const int ob_lo = cg * nob / CG, ob_hi = (cg + 1) * nob / CG;
+  // tiles of this wavefront; the workgroups of one XCD take a contiguous run of each round
+  const int64_t G = gridDim.x;
+  int64_t wg = blockIdx.x;
+  if (G % 8 == 0) wg = (int64_t)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
+  int64_t tile = (wg * WAVES + wave) / CG;
+  const int64_t stride = G * WAVES / CG;
+  int64_t P = 0, k64 = 0, pix0 = 0, t_lo = 0, t_hi = 0;
+  // goes to the next tile with pixels (the last of an image has none); false: there is none
+  auto locate = [&]() {
+    for (; tile < total_tiles; tile += stride) {
+      if (tile >= t_hi) {
+        const int64_t img = find_segment_uniform(tile_offsets, B, tile);
+        t_lo = tile_offsets[img];
+        t_hi = tile_offsets[img + 1];
+        pix0 = pix_offsets[img];
+        P = pix_offsets[img + 1] - pix0;
+      }
+      k64 = (tile - t_lo) * kConvTile;
+      if (k64 < P) return true;
+    }
+    return false;
+  };
+  uint32_t stage[KS][8];                        // channels 16 ks + 8 g + j
+  auto fetch = [&]() {
+    const T* p = x + pix0 * c_in + k64 + 8 * g * P + 2 * n;
+    const int64_t left = P - k64 - 2 * n;       // pixels from this lane's first on
+    const bool whole = k64 + kConvTile <= P;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      if (16 * ks >= c_in) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const T* q = p + (16 * ks + j) * P;
+        if (whole || left >= 2) {
+          stage[ks][j] = *reinterpret_cast<const Pair*>(q);
+        } else {
+          stage[ks][j] = left == 1 ? *reinterpret_cast<const uint16_t*>(q) : 0u;
+        }
+      }
+    }
+  };
+  bool have = locate();
+  if (have) fetch();
+  while (have) {
+    const int64_t cur_P = P, cur_k64 = k64, cur_pix0 = pix0;
+    Frag xf[KS][2];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      if (16 * ks >= c_in) continue;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        u32x4 f;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          f[d] = __builtin_amdgcn_perm(stage[ks][2 * d + 1], stage[ks][2 * d], i ? 0x07060302u : 0x05040100u);
+        __builtin_memcpy(&xf[ks][i], &f, 16);
+      }
+    }
+    tile += stride;
+    have = locate();
+    if (have) fetch();                          // in flight during the products and stores below
+    T* out = y + cur_pix0 * c_out + cur_k64 + (32 * ob_lo + 4 * g) * cur_P + 2 * n;
+    const int64_t left = cur_P - cur_k64 - 2 * n;
+    const bool whole = cur_k64 + kConvTile <= cur_P;
+    for (int ob = ob_lo; ob < ob_hi; ++ob) {
+      acc16 acc[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (16 * ks >= c_in) continue;
+        const Frag wf = *reinterpret_cast<const Frag*>(Wl + (size_t)(ob * 32 + n) * SW + 16 * ks + 8 * g);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i] = AT::mma(wf, xf[ks][i], acc[i]);
+      }
+      // accumulator e: channel 32 ob + 8 (e / 4) + 4 g + e % 4
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const uint32_t two = AT::cvt2(acc[0][e], acc[1][e]);
+        T* q = out + (8 * (e / 4) + e % 4) * cur_P;
+        if (whole || left >= 2) {
+          *reinterpret_cast<Pair*>(q) = two;
+        } else if (left == 1) {
+          *reinterpret_cast<uint16_t*>(q) = (uint16_t)two;
+        }
+      }
+      out += 32 * cur_P;
+    }
+  }
+}
+
 static size_t conv_lds_bytes(int c_in, int c_out, int waves, size_t elem) {
   const size_t x_bytes = (size_t)c_in * (kConvTile + 1) * 4, strip_bytes = (size_t)32 * (kConvTile + 4) * 4;
   return (size_t)c_out * (c_in + 8) * elem + (size_t)waves * (x_bytes > strip_bytes ? x_bytes : strip_bytes);
@@ -314,6 +451,39 @@ static int launch_conv_w(const void* x, const void* w, void* y, const int64_t* p
 #undef NT_CONV_ARGS
 }
 
+template <typename T, int KS, int CG>
+static int launch_direct(const void* x, const void* w, void* y, const int64_t* pix_offsets, const int64_t* tile_offsets,
+                         int64_t B, int64_t total_tiles, int c_in, int c_out, int cus, hipStream_t stream) {
+  auto kernel = conv1x1_direct_kernel<T, KS, CG>;
+  static bool configured = false;      // one attribute call per instantiation (and process)
+  if (!configured) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            160 * 1024) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(NT_ERR_HIP, "conv1x1: cannot raise the dynamic LDS limit");
+    }
+    configured = true;
+  }
+  int64_t grid = cus;
+  const int64_t needed = (total_tiles * CG + 7) / 8;
+  if (grid > needed) grid = needed;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), (size_t)c_out * (c_in + 8) * sizeof(T), stream,
+                     static_cast<const T*>(x), static_cast<const T*>(w), static_cast<T*>(y), pix_offsets, tile_offsets, B,
+                     total_tiles, c_in, c_out);
+  return check_launch("conv1x1_direct_kernel");
+}
+
+template <typename T, int CG>
+static int launch_direct_ks(const void* x, const void* w, void* y, const int64_t* pix_offsets, const int64_t* tile_offsets,
+                            int64_t B, int64_t total_tiles, int c_in, int c_out, int cus, hipStream_t stream) {
+#define NT_CONV_ARGS x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream
+  if (c_in <= 16) return launch_direct<T, 1, CG>(NT_CONV_ARGS);
+  if (c_in <= 32) return launch_direct<T, 2, CG>(NT_CONV_ARGS);
+  if (c_in <= 64) return launch_direct<T, 4, CG>(NT_CONV_ARGS);
+  return launch_direct<T, 8, CG>(NT_CONV_ARGS);
+#undef NT_CONV_ARGS
+}
+
 // The most wavefronts per workgroup (8, 7, 6, 4 or 2) whose tiles fit the LDS beside the weight; 0: none.
 static int conv_waves(int c_in, int c_out, size_t elem) {
   const int choices[] = {8, 7, 6, 4, 2};
@@ -326,6 +496,17 @@ static int conv_waves(int c_in, int c_out, size_t elem) {
 template <typename T>
 static int launch_conv_t(const void* x, const void* w, void* y, const int64_t* pix_offsets, const int64_t* tile_offsets,
                          int64_t B, int64_t total_tiles, int c_in, int c_out, int cus, hipStream_t stream) {
+  // Which kernel: see conv1x1_direct_kernel.  (total_tiles counts one tile too many per image.)
+  const int64_t windows = total_tiles - B > 0 ? total_tiles - B : 0;
+  const bool small = windows <= (int64_t(64) << 20) / (kConvTile * (int64_t)sizeof(T)) / c_out;
+  if (small || c_in > 96 || (c_in > 64 && c_out <= 2 * c_in)) {
+    // Four wavefronts per window while two would leave half of them idle or nearly so (128 -> 256
+    // on 3 200 and 35 000 pixels 22 -> 16 and 25 -> 21), two from there on (on 110 000 28 against 32).
+    if (c_out % 128 == 0 && windows <= 4 * (int64_t)cus) {
+      return launch_direct_ks<T, 4>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
+    }
+    return launch_direct_ks<T, 2>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
+  }
   switch (conv_waves(c_in, c_out, sizeof(T))) {
     case 8: return launch_conv_w<T, 8>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
     case 7: return launch_conv_w<T, 7>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);

@@ -1,0 +1,41 @@
+"""Row-major 1x1 convolution on both kernels and on either side of the lines between them: pixel
+counts around one and two 64-pixel windows, next to images that make the batch small or large."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+EDGES = [1, 2, 31, 32, 33, 63, 64, 65, 66, 127, 128, 129, 191, 193, 640]
+
+
+def _check(pixels, c_in, c_out, dtype):
+    import nestedtensor_amd as nt
+    g = torch.Generator("cuda").manual_seed(c_in + c_out)
+    maps = [torch.randn(c_in, 1, n, device=DEV, generator=g).to(dtype) for n in pixels]
+    w = (torch.randn(c_out, c_in, 1, 1, device=DEV, generator=g) * c_in ** -0.5).to(dtype)
+    got = torch.conv2d(nt.nested_tensor(maps, dtype=dtype, device=DEV), w)
+    # one rounding to the type, and fp32 sums of c_in products
+    unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    a = w.double().reshape(c_out, c_in)
+    for m, y in zip(maps, got.unbind()):
+        b = m.double().reshape(c_in, -1)
+        exact, size = a @ b, a.abs() @ b.abs()
+        err = (y.double().reshape(c_out, -1) - exact).abs()
+        assert bool((err <= unit * exact.abs() + c_in * 2.0 ** -23 * size + 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c_in,c_out", [(16, 32), (32, 128), (64, 256), (80, 96), (96, 512), (128, 64), (128, 384)])
+def test_conv1x1_small_batches(c_in, c_out, dtype):
+    _check(EDGES, c_in, c_out, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c_in,c_out,pixels", [
+    (64, 256, 131072 - 200), (64, 256, 131072 + 200),        # 64 MiB of result
+    (48, 128, 270001), (96, 256, 131072 + 200),              # whole lines
+    (112, 128, 270001), (96, 64, 540001),                    # too many channels for those
+    (128, 256, 1024 * 64 - 2000), (128, 256, 1024 * 64 + 200)])   # four, two wavefronts per window
+def test_conv1x1_large_batches(c_in, c_out, pixels, dtype):
+    _check(EDGES + [pixels] + EDGES, c_in, c_out, dtype)
