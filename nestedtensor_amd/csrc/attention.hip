@@ -842,22 +842,27 @@ __device__ __forceinline__ void attention_f32_tile(
 //  * V: transposed by the loads themselves, a lane fetching eight keys of its head dim
 //    (whole rows over the lanes): the keys that the score accumulators 8 s .. 8 s + 7 of a
 //    lane half hold, which makes those accumulators, split, the other operand.
-// The next tile but one is in flight in registers, the next one is split between the matrix
-// instructions of the current one.  Wavefronts without a query row only fetch.
+// Wavefronts without a query row only fetch.
+//
 // Bound by matrix and vector instructions, which share a SIMD badly: 48 matrix and some 300
 // vector instructions per tile of head_dim 64, of which the splits of P, K and V are 200
 // (measured apart, a SIMD keeps its matrix pipe full beside four vector instructions per
-// matrix instruction of each of two wavefronts; each further one costs its own time).
-// Against attention_f32_tile: 32 sequences of 32 to 512, 12 heads of 64: 126 -> 82 us; 8 of
-// 256 to 2048, 8 heads of 64: 239 -> 148; 8 heads of 32: 52 -> 38; 16 of 64 to 1024, 16 heads of
-// 128: 556 -> 456 (one wavefront per SIMD: its Q parts alone take 96 registers); 64 of 10 to 200,
-// 8 heads of 128: 79 -> 77.  Error against 64 bits 0.78 to 0.85 of what it was.
+// matrix instruction of each of two wavefronts; each further one costs its own time).  What
+// hides the fetch of a tile and the rest is other workgroups: one tile buffer and nothing
+// in flight in registers leave room for three per CU (128: two).  With two buffers and the
+// next tile in registers it was two (one): 100 sequences of 64 to 1024, 12 heads of 64 680 us, of
+// 128 1850, 200 of 1 to 16, 12 heads of 128 103; only a launch that does not fill those places is
+// slower for it (8 of 256 to 2048, 8 heads of 64 148, now 167).
+// Against attention_f32_tile, us: 32 sequences of 32 to 512, 12 heads of 64 126 -> 81; 100 of 64 to
+// 1024, 12 heads of 64 889 -> 573, of 32 529 -> 388, of 128 1976 -> 1139; 8 of 256 to 2048, 8 heads of
+// 64 239 -> 167; 256 of 4 to 64, 12 heads of 64 61 -> 41; 100 of 1 to 16, 12 heads of 128 36 -> 25.
+// Error against 64 bits 0.78 to 0.85 of what it was.
 template <int HD>
 struct SplitAttention {
   static constexpr int kKT = 32;
   static constexpr int kKPart = kKT * HD * 2, kBuf = 6 * kKPart;   // three parts of K, three of V
-  static constexpr int kLdsBytes = 2 * kBuf;
-  static_assert(kLdsBytes >= 2 * 32 * (2 * HD + 12) * (int)sizeof(float), "attention_f32_tile runs in the same LDS");
+  static constexpr int kF32Bytes = 2 * 32 * (2 * HD + 12) * (int)sizeof(float);   // attention_f32_tile's, in the same LDS
+  static constexpr int kLdsBytes = kBuf > kF32Bytes ? kBuf : kF32Bytes;
 };
 
 template <int HD>
@@ -915,9 +920,9 @@ __device__ __forceinline__ void attention_split_tile(
   const char* kbase = reinterpret_cast<const char*>(Kp + kv_begin * ldk + (int64_t)h * HD);
   const char* vbase = reinterpret_cast<const char*>(Vp + kv_begin * ldv + (int64_t)h * HD);
   const int64_t kld = ldk * 4, vld = ldv * 4;
-  float kraw[kPer][8], vraw[kPer][8];
   constexpr int kKeyPieces = HD / 8;
-  auto gload = [&](int64_t t) __attribute__((always_inline)) {
+  auto fetch = [&](int64_t t) __attribute__((always_inline)) {     // tile t into LDS
+    float kraw[kPer][8], vraw[kPer][8];
     const int64_t rest = Lk - t * kKT;
     const int last = rest < kKT ? (int)rest - 1 : kKT - 1;
     const char* kt = kbase + t * kKT * kld;
@@ -945,8 +950,6 @@ __device__ __forceinline__ void attention_split_tile(
         }
       }
     }
-  };
-  auto put = [&](char* buf) __attribute__((always_inline)) {
     if (fetches_k) {
 #pragma unroll
       for (int i = 0; i < kPer; ++i) {
@@ -956,7 +959,7 @@ __device__ __forceinline__ void attention_split_tile(
         split8(kraw[i], part);
 #pragma unroll
         for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
-        char* dst = buf + (piece * 32 + (key ^ (piece * (128 / HD) & 15))) * 16;
+        char* dst = lds + (piece * 32 + (key ^ (piece * (128 / HD) & 15))) * 16;
 #pragma unroll
         for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dst + p * kPart) = part[p];
       }
@@ -969,7 +972,7 @@ __device__ __forceinline__ void attention_split_tile(
 #pragma unroll
         for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
         // piece (sg, d): sg * HD + d counts the threads
-        char* dst = buf + 3 * kPart + (HD >= 64 ? tid + 256 * i : tid - 128) * 16;
+        char* dst = lds + 3 * kPart + (HD >= 64 ? tid + 256 * i : tid - 128) * 16;
 #pragma unroll
         for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dst + p * kPart) = part[p];
       }
@@ -986,26 +989,18 @@ __device__ __forceinline__ void attention_split_tile(
 
   const int64_t n_tiles = (Lk + kKT - 1) / kKT;
   if (n_tiles > 0) {
-    gload(0);
-    put(lds);
-    gload(n_tiles > 1 ? 1 : 0);
+    fetch(0);
   }
   __syncthreads();
   for (int64_t t = 0; t < n_tiles; ++t) {
-    const char* cur = lds + (t & 1) * S::kBuf;
-    char* next = lds + ((t + 1) & 1) * S::kBuf;
-    const int64_t ahead = t + 2 < n_tiles ? t + 2 : n_tiles - 1;     // past the end: not used
-    if (!active) {
-      put(next);
-      gload(ahead);
-    } else {
+    if (active) {
       acc16 s;
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = 0.0f;
 #pragma unroll
       for (int tt = 0; tt < kT; ++tt) {
         const int piece = 2 * tt + half;
-        const char* kp = cur + (piece * 32 + (col ^ (piece * (128 / HD) & 15))) * 16;
+        const char* kp = lds + (piece * 32 + (col ^ (piece * (128 / HD) & 15))) * 16;
         bf16x8 kf[3];
 #pragma unroll
         for (int p = 0; p < 3; ++p) kf[p] = *reinterpret_cast<const bf16x8*>(kp + p * kPart);
@@ -1013,8 +1008,6 @@ __device__ __forceinline__ void attention_split_tile(
         for (int p = 0; p < 6; ++p)
           s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kPa[p]], qf[tt][kPb[p]], s, 0, 0, 0);
       }
-      put(next);
-      gload(ahead);
       // accumulator i: key 8 (i / 4) + 4 half + i % 4 of the tile, query col
       const int64_t left = Lk - t * kKT;
       if (left < kKT) {
@@ -1053,7 +1046,7 @@ __device__ __forceinline__ void attention_split_tile(
         split8(x, part);
 #pragma unroll
         for (int j = 0; j < kJ; ++j) {
-          const char* vp = cur + 3 * kPart + ((2 * st + half) * HD + 32 * j + col) * 16;
+          const char* vp = lds + 3 * kPart + ((2 * st + half) * HD + 32 * j + col) * 16;
           bf16x8 vf[3];
 #pragma unroll
           for (int p = 0; p < 3; ++p) vf[p] = *reinterpret_cast<const bf16x8*>(vp + p * kPart);
@@ -1065,6 +1058,10 @@ __device__ __forceinline__ void attention_split_tile(
       }
     }
     __syncthreads();
+    if (t + 1 < n_tiles) {
+      fetch(t + 1);
+      __syncthreads();
+    }
   }
 
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
@@ -1100,7 +1097,7 @@ __device__ __forceinline__ void attention_split_tile(
 // Workgroup = (128 query rows, head, sequence) on a padded grid: tiles past a
 // sequence's last query row leave at once.
 template <int HD>
-__global__ __launch_bounds__(256, HD < 128 ? 2 : 1) void varlen_attention_f32_kernel(
+__global__ __launch_bounds__(256, HD < 128 ? 3 : 2) void varlen_attention_f32_kernel(
     const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
     const float* __restrict__ Vp, int64_t ldv, float* __restrict__ O, int64_t ldo,
     const int64_t* __restrict__ q_offsets, const int64_t* __restrict__ kv_offsets,
@@ -1119,7 +1116,7 @@ __global__ __launch_bounds__(256, HD < 128 ? 2 : 1) void varlen_attention_f32_ke
 // The same tiles from a work list (the items of nt_varlen_attention_vt): only
 // tiles that exist are launched, longest key sequences first, head fastest.
 template <int HD>
-__global__ __launch_bounds__(256, HD < 128 ? 2 : 1) void varlen_attention_f32_sched_kernel(
+__global__ __launch_bounds__(256, HD < 128 ? 3 : 2) void varlen_attention_f32_sched_kernel(
     const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
     const float* __restrict__ Vp, int64_t ldv, float* __restrict__ O, int64_t ldo,
     const int4* __restrict__ schedule, unsigned num_heads, float scale_log2e) {
