@@ -1535,18 +1535,26 @@ Tensor mha_rowmajor_packed(const Tensor& xq, const Tensor& xk, const Tensor& xv,
   Tensor out = at::empty({Tq, N}, xq.options());
   if (Tq == 0) return out;
   Tensor q, k, v;
-  int64_t qc = 0, kc = 0, vc = 0, ld = E;
+  int64_t qc = 0, kc = 0, vc = 0, ld = E, ld_kv = E;
   if (same) {
     q = project_rows(xq, W, b_in, 0, 3 * E, stream);     // [T, 3E]
     k = q;
     v = q;
     kc = E;
     vc = 2 * E;
-    ld = 3 * E;
+    ld = ld_kv = 3 * E;
   } else {
     q = project_rows(xq, W, b_in, 0, E, stream);
-    k = project_rows(xk, W, b_in, E, E, stream);
-    v = project_rows(xv, W, b_in, 2 * E, E, stream);
+    if (xk.const_data_ptr() == xv.const_data_ptr() && xk.stride(0) == xv.stride(0) && xk.size(0) == xv.size(0)) {
+      // key and value are one buffer: one projection [T, 2E], the buffer read once
+      k = project_rows(xk, W, b_in, E, 2 * E, stream);
+      v = k;
+      vc = E;
+      ld_kv = 2 * E;
+    } else {
+      k = project_rows(xk, W, b_in, E, E, stream);
+      v = project_rows(xv, W, b_in, 2 * E, E, stream);
+    }
   }
   const int64_t es = static_cast<int64_t>(xq.element_size());
   const char* qp = static_cast<const char*>(q.const_data_ptr()) + qc * es;
@@ -1559,10 +1567,10 @@ Tensor mha_rowmajor_packed(const Tensor& xq, const Tensor& xk, const Tensor& xv,
     TORCH_CHECK(schedule->scalar_type() == at::kInt && schedule->dim() == 2 && schedule->size(1) == 8 &&
                     schedule->is_contiguous() && schedule->device() == xq.device(),
                 "mha: schedule must be a contiguous int32 [n_work, 8] tensor on the input's device");
-    check(nt_varlen_attention_scheduled(qp, ld, kp, ld, vp, ld, attn.data_ptr(), E, schedule->const_data_ptr<int32_t>(),
+    check(nt_varlen_attention_scheduled(qp, ld, kp, ld_kv, vp, ld_kv, attn.data_ptr(), E, schedule->const_data_ptr<int32_t>(),
                                         schedule->size(0), num_heads, head_dim, static_cast<float>(scaling), dt, stream));
   } else {
-    check(nt_varlen_attention(qp, ld, kp, ld, vp, ld, attn.data_ptr(), E, q_offsets.const_data_ptr<int64_t>(),
+    check(nt_varlen_attention(qp, ld, kp, ld_kv, vp, ld_kv, attn.data_ptr(), E, q_offsets.const_data_ptr<int64_t>(),
                               kv_offsets.const_data_ptr<int64_t>(), B, num_heads, head_dim, max_q,
                               static_cast<float>(scaling), dt, stream));
   }
