@@ -343,14 +343,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> pack_device(at::TensorList tensors) {
   // launch, which also writes the device copy; a large one is uploaded from pinned
   // memory first
   const bool in_args = n <= nt_pack_table_max_entries();
-  Tensor host;
-  std::vector<int64_t> args;
-  if (in_args) {
-    args.resize(static_cast<size_t>(n));
-  } else {
-    host = at::empty({n}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-  }
-  int64_t* h = in_args ? args.data() : host.data_ptr<int64_t>();
+  Tensor host = in_args ? at::empty({n}, at::kLong)
+                        : at::empty({n}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  int64_t* h = host.data_ptr<int64_t>();
   int64_t* off = h + B * D;
   int64_t* ptrs = off + B + 1;
   int64_t acc = 0;
@@ -1051,19 +1046,19 @@ void check_attention_schedule(const Tensor& schedule, const Tensor& x) {
               "input's device");
 }
 
-void launch_attention_vt(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* vt, int64_t ldvt,
-                         void* attn, int64_t E, const Tensor& schedule, int64_t num_heads, int64_t head_dim,
+void launch_attention_vt(const void* q, int64_t ldq, const void* k, int64_t ldk, const Tensor& vt, int64_t ldvt,
+                         Tensor& attn, int64_t E, const Tensor& schedule, int64_t num_heads, int64_t head_dim,
                          int64_t total_kv, double scaling, int dt, void* stream) {
   if (schedule.dim() == 1) {
     TORCH_CHECK(head_dim == 64, "mha: the planned attention kernel covers head_dim 64 only");
     // the plan was made for one workgroup per compute unit of this device (attention_plan
     // below); a workgroup beyond the plan's own count returns at once
-    check(nt_varlen_attention_planned(q, ldq, k, ldk, vt, ldvt, attn, E,
-                                      schedule.const_data_ptr<int32_t>(), compute_units_of(schedule.device()), num_heads,
+    check(nt_varlen_attention_planned(q, ldq, k, ldk, vt.const_data_ptr(), ldvt, attn.data_ptr(), E,
+                                      schedule.const_data_ptr<int32_t>(), compute_units_of(attn.device()), num_heads,
                                       head_dim, total_kv, static_cast<float>(scaling), dt, stream));
     return;
   }
-  check(nt_varlen_attention_vt(q, ldq, k, ldk, vt, ldvt, attn, E,
+  check(nt_varlen_attention_vt(q, ldq, k, ldk, vt.const_data_ptr(), ldvt, attn.data_ptr(), E,
                                schedule.const_data_ptr<int32_t>(), schedule.size(0), num_heads, head_dim, total_kv,
                                static_cast<float>(scaling), dt, stream));
 }
@@ -1147,20 +1142,17 @@ Tensor mha_self_packed(const Tensor& x, const Tensor& schedule, int64_t num_head
   c10::hip::HIPGuard guard(x.device().index());
   void* stream = stream_of(x);
   const int dt = dtype_code(st);
+  Tensor qk = at::empty({T, 2 * E}, x.options());
+  Tensor vt = at::empty({E, ldvt}, x.options());
+  Tensor attn = at::empty({T, E}, x.options());
   Tensor out = at::empty({T, N}, x.options());
   if (T == 0) return out;
-  // Q | K, V transposed and the heads' outputs in one block, each from a 256-byte boundary on
-  const int64_t es = static_cast<int64_t>(x.element_size());
-  const int64_t qk_bytes = (T * 2 * E * es + 255) / 256 * 256, vt_bytes = (E * ldvt * es + 255) / 256 * 256;
-  Tensor block = at::empty({qk_bytes + vt_bytes + T * E * es}, x.options().dtype(at::kByte));
-  char* qk = static_cast<char*>(block.data_ptr());
-  char* vt = qk + qk_bytes;
-  char* attn = vt + vt_bytes;
   check(nt_linear_qkv(x.const_data_ptr(), x.stride(0), W.const_data_ptr(), b_in.defined() ? b_in.const_data_ptr() : nullptr,
-                      qk, 2 * E, vt, ldvt, T, E, E, dt, stream));
-  launch_attention_vt(qk, 2 * E, qk + E * es, 2 * E, vt, ldvt, attn, E, schedule, num_heads, head_dim, T, scaling, dt,
-                      stream);
-  check(nt_linear_act(attn, E, Wo.const_data_ptr(), b_out.defined() ? b_out.const_data_ptr() : nullptr,
+                      qk.data_ptr(), 2 * E, vt.data_ptr(), ldvt, T, E, E, dt, stream));
+  const char* kptr = static_cast<const char*>(qk.const_data_ptr()) + E * static_cast<int64_t>(x.element_size());
+  launch_attention_vt(qk.const_data_ptr(), 2 * E, kptr, 2 * E, vt, ldvt, attn, E, schedule, num_heads, head_dim, T,
+                      scaling, dt, stream);
+  check(nt_linear_act(attn.const_data_ptr(), E, Wo.const_data_ptr(), b_out.defined() ? b_out.const_data_ptr() : nullptr,
                       out.data_ptr(), N, T, N, E, 0, dt, stream));
   return out;
 }
@@ -1502,8 +1494,8 @@ Tensor mha_cross_packed(const Tensor& xq, const Tensor& xk, const Tensor& xv, co
                                vt.data_ptr(), ldvt, Tk, E, E, dt, stream));
   }
   Tensor attn = at::empty({Tq, E}, xq.options());
-  launch_attention_vt(q.const_data_ptr(), E, k.const_data_ptr(), E, vt.const_data_ptr(), ldvt, attn.data_ptr(), E, schedule,
-                      num_heads, head_dim, Tk, scaling, dt, stream);
+  launch_attention_vt(q.const_data_ptr(), E, k.const_data_ptr(), E, vt, ldvt, attn, E, schedule, num_heads, head_dim, Tk,
+                      scaling, dt, stream);
   check(nt_linear_act(attn.const_data_ptr(), E, Wo.const_data_ptr(), b_out.defined() ? b_out.const_data_ptr() : nullptr,
                       out.data_ptr(), N, Tq, N, E, 0, dt, stream));
   return out;

@@ -58,7 +58,12 @@ def _n_ragged(impl):
     """Number of leading constituent dims the row decode must walk: up to and
     including the last irregular dim.  Trailing regular dims are one contiguous
     run (the generalisation of _collapse_two_dims_3, masking.cpp:535-556)."""
-    return impl.ragged_dims()[0]
+    opt = impl.opt_sizes()[1:]
+    n = 1
+    for k, v in enumerate(opt):
+        if v is None:
+            n = k + 1
+    return n
 
 
 def _check_no_empty(impl):
@@ -403,24 +408,21 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
     if opt[2] != E:
         raise RuntimeError("query's embedding dimension %d does not match num_heads * head_dim = %d"
                            % (opt[2], E))
-    one = key is query and value is query           # self-attention: nothing to compare
-    if not one:
-        if key.opt_sizes()[2] != E or value.opt_sizes()[2] != E:
-            raise RuntimeError("key and value must have the embedding dimension of query.")
-        if key.B != query.B or value.B != query.B:
-            raise RuntimeError("query, key and value must hold the same number of sequences.")
-        if not _same_sizes(key, value):
-            raise RuntimeError("key and value must have the same nested size.")
-    buffer = query.buffer
-    _C.require_device(buffer, "multi-head attention")
-    dtype = buffer.dtype
+    if key.opt_sizes()[2] != E or value.opt_sizes()[2] != E:
+        raise RuntimeError("key and value must have the embedding dimension of query.")
+    if key.B != query.B or value.B != query.B:
+        raise RuntimeError("query, key and value must hold the same number of sequences.")
+    if not _same_sizes(key, value):
+        raise RuntimeError("key and value must have the same nested size.")
+    _C.require_device(query.buffer, "multi-head attention")
+    dtype = query.buffer.dtype
     W = in_proj_weight.contiguous()
-    if W.shape != (3 * E, E):
+    if tuple(W.shape) != (3 * E, E):
         raise RuntimeError("in_proj_weight must have shape [3 * embed_dim, embed_dim].")
-    xq = buffer.view(-1, E)
-    same = one or ((key is query or key.buffer.data_ptr() == buffer.data_ptr()) and
-                   (value is query or value.buffer.data_ptr() == buffer.data_ptr()) and
-                   _same_sizes(key, query))
+    xq = query.buffer.reshape(-1, E)
+    same = (key is query or key.buffer.data_ptr() == query.buffer.data_ptr()) and \
+        (value is query or value.buffer.data_ptr() == query.buffer.data_ptr()) and \
+        _same_sizes(key, query)
     mfma_path = head_dim in (32, 64, 128) and dtype in (torch.float16, torch.bfloat16)
     fused = same and mfma_path and (2 * E) % 128 == 0
     if in_proj_bias is not None:
@@ -435,7 +437,7 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
         # output projection: three launches, issued by one call into the extension
         out = _mha_self_packed(xq, _attention_work(query, None, num_heads, head_dim), num_heads, head_dim, W, in_proj_bias,
                                float(scaling), out_proj_weight, out_proj_bias)
-        return query.with_buffer(out.view(-1))
+        return query.with_buffer(out.reshape(-1))
     xk, xv = key.buffer.reshape(-1, E), value.buffer.reshape(-1, E)
     if mfma_path and (key.B == 0 or key.min_sizes()[0] > 0):
         # cross-attention (or an embedding size the fused projection does not tile),
