@@ -210,6 +210,158 @@ Tensor upload_table(const Tensor& table_in, c10::Device device) {
   return out;
 }
 
+// ---- ragged images: tables and launches of transposes and 1x1 convolutions ---------
+//
+// Bound by the host for all but large images.  One pass over the [B, 3] table builds what a
+// launch needs; built from a dozen small tensor operations each, the tables were most of
+// the 232 to 245 us that a 1x1 convolution, its activation, a channels-last conversion, a
+// second convolution and the way back took on images up to 128 pixels wide: 87 to 90 us now.
+
+// `sizes` with extent `dim` set to `value`.
+Tensor sizes_with_extent(const Tensor& sizes, int64_t dim, int64_t value) {
+  TORCH_CHECK(sizes.device().is_cpu() && sizes.scalar_type() == at::kLong && sizes.dim() == 2 && dim >= 0 &&
+                  dim < sizes.size(1),
+              "sizes_with_extent: the nested size must be a host int64 [B, D] table with that extent");
+  Tensor out = sizes.clone(at::MemoryFormat::Contiguous);
+  int64_t* o = out.data_ptr<int64_t>();
+  const int64_t B = out.size(0), D = out.size(1);
+  for (int64_t b = 0; b < B; ++b) o[b * D + dim] = value;
+  return out;
+}
+
+// Tile shape of nt_transpose_ragged: the strip kernels (a workgroup per 2048 bytes of the
+// long side) when the other side is at most 16, images of a few channels; 64 x 64 otherwise.
+// The larger tiles the library also accepts keep fewer workgroups in flight and measured
+// slower on every image shape tried.
+std::tuple<int64_t, int64_t> transpose_tile(int64_t max_rows, int64_t max_cols, int64_t elem_bytes) {
+  const int64_t strip = 2048 / elem_bytes;
+  if (max_rows <= 16 && max_cols > 64) return std::make_tuple(int64_t(16), strip);
+  if (max_cols <= 16 && max_rows > 64) return std::make_tuple(strip, int64_t(16));
+  return std::make_tuple(int64_t(64), int64_t(64));
+}
+
+// Which constituents a transpose sees: [C, H, W] stored row-major, to [H, W, C]; [H, W, C]
+// stored row-major, to [C, H, W]; [C, H, W] stored channels-last, to row-major.
+enum { kNchwToNhwc = 0, kNhwcToNchw = 1, kChannelsLastToRowMajor = 2 };
+
+// (device table, nested size of the result, tiles, tile rows, tile columns) of
+// nt_transpose_ragged for every constituent as a row-major [rows, cols] matrix.  The table
+// is int64 [4, B + 1]: rows, cols, first tile and first element of every constituent.  A
+// tile of 0 x 0: nt_transpose_ragged_lines, for 2-byte output rows that do not begin on
+// 128-byte lines.  With a
+// host device the table stays on the host.
+std::tuple<Tensor, Tensor, int64_t, int64_t, int64_t> transpose_tables(const Tensor& sizes_in, int64_t mode,
+                                                                       int64_t elem_bytes, c10::Device device) {
+  TORCH_CHECK(sizes_in.device().is_cpu() && sizes_in.scalar_type() == at::kLong && sizes_in.dim() == 2 &&
+                  sizes_in.size(1) == 3 && mode >= kNchwToNhwc && mode <= kChannelsLastToRowMajor && elem_bytes > 0,
+              "transpose_tables: the nested size must be a host int64 [B, 3] table");
+  const Tensor sizes = sizes_in.contiguous();
+  const int64_t B = sizes.size(0);
+  const int64_t* s = sizes.const_data_ptr<int64_t>();
+  Tensor result = mode == kChannelsLastToRowMajor ? sizes.clone() : at::empty({B, 3}, at::kLong);
+  Tensor meta = at::zeros({4, B + 1}, at::kLong);
+  int64_t* rows = meta.data_ptr<int64_t>();
+  int64_t *cols = rows + B + 1, *tiles = cols + B + 1, *elems = tiles + B + 1;
+  int64_t max_rows = 0, max_cols = 0;
+  bool whole_lines = true;
+  for (int64_t b = 0; b < B; ++b) {
+    const int64_t x = s[3 * b], y = s[3 * b + 1], z = s[3 * b + 2];
+    if (mode == kNchwToNhwc) {
+      rows[b] = x;
+      cols[b] = y * z;
+    } else if (mode == kNhwcToNchw) {
+      rows[b] = x * y;
+      cols[b] = z;
+    } else {
+      rows[b] = y * z;
+      cols[b] = x;
+    }
+    if (mode != kChannelsLastToRowMajor) {
+      int64_t* r = result.data_ptr<int64_t>() + 3 * b;
+      r[0] = mode == kNchwToNhwc ? y : z;
+      r[1] = mode == kNchwToNhwc ? z : x;
+      r[2] = mode == kNchwToNhwc ? x : y;
+    }
+    max_rows = std::max(max_rows, rows[b]);
+    max_cols = std::max(max_cols, cols[b]);
+    whole_lines = whole_lines && rows[b] % 64 == 0;
+  }
+  int64_t tr, tc;
+  std::tie(tr, tc) = transpose_tile(max_rows, max_cols, elem_bytes);
+  const bool lines = tr == 64 && tc == 64 && elem_bytes == 2 && !whole_lines;
+  for (int64_t b = 0; b < B; ++b) {
+    int64_t n = ((rows[b] + tr - 1) / tr) * ((cols[b] + tc - 1) / tc);
+    if (lines) n = rows[b] > 0 && cols[b] > 0 ? ((rows[b] + 63) / 64 + 1) * ((cols[b] + 63) / 64) : 0;
+    tiles[b + 1] = tiles[b] + n;
+    elems[b + 1] = elems[b] + rows[b] * cols[b];
+  }
+  if (lines) tr = tc = 0;
+  const int64_t total = tiles[B];
+  return std::make_tuple(device.is_cpu() ? meta : upload_table(meta, device), result, total, tr, tc);
+}
+
+Tensor transpose_packed(const Tensor& buffer, const Tensor& table, int64_t total_tiles, int64_t tr, int64_t tc) {
+  require_device(buffer, "transpose");
+  TORCH_CHECK(buffer.dim() == 1 && buffer.is_contiguous() && table.dim() == 2 && table.size(0) == 4 &&
+                  table.scalar_type() == at::kLong && table.is_contiguous() && table.device() == buffer.device(),
+              "transpose: a packed buffer and its table on one device");
+  c10::hip::HIPGuard guard(buffer.device().index());
+  Tensor out = at::empty_like(buffer);
+  if (total_tiles == 0) return out;
+  const int64_t B = table.size(1) - 1, es = static_cast<int64_t>(buffer.element_size());
+  const int64_t* rows = table.const_data_ptr<int64_t>();
+  const int64_t *cols = rows + B + 1, *tiles = cols + B + 1, *elems = tiles + B + 1;
+  if (tr == 0) {
+    check(nt_transpose_ragged_lines(buffer.const_data_ptr(), out.data_ptr(), elems, rows, cols, tiles, B, total_tiles,
+                                    static_cast<int>(es), stream_of(buffer)));
+  } else {
+    check(nt_transpose_ragged(buffer.const_data_ptr(), out.data_ptr(), elems, rows, cols, tiles, B, total_tiles,
+                              static_cast<int>(tr), static_cast<int>(tc), static_cast<int>(es), stream_of(buffer)));
+  }
+  return out;
+}
+
+// (device table, tiles, pixels) of nt_conv1x1_nchw: int64 [2, B + 1], the first pixel and the
+// first tile of every image.  A tile is one 128-byte line of every output row; the rows'
+// lines start up to a tile less one pixel before a multiple of the tile, hence one tile
+// more than the pixels fill.
+std::tuple<Tensor, int64_t, int64_t> conv1x1_tables(const Tensor& sizes_in, c10::Device device) {
+  TORCH_CHECK(sizes_in.device().is_cpu() && sizes_in.scalar_type() == at::kLong && sizes_in.dim() == 2 &&
+                  sizes_in.size(1) == 3,
+              "conv1x1_tables: the nested size must be a host int64 [B, 3] table");
+  const Tensor sizes = sizes_in.contiguous();
+  const int64_t B = sizes.size(0), tile = nt_conv1x1_tile_pixels();
+  const int64_t* s = sizes.const_data_ptr<int64_t>();
+  Tensor meta = at::zeros({2, B + 1}, at::kLong);
+  int64_t *pixels = meta.data_ptr<int64_t>(), *tiles = pixels + B + 1;
+  for (int64_t b = 0; b < B; ++b) {
+    const int64_t p = s[3 * b + 1] * s[3 * b + 2];
+    pixels[b + 1] = pixels[b] + p;
+    tiles[b + 1] = tiles[b] + (p > 0 ? (p + tile - 1) / tile + 1 : 0);
+  }
+  const int64_t total_tiles = tiles[B], total_pixels = pixels[B];
+  return std::make_tuple(device.is_cpu() ? meta : upload_table(meta, device), total_tiles, total_pixels);
+}
+
+Tensor conv1x1_packed(const Tensor& buffer, const Tensor& weight_in, const Tensor& table, int64_t total_tiles,
+                      int64_t total_pixels) {
+  require_device(buffer, "conv2d");
+  const Tensor weight = weight_in.contiguous();
+  TORCH_CHECK(weight.dim() == 2 && weight.scalar_type() == buffer.scalar_type() && weight.device() == buffer.device() &&
+                  buffer.dim() == 1 && buffer.is_contiguous() && buffer.numel() == total_pixels * weight.size(1) &&
+                  table.dim() == 2 && table.size(0) == 2 && table.scalar_type() == at::kLong && table.is_contiguous() &&
+                  table.device() == buffer.device(),
+              "conv1x1: a packed buffer, its table and a [C_out, C_in] weight of one dtype and device");
+  c10::hip::HIPGuard guard(buffer.device().index());
+  Tensor out = at::empty({total_pixels * weight.size(0)}, buffer.options());
+  if (total_tiles == 0) return out;
+  const int64_t B = table.size(1) - 1;
+  const int64_t* pixels = table.const_data_ptr<int64_t>();
+  check(nt_conv1x1_nchw(buffer.const_data_ptr(), weight.const_data_ptr(), out.data_ptr(), pixels, pixels + B + 1, B,
+                        total_tiles, weight.size(1), weight.size(0), dtype_code(buffer.scalar_type()), stream_of(buffer)));
+  return out;
+}
+
 // ---- packed <-> padded --------------------------------------------------------
 
 struct PadArgs {
@@ -343,9 +495,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> pack_device(at::TensorList tensors) {
   // launch, which also writes the device copy; a large one is uploaded from pinned
   // memory first
   const bool in_args = n <= nt_pack_table_max_entries();
-  Tensor host = in_args ? at::empty({n}, at::kLong)
-                        : at::empty({n}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-  int64_t* h = host.data_ptr<int64_t>();
+  Tensor host;
+  std::vector<int64_t> args;
+  if (in_args) {
+    args.resize(static_cast<size_t>(n));
+  } else {
+    host = at::empty({n}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  }
+  int64_t* h = in_args ? args.data() : host.data_ptr<int64_t>();
   int64_t* off = h + B * D;
   int64_t* ptrs = off + B + 1;
   int64_t acc = 0;
@@ -1046,19 +1203,19 @@ void check_attention_schedule(const Tensor& schedule, const Tensor& x) {
               "input's device");
 }
 
-void launch_attention_vt(const void* q, int64_t ldq, const void* k, int64_t ldk, const Tensor& vt, int64_t ldvt,
-                         Tensor& attn, int64_t E, const Tensor& schedule, int64_t num_heads, int64_t head_dim,
+void launch_attention_vt(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* vt, int64_t ldvt,
+                         void* attn, int64_t E, const Tensor& schedule, int64_t num_heads, int64_t head_dim,
                          int64_t total_kv, double scaling, int dt, void* stream) {
   if (schedule.dim() == 1) {
     TORCH_CHECK(head_dim == 64, "mha: the planned attention kernel covers head_dim 64 only");
     // the plan was made for one workgroup per compute unit of this device (attention_plan
     // below); a workgroup beyond the plan's own count returns at once
-    check(nt_varlen_attention_planned(q, ldq, k, ldk, vt.const_data_ptr(), ldvt, attn.data_ptr(), E,
-                                      schedule.const_data_ptr<int32_t>(), compute_units_of(attn.device()), num_heads,
+    check(nt_varlen_attention_planned(q, ldq, k, ldk, vt, ldvt, attn, E,
+                                      schedule.const_data_ptr<int32_t>(), compute_units_of(schedule.device()), num_heads,
                                       head_dim, total_kv, static_cast<float>(scaling), dt, stream));
     return;
   }
-  check(nt_varlen_attention_vt(q, ldq, k, ldk, vt.const_data_ptr(), ldvt, attn.data_ptr(), E,
+  check(nt_varlen_attention_vt(q, ldq, k, ldk, vt, ldvt, attn, E,
                                schedule.const_data_ptr<int32_t>(), schedule.size(0), num_heads, head_dim, total_kv,
                                static_cast<float>(scaling), dt, stream));
 }
@@ -1142,17 +1299,20 @@ Tensor mha_self_packed(const Tensor& x, const Tensor& schedule, int64_t num_head
   c10::hip::HIPGuard guard(x.device().index());
   void* stream = stream_of(x);
   const int dt = dtype_code(st);
-  Tensor qk = at::empty({T, 2 * E}, x.options());
-  Tensor vt = at::empty({E, ldvt}, x.options());
-  Tensor attn = at::empty({T, E}, x.options());
   Tensor out = at::empty({T, N}, x.options());
   if (T == 0) return out;
+  // Q | K, V transposed and the heads' outputs in one block, each from a 256-byte boundary on
+  const int64_t es = static_cast<int64_t>(x.element_size());
+  const int64_t qk_bytes = (T * 2 * E * es + 255) / 256 * 256, vt_bytes = (E * ldvt * es + 255) / 256 * 256;
+  Tensor block = at::empty({qk_bytes + vt_bytes + T * E * es}, x.options().dtype(at::kByte));
+  char* qk = static_cast<char*>(block.data_ptr());
+  char* vt = qk + qk_bytes;
+  char* attn = vt + vt_bytes;
   check(nt_linear_qkv(x.const_data_ptr(), x.stride(0), W.const_data_ptr(), b_in.defined() ? b_in.const_data_ptr() : nullptr,
-                      qk.data_ptr(), 2 * E, vt.data_ptr(), ldvt, T, E, E, dt, stream));
-  const char* kptr = static_cast<const char*>(qk.const_data_ptr()) + E * static_cast<int64_t>(x.element_size());
-  launch_attention_vt(qk.const_data_ptr(), 2 * E, kptr, 2 * E, vt, ldvt, attn, E, schedule, num_heads, head_dim, T,
-                      scaling, dt, stream);
-  check(nt_linear_act(attn.const_data_ptr(), E, Wo.const_data_ptr(), b_out.defined() ? b_out.const_data_ptr() : nullptr,
+                      qk, 2 * E, vt, ldvt, T, E, E, dt, stream));
+  launch_attention_vt(qk, 2 * E, qk + E * es, 2 * E, vt, ldvt, attn, E, schedule, num_heads, head_dim, T, scaling, dt,
+                      stream);
+  check(nt_linear_act(attn, E, Wo.const_data_ptr(), b_out.defined() ? b_out.const_data_ptr() : nullptr,
                       out.data_ptr(), N, T, N, E, 0, dt, stream));
   return out;
 }
@@ -1494,8 +1654,8 @@ Tensor mha_cross_packed(const Tensor& xq, const Tensor& xk, const Tensor& xv, co
                                vt.data_ptr(), ldvt, Tk, E, E, dt, stream));
   }
   Tensor attn = at::empty({Tq, E}, xq.options());
-  launch_attention_vt(q.const_data_ptr(), E, k.const_data_ptr(), E, vt, ldvt, attn, E, schedule, num_heads, head_dim, Tk,
-                      scaling, dt, stream);
+  launch_attention_vt(q.const_data_ptr(), E, k.const_data_ptr(), E, vt.const_data_ptr(), ldvt, attn.data_ptr(), E, schedule,
+                      num_heads, head_dim, Tk, scaling, dt, stream);
   check(nt_linear_act(attn.const_data_ptr(), E, Wo.const_data_ptr(), b_out.defined() ? b_out.const_data_ptr() : nullptr,
                       out.data_ptr(), N, Tq, N, E, 0, dt, stream));
   return out;
@@ -1635,6 +1795,12 @@ TORCH_LIBRARY(nestedtensor, m) {
   m.def("sizes_with_last(Tensor sizes, int last, bool append) -> Tensor");
   m.def("upload_sizes(Tensor sizes, Device device) -> (Tensor, Tensor)");
   m.def("upload_table(Tensor table, Device device) -> Tensor");
+  m.def("sizes_with_extent(Tensor sizes, int dim, int value) -> Tensor");
+  m.def("transpose_tile(int max_rows, int max_cols, int elem_bytes) -> (int, int)", transpose_tile);
+  m.def("transpose_tables(Tensor sizes, int mode, int elem_bytes, Device device) -> (Tensor, Tensor, int, int, int)");
+  m.def("transpose_packed(Tensor buffer, Tensor table, int total_tiles, int tile_rows, int tile_cols) -> Tensor");
+  m.def("conv1x1_tables(Tensor sizes, Device device) -> (Tensor, int, int)");
+  m.def("conv1x1_packed(Tensor buffer, Tensor weight, Tensor table, int total_tiles, int total_pixels) -> Tensor");
   m.def("attention_schedule(Tensor q_sizes, Tensor k_sizes, int q_tile, Device device) -> Tensor");
   m.def("attention_plan(Tensor q_lens, Tensor k_lens, int num_heads, int head_dim, Device device) -> Tensor");
   m.def("mha_self_packed(Tensor x, Tensor schedule, int num_heads, int head_dim, Tensor in_proj_weight, "
@@ -1657,6 +1823,8 @@ TORCH_LIBRARY_IMPL(nestedtensor, CUDA, m) {
   m.impl("build_mask", build_mask);
   m.impl("from_padded_value_lowered", from_padded_value_lowered);
   m.impl("nt_from_padded_tensor", nt_from_padded_tensor_op);
+  m.impl("transpose_packed", transpose_packed);
+  m.impl("conv1x1_packed", conv1x1_packed);
   m.impl("linear_packed", linear_packed);
   m.impl("mha_self_packed", mha_self_packed);
   m.impl("mha_cross_packed", mha_cross_packed);
@@ -1674,12 +1842,20 @@ TORCH_LIBRARY_IMPL(nestedtensor, CUDA, m) {
 // Operators on plain tensors of any device: merge_tensor_mask is host logic over
 // torch reductions; nt_from_tensor_mask answers the trivial masks (empty, one
 // element) for any device and raises for host tensors otherwise.
+// These two pass no gradient on: their results require none, also where a weight does.
+TORCH_LIBRARY_IMPL(nestedtensor, AutogradCUDA, m) {
+  m.impl("transpose_packed", torch::CppFunction::makeFallthrough());
+  m.impl("conv1x1_packed", torch::CppFunction::makeFallthrough());
+}
 TORCH_LIBRARY_IMPL(nestedtensor, CompositeExplicitAutograd, m) {
   m.impl("merge_tensor_mask", merge_tensor_mask);
   m.impl("size_summary", size_summary);
   m.impl("sizes_with_last", sizes_with_last);
   m.impl("upload_sizes", upload_sizes);
   m.impl("upload_table", upload_table);
+  m.impl("sizes_with_extent", sizes_with_extent);
+  m.impl("transpose_tables", transpose_tables);
+  m.impl("conv1x1_tables", conv1x1_tables);
   m.impl("attention_schedule", attention_schedule);
   m.impl("attention_plan", attention_plan);   // host lengths in, device plan out
   m.impl("nt_from_tensor_mask", nt_from_tensor_mask_op);

@@ -24,7 +24,7 @@ from . import _C
 
 
 class NestedTensorImpl:
-    __slots__ = ("buffer", "sizes", "_opt_sizes", "_given", "_summary", "_attn_plan", "_kept", "channels_last")
+    __slots__ = ("buffer", "sizes", "_opt_sizes", "_given", "_summary", "_attn_plan", "_kept", "_ragged", "channels_last")
 
     def __init__(self, buffer, sizes, channels_last=False):
         """buffer: 1-D contiguous tensor; sizes: CPU int64 [B, D], or 0-d for an
@@ -45,6 +45,7 @@ class NestedTensorImpl:
         self._summary = None
         self._attn_plan = None
         self._kept = {}
+        self._ragged = None
 
     # ---- host metadata ----------------------------------------------------
     @property
@@ -101,8 +102,19 @@ class NestedTensorImpl:
     def min_sizes(self):
         return self._extents(2)
 
+    def ragged_dims(self):
+        """(number of leading constituent dims up to and including the last irregular one, at
+        least 1; whether a constituent is empty): what every padding call asks, answered once."""
+        if self._ragged is None:
+            n = 1
+            for k, v in enumerate(self._extents(0)):
+                if v < 0:
+                    n = k + 1
+            self._ragged = n, 0 in self._extents(2)
+        return self._ragged
+
     def has_empty_constituent(self):
-        return 0 in self._extents(2)
+        return self.ragged_dims()[1]
 
     def shapes(self):
         return [tuple(int(v) for v in row) for row in self.sizes] if self.sizes.dim() > 0 else []
@@ -247,6 +259,7 @@ class NestedTensorImpl:
                                self.channels_last if channels_last is None else channels_last)
         out._opt_sizes = self._opt_sizes
         out._summary = self._summary
+        out._ragged = self._ragged
         if buffer.device == self.buffer.device:
             out._given = self._given
             out._attn_plan = self._attn_plan

@@ -56,7 +56,13 @@ def _wrap_result(result):
     return NestedTensor(result) if isinstance(result, NestedTensorImpl) else result
 
 
+# what most arguments beside the nested tensors are: nothing to look into
+_AS_THEY_ARE = {torch.Tensor, torch.nn.Parameter, int, float, bool, str, type(None)}
+
+
 def _unwrap(a):
+    if type(a) in _AS_THEY_ARE:
+        return a
     if isinstance(a, NestedTensor):
         return a._impl
     if isinstance(a, (list, tuple)):
@@ -68,6 +74,8 @@ def _unwrap_row_major(a):
     """_unwrap for handlers that read the buffer as row-major constituents: a
     channels-last operand is brought back first, as the reference's ops do with
     NestedTensor_contiguous (e.g. BinaryOps.cpp:47, masking.cpp:562)."""
+    if type(a) in _AS_THEY_ARE:
+        return a
     if isinstance(a, NestedTensor):
         return ops.contiguous(a._impl)
     if isinstance(a, (list, tuple)):
@@ -369,7 +377,8 @@ class NestedTensor:
             handler = _HANDLERS.get(func.overloadpacket)
         if handler is not None:
             unwrap = _unwrap if handler in _LAYOUT_AWARE else _unwrap_row_major
-            return _wrap_result(handler(*unwrap(args), **unwrap(kwargs)))
+            result = handler(*[unwrap(a) for a in args], **kwargs)
+            return NestedTensor(result) if type(result) is NestedTensorImpl else _wrap_result(result)
         if func is torch.nn.functional.linear:
             return _wrap_result(_nn_functional_linear(*_unwrap_row_major(args), **_unwrap_row_major(kwargs)))
         raise NotImplementedError(

@@ -22,7 +22,11 @@ from .impl import NestedTensorImpl
 # operators that do the work live in the C++ extension csrc/torch_ops.cpp
 # (TORCH_LIBRARY(nestedtensor, ...)), loaded by _C.  Overloads are resolved once.
 _sizes_with_last = _C.ops.sizes_with_last.default
-_upload_table = _C.ops.upload_table.default
+_sizes_with_extent = _C.ops.sizes_with_extent.default
+_transpose_tables = _C.ops.transpose_tables.default
+_transpose_packed = _C.ops.transpose_packed.default
+_conv1x1_tables = _C.ops.conv1x1_tables.default
+_conv1x1_packed = _C.ops.conv1x1_packed.default
 _add_padding = _C.ops.add_padding.default
 _add_padding_mask = _C.ops.add_padding_mask.default
 _remove_padding = _C.ops.remove_padding.default
@@ -58,12 +62,7 @@ def _n_ragged(impl):
     """Number of leading constituent dims the row decode must walk: up to and
     including the last irregular dim.  Trailing regular dims are one contiguous
     run (the generalisation of _collapse_two_dims_3, masking.cpp:535-556)."""
-    opt = impl.opt_sizes()[1:]
-    n = 1
-    for k, v in enumerate(opt):
-        if v is None:
-            n = k + 1
-    return n
+    return impl.ragged_dims()[0]
 
 
 def _check_no_empty(impl):
@@ -408,21 +407,24 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
     if opt[2] != E:
         raise RuntimeError("query's embedding dimension %d does not match num_heads * head_dim = %d"
                            % (opt[2], E))
-    if key.opt_sizes()[2] != E or value.opt_sizes()[2] != E:
-        raise RuntimeError("key and value must have the embedding dimension of query.")
-    if key.B != query.B or value.B != query.B:
-        raise RuntimeError("query, key and value must hold the same number of sequences.")
-    if not _same_sizes(key, value):
-        raise RuntimeError("key and value must have the same nested size.")
-    _C.require_device(query.buffer, "multi-head attention")
-    dtype = query.buffer.dtype
+    one = key is query and value is query           # self-attention: nothing to compare
+    if not one:
+        if key.opt_sizes()[2] != E or value.opt_sizes()[2] != E:
+            raise RuntimeError("key and value must have the embedding dimension of query.")
+        if key.B != query.B or value.B != query.B:
+            raise RuntimeError("query, key and value must hold the same number of sequences.")
+        if not _same_sizes(key, value):
+            raise RuntimeError("key and value must have the same nested size.")
+    buffer = query.buffer
+    _C.require_device(buffer, "multi-head attention")
+    dtype = buffer.dtype
     W = in_proj_weight.contiguous()
-    if tuple(W.shape) != (3 * E, E):
+    if W.shape != (3 * E, E):
         raise RuntimeError("in_proj_weight must have shape [3 * embed_dim, embed_dim].")
-    xq = query.buffer.reshape(-1, E)
-    same = (key is query or key.buffer.data_ptr() == query.buffer.data_ptr()) and \
-        (value is query or value.buffer.data_ptr() == query.buffer.data_ptr()) and \
-        _same_sizes(key, query)
+    xq = buffer.view(-1, E)
+    same = one or ((key is query or key.buffer.data_ptr() == buffer.data_ptr()) and
+                   (value is query or value.buffer.data_ptr() == buffer.data_ptr()) and
+                   _same_sizes(key, query))
     mfma_path = head_dim in (32, 64, 128) and dtype in (torch.float16, torch.bfloat16)
     fused = same and mfma_path and (2 * E) % 128 == 0
     if in_proj_bias is not None:
@@ -437,7 +439,7 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
         # output projection: three launches, issued by one call into the extension
         out = _mha_self_packed(xq, _attention_work(query, None, num_heads, head_dim), num_heads, head_dim, W, in_proj_bias,
                                float(scaling), out_proj_weight, out_proj_bias)
-        return query.with_buffer(out.reshape(-1))
+        return query.with_buffer(out.view(-1))
     xk, xv = key.buffer.reshape(-1, E), value.buffer.reshape(-1, E)
     if mfma_path and (key.B == 0 or key.min_sizes()[0] > 0):
         # cross-attention (or an embedding size the fused projection does not tile),
@@ -697,29 +699,9 @@ def _conv1x1_row_major(impl, w2d):
     if impl.channels_last or buf.dtype not in (torch.float16, torch.bfloat16) or \
             not _C.lib.nt_conv1x1_supported(c_in, c_out, _C.dtype_code(buf.dtype)):
         return None
-    tn = int(_C.lib.nt_conv1x1_tile_pixels())
-    B = impl.B
-
-    def tables():
-        pix = impl.sizes[:, 1] * impl.sizes[:, 2]
-        meta = torch.zeros((2, B + 1), dtype=torch.int64)
-        meta[0, 1:] = torch.cumsum(pix, 0)
-        # a tile is one 128-byte line of every output row; the rows' lines start up to
-        # tn - 1 pixels before a multiple of tn, hence one tile more than ceil(P / tn)
-        meta[1, 1:] = torch.cumsum(torch.where(pix > 0, (pix + tn - 1) // tn + 1, pix), 0)
-        return _upload_table(meta, buf.device).unbind(0), int(meta[1, B])
-
-    (pixels_dev, tiles_dev), total_tiles = impl.kept(("conv1x1", tn), tables)
-    w2d = w2d.contiguous()
-    sizes = impl.sizes.clone()
-    sizes[:, 0] = c_out
-    out = torch.empty(int(sizes.prod(1).sum()), dtype=buf.dtype, device=buf.device)
-    if total_tiles:
-        with _C.on_device(buf.device):
-            _C.check(_C.lib.nt_conv1x1_nchw(_C.ptr(buf), _C.ptr(w2d), _C.ptr(out), _C.ptr(pixels_dev),
-                                            _C.ptr(tiles_dev), B, total_tiles, c_in, c_out,
-                                            _C.dtype_code(buf.dtype), _C.current_stream(buf.device)))
-    return NestedTensorImpl(out, sizes)
+    table, total_tiles, total_pixels = impl.kept("conv1x1", lambda: _conv1x1_tables(impl.sizes, buf.device))
+    out = _conv1x1_packed(buf, w2d, table, total_tiles, total_pixels)
+    return NestedTensorImpl(out, _sizes_with_extent(impl.sizes, 0, c_out))
 
 
 def conv2d(impl, weight, bias=None, stride=1, padding=0, dilation=1, groups=1):
@@ -738,19 +720,14 @@ def conv2d(impl, weight, bias=None, stride=1, padding=0, dilation=1, groups=1):
             # the buffer already is the [pixels, C_in] matrix, and the product is
             # the channels-last result (conv2d.cpp:43-60): no transposes
             y = linear(impl.buffer.reshape(-1, c_in), weight.reshape(c_out, c_in), None)
-            sizes = impl.sizes.clone()
-            sizes[:, 0] = c_out
-            res = NestedTensorImpl(y.reshape(-1), sizes, channels_last=True)
-            return res
+            return NestedTensorImpl(y.reshape(-1), _sizes_with_extent(impl.sizes, 0, c_out), channels_last=True)
         y = _conv1x1_row_major(impl, weight.reshape(c_out, c_in))
         if y is not None:
             return y
         # NCHW -> NHWC on the packed buffer, [pixels, C_in] x W^T, and back (conv2d.cpp:61-73)
         nhwc = transpose_nchw_nhwc(impl)
         y = linear(nhwc.buffer.reshape(-1, c_in), weight.reshape(c_out, c_in), None)
-        sizes = nhwc.sizes.clone()
-        sizes[:, 2] = c_out
-        return transpose_nhwc_nchw(NestedTensorImpl(y.reshape(-1), sizes))
+        return transpose_nhwc_nchw(NestedTensorImpl(y.reshape(-1), _sizes_with_extent(nhwc.sizes, 2, c_out)))
     return _dense_via_padding(
         impl, 0.0, lambda x: torch.conv2d(x, weight, bias, s, p, d, groups), weight.size(0), k, s, p, d)
 
@@ -963,60 +940,29 @@ def to_packed_sequence(impl):
 # ---- channels-last ragged images: per-constituent transposes ------------------------
 
 def _transpose_tile(max_rows, max_cols, elem_bytes):
-    """Tile shape for nt_transpose_ragged: the strip kernels (a workgroup per 2048
-    bytes of the long side) when the other side is at most 16, images of a few
-    channels; 64 x 64 otherwise.  The larger tiles the library also accepts keep
-    fewer workgroups in flight and measured slower on every image shape tried."""
-    strip = 2048 // elem_bytes
-    if max_rows <= 16 and max_cols > 64:
-        return 16, strip
-    if max_cols <= 16 and max_rows > 64:
-        return strip, 16
-    return 64, 64
+    """Tile shape for nt_transpose_ragged (transpose_tile in the extension)."""
+    return _C.ops.transpose_tile.default(max_rows, max_cols, elem_bytes)
 
 
-def _transpose_constituents(impl, rows, cols, new_sizes, which):
-    """Every constituent, seen as a row-major [rows[b], cols[b]] matrix, is
-    transposed in place of its slot of the packed buffer (nt_transpose_ragged).
-    The device copy of (rows, cols, tile offsets) depends on the nested size and
-    the direction `which` only and is kept with the nested size."""
+# what a transpose sees of its constituents (transpose_tables in the extension)
+_NCHW_TO_NHWC, _NHWC_TO_NCHW, _CHANNELS_LAST_TO_ROW_MAJOR = 0, 1, 2
+
+
+def _transpose_constituents(impl, mode):
+    """Every constituent, seen as a row-major [rows, cols] matrix, is transposed in place of
+    its slot of the packed buffer (nt_transpose_ragged): (buffer, nested size of the result).
+    The device table of the launch depends on the nested size, the mode and the element
+    size only and is kept with the nested size."""
     buf = impl.buffer
     _C.require_device(buf, "transpose")
-    B = impl.B
-    which = (which, buf.element_size())       # the tile shape depends on the element size
+    elem_bytes = buf.element_size()
+    table, sizes, total_tiles, tr, tc = impl.kept(
+        ("transpose", mode, elem_bytes), lambda: _transpose_tables(impl.sizes, mode, elem_bytes, buf.device))
+    return _transpose_packed(buf, table, total_tiles, tr, tc), sizes
 
-    def tables():
-        tr, tc = _transpose_tile(int(rows.max()) if B else 0, int(cols.max()) if B else 0, buf.element_size())
-        if (tr, tc) == (64, 64) and buf.element_size() == 2 and bool((rows % 64 != 0).any()):
-            # output rows that do not begin on 128-byte lines: the kernel that gives every
-            # output row its own line-aligned window (tile shape recorded as 0 x 0)
-            tr = tc = 0
-            tiles = torch.where((rows > 0) & (cols > 0), ((rows + 63) // 64 + 1) * ((cols + 63) // 64),
-                                torch.zeros_like(rows))
-        else:
-            tiles = ((rows + tr - 1) // tr) * ((cols + tc - 1) // tc)
-        # one table, one launch: rows, cols, first tile and first element of every constituent
-        meta = torch.zeros((4, B + 1), dtype=torch.int64)
-        meta[0, :B], meta[1, :B] = rows, cols
-        meta[2, 1:] = torch.cumsum(tiles, 0)
-        meta[3, 1:] = torch.cumsum(rows * cols, 0)
-        return _upload_table(meta, buf.device).unbind(0), int(meta[2, B]), tr, tc
 
-    (rows_dev, cols_dev, tiles_dev, offsets_dev), total_tiles, tr, tc = impl.kept(which, tables)
-    out = torch.empty_like(buf)
-    if total_tiles:
-        with _C.on_device(buf.device):
-            if tr == 0:
-                _C.check(_C.lib.nt_transpose_ragged_lines(
-                    _C.ptr(buf), _C.ptr(out), _C.ptr(offsets_dev), _C.ptr(rows_dev),
-                    _C.ptr(cols_dev), _C.ptr(tiles_dev), B, total_tiles, buf.element_size(),
-                    _C.current_stream(buf.device)))
-            else:
-                _C.check(_C.lib.nt_transpose_ragged(
-                    _C.ptr(buf), _C.ptr(out), _C.ptr(offsets_dev), _C.ptr(rows_dev),
-                    _C.ptr(cols_dev), _C.ptr(tiles_dev), B, total_tiles, tr, tc, buf.element_size(),
-                    _C.current_stream(buf.device)))
-    res = NestedTensorImpl(out, new_sizes)
+def _transposed(impl, mode):
+    res = NestedTensorImpl(*_transpose_constituents(impl, mode))
     res.share_offsets(impl)       # the constituents keep their extents
     return res
 
@@ -1029,9 +975,7 @@ def transpose_nchw_nhwc(impl):
         raise RuntimeError("transpose_nchw_nhwc needs 4d input.")
     if impl.opt_sizes()[1] is None:
         raise RuntimeError("Expected first dimension to be regular.")
-    s = impl.sizes
-    return _transpose_constituents(impl, s[:, 0], s[:, 1] * s[:, 2],
-                                   torch.stack([s[:, 1], s[:, 2], s[:, 0]], 1).contiguous(), "nchw_nhwc")
+    return _transposed(impl, _NCHW_TO_NHWC)
 
 
 def transpose_nhwc_nchw(impl):
@@ -1042,9 +986,7 @@ def transpose_nhwc_nchw(impl):
         raise RuntimeError("transpose_nhwc_nchw needs 4d input.")
     if impl.opt_sizes()[3] is None:
         raise RuntimeError("Expected last dimension to be regular.")
-    s = impl.sizes
-    return _transpose_constituents(impl, s[:, 0] * s[:, 1], s[:, 2],
-                                   torch.stack([s[:, 2], s[:, 0], s[:, 1]], 1).contiguous(), "nhwc_nchw")
+    return _transposed(impl, _NHWC_TO_NCHW)
 
 
 def is_contiguous(impl, memory_format=torch.contiguous_format):
@@ -1068,11 +1010,9 @@ def contiguous(impl, memory_format=torch.contiguous_format):
     if memory_format == torch.contiguous_format:
         if not impl.channels_last:
             return impl
-        s = impl.sizes
-        as_nhwc = NestedTensorImpl(impl.buffer, torch.stack([s[:, 1], s[:, 2], s[:, 0]], 1).contiguous())
-        as_nhwc.share_offsets(impl)
-        out = transpose_nhwc_nchw(as_nhwc)
-        return impl.with_buffer(out.buffer, channels_last=False)
+        if impl.opt_sizes()[1] is None:
+            raise RuntimeError("Expected last dimension to be regular.")
+        return impl.with_buffer(_transpose_constituents(impl, _CHANNELS_LAST_TO_ROW_MAJOR)[0], channels_last=False)
     if memory_format == torch.channels_last:
         if impl.channels_last:
             return impl
