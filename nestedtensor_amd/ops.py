@@ -449,7 +449,7 @@ def mha_packed(num_heads, head_dim, query, key, value, in_proj_weight, in_proj_b
         out = _mha_cross_packed(xq, xk, xv, _attention_work(query, key, num_heads, head_dim), num_heads, head_dim, W,
                                 in_proj_bias, float(scaling), out_proj_weight, out_proj_bias)
         return query.with_buffer(out.reshape(-1))
-    # V row-major: fp32 with head_dim 32 / 64 / 128 on the fp32 matrix instruction from
+    # V row-major: fp32 with head_dim 32 / 64 / 128 on the matrix instruction from
     # the work list (only tiles that exist, longest key sequences first), anything else
     # (other head dims, key sequences without keys) on the generic kernels over the
     # device row offsets
