@@ -908,20 +908,26 @@ static int launch_phased(const GemmArgs<T>& a, hipStream_t stream) {
 // The fp32 matrix instruction does a sixteenth of the bf16 one's work per cycle, and a
 // product of fp32 operands is bound by it (phased_kernel reached 0.8 of its rate).  An fp32
 // number is the sum of three bf16 ones (24 significant bits in three of 8, each the rounded
-// rest of the one before: exact), so a product of two is nine bf16 products, of which the
-// six largest are kept: what is left out is below 2^-25 of |x| |w|, half the rounding of one
-// fp32 product.  (Splitting by rounding and rest is Dekker's; products of bf16 numbers are exact
-// in the fp32 accumulators.)  The error against 64 bits is smaller than the fp32
-// instruction's, which rounds more partial sums: 2.1e-7 against 2.5e-7 of the 2-norm at K 768,
-// 2.7e-7 against 3.1e-7 at 1024, 7.8e-8 against 9.2e-8 at 256.
+// rest of the one before: exact), so a product of two is nine bf16 products, each exact in the
+// fp32 accumulators.  Eight are kept; that of the two third parts, below 2^-34 of |x| |w|, is
+// left out.  (Splitting by rounding and rest is Dekker's.)  The product of the first parts is
+// summed in accumulators of its own and the seven others, below 2^-7 of it, in a second set,
+// added once at the end: so a partial sum is rounded no oftener than by the fp32 instruction,
+// however few of the products are other than zero.  All in one set, a row with one product per
+// 16 k was rounded up to eight times per product.  Error against 64 bits, 2-norm, fp32
+// instruction / here: N(0, 1) operands of K 256 2.9e-7 / 0.9e-7, 768 5.0e-7 / 1.6e-7, 2048
+// 8.1e-7 / 2.7e-7; one product per 16 k, over 1, 4, 48 steps 2.53e-8 / 2.53e-8, 4.0e-8 / 2.6e-8, 1.25e-7 /
+// 0.51e-7; rows behind a relu, K 768 3.5e-7 / 1.2e-7.  (Of six products, without the two next
+// smallest, a single one has 1.03 times the error of the fp32 instruction, up to a whole
+// rounding more; they would take 0.85 of the time.)
 //
 // The operands are split on the way from global memory to LDS, once per tile: a step of 16
 // k of all its rows is fetched into registers kDepth steps ahead, split between the matrix
 // instructions of the step before its own and written to the other of two tile buffers.
-// Bound by the matrix pipe at the clock that random operands leave (8040 x 2304 x 768 on
-// zeros 111 us, on N(0, 1) operands 137 to 160); before, on the fp32 instruction: 260.
-// 8040 x 768 x 768 76-84 -> 52-56, 20000 x 3072 x 1024 900 -> 545, 2000 x 1536 x 512 39.5 -> 24,
-// 300 x 768 x 256 19.4 -> 8.9, and 0.49 of the time over 174 products of K 192 to 2048 (0.74 at most).
+// Two sets of accumulators leave room for tiles of up to 320 x 128 at two wavefronts per SIMD.
+// Bound by the matrix pipe at the clock that random operands leave.  Fp32 instruction / here, us:
+// 8040 x 2304 x 768 216 / 185, 8040 x 768 x 768 76 / 63, 20000 x 3072 x 1024 894 / 744, 2000 x 1536 x 512 36 / 26,
+// 300 x 768 x 256 19.1 / 8.9; 0.55 of the time over 174 products of K 192 to 2048 (0.86 at most).
 template <int GM_, int GN_, int NI_, int NJ_, int DEPTH_>
 struct SplitCfg {
   static constexpr int kGM = GM_, kGN = GN_, kNI = NI_, kNJ = NJ_;   // wavefronts, 32 x 32 blocks of each
@@ -995,13 +1001,13 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
-  acc16 acc[NI][NJ];
+  acc16 acc[NI][NJ], low[NI][NJ];        // products of the first parts; the seven others
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.0f;
 
   float* lds_bias = reinterpret_cast<float*>(lds + Cfg::kLdsBytes);
   int* lds_tiny = reinterpret_cast<int*>(lds_bias + Cfg::kBN);
@@ -1095,13 +1101,16 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
           for (int p = 0; p < 3; ++p)
             fb_next[j][p] = *reinterpret_cast<const bf16x8*>(w_lds + other + j * 3072 + p * 1024);
       }
-      // smallest products first
-      constexpr int kPa[6] = {0, 1, 2, 1, 0, 0}, kPw[6] = {2, 1, 0, 0, 1, 0};
+      // smallest products first; the first parts' among them, for a break in the chain of sums
+      constexpr int kPa[7] = {1, 2, 0, 1, 2, 0, 1}, kPw[7] = {2, 1, 2, 1, 0, 1, 0};
 #pragma unroll
-      for (int p = 0; p < 6; ++p)
+      for (int p = 0; p < 7; ++p) {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
-          acc[i][j] = Mma<__bf16>::run(fb[j][kPw[p]], fa[i & 1][kPa[p]], acc[i][j]);
+        for (int j = 0; j < NJ; ++j) {
+          low[i][j] = Mma<__bf16>::run(fb[j][kPw[p]], fa[i & 1][kPa[p]], low[i][j]);
+          if (p == 4) acc[i][j] = Mma<__bf16>::run(fb[j][0], fa[i & 1][0], acc[i][j]);
+        }
+      }
       if (i + 1 < NI) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // the next block's reads first
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1135,7 +1144,10 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) probe = fmaf(acc[i][j][e], 0.0f, probe);
+      for (int e = 0; e < 16; ++e) {
+        acc[i][j][e] += low[i][j][e];
+        probe = fmaf(acc[i][j][e], 0.0f, probe);
+      }
   __syncthreads();
   char* strip = lds + wave * strip_bytes<float, NI, NJ, false>();
   if (*lds_tiny == 0 && __ballot(probe != probe) == 0) {
@@ -1295,18 +1307,18 @@ static int pick_phased_f32(int64_t M, int64_t N, int64_t nk, int num_cus) {
 
 // Tiles of split_kernel and what one takes, in microseconds per 16 k; fitted like the above on
 // 174 products (16 to 60000 rows, K 192 to 2048): what it picks takes 1.002 times the fastest
-// shape's time on average, 1.03 at most.
+// shape's time on average, 1.02 at most.
 struct SplitShape {
   int bm, bn;
   TileCost cost;
 };
 static const SplitShape kSplitShapes[] = {
-    {320, 256, {2.167, 2.421, 15.83, 1.72, 0.0}},
-    {256, 256, {1.58, 1.951, 17.17, 7.19, 0.0}},
-    {192, 128, {0.752, 0.842, 5.86, 2.52, 0.0}},
-    {128, 128, {0.552, 0.623, 4.1, 2.25, 0.0}},
-    {64, 128, {0.451, 0.368, 1.33, 1.33, 0.0}},
-    {128, 64, {0.306, 0.361, 4.55, 0.974, 0.0}}};
+    {320, 128, {1.471, 1.85, 13.606, 1.721, 0.0}},
+    {256, 128, {1.317, 1.519, 7.484, 1.847, 0.0}},
+    {192, 128, {1.105, 1.207, 3.214, 6.064, 0.0}},
+    {128, 128, {0.664, 0.835, 3.496, 6.615, 0.0}},
+    {64, 128, {0.402, 0.481, 2.089, 1.249, 0.0}},
+    {128, 64, {0.31, 0.476, 3.686, 0.603, 0.0}}};
 constexpr int kSplitCount = (int)(sizeof(kSplitShapes) / sizeof(kSplitShapes[0]));
 
 static int pick_split(int64_t M, int64_t N, int64_t K, int num_cus) {
@@ -1441,9 +1453,9 @@ static int launch_epi(const GemmArgs<T>& a, hipStream_t stream) {
   }
   if constexpr (sizeof(T) == 4 && EPI != kEpiQkv) {
     switch (tile) {
-      case kTileSplit + 0: return launch_split<SplitCfg<2, 4, 5, 2, 1>, EPI>(a, stream);
-      case kTileSplit + 1: return launch_split<SplitCfg<2, 4, 4, 2, 1>, EPI>(a, stream);
-      case kTileSplit + 2: return launch_split<SplitCfg<2, 4, 3, 1, 2>, EPI>(a, stream);
+      case kTileSplit + 0: return launch_split<SplitCfg<2, 4, 5, 1, 1>, EPI>(a, stream);
+      case kTileSplit + 1: return launch_split<SplitCfg<2, 4, 4, 1, 1>, EPI>(a, stream);
+      case kTileSplit + 2: return launch_split<SplitCfg<2, 4, 3, 1, 1>, EPI>(a, stream);
       case kTileSplit + 3: return launch_split<SplitCfg<2, 4, 2, 1, 4>, EPI>(a, stream);
       case kTileSplit + 4: return launch_split<SplitCfg<2, 4, 1, 1, 2>, EPI>(a, stream);
       case kTileSplit + 5: return launch_split<SplitCfg<4, 2, 1, 1, 2>, EPI>(a, stream);

@@ -27,19 +27,20 @@ def _case(M, N, K, seed=0):
 
 
 def _bound(x, w, ref):
-    # six products per k; were the sums of an instruction rounded after every four k, 1.5 K
-    # roundings of partial sums below sum |x||w|; half a rounding per k for the products left
-    # out; the bias and the store
-    return (x.double().abs() @ w.double().abs().t()) * (2 * x.size(1) * 2.0 ** -24) + ref.abs() * 2.0 ** -24 + 1e-30
+    # Were the sums of an instruction cut off, not rounded, after every four k: K / 4 units of
+    # 2^-23 of partial sums below sum |x||w| for the first parts, 7 K / 4 of them at 2^-7 of it
+    # for the other products (0.53 K roundings of 2^-24 in all), 2^-34 per k for the product left
+    # out; the two sums added, the bias and the store
+    return (x.double().abs() @ w.double().abs().t()) * ((0.55 * x.size(1) + 4) * 2.0 ** -24) + ref.abs() * 2.0 ** -24 + 1e-30
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
     (1, 1, 192, (64, 128, -1)), (3, 130, 192, (64, 128, -1)), (64, 129, 208, (64, 128, -1)),
     (1000, 300, 224, (64, 128, -1)), (500, 2050, 2064, (128, 64, -1)), (60001, 33, 192, (128, 64, -1)),
     (2000, 1536, 512, (128, 128, -1)), (2001, 1537, 528, (128, 128, -1)), (129, 12000, 208, (128, 128, -1)),
-    (8040, 768, 768, (192, 128, -1)), (20001, 1026, 208, (192, 128, -1)), (16001, 1025, 1040, (192, 128, -1)),
-    (16001, 1024, 208, (256, 256, -1)), (16001, 1022, 240, (256, 256, -1)),
-    (8040, 2304, 768, (320, 256, -1)), (8167, 2300, 304, (320, 256, -1)),
+    (8040, 768, 768, (192, 128, -1)), (40000, 128, 208, (192, 128, -1)),
+    (20001, 1026, 208, (256, 128, -1)), (16001, 1024, 208, (256, 128, -1)), (16001, 1022, 240, (256, 128, -1)),
+    (16001, 1025, 1040, (320, 128, -1)), (8040, 2304, 768, (320, 128, -1)), (8167, 2300, 304, (320, 128, -1)),
 ])
 def test_linear_split_shapes(M, N, K, tile):
     from nestedtensor_amd import ops
@@ -114,3 +115,45 @@ def test_linear_split_precision(M, N, K):
         acc = (acc.double() + x[:, k:k + 1].double() * w[:, k].double()).float()
     chain = ((acc + b).double() - ref).norm()
     assert (ops.linear(x, w, b).double() - ref).norm() <= chain
+
+
+def _chain(x, w):
+    """fp32 multiply-adds, one rounding per product."""
+    acc = torch.zeros(x.size(0), w.size(0), device=DEV)
+    for k in range(x.size(1)):
+        acc = (acc.double() + x[:, k:k + 1].double() * w[:, k].double()).float()
+    return acc
+
+
+@pytest.mark.parametrize("steps", [1, 2, 4, 16, 48])
+@pytest.mark.parametrize("positive", [False, True])
+@pytest.mark.parametrize("M,N", [(9000, 1030), (200, 100)])
+def test_linear_split_one_product_per_step(M, N, steps, positive):
+    """Sums of few products, one in 16 k, are no less precise than chains of fp32 multiply-adds.
+    (1.01: seven roundings of products below 2^-7 of the largest add sqrt(7) 2^-7 of one
+    rounding, in quadrature; the product left out is below 2^-34.)"""
+    from nestedtensor_amd import ops
+    K = 16 * max(steps, 12)
+    g = torch.Generator("cuda").manual_seed(steps)
+    at = torch.randint(0, 16, (M, steps), device=DEV, generator=g) + 16 * torch.arange(steps, device=DEV)
+    x = torch.zeros(M, K, device=DEV).scatter_(1, at, torch.randn(M, steps, device=DEV, generator=g))
+    w = torch.randn(N, K, device=DEV, generator=g)
+    if positive:
+        x, w = x.abs(), w.abs()
+    assert _tile(M, N, K)[2] == -1
+    ref = x.double() @ w.double().t()
+    err, chain = ((t.double() - ref).norm() for t in (ops.linear(x, w, None), _chain(x, w)))
+    assert err <= 1.01 * chain
+
+
+def test_linear_split_largest_rests():
+    """1 + 2^-8 - 2^-17: the second and third parts are as large as they can be."""
+    from nestedtensor_amd import ops
+    v = 1 + 2.0 ** -8 - 2.0 ** -17
+    x, w = torch.zeros(300, 768, device=DEV), torch.full((256, 768), v, device=DEV)
+    x[:, 5] = v
+    assert torch.equal(ops.linear(x, w, None), (x.double() @ w.double().t()).float())
+    x.fill_(v)
+    y = ops.linear(x, w, None)
+    # 48 steps of exact sums, one rounding each
+    assert bool(((y.double() - 768 * v * v).abs() <= 48 * 2.0 ** -24 * 768 * v * v).all())
