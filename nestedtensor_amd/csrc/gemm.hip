@@ -938,7 +938,7 @@ struct SplitCfg {
   static constexpr int kBufBytes = kBlocks * 3 * 1024;               // 16 k of all rows, three parts
   static constexpr int kLdsBytes = 2 * kBufBytes;
   static_assert(8 * strip_bytes<float, NI_, NJ_, false>() <= kLdsBytes, "strips must fit");
-  static_assert(kLdsBytes + kBN * 4 + 16 <= 160 * 1024, "tile buffers must fit the LDS");
+  static_assert(kLdsBytes + kBN * 4 <= 160 * 1024, "tile buffers must fit the LDS");
 };
 
 // 32-row blocks of A and W lie in LDS as three parts of 1 KiB, a part as the 16-byte pieces
@@ -975,13 +975,12 @@ struct SplitPiece {
     __builtin_memcpy(raw[slot], src + off, FLOATS < 8 ? FLOATS * 4 : 16);
     if constexpr (FLOATS == 8) __builtin_memcpy(raw[slot] + 4, src + off + 32, 16);
   }
-  __device__ __forceinline__ void put(char* buf, int slot, SmallestBf16& smallest) const {
+  __device__ __forceinline__ void put(char* buf, int slot) const {
     uint32_t part[3][FLOATS / 2];
 #pragma unroll
     for (int e = 0; e < FLOATS / 2; ++e) {
-      split_bf16_pair(__builtin_bit_cast(float, raw[slot][2 * e]), __builtin_bit_cast(float, raw[slot][2 * e + 1]),
-                      part[0][e], part[1][e], part[2][e]);
-      smallest.add(part[0][e]);
+      split_bf16_pair(__builtin_bit_cast(float, raw[slot][2 * e]) * kSplitScale,
+                      __builtin_bit_cast(float, raw[slot][2 * e + 1]) * kSplitScale, part[0][e], part[1][e], part[2][e]);
     }
 #pragma unroll
     for (int p = 0; p < 3; ++p)
@@ -1010,12 +1009,10 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
       for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.0f;
 
   float* lds_bias = reinterpret_cast<float*>(lds + Cfg::kLdsBytes);
-  int* lds_tiny = reinterpret_cast<int*>(lds_bias + Cfg::kBN);
   if (tid < Cfg::kBN) {
     const int64_t col = n0 + tid;
     lds_bias[tid] = (a.bias && col < a.N) ? a.bias[col] : 0.0f;
   }
-  if (tid == 0) *lds_tiny = 0;
 
   const int n_steps = (int)(a.K / 16);
   constexpr int kABlocks = Cfg::kBM / 32;
@@ -1029,7 +1026,6 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
     half.place(a, m0, n0, kABlocks, 8 * kUnits + (wave >> 1), (wave & 1) * 16 + (lane >> 2), lane & 3);
   if (kTail2)
     quarter.place(a, m0, n0, kABlocks, 8 * kUnits + kTail4 + (wave >> 2), (wave & 3) * 8 + (lane >> 3), lane & 7);
-  SmallestBf16 smallest;
 
   constexpr int kPuts = kUnits + (kTail4 ? 1 : 0) + (kTail2 ? 1 : 0);
   auto fetch = [&](int u, int step, int slot) __attribute__((always_inline)) {
@@ -1039,9 +1035,9 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
     else quarter.fetch(step, slot);
   };
   auto put = [&](int u, char* buf, int slot) __attribute__((always_inline)) {
-    if (u < kUnits) unit[u < kUnits ? u : 0].put(buf, slot, smallest);
-    else if (u == kUnits && kTail4) half.put(buf, slot, smallest);
-    else quarter.put(buf, slot, smallest);
+    if (u < kUnits) unit[u < kUnits ? u : 0].put(buf, slot);
+    else if (u == kUnits && kTail4) half.put(buf, slot);
+    else quarter.put(buf, slot);
   };
   auto publish = [] __attribute__((always_inline)) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1133,11 +1129,10 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
   for (int d = 0; d + 1 < kDepth; ++d)
     if (step + d < n_steps) one_step(step + d, (d + 1) % kDepth);
 
-  // A magnitude below 2^-100 other than zero: its third part may be lost below the smallest
-  // bf16 number.  A result that is no finite number: an infinity or NaN went in (their rests
-  // are NaN), a first part rounded up to infinity, or the sum overflowed.  Both are computed
-  // again by the fp32 instruction.
-  if (smallest.tiny()) *lds_tiny = 1;
+  // A result that is no finite number: an infinity, a NaN or a magnitude from 2^111 on went in,
+  // or a sum, 2^32 times the result's, overflowed.  The wavefront's part is computed again by the
+  // fp32 instruction, straight from global memory: one row of 8040 x 2304 x 768 not finite costs
+  // 190 us more, all of them take 575 us (the fp32 instruction alone 215).
   float probe = 0.0f;
 #pragma unroll
   for (int i = 0; i < NI; ++i)
@@ -1147,10 +1142,11 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
       for (int e = 0; e < 16; ++e) {
         acc[i][j][e] += low[i][j][e];
         probe = fmaf(acc[i][j][e], 0.0f, probe);
+        acc[i][j][e] *= kSplitUnscale;
       }
   __syncthreads();
   char* strip = lds + wave * strip_bytes<float, NI, NJ, false>();
-  if (*lds_tiny == 0 && __ballot(probe != probe) == 0) {
+  if (__ballot(probe != probe) == 0) {
     store_tile<float, NI, NJ, false, ACT>(a, acc, m0 + wm * (32 * NI), n0, wn * (32 * NJ), strip, lds_bias);
     return;
   }
@@ -1210,7 +1206,7 @@ __global__ __launch_bounds__(512, 2) void split_kernel(GemmArgs<float> a) {
 template <class Cfg, int EPI>
 static int launch_split(const GemmArgs<float>& a, hipStream_t stream) {
   const int64_t tiles = ((a.M + Cfg::kBM - 1) / Cfg::kBM) * ((a.N + Cfg::kBN - 1) / Cfg::kBN);
-  const int lds_bytes = Cfg::kLdsBytes + Cfg::kBN * (int)sizeof(float) + 16;
+  const int lds_bytes = Cfg::kLdsBytes + Cfg::kBN * (int)sizeof(float);
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_kernel<Cfg, EPI>),

@@ -48,10 +48,15 @@ __device__ __forceinline__ void store16_stream(char* p, u32x4 v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
-// Two fp32 numbers as three packed pairs of bf16 each, every one the rounded rest of the one
-// before: x is the exact sum of its parts unless it lies below 2^-110 (the third part may
-// fall below the smallest bf16 number), is no finite number or next to the largest
-// (NaN among the parts).
+// fp32 operands of products on the bf16 matrix instruction are taken times 2^16 and split into
+// three bf16 parts, each the rounded rest of the one before.  Of any fp32 number below 2^111 the
+// parts are exact: it is a multiple of 2^-149, 2^16 times it one of 2^-133, the smallest bf16
+// number, so no rest falls below what a part can hold.  From 2^111 on (and of what is no
+// finite number) a part is infinite or NaN, and so is every sum that it enters.
+constexpr float kSplitScale = 0x1p16f;
+constexpr float kSplitUnscale = 0x1p-32f;      // of a product of two
+
+// The parts of two scaled numbers, a packed pair each.
 __device__ __forceinline__ void split_bf16_pair(float x, float y, uint32_t& first, uint32_t& second, uint32_t& third) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));

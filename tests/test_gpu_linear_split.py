@@ -30,8 +30,8 @@ def _bound(x, w, ref):
     # Were the sums of an instruction cut off, not rounded, after every four k: K / 4 units of
     # 2^-23 of partial sums below sum |x||w| for the first parts, 7 K / 4 of them at 2^-7 of it
     # for the other products (0.53 K roundings of 2^-24 in all), 2^-34 per k for the product left
-    # out; the two sums added, the bias and the store
-    return (x.double().abs() @ w.double().abs().t()) * ((0.55 * x.size(1) + 4) * 2.0 ** -24) + ref.abs() * 2.0 ** -24 + 1e-30
+    # out; the two sums added, the bias and the store; twice half the smallest fp32 number
+    return (x.double().abs() @ w.double().abs().t()) * ((0.55 * x.size(1) + 4) * 2.0 ** -24) + ref.abs() * 2.0 ** -24 + 2.0 ** -148
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
@@ -94,14 +94,36 @@ def test_linear_split_special_values(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(5, 7, 192), (300, 200, 256), (2001, 1537, 224)])
-def test_linear_split_small_magnitudes(M, N, K):
-    """The third part of a number below 2^-110 lies below the smallest bf16 number."""
+@pytest.mark.parametrize("ex,ew", [
+    (-118, 100), (90, -120), (-60, -40), (-100, 0), (0, -101),
+    (-128, 100), (-134, 100), (-140, 105), (-147, 105), (105, -140), (-1, -130),      # denormal operands
+    (-66, -64), (-70, -75),                                                            # denormal results
+    (60, 50), (107, -10), (113, -20), (-20, 124)])                                     # results or operands too large to split
+def test_linear_split_magnitudes(M, N, K, ex, ew):
     from nestedtensor_amd import ops
     x, w, _ = _case(M, N, K)
-    for ex, ew in ((-118, 100), (90, -120), (-60, -40), (-100, 0)):
-        xs, ws = torch.ldexp(x, torch.tensor(ex, device=DEV)), torch.ldexp(w, torch.tensor(ew, device=DEV))
-        ref = xs.double() @ ws.double().t()
-        assert bool(((ops.linear(xs, ws, None).double() - ref).abs() <= _bound(xs, ws, ref)).all()), (ex, ew)
+    xs, ws = torch.ldexp(x, torch.tensor(ex, device=DEV)), torch.ldexp(w, torch.tensor(ew, device=DEV))
+    xs, ws = xs.nan_to_num(posinf=0.0, neginf=0.0), ws.nan_to_num(posinf=0.0, neginf=0.0)
+    ref = xs.double() @ ws.double().t()
+    y = ops.linear(xs, ws, None).double()
+    # (a result that fp32 recomputes: one rounding per k of partial sums)
+    bound = _bound(xs, ws, ref) if ex + ew < 80 and max(ex, ew) < 108 else \
+        xs.double().abs() @ ws.double().abs().t() * ((K + 2) * 2.0 ** -24) + 2.0 ** -148
+    assert bool(((y - ref).abs() <= bound).all())
+
+
+def test_linear_split_mixed_magnitudes():
+    """One operand below the smallest bf16 number among ordinary ones is not taken for zero."""
+    from nestedtensor_amd import ops
+    x, w, _ = _case(300, 200, 256)
+    x[17, 9] = 2.0 ** -140
+    x[17, 10:] = 0.0
+    x[17, :9] = 0.0
+    w[:, 9] = torch.ldexp(w[:, 9], torch.tensor(100, device=DEV))
+    ref = x.double() @ w.double().t()
+    y = ops.linear(x, w, None).double()
+    assert bool(((y - ref).abs() <= _bound(x, w, ref)).all())
+    assert bool((y[17] != 0).all())
 
 
 @pytest.mark.parametrize("M,N,K", [(4000, 512, 256), (4000, 768, 768), (2000, 1024, 1024)])
