@@ -1130,12 +1130,11 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
     if (step + d < n_steps) one_step(step + d, (d + 1) % kDepth);
 
   // A result that is no finite number: an infinity, a NaN or a magnitude from 2^111 on went in,
-  // or a sum, 2^32 times the result's, overflowed.  The wavefront's part is computed again by the
-  // fp32 instruction, straight from global memory: one row of 8040 x 2304 x 768 not finite costs
-  // 190 us more, all of them take 575 us (the fp32 instruction alone 215).
-  float probe = 0.0f;
+  // or a sum, 2^32 times the result's, overflowed.
+  unsigned redo = 0;                            // a bit per block of 32 rows, the same in a wavefront
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
+  for (int i = 0; i < NI; ++i) {
+    float probe = 0.0f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -1144,14 +1143,19 @@ __device__ __forceinline__ void split_tile(const GemmArgs<float>& a, int64_t m0,
         probe = fmaf(acc[i][j][e], 0.0f, probe);
         acc[i][j][e] *= kSplitUnscale;
       }
+    if (__ballot(probe != probe) != 0) redo |= 1u << i;
+  }
   __syncthreads();
   char* strip = lds + wave * strip_bytes<float, NI, NJ, false>();
-  if (__ballot(probe != probe) == 0) {
-    store_tile<float, NI, NJ, false, ACT>(a, acc, m0 + wm * (32 * NI), n0, wn * (32 * NJ), strip, lds_bias);
-    return;
-  }
+  store_tile<float, NI, NJ, false, ACT>(a, acc, m0 + wm * (32 * NI), n0, wn * (32 * NJ), strip, lds_bias);
+  if (redo == 0) return;
+  // Those blocks once more by the fp32 instruction, operands straight from global memory, and over
+  // what has been stored.  Seldom worth more: one row of 8040 x 2304 x 768 not finite costs 35 us more (190 with
+  // all rows of the wavefront done again), all of them take 590 us (the fp32 instruction alone 215).
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll 1
   for (int i = 0; i < NI; ++i) {
+    if (!(redo >> i & 1)) continue;
     acc16 row[1][NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
