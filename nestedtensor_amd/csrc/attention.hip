@@ -831,8 +831,16 @@ __device__ __forceinline__ void attention_f32_tile(
 }
 
 // The same tile on the bf16 matrix instruction (v_mfma_f32_32x32x16_bf16): Q, K, V and P are
-// split into three bf16 parts each and the six largest of the nine products kept, an
-// error below half a rounding of one fp32 product; scores, softmax and sums stay fp32.
+// split into three bf16 parts each, and eight of the nine products
+// kept: that of two third parts, below 2^-34 of the whole, is left out.  Scores, softmax and
+// sums stay fp32.  The seven small products are summed apart from the product of the first
+// parts: in the scores in accumulators of their own, added at the end; in the second product
+// a tile of 32 keys sums the seven first and then the first parts' in fresh accumulators,
+// which go to the running ones by one multiply-add with the rescaling.  So a product of few is
+// rounded twice at most, in its tile's sum and in the running one, of many once in 16.  Error against 64 bits, 2-norm, fp32 instruction / here: N(0, 1), 2000 keys of 64
+// 8.7e-7 / 2.4e-7, of 128 9.1e-7 / 2.6e-7; 3 to 17 keys of 64 1.7e-7 / 0.9e-7; one probability per 32 keys, 2, 4, 32
+// of 64 8.3e-8 / 5.9e-8, 1.1e-7 / 7.6e-8, 2.4e-7 / 1.7e-7; at most 0.90 of it over 19 distributions per
+// head_dim.  (With all products but the three smallest in one accumulator up to 1.22.)
 // The fp32 instruction does a sixteenth of the work per cycle and was what bounded the tile.
 //
 // A K tile of 32 keys is split on its way into LDS, one 16-byte piece (8 k) per part:
@@ -844,19 +852,15 @@ __device__ __forceinline__ void attention_f32_tile(
 //    lane half hold, which makes those accumulators, split, the other operand.
 // Wavefronts without a query row only fetch.
 //
-// Bound by matrix and vector instructions, which share a SIMD badly: 48 matrix and some 300
+// Bound by matrix and vector instructions, which share a SIMD badly: 64 matrix and some 350
 // vector instructions per tile of head_dim 64, of which the splits of P, K and V are 200
 // (measured apart, a SIMD keeps its matrix pipe full beside four vector instructions per
 // matrix instruction of each of two wavefronts; each further one costs its own time).  What
 // hides the fetch of a tile and the rest is other workgroups: one tile buffer and nothing
-// in flight in registers leave room for three per CU (128: two).  With two buffers and the
-// next tile in registers it was two (one): 100 sequences of 64 to 1024, 12 heads of 64 680 us, of
-// 128 1850, 200 of 1 to 16, 12 heads of 128 103; only a launch that does not fill those places is
-// slower for it (8 of 256 to 2048, 8 heads of 64 148, now 167).
-// Against attention_f32_tile, us: 32 sequences of 32 to 512, 12 heads of 64 126 -> 81; 100 of 64 to
-// 1024, 12 heads of 64 889 -> 573, of 32 529 -> 388, of 128 1976 -> 1139; 8 of 256 to 2048, 8 heads of
-// 64 239 -> 167; 256 of 4 to 64, 12 heads of 64 61 -> 41; 100 of 1 to 16, 12 heads of 128 36 -> 25.
-// Error against 64 bits 0.78 to 0.85 of what it was.
+// in flight in registers leave room for three per CU (128: two).
+// Fp32 instruction / here, us: 32 sequences of 32 to 512, 12 heads of 32 56 / 43, of 64 103 / 74, of 128 208 / 147;
+// 100 of 64 to 1024, 12 heads of 32 645 / 523, of 64 1235 / 907, of 128 2690 / 1920; 8 of 256 to 2048, 8 heads of
+// 64 225 / 169; 256 of 4 to 64, 12 heads of 64 57 / 38; 100 of 1 to 16, 12 heads of 128 37 / 27.
 template <int HD>
 struct SplitAttention {
   static constexpr int kKT = 32;
@@ -985,7 +989,7 @@ __device__ __forceinline__ void attention_split_tile(
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[j][i] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;       // l_run: this lane half's keys only
-  constexpr int kPa[6] = {0, 1, 2, 1, 0, 0}, kPb[6] = {2, 1, 0, 0, 1, 0};   // smallest products first
+  constexpr int kPa[7] = {1, 2, 0, 1, 2, 0, 1}, kPb[7] = {2, 1, 2, 1, 0, 1, 0};   // smallest products first
 
   const int64_t n_tiles = (Lk + kKT - 1) / kKT;
   if (n_tiles > 0) {
@@ -994,26 +998,32 @@ __device__ __forceinline__ void attention_split_tile(
   __syncthreads();
   for (int64_t t = 0; t < n_tiles; ++t) {
     if (active) {
-      acc16 s;
+      int key_place = (col ^ half * (128 / HD)) * 16;      // in a piece 2 tt + half; XOR-ed with tt's share below
+      // at 128 one v_xor per tt instead of an address kept for each: no registers are left for those
+      if constexpr (HD == 128) asm volatile("" : "+v"(key_place));
+      acc16 s, s_low;                                      // products of the first parts; the seven others
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+      for (int i = 0; i < 16; ++i) s[i] = s_low[i] = 0.0f;
 #pragma unroll
       for (int tt = 0; tt < kT; ++tt) {
-        const int piece = 2 * tt + half;
-        const char* kp = lds + (piece * 32 + (col ^ (piece * (128 / HD) & 15))) * 16;
+        const char* kp = lds + half * 512 + tt * 1024 + (key_place ^ tt * (128 / HD) * 32);
         bf16x8 kf[3];
 #pragma unroll
         for (int p = 0; p < 3; ++p) kf[p] = *reinterpret_cast<const bf16x8*>(kp + p * kPart);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[tt][0], s, 0, 0, 0);
 #pragma unroll
-        for (int p = 0; p < 6; ++p)
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kPa[p]], qf[tt][kPb[p]], s, 0, 0, 0);
+        for (int p = 0; p < 7; ++p)
+          s_low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kPa[p]], qf[tt][kPb[p]], s_low, 0, 0, 0);
       }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] += s_low[i];
       // accumulator i: key 8 (i / 4) + 4 half + i % 4 of the tile, query col
       const int64_t left = Lk - t * kKT;
       if (left < kKT) {
+        const int valid = (int)left - 4 * half;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          if (8 * (i / 4) + 4 * half + (i % 4) >= left) s[i] = -INFINITY;
+          if (8 * (i / 4) + (i % 4) >= valid) s[i] = -INFINITY;
         }
       }
       float m_tile = s[0];
@@ -1030,13 +1040,7 @@ __device__ __forceinline__ void attention_split_tile(
         l_tile += s[i];
       }
       l_run = l_run * alpha + l_tile;
-      if (__ballot(alpha != 1.0f) != 0) {
-#pragma unroll
-        for (int j = 0; j < kJ; ++j) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[j][i] *= alpha;
-        }
-      }
+      bf16x8 pf[2][3];
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         float x[8];
@@ -1045,16 +1049,30 @@ __device__ __forceinline__ void attention_split_tile(
         u32x4 part[3];
         split8(x, part);
 #pragma unroll
-        for (int j = 0; j < kJ; ++j) {
-          const char* vp = lds + 3 * kPart + ((2 * st + half) * HD + 32 * j + col) * 16;
-          bf16x8 vf[3];
+        for (int p = 0; p < 3; ++p) pf[st][p] = __builtin_bit_cast(bf16x8, part[p]);
+      }
+      auto read_v = [&](bf16x8 (&vf)[3], int st, int j) __attribute__((always_inline)) {
+        const char* vp = lds + 3 * kPart + ((2 * st + half) * HD + 32 * j + col) * 16;
 #pragma unroll
-          for (int p = 0; p < 3; ++p) vf[p] = *reinterpret_cast<const bf16x8*>(vp + p * kPart);
+        for (int p = 0; p < 3; ++p) vf[p] = *reinterpret_cast<const bf16x8*>(vp + p * kPart);
+      };
 #pragma unroll
-          for (int p = 0; p < 6; ++p)
-            o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[kPa[p]], __builtin_bit_cast(bf16x8, part[kPb[p]]), o[j],
-                                                           0, 0, 0);
-        }
+      for (int j = 0; j < kJ; ++j) {
+        bf16x8 vf[2][3];
+        acc16 x;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = 0.0f;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) read_v(vf[st], st, j);
+#pragma unroll
+        for (int p = 0; p < 7; ++p)
+#pragma unroll
+          for (int st = 0; st < 2; ++st)
+            x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[st][kPa[p]], pf[st][kPb[p]], x, 0, 0, 0);
+#pragma unroll
+        for (int st = 0; st < 2; ++st) x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[st][0], pf[st][0], x, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[j][i] = fmaf(o[j][i], alpha, x[i]);
       }
     }
     __syncthreads();

@@ -99,3 +99,54 @@ def test_attention_f32_magnitudes(hd, eq, ek, ev):
 
     y, (ref, bound) = _run((37, 130), (37, 130), 2, hd, scale)
     assert bool(((y.double() - ref).abs() <= bound + 2.0 ** -148).all())
+
+
+def _chain(q, k, v, lens, H, hd, scale):
+    """The layer in fp32 with one rounding per product: chains of multiply-adds."""
+    out, a = torch.zeros_like(q), 0
+    scale = (torch.tensor(scale, dtype=torch.float32) * torch.tensor(1.4426950408889634, dtype=torch.float32)).item()
+    for L in lens:
+        qh, kh, vh = (t[a:a + L].reshape(L, H, hd).transpose(0, 1).contiguous() for t in (q, k, v))
+        qh = qh * scale
+        s = torch.zeros(H, L, L, device=DEV)
+        for d in range(hd):
+            s = (s.double() + qh[:, :, d:d + 1].double() * kh[:, None, :, d].double()).float()
+        p = torch.exp2(s - s.amax(-1, keepdim=True))
+        o = torch.zeros_like(qh)
+        for n in range(L):
+            o = (o.double() + p[:, :, n:n + 1].double() * vh[:, n:n + 1].double()).float()
+        out[a:a + L] = (o * (1.0 / p.sum(-1, keepdim=True))).transpose(0, 1).reshape(L, H * hd)
+        a += L
+    return out
+
+
+def _one_key_in(every):
+    def scores(q, k, v):
+        hd = q.size(1) // 3
+        for h in range(3):
+            q[:, h * hd] = 2.0 * hd ** 0.5
+            k[:, h * hd] = -1000.0               # probabilities of zero
+            k[::every, h * hd] = 0.0
+    return scores
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128])
+@pytest.mark.parametrize("lens,qkv", [
+    ((37, 130, 300), None), ((5, 9, 17, 3, 12), None), ((40, 200), lambda q, k, v: q.mul_(16)),
+    ((40, 200), lambda q, k, v: v.abs_()),
+    ((64,) * 20, _one_key_in(32)), ((128,) * 10, _one_key_in(32)), ((512,), _one_key_in(32)),
+    ((32,) * 20, _one_key_in(16)), ((64,) * 20, _one_key_in(16)), ((256, 256), _one_key_in(16))])
+def test_attention_f32_precision(hd, lens, qkv):
+    """The 2-norm of the error is no larger than that of fp32 multiply-adds, also where few
+    probabilities of a tile are other than zero.  (Two parts and three products are off by
+    more than ten times that.)"""
+    kept = []
+
+    def inputs(q, k, v):
+        if qkv is not None:
+            qkv(q, k, v)
+        kept.extend((q, k, v))
+
+    y, (ref, _) = _run(lens, lens, 3, hd, inputs)
+    err, chain = ((t.double() - ref).norm() for t in (y, _chain(*kept, lens, 3, hd, hd ** -0.5)))
+    assert err <= chain, float(err / chain)
