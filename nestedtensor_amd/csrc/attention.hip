@@ -689,8 +689,11 @@ __global__ __launch_bounds__(64) void attention_rows_kernel(
 // of the K row); in the second, step i contracts the key that accumulator i of
 // that lane half holds, 8 (i / 4) + 4 g + i % 4.  Everything stays fp32
 // (exp2 on scores prescaled by log2 e).  A workgroup owns 128 query rows of
-// (sequence, head) and walks the sequence's keys in tiles of 32, the next tile's
-// global loads in flight while the current one is multiplied, two LDS buffers.
+// (sequence, head) and walks the sequence's keys in tiles of 32.
+//
+// Only what attention_split_tile cannot do comes here (infinities, NaN, magnitudes above
+// 2^96), out of its kernel and within its registers: query rows are read again for every
+// tile and nothing is fetched ahead.
 template <int HD>
 __device__ __forceinline__ void attention_f32_tile(
     const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
@@ -701,50 +704,18 @@ __device__ __forceinline__ void attention_f32_tile(
   constexpr int kKT = 32;                      // keys per tile
   constexpr int kKs = HD + 4;                  // K row stride in floats: 16-byte reads of 16 rows hit 16 bank groups
   constexpr int kVs = HD + 8;                  // V row stride: the two lane halves (keys 4 apart) use different banks
-  constexpr int kBuf = kKT * (kKs + kVs);
   constexpr int kC4 = HD / 4;                  // 16-byte pieces per row
   constexpr int kPieces = kKT * kC4 / 256;     // pieces per thread and operand: 1, 2, 4
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 31, half = lane >> 5;
 
-  // this lane's query row, prescaled: dims 8t + 4 half + u  ->  qf[4t + u]
   const int64_t qrow = q0 + wave * 32 + col;
   const bool q_ok = qrow < Lq;
-  float qf[HD / 2];
-  {
-    const float* qp = Q + (q_begin + (q_ok ? qrow : q0)) * ldq + (int64_t)h * HD + 4 * half;
-#pragma unroll
-    for (int t = 0; t < HD / 8; ++t) {
-      f32x4 v = *reinterpret_cast<const f32x4*>(qp + 8 * t);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) qf[4 * t + u] = q_ok ? v[u] * scale_log2e : 0.0f;
-    }
-  }
-
-  f32x4 kreg[kPieces], vreg[kPieces];
+  const float* qp = Q + (q_begin + (q_ok ? qrow : q0)) * ldq + (int64_t)h * HD + 4 * half;
+  const float q_scale = q_ok ? scale_log2e : 0.0f;
   const float* kbase = Kp + kv_begin * ldk + (int64_t)h * HD;
   const float* vbase = Vp + kv_begin * ldv + (int64_t)h * HD;
-  auto gload = [&](int64_t k0) {
-#pragma unroll
-    for (int i = 0; i < kPieces; ++i) {
-      const int p = tid + 256 * i;
-      const int row = p / kC4, c4 = p % kC4;
-      const int64_t key = k0 + row;
-      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-      // rows past the last key are zero: 0 * V must not meet a NaN
-      kreg[i] = key < Lk ? *reinterpret_cast<const f32x4*>(kbase + key * ldk + 4 * c4) : zero;
-      vreg[i] = key < Lk ? *reinterpret_cast<const f32x4*>(vbase + key * ldv + 4 * c4) : zero;
-    }
-  };
-  auto lstore = [&](float* buf) {
-#pragma unroll
-    for (int i = 0; i < kPieces; ++i) {
-      const int p = tid + 256 * i;
-      const int row = p / kC4, c4 = p % kC4;
-      *reinterpret_cast<f32x4*>(buf + row * kKs + 4 * c4) = kreg[i];
-      *reinterpret_cast<f32x4*>(buf + kKT * kKs + row * kVs + 4 * c4) = vreg[i];
-    }
-  };
+  float* Vl = lds + kKT * kKs;
 
   acc16 o[HD / 32];
 #pragma unroll
@@ -754,26 +725,35 @@ __device__ __forceinline__ void attention_f32_tile(
   float m_run = -INFINITY, l_run = 0.0f;       // l_run: this lane half's keys only
 
   const int64_t n_tiles = (Lk + kKT - 1) / kKT;
-  if (n_tiles > 0) {
-    gload(0);
-    lstore(lds);
-  }
-  __syncthreads();
+#pragma unroll 1
   for (int64_t t = 0; t < n_tiles; ++t) {
-    float* cur = lds + (t & 1) * kBuf;
-    const bool more = t + 1 < n_tiles;
-    if (more) gload((t + 1) * kKT);
-    const float* Ks = cur + col * kKs + 4 * half;
-    const float* Vs = cur + kKT * kKs + 4 * half * kVs + col;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int p = tid + 256 * i;
+      const int row = p / kC4, c4 = p % kC4;
+      const int64_t key = t * kKT + row;
+      f32x4 kv = {0.0f, 0.0f, 0.0f, 0.0f}, vv = kv;
+      if (key < Lk) {                          // rows past the last key are zero: 0 * V must not meet a NaN
+        kv = *reinterpret_cast<const f32x4*>(kbase + key * ldk + 4 * c4);
+        vv = *reinterpret_cast<const f32x4*>(vbase + key * ldv + 4 * c4);
+      }
+      *reinterpret_cast<f32x4*>(lds + row * kKs + 4 * c4) = kv;
+      *reinterpret_cast<f32x4*>(Vl + row * kVs + 4 * c4) = vv;
+    }
+    __syncthreads();
+    const float* Ks = lds + col * kKs + 4 * half;
+    const float* Vs = Vl + 4 * half * kVs + col;
 
     acc16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-#pragma unroll
+#pragma unroll 2
     for (int tt = 0; tt < HD / 8; ++tt) {
       const f32x4 kf = *reinterpret_cast<const f32x4*>(Ks + 8 * tt);
+      const f32x4 q = *reinterpret_cast<const f32x4*>(qp + 8 * tt);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[u], qf[4 * tt + u], s, 0, 0, 0);
+      for (int u = 0; u < 4; ++u) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[u], q[u] * q_scale, s, 0, 0, 0);
     }
     // accumulator i: key 8 (i / 4) + 4 half + i % 4 of the tile, query col
     const int64_t left = Lk - t * kKT;
@@ -810,8 +790,6 @@ __device__ __forceinline__ void attention_f32_tile(
         o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * j], s[i], o[j], 0, 0, 0);
       }
     }
-    if (more) lstore(lds + ((t + 1) & 1) * kBuf);
-    __syncthreads();
   }
 
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
@@ -831,7 +809,7 @@ __device__ __forceinline__ void attention_f32_tile(
 }
 
 // The same tile on the bf16 matrix instruction (v_mfma_f32_32x32x16_bf16): Q, K, V and P are
-// split into three bf16 parts each, and eight of the nine products
+// scaled and split into three bf16 parts each (split_bf16_pair), and eight of the nine products
 // kept: that of two third parts, below 2^-34 of the whole, is left out.  Scores, softmax and
 // sums stay fp32.  The seven small products are summed apart from the product of the first
 // parts: in the scores in accumulators of their own, added at the end; in the second product
@@ -857,16 +835,16 @@ __device__ __forceinline__ void attention_f32_tile(
 // (measured apart, a SIMD keeps its matrix pipe full beside four vector instructions per
 // matrix instruction of each of two wavefronts; each further one costs its own time).  What
 // hides the fetch of a tile and the rest is other workgroups: one tile buffer and nothing
-// in flight in registers leave room for three per CU (128: two).
+// in flight in registers leave room for three per CU (32: four, 128: two).
 // Fp32 instruction / here, us: 32 sequences of 32 to 512, 12 heads of 32 56 / 43, of 64 103 / 74, of 128 208 / 147;
 // 100 of 64 to 1024, 12 heads of 32 645 / 523, of 64 1235 / 907, of 128 2690 / 1920; 8 of 256 to 2048, 8 heads of
 // 64 225 / 169; 256 of 4 to 64, 12 heads of 64 57 / 38; 100 of 1 to 16, 12 heads of 128 37 / 27.
 template <int HD>
 struct SplitAttention {
   static constexpr int kKT = 32;
+  static constexpr int kWorkgroups = HD == 32 ? 4 : HD == 64 ? 3 : 2;              // per CU
   static constexpr int kKPart = kKT * HD * 2, kBuf = 6 * kKPart;   // three parts of K, three of V
-  static constexpr int kF32Bytes = 2 * 32 * (2 * HD + 12) * (int)sizeof(float);   // attention_f32_tile's, in the same LDS
-  static constexpr int kLdsBytes = kBuf > kF32Bytes ? kBuf : kF32Bytes;
+  static_assert(kKT * (2 * HD + 12) * 4 <= kBuf, "attention_f32_tile's tile lies in the same LDS");
 };
 
 template <int HD>
@@ -884,13 +862,12 @@ __device__ __forceinline__ void attention_split_tile(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, half = lane >> 5;
   const bool fetches_k = HD >= 64 || wave < 2, fetches_v = HD >= 64 || wave >= 2;
-  SmallestBf16 smallest;
 
-  auto split8 = [&](const float (&x)[8], u32x4 (&part)[3]) __attribute__((always_inline)) {
+  auto split8 = [&](const float (&x)[8], float factor, u32x4 (&part)[3]) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       uint32_t a, b, c;
-      split_bf16_pair(x[2 * e], x[2 * e + 1], a, b, c);
+      split_bf16_pair(x[2 * e] * factor, x[2 * e + 1] * factor, a, b, c);
       part[0][e] = a;
       part[1][e] = b;
       part[2][e] = c;
@@ -901,6 +878,7 @@ __device__ __forceinline__ void attention_split_tile(
   const int64_t qrow = q0 + wave * 32 + col;
   const bool q_ok = qrow < Lq;
   const bool active = q0 + wave * 32 < Lq;         // uniform
+  const float q_scale = q_ok ? scale_log2e * kSplitScale : 0.0f;
   bf16x8 qf[kT][3];
   {
     const float* qp = Q + (q_begin + (q_ok ? qrow : q0)) * ldq + (int64_t)h * HD + 8 * half;
@@ -909,11 +887,7 @@ __device__ __forceinline__ void attention_split_tile(
       float x[8];
       __builtin_memcpy(x, __builtin_assume_aligned(qp + 16 * t, 16), 32);
       u32x4 part[3];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = q_ok ? x[e] * scale_log2e : 0.0f;
-      split8(x, part);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
+      split8(x, q_scale, part);
 #pragma unroll
       for (int p = 0; p < 3; ++p) qf[t][p] = __builtin_bit_cast(bf16x8, part[p]);
     }
@@ -960,9 +934,7 @@ __device__ __forceinline__ void attention_split_tile(
         const int c = tid + 256 * i;
         const int key = c / kKeyPieces, piece = c % kKeyPieces;
         u32x4 part[3];
-        split8(kraw[i], part);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
+        split8(kraw[i], kSplitScale, part);
         char* dst = lds + (piece * 32 + (key ^ (piece * (128 / HD) & 15))) * 16;
 #pragma unroll
         for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dst + p * kPart) = part[p];
@@ -972,9 +944,7 @@ __device__ __forceinline__ void attention_split_tile(
 #pragma unroll
       for (int i = 0; i < kPer; ++i) {
         u32x4 part[3];
-        split8(vraw[i], part);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) smallest.add(part[0][e]);
+        split8(vraw[i], kSplitScale, part);
         // piece (sg, d): sg * HD + d counts the threads
         char* dst = lds + 3 * kPart + (HD >= 64 ? tid + 256 * i : tid - 128) * 16;
 #pragma unroll
@@ -1029,14 +999,14 @@ __device__ __forceinline__ void attention_split_tile(
       float m_tile = s[0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) m_tile = fmaxf(m_tile, s[i]);
-      m_tile = max_across_halves(m_tile);                      // finite: the tile holds a valid key
+      m_tile = max_across_halves(m_tile) * kSplitUnscale;      // finite: the tile holds a valid key
       const float m_new = fmaxf(m_run, m_tile);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
       float l_tile = 0.0f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        s[i] = __builtin_amdgcn_exp2f(s[i] - m_new);
+        s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], kSplitUnscale, -m_new));
         l_tile += s[i];
       }
       l_run = l_run * alpha + l_tile;
@@ -1047,7 +1017,7 @@ __device__ __forceinline__ void attention_split_tile(
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = s[8 * st + e];
         u32x4 part[3];
-        split8(x, part);
+        split8(x, kSplitScale, part);
 #pragma unroll
         for (int p = 0; p < 3; ++p) pf[st][p] = __builtin_bit_cast(bf16x8, part[p]);
       }
@@ -1083,20 +1053,21 @@ __device__ __forceinline__ void attention_split_tile(
   }
 
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-  // No finite result: an infinity or NaN went in or came out of a product or a split.  Those
-  // tiles, and the ones with magnitudes that the split cannot carry, run on the fp32
-  // instruction instead.
+  // No finite result: an infinity, a NaN or a number too large to be scaled went in, or a
+  // score from 2^96 or a sum of that size, scaled, came out.  Those items run again on the fp32
+  // instruction: one of 32 sequences of 32 to 512, 12 heads of 64 75 -> 120 us, one of 100 of 64 to 1024 nothing to
+  // be seen, all of those 907 -> 2050 (of 128 1870 -> 4550; the fp32 instruction alone 1190, 2650).
   float probe = l_tot * 0.0f;
 #pragma unroll
   for (int j = 0; j < kJ; ++j)
 #pragma unroll
     for (int i = 0; i < 16; ++i) probe = fmaf(o[j][i], 0.0f, probe);
-  if (__syncthreads_or(smallest.tiny() || probe != probe)) {
+  if (__syncthreads_or(probe != probe)) {
     attention_f32_tile<HD>(Q, ldq, Kp, ldk, Vp, ldv, O, ldo, q_begin, Lq, q0, kv_begin, Lk, h, scale_log2e,
                            reinterpret_cast<float*>(lds));
     return;
   }
-  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;     // no keys: zeros
+  const float inv = l_tot > 0.0f ? kSplitUnscale / l_tot : 0.0f;     // no keys: zeros
   if (q_ok) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     // accumulator i of block j: head dim 32 j + 8 (i / 4) + 4 half + i % 4
@@ -1115,7 +1086,7 @@ __device__ __forceinline__ void attention_split_tile(
 // Workgroup = (128 query rows, head, sequence) on a padded grid: tiles past a
 // sequence's last query row leave at once.
 template <int HD>
-__global__ __launch_bounds__(256, HD < 128 ? 3 : 2) void varlen_attention_f32_kernel(
+__global__ __launch_bounds__(256, SplitAttention<HD>::kWorkgroups) void varlen_attention_f32_kernel(
     const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
     const float* __restrict__ Vp, int64_t ldv, float* __restrict__ O, int64_t ldo,
     const int64_t* __restrict__ q_offsets, const int64_t* __restrict__ kv_offsets,
@@ -1134,7 +1105,7 @@ __global__ __launch_bounds__(256, HD < 128 ? 3 : 2) void varlen_attention_f32_ke
 // The same tiles from a work list (the items of nt_varlen_attention_vt): only
 // tiles that exist are launched, longest key sequences first, head fastest.
 template <int HD>
-__global__ __launch_bounds__(256, HD < 128 ? 3 : 2) void varlen_attention_f32_sched_kernel(
+__global__ __launch_bounds__(256, SplitAttention<HD>::kWorkgroups) void varlen_attention_f32_sched_kernel(
     const float* __restrict__ Q, int64_t ldq, const float* __restrict__ Kp, int64_t ldk,
     const float* __restrict__ Vp, int64_t ldv, float* __restrict__ O, int64_t ldo,
     const int4* __restrict__ schedule, unsigned num_heads, float scale_log2e) {
@@ -1165,9 +1136,9 @@ static int launch_f32(const void* q, int64_t ldq, const void* k, int64_t ldk, co
                       int64_t ldv, void* out, int64_t ldo, const int64_t* qo, const int64_t* kvo,
                       int64_t B, int64_t H, int64_t max_q, float scale, hipStream_t s) {
   dim3 grid((unsigned)((max_q + 127) / 128), (unsigned)H, (unsigned)B);
-  const int rc = allow_lds<varlen_attention_f32_kernel<HD>>(SplitAttention<HD>::kLdsBytes);
+  const int rc = allow_lds<varlen_attention_f32_kernel<HD>>(SplitAttention<HD>::kBuf);
   if (rc != NT_OK) return rc;
-  hipLaunchKernelGGL((varlen_attention_f32_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kLdsBytes, s,
+  hipLaunchKernelGGL((varlen_attention_f32_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kBuf, s,
                      static_cast<const float*>(q), ldq, static_cast<const float*>(k), ldk,
                      static_cast<const float*>(v), ldv, static_cast<float*>(out), ldo, qo, kvo,
                      scale * 1.4426950408889634f);
@@ -1278,9 +1249,9 @@ template <int HD>
 static int launch_f32_sched(dim3 grid, hipStream_t s, const void* q, int64_t ldq, const void* k, int64_t ldk,
                              const void* v, int64_t ldv, void* out, int64_t ldo, const int4* sched,
                              unsigned num_heads, float scale_log2e) {
-  const int rc = allow_lds<varlen_attention_f32_sched_kernel<HD>>(SplitAttention<HD>::kLdsBytes);
+  const int rc = allow_lds<varlen_attention_f32_sched_kernel<HD>>(SplitAttention<HD>::kBuf);
   if (rc != NT_OK) return rc;
-  hipLaunchKernelGGL((varlen_attention_f32_sched_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kLdsBytes, s,
+  hipLaunchKernelGGL((varlen_attention_f32_sched_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kBuf, s,
                      static_cast<const float*>(q), ldq, static_cast<const float*>(k), ldk,
                      static_cast<const float*>(v), ldv, static_cast<float*>(out), ldo, sched, num_heads,
                      scale_log2e);

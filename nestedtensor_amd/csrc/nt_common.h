@@ -72,20 +72,6 @@ __device__ __forceinline__ void split_bf16_pair(float x, float y, uint32_t& firs
   third = round_pair();
 }
 
-// The smallest magnitudes, other than zero, of the first parts of a number of pairs.
-struct SmallestBf16 {
-  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-  u16x2 bits = {0xffff, 0xffff};       // twice the magnitude's bits less one: of a zero the largest
-  __device__ __forceinline__ void add(uint32_t first) {
-    bits = __builtin_elementwise_min(bits, (u16x2)(__builtin_bit_cast(u16x2, first) * (uint16_t)2 - (uint16_t)1));
-  }
-  // one of them below 2^-100
-  __device__ __forceinline__ bool tiny() const {
-    constexpr uint16_t kTiny = 2 * (27 << 7) - 1;
-    return bits[0] < kTiny || bits[1] < kTiny;
-  }
-};
-
 // gelu(x) = x Phi(x), Phi the normal distribution function, from its tail: Phi(-|x|) is
 // 2^Q(|x|) with Q a polynomial of degree 8 fitted to log2 Phi(-u) on [0, 5] (least
 // squares reweighted towards the smallest largest error of Phi).  Q falls without end past 5, so the tail

@@ -91,7 +91,10 @@ def test_attention_f32_special_values(hd):
 
 
 @pytest.mark.parametrize("hd", [32, 64, 128])
-@pytest.mark.parametrize("eq,ek,ev", [(-118, 118, 0), (120, -119, 0), (0, 0, -116), (-60, 58, 90)])
+@pytest.mark.parametrize("eq,ek,ev", [
+    (-118, 118, 0), (120, -119, 0), (0, 0, -116), (-60, 58, 90),
+    (0, 0, -128), (0, 0, -134), (0, 0, -140), (100, -128, 0), (100, -134, 0), (105, -140, 0), (105, -147, 0),   # denormal K, V
+    (-105, 106, 0), (60, -59, 110), (113, -112, 0), (-118, 119, 0)])                                           # up to those too large to split
 def test_attention_f32_magnitudes(hd, eq, ek, ev):
     def scale(q, k, v):
         for t, e in ((q, eq), (k, ek), (v, ev)):
@@ -150,3 +153,35 @@ def test_attention_f32_precision(hd, lens, qkv):
     y, (ref, _) = _run(lens, lens, 3, hd, inputs)
     err, chain = ((t.double() - ref).norm() for t in (y, _chain(*kept, lens, 3, hd, hd ** -0.5)))
     assert err <= chain, float(err / chain)
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128])
+def test_attention_f32_small_probabilities(hd):
+    """A probability of 2^-124 keeps its 24 bits: two keys, the one with all the weight worth 0."""
+    # a scale that times log2 e is one in fp32, so that the scores, of at most 24 bits, are exact
+    log2e = torch.tensor(1.4426950408889634, dtype=torch.float32)
+    scale = torch.tensor(0.6931471805599453, dtype=torch.float32)
+    near = [scale]
+    for towards in (0.0, 1.0):
+        x = scale
+        for _ in range(4):
+            x = torch.nextafter(x, torch.tensor(towards, dtype=torch.float32))
+            near.append(x)
+    scale = next(float(x) for x in near if float(x * log2e) == 1.0)
+    g = torch.Generator("cuda").manual_seed(hd)
+    B = 400
+    score = -(104 + 21 * torch.rand(B, device=DEV, generator=g)).mul(2 ** 16).round().div(2 ** 16)
+    worth = (1 + torch.rand(B, hd, device=DEV, generator=g)) * 2.0 ** 90
+
+    def plant(q, k, v):
+        q.zero_()
+        k.zero_()
+        q[:, 0] = 1.0
+        k[1::2, 0] = score
+        v[0::2] = 0.0
+        v[1::2] = worth
+
+    y, _ = _run((2,) * B, (2,) * B, 1, hd, plant, scale=scale)
+    ref = torch.exp2(score.double())[:, None] * worth.double()       # (the sum is 1 within 2^-104)
+    # two units of 2^-23 for the exponential, a rounding each for the sums and the quotient
+    assert bool(((y[0::2].double() - ref).abs() <= 6 * 2.0 ** -24 * ref).all())
