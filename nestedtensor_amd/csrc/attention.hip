@@ -845,6 +845,7 @@ struct SplitAttention {
   static constexpr int kWorkgroups = HD == 32 ? 4 : HD == 64 ? 3 : 2;              // per CU
   static constexpr int kKPart = kKT * HD * 2, kBuf = 6 * kKPart;   // three parts of K, three of V
   static_assert(kKT * (2 * HD + 12) * 4 <= kBuf, "attention_f32_tile's tile lies in the same LDS");
+  static_assert(kBuf <= 48 * 1024, "more has to be allowed (allow_lds)");
 };
 
 template <int HD>
@@ -1118,26 +1119,11 @@ __global__ __launch_bounds__(256, SplitAttention<HD>::kWorkgroups) void varlen_a
                            item_kv.y > 0 ? item_kv.y : 0, h, scale_log2e, lds);
 }
 
-// Dynamic LDS beyond 48 KiB has to be asked for, once per kernel.
-template <auto KERNEL>
-static int allow_lds(int bytes) {
-  static bool done = false;
-  if (!done && bytes > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       bytes);
-    if (e != hipSuccess) return fail(NT_ERR_HIP, "attention: %s", hipGetErrorString(e));
-    done = true;
-  }
-  return NT_OK;
-}
-
 template <int HD>
 static int launch_f32(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v,
                       int64_t ldv, void* out, int64_t ldo, const int64_t* qo, const int64_t* kvo,
                       int64_t B, int64_t H, int64_t max_q, float scale, hipStream_t s) {
   dim3 grid((unsigned)((max_q + 127) / 128), (unsigned)H, (unsigned)B);
-  const int rc = allow_lds<varlen_attention_f32_kernel<HD>>(SplitAttention<HD>::kBuf);
-  if (rc != NT_OK) return rc;
   hipLaunchKernelGGL((varlen_attention_f32_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kBuf, s,
                      static_cast<const float*>(q), ldq, static_cast<const float*>(k), ldk,
                      static_cast<const float*>(v), ldv, static_cast<float*>(out), ldo, qo, kvo,
@@ -1249,8 +1235,6 @@ template <int HD>
 static int launch_f32_sched(dim3 grid, hipStream_t s, const void* q, int64_t ldq, const void* k, int64_t ldk,
                              const void* v, int64_t ldv, void* out, int64_t ldo, const int4* sched,
                              unsigned num_heads, float scale_log2e) {
-  const int rc = allow_lds<varlen_attention_f32_sched_kernel<HD>>(SplitAttention<HD>::kBuf);
-  if (rc != NT_OK) return rc;
   hipLaunchKernelGGL((varlen_attention_f32_sched_kernel<HD>), grid, dim3(256), SplitAttention<HD>::kBuf, s,
                      static_cast<const float*>(q), ldq, static_cast<const float*>(k), ldk,
                      static_cast<const float*>(v), ldv, static_cast<float*>(out), ldo, sched, num_heads,

@@ -657,13 +657,8 @@ extern "C" int nt_varlen_attention_planned(const void* q, int64_t ldq, const voi
   const float scale_log2e = scale * 1.4426950408889634f;
 #define NT_CHAIN_LAUNCH(TYPE)                                                                              \
   {                                                                                                        \
-    static bool attr_set = false;                                                                          \
-    if (!attr_set) {                                                                                       \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_chain_kernel<TYPE>),      \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);           \
-      if (e != hipSuccess) return fail(NT_ERR_HIP, "attention_planned: %s", hipGetErrorString(e));         \
-      attr_set = true;                                                                                     \
-    }                                                                                                      \
+    const int rc = allow_lds<attention_chain_kernel<TYPE>>(lds_bytes, "attention_planned");                \
+    if (rc != NT_OK) return rc;                                                                            \
     hipLaunchKernelGGL((attention_chain_kernel<TYPE>), dim3((unsigned)n_workgroups), dim3(64 * kChainWaves), \
                        lds_bytes, s, static_cast<const TYPE*>(q), ldq, static_cast<const TYPE*>(k), ldk,   \
                        static_cast<const TYPE*>(vt), ldvt, static_cast<TYPE*>(out), ldo, plan, scale_log2e); \

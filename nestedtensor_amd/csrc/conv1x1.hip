@@ -421,15 +421,8 @@ static int launch_conv(const void* x, const void* w, void* y, const int64_t* pix
                        int64_t B, int64_t total_tiles, int c_in, int c_out, int cus, hipStream_t stream) {
   const size_t lds = conv_lds_bytes(c_in, c_out, WAVES, sizeof(T));
   auto kernel = conv1x1_nchw_kernel<T, WAVES, LOADS>;
-  static bool configured = false;      // one attribute call per instantiation (and process)
-  if (!configured) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            160 * 1024) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail(NT_ERR_HIP, "conv1x1: cannot raise the dynamic LDS limit");
-    }
-    configured = true;
-  }
+  const int rc = allow_lds<conv1x1_nchw_kernel<T, WAVES, LOADS>>(160 * 1024, "conv1x1");
+  if (rc != NT_OK) return rc;
   int64_t grid = cus;
   const int64_t needed = (total_tiles + WAVES - 1) / WAVES;
   if (grid > needed) grid = needed;
@@ -455,15 +448,8 @@ template <typename T, int KS, int CG>
 static int launch_direct(const void* x, const void* w, void* y, const int64_t* pix_offsets, const int64_t* tile_offsets,
                          int64_t B, int64_t total_tiles, int c_in, int c_out, int cus, hipStream_t stream) {
   auto kernel = conv1x1_direct_kernel<T, KS, CG>;
-  static bool configured = false;      // one attribute call per instantiation (and process)
-  if (!configured) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            160 * 1024) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail(NT_ERR_HIP, "conv1x1: cannot raise the dynamic LDS limit");
-    }
-    configured = true;
-  }
+  const int rc = allow_lds<conv1x1_direct_kernel<T, KS, CG>>(160 * 1024, "conv1x1");
+  if (rc != NT_OK) return rc;
   int64_t grid = cus;
   const int64_t needed = (total_tiles * CG + 7) / 8;
   if (grid > needed) grid = needed;

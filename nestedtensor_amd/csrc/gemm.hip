@@ -581,14 +581,8 @@ static int launch_kernel(const GemmArgs<T>& a, hipStream_t stream) {
   const int64_t wgs = ((tiles_m + 7) / 8) * 8 * tiles_n;
   if (wgs > 0x7fffffffLL) return fail(NT_ERR_UNSUPPORTED, "linear: too many tiles");
   const int lds_bytes = Cfg::kLdsBytes + Cfg::kBN * (int)sizeof(float);
-  static bool attr_set = false;
-  if (!attr_set && lds_bytes > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(linear_kernel<T, Cfg, EPI, ALIGNED_K>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (e != hipSuccess) return fail(NT_ERR_HIP, "linear: %s", hipGetErrorString(e));
-    attr_set = true;
-  }
+  const int rc = allow_lds<linear_kernel<T, Cfg, EPI, ALIGNED_K>>(lds_bytes, "linear");
+  if (rc != NT_OK) return rc;
   hipLaunchKernelGGL((linear_kernel<T, Cfg, EPI, ALIGNED_K>), dim3((unsigned)wgs),
                      dim3(Cfg::kThreads), lds_bytes, stream, a);
   return check_launch("linear_kernel");
@@ -891,13 +885,8 @@ template <typename T, class Cfg, int EPI>
 static int launch_phased(const GemmArgs<T>& a, hipStream_t stream) {
   const int64_t tiles = ((a.M + Cfg::kBM - 1) / Cfg::kBM) * ((a.N + Cfg::kBN - 1) / Cfg::kBN);
   const int lds_bytes = Cfg::kLdsBytes + Cfg::kBN * (int)sizeof(float);
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(phased_kernel<T, Cfg, EPI>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (e != hipSuccess) return fail(NT_ERR_HIP, "linear: %s", hipGetErrorString(e));
-    attr_set = true;
-  }
+  const int rc = allow_lds<phased_kernel<T, Cfg, EPI>>(lds_bytes, "linear");
+  if (rc != NT_OK) return rc;
   hipLaunchKernelGGL((phased_kernel<T, Cfg, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds_bytes, stream,
                      a);
   return check_launch("phased_kernel");
@@ -1211,13 +1200,8 @@ template <class Cfg, int EPI>
 static int launch_split(const GemmArgs<float>& a, hipStream_t stream) {
   const int64_t tiles = ((a.M + Cfg::kBM - 1) / Cfg::kBM) * ((a.N + Cfg::kBN - 1) / Cfg::kBN);
   const int lds_bytes = Cfg::kLdsBytes + Cfg::kBN * (int)sizeof(float);
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_kernel<Cfg, EPI>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (e != hipSuccess) return fail(NT_ERR_HIP, "linear: %s", hipGetErrorString(e));
-    attr_set = true;
-  }
+  const int rc = allow_lds<split_kernel<Cfg, EPI>>(lds_bytes, "linear");
+  if (rc != NT_OK) return rc;
   hipLaunchKernelGGL((split_kernel<Cfg, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds_bytes, stream, a);
   return check_launch("split_kernel");
 }

@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <atomic>
 
 #include "../../include/nestedtensor_amd.h"
 
@@ -28,6 +29,24 @@ inline int check_launch(const char* what) {
     return fail(NT_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
   }
   return NT_OK;
+}
+
+// Dynamic LDS beyond 48 KiB has to be allowed on every device that a kernel runs on: once per
+// kernel and device (the first 64 of them; on any other every time).
+template <auto KERNEL>
+inline int allow_lds(int bytes, const char* what) {
+  static std::atomic<uint64_t> allowed{0};
+  if (bytes <= 48 * 1024) return NT_OK;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  const uint64_t bit = dev >= 0 && dev < 64 ? uint64_t(1) << dev : 0;
+  if (e == hipSuccess && (allowed.load(std::memory_order_relaxed) & bit) == 0) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess) allowed.fetch_or(bit, std::memory_order_relaxed);
+  }
+  if (e == hipSuccess) return NT_OK;
+  (void)hipGetLastError();
+  return fail(NT_ERR_HIP, "%s: cannot raise the dynamic LDS limit: %s", what, hipGetErrorString(e));
 }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
