@@ -530,13 +530,18 @@ int nt_transpose_ragged_lines(const void* in, void* out, const int64_t* offsets,
  * to t - 1 pixels before a multiple of t); total_tiles their sum.  y must be
  * 128-byte aligned.  f16 / bf16, fp32 accumulation; nt_conv1x1_supported() says
  * whether a pair of depths is covered (c_in a multiple of 16 up to 128, c_out a
- * multiple of 32 up to 512, and the weight plus two wavefronts' tiles must fit the
- * 160 KiB of LDS), otherwise NT_ERR_UNSUPPORTED.  Replaces transpose_nchw_nhwc +
+ * multiple of 32 up to 512, and what the kernels keep in LDS, the weight above
+ * all, must fit its 160 KiB), otherwise NT_ERR_UNSUPPORTED.  Replaces transpose_nchw_nhwc +
  * matmul + transpose_nhwc_nchw of the reference's 1x1 path
  * (nestedtensor/csrc/conv2d.cpp:33-75) by one launch that reads and writes every
  * element once. */
 int nt_conv1x1_supported(int64_t c_in, int64_t c_out, int dtype);
 int64_t nt_conv1x1_tile_pixels(void);
+/* What nt_conv1x1_nchw runs on, for num_cus compute units (0: those of the current device):
+ * route[0] wavefronts per workgroup of the kernel that writes whole lines, or, where that is 0,
+ * the kernel without LDS for pixels and results, route[1] wavefronts sharing a window. */
+int nt_conv1x1_route(int64_t B, int64_t total_tiles, int64_t c_in, int64_t c_out, int dtype, int num_cus,
+                     int* route);
 int nt_conv1x1_nchw(const void* x, const void* weight, void* y, const int64_t* pix_offsets,
                     const int64_t* tile_offsets, int64_t B, int64_t total_tiles, int64_t c_in,
                     int64_t c_out, int dtype, void* stream);

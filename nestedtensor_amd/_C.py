@@ -99,6 +99,7 @@ SIGNATURES = {
                                          _int, _c_void_p]),
     "nt_conv1x1_tile_pixels": (_i64, []),
     "nt_conv1x1_supported": (_int, [_i64, _i64, _int]),
+    "nt_conv1x1_route": (_int, [_i64, _i64, _i64, _i64, _int, _int, _c_void_p]),
     "nt_conv1x1_nchw": (_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i64, _int,
                                _c_void_p]),
     "nt_embedding_bag": (_int, [_c_void_p, _i64, _i64, _c_void_p, _i64, _c_void_p, _c_void_p, _i64, _i64, _int,

@@ -286,7 +286,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
 // so the even and the odd accumulator of a channel are one dword of the result: 128 contiguous
 // bytes of a row per store and lane half.  Nothing is transposed, no window is
 // multiplied twice, and CG wavefronts share a window, a CG-th of the output channels each, so
-// that a small batch still spreads over the chip (us, in the cache / not):
+// that a small batch still spreads over the chip (us, in the cache / not; with CG 2 throughout):
 //   64 -> 256 on 2 600, 29 000, 127 000 pixels    27 -> 9, 30 -> 11, 41 / 42 -> 27 / 29
 //   64 -> 64  on 2 800, 32 000, 128 000           15 -> 9, 16 -> 9, 18 / 21 -> 14 / 17
 //   32 -> 128 on 3 400, 31 000, 122 000           14 -> 8, 16 -> 9, 16 / 17 -> 14 / 15
@@ -479,42 +479,88 @@ static int conv_waves(int c_in, int c_out, size_t elem) {
   return 0;
 }
 
+// What a convolution runs on: `waves` wavefronts per workgroup of conv1x1_nchw_kernel, or `parts`
+// wavefronts per window of conv1x1_direct_kernel.  Both 0: it does not fit the LDS.
+struct ConvRoute {
+  int waves, parts;
+};
+
+static ConvRoute choose_conv(int64_t B, int64_t total_tiles, int c_in, int c_out, int cus, size_t elem) {
+  // Which kernel: see conv1x1_direct_kernel.  (total_tiles counts one tile too many per image.)
+  const int64_t windows = total_tiles - B > 0 ? total_tiles - B : 0;
+  const bool small = windows <= (int64_t(64) << 20) / (kConvTile * (int64_t)elem) / c_out;
+  if (small || c_in > 96 || (c_in > 64 && c_out <= 2 * c_in)) {
+    if ((size_t)c_out * (c_in + 8) * elem > 160 * 1024) return {0, 0};
+    // Four wavefronts per window while two would leave half of them idle or nearly so (128 -> 256
+    // on 3 200 and 35 000 pixels 22 -> 16 and 25 -> 21), two from there on (on 110 000 28 against 32).
+    return {0, c_out % 128 == 0 && windows <= 4 * (int64_t)cus ? 4 : 2};
+  }
+  return {conv_waves(c_in, c_out, elem), 0};
+}
+
 template <typename T>
 static int launch_conv_t(const void* x, const void* w, void* y, const int64_t* pix_offsets, const int64_t* tile_offsets,
                          int64_t B, int64_t total_tiles, int c_in, int c_out, int cus, hipStream_t stream) {
-  // Which kernel: see conv1x1_direct_kernel.  (total_tiles counts one tile too many per image.)
-  const int64_t windows = total_tiles - B > 0 ? total_tiles - B : 0;
-  const bool small = windows <= (int64_t(64) << 20) / (kConvTile * (int64_t)sizeof(T)) / c_out;
-  if (small || c_in > 96 || (c_in > 64 && c_out <= 2 * c_in)) {
-    // Four wavefronts per window while two would leave half of them idle or nearly so (128 -> 256
-    // on 3 200 and 35 000 pixels 22 -> 16 and 25 -> 21), two from there on (on 110 000 28 against 32).
-    if (c_out % 128 == 0 && windows <= 4 * (int64_t)cus) {
-      return launch_direct_ks<T, 4>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
-    }
-    return launch_direct_ks<T, 2>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
-  }
-  switch (conv_waves(c_in, c_out, sizeof(T))) {
-    case 8: return launch_conv_w<T, 8>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
-    case 7: return launch_conv_w<T, 7>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
-    case 6: return launch_conv_w<T, 6>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
-    case 4: return launch_conv_w<T, 4>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
-    case 2: return launch_conv_w<T, 2>(x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream);
+#define NT_CONV_ARGS x, w, y, pix_offsets, tile_offsets, B, total_tiles, c_in, c_out, cus, stream
+  const ConvRoute route = choose_conv(B, total_tiles, c_in, c_out, cus, sizeof(T));
+  switch (route.parts) {
+    case 4: return launch_direct_ks<T, 4>(NT_CONV_ARGS);
+    case 2: return launch_direct_ks<T, 2>(NT_CONV_ARGS);
     default: break;
   }
-  return fail(NT_ERR_UNSUPPORTED, "conv1x1: %d -> %d channels do not fit the LDS (%zu bytes with two wavefronts)",
-              c_in, c_out, conv_lds_bytes(c_in, c_out, 2, sizeof(T)));
+  switch (route.waves) {
+    case 8: return launch_conv_w<T, 8>(NT_CONV_ARGS);
+    case 7: return launch_conv_w<T, 7>(NT_CONV_ARGS);
+    case 6: return launch_conv_w<T, 6>(NT_CONV_ARGS);
+    case 4: return launch_conv_w<T, 4>(NT_CONV_ARGS);
+    case 2: return launch_conv_w<T, 2>(NT_CONV_ARGS);
+    default: break;
+  }
+#undef NT_CONV_ARGS
+  return fail(NT_ERR_UNSUPPORTED, "conv1x1: %d -> %d channels do not fit the LDS", c_in, c_out);
 }
 
 }  // namespace nt
 
 using namespace nt;
 
+static int compute_units(int* cus) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || *cus < 1) {
+    (void)hipGetLastError();
+    return fail(NT_ERR_HIP, "conv1x1: cannot query the device");
+  }
+  return NT_OK;
+}
+
 extern "C" int64_t nt_conv1x1_tile_pixels(void) { return kConvTile; }
 
 extern "C" int nt_conv1x1_supported(int64_t c_in, int64_t c_out, int dtype) {
   if (dtype != NT_F16 && dtype != NT_BF16) return 0;
   if (c_in < 16 || c_in % 16 != 0 || c_in > kConvMaxIn || c_out < 32 || c_out % 32 != 0 || c_out > kConvMaxOut) return 0;
-  return conv_waves((int)c_in, (int)c_out, 2) != 0;
+  // of a small batch and of a large one
+  for (int64_t tiles : {int64_t(1), int64_t(0x7fffffff)}) {
+    const ConvRoute route = choose_conv(0, tiles, (int)c_in, (int)c_out, 256, 2);
+    if (route.waves == 0 && route.parts == 0) return 0;
+  }
+  return 1;
+}
+
+extern "C" int nt_conv1x1_route(int64_t B, int64_t total_tiles, int64_t c_in, int64_t c_out, int dtype, int num_cus,
+                                int* route) {
+  if (B < 0 || total_tiles < 0 || num_cus < 0 || !route) return fail(NT_ERR_INVALID_ARGUMENT, "conv1x1_route: bad arguments");
+  if (!nt_conv1x1_supported(c_in, c_out, dtype)) {
+    return fail(NT_ERR_UNSUPPORTED, "conv1x1: %lld -> %lld channels", (long long)c_in, (long long)c_out);
+  }
+  if (num_cus == 0) {
+    const int rc = compute_units(&num_cus);
+    if (rc != NT_OK) return rc;
+  }
+  const ConvRoute r = choose_conv(B, total_tiles, (int)c_in, (int)c_out, num_cus, 2);
+  route[0] = r.waves;
+  route[1] = r.parts;
+  return NT_OK;
 }
 
 extern "C" int nt_conv1x1_nchw(const void* x, const void* weight, void* y, const int64_t* pix_offsets,
@@ -535,12 +581,9 @@ extern "C" int nt_conv1x1_nchw(const void* x, const void* weight, void* y, const
     return fail(NT_ERR_INVALID_ARGUMENT, "conv1x1: the weight must be 16-byte and the output 128-byte aligned");
   }
   if (total_tiles > 0x7fffffffLL) return fail(NT_ERR_UNSUPPORTED, "conv1x1: too many tiles");
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
-    (void)hipGetLastError();
-    return fail(NT_ERR_HIP, "conv1x1: cannot query the device");
-  }
+  int cus = 0;
+  const int rc = compute_units(&cus);
+  if (rc != NT_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == NT_F16) {
     return launch_conv_t<_Float16>(x, weight, y, pix_offsets, tile_offsets, B, total_tiles, (int)c_in, (int)c_out, cus, s);

@@ -1,5 +1,7 @@
 """Row-major 1x1 convolution on both kernels and on either side of the lines between them: pixel
 counts around one and two 64-pixel windows, next to images that make the batch small or large."""
+import ctypes
+
 import pytest
 import torch
 
@@ -9,8 +11,19 @@ DEV = torch.device("cuda", 0)
 EDGES = [1, 2, 31, 32, 33, 63, 64, 65, 66, 127, 128, 129, 191, 193, 640]
 
 
+def _route(pixels, c_in, c_out):
+    """(wavefronts of the kernel that writes whole lines or 0, wavefronts per window of the other one)."""
+    from nestedtensor_amd import _C
+    route = (ctypes.c_int * 2)()
+    tiles = sum((n + 63) // 64 + 1 for n in pixels)
+    _C.check(_C.lib.nt_conv1x1_route(len(pixels), tiles, c_in, c_out, _C.dtype_code(torch.float16), 0, route))
+    return tuple(route)
+
+
 def _check(pixels, c_in, c_out, dtype):
     import nestedtensor_amd as nt
+    from nestedtensor_amd import _C
+    assert _C.lib.nt_conv1x1_supported(c_in, c_out, _C.dtype_code(dtype))
     g = torch.Generator("cuda").manual_seed(c_in + c_out)
     maps = [torch.randn(c_in, 1, n, device=DEV, generator=g).to(dtype) for n in pixels]
     w = (torch.randn(c_out, c_in, 1, 1, device=DEV, generator=g) * c_in ** -0.5).to(dtype)
@@ -39,3 +52,25 @@ def test_conv1x1_small_batches(c_in, c_out, dtype):
     (128, 256, 1024 * 64 - 2000), (128, 256, 1024 * 64 + 200)])   # four, two wavefronts per window
 def test_conv1x1_large_batches(c_in, c_out, pixels, dtype):
     _check(EDGES + [pixels] + EDGES, c_in, c_out, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c_in,c_out,pixels,waves", [
+    (16, 32, 1100001, 8), (32, 96, 360001, 8), (48, 512, 70001, 8),
+    (64, 224, 160001, 7), (64, 384, 90001, 6), (80, 192, 180001, 6), (64, 512, 70001, 4), (96, 256, 140001, 4),
+    (80, 480, 75001, 2), (96, 512, 70001, 2)])
+def test_conv1x1_whole_lines(c_in, c_out, pixels, waves, dtype):
+    """Every number of wavefronts that the LDS leaves room for, and every depth of the loads."""
+    pixels = [7, 192, 255, 256, 257, 1001] + EDGES + [pixels] + EDGES
+    assert _route(pixels, c_in, c_out) == (waves, 0)
+    _check(pixels, c_in, c_out, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c_in,c_out", [(128, 384), (128, 512), (112, 448)])
+@pytest.mark.parametrize("large", [0, 200001])
+def test_conv1x1_weight_fills_the_lds(c_in, c_out, large, dtype):
+    """Weights beside which the pixels of the other kernel find no room."""
+    pixels = EDGES + [large] * (large > 0)
+    assert _route(pixels, c_in, c_out)[0] == 0
+    _check(pixels, c_in, c_out, dtype)

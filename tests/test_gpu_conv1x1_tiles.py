@@ -1,5 +1,6 @@
-"""Row-major 1x1 convolution where its tiles meet the ends of an image: pixel counts around one, two
-and three 64-pixel lines, where a tile's 128-pixel window is first or no longer wholly inside."""
+"""Row-major 1x1 convolution of small batches where its tiles meet the ends of an image: pixel counts
+around one, two and three 64-pixel windows.  (The kernel that writes whole lines, for large
+results, is run on such images by test_gpu_conv1x1_routes.py.)"""
 import pytest
 import torch
 
