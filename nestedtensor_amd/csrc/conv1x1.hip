@@ -489,11 +489,26 @@ static ConvRoute choose_conv(int64_t B, int64_t total_tiles, int c_in, int c_out
   // Which kernel: see conv1x1_direct_kernel.  (total_tiles counts one tile too many per image.)
   const int64_t windows = total_tiles - B > 0 ? total_tiles - B : 0;
   const bool small = windows <= (int64_t(64) << 20) / (kConvTile * (int64_t)elem) / c_out;
-  if (small || c_in > 96 || (c_in > 64 && c_out <= 2 * c_in)) {
+  const int64_t round = 8 * (int64_t)cus;         // wavefronts in flight
+  // Few channels leave little to save: whole lines win from two or three rounds of windows on (16 -> 64 on
+  // 300 000 pixels 17.1 against 17.8, on 400 000 19.6 against 23.0, 32 -> 96 on 300 000 25.5 against 27.5, 16 -> 32 on
+  // 400 000 15.3 against 15.4, on 900 000 22.7 against 25.8; but 32 -> 32 34.8 against 34.2).
+  const bool few_channels = c_out == 32 ? c_in == 16 && windows > 3 * round : c_in <= 32 && c_out <= 96 && windows > 2 * round;
+  if ((small && !few_channels) || c_in > 96 || (c_in > 64 && c_out <= 2 * c_in)) {
     if ((size_t)c_out * (c_in + 8) * elem > 160 * 1024) return {0, 0};
-    // Four wavefronts per window while two would leave half of them idle or nearly so (128 -> 256
-    // on 3 200 and 35 000 pixels 22 -> 16 and 25 -> 21), two from there on (on 110 000 28 against 32).
-    return {0, c_out % 128 == 0 && windows <= 4 * (int64_t)cus ? 4 : 2};
+    // As many wavefronts per window as one round of them can take (4 / 2 / 1, us: 64 -> 256 on 24 000
+    // pixels 9.5 / 11.6 / 16.0, on 40 000 18.4 / 12.4 / 16.7, on 75 000 28.9 / 27.0 / 20.0).
+    if (c_out % 128 == 0 && 4 * windows <= round) return {0, 4};
+    if (2 * windows <= round) return {0, 2};
+    if (windows <= round) return {0, 1};
+    // Beyond one round two to a window while three half rounds do for two whole ones (2 / 1: 64 -> 96 on
+    // 150 000 24.7 / 27.5, on 200 000 31.0 / 27.9), and for many input channels, whose windows take longest
+    // to fetch (128 -> 64 on 200 000 31.1 / 39.2, on 700 000 82.5 / 89.7).
+    // With 32 output channels the second wavefront only fetches the same pixels: worth it where the
+    // windows are few (32 -> 32 on 30 000 5.4 / 6.0, 96 -> 32 on 150 000 18.8 / 27.9), but not for few channels
+    // beyond a round (32 -> 32 on 900 000 44.8 / 34.2) or beyond four rounds (96 -> 32 on 900 000 77.6 / 67.5).
+    const bool two = 2 * windows <= 3 * round ? c_out > 32 || c_in > 32 : c_in > 64 && (c_out > 32 || windows <= 4 * round);
+    return {0, two ? 2 : 1};
   }
   return {conv_waves(c_in, c_out, elem), 0};
 }
@@ -506,6 +521,7 @@ static int launch_conv_t(const void* x, const void* w, void* y, const int64_t* p
   switch (route.parts) {
     case 4: return launch_direct_ks<T, 4>(NT_CONV_ARGS);
     case 2: return launch_direct_ks<T, 2>(NT_CONV_ARGS);
+    case 1: return launch_direct_ks<T, 1>(NT_CONV_ARGS);
     default: break;
   }
   switch (route.waves) {

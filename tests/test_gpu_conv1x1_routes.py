@@ -49,7 +49,7 @@ def test_conv1x1_small_batches(c_in, c_out, dtype):
     (64, 256, 131072 - 200), (64, 256, 131072 + 200),        # 64 MiB of result
     (48, 128, 270001), (96, 256, 131072 + 200),              # whole lines
     (112, 128, 270001), (96, 64, 540001),                    # too many channels for those
-    (128, 256, 1024 * 64 - 2000), (128, 256, 1024 * 64 + 200)])   # four, two wavefronts per window
+    (128, 256, 1024 * 64 - 2000), (128, 256, 1024 * 64 + 200)])   # two wavefronts per window and one
 def test_conv1x1_large_batches(c_in, c_out, pixels, dtype):
     _check(EDGES + [pixels] + EDGES, c_in, c_out, dtype)
 
@@ -73,4 +73,14 @@ def test_conv1x1_weight_fills_the_lds(c_in, c_out, large, dtype):
     """Weights beside which the pixels of the other kernel find no room."""
     pixels = EDGES + [large] * (large > 0)
     assert _route(pixels, c_in, c_out)[0] == 0
+    _check(pixels, c_in, c_out, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c_in,c_out,pixels,parts", [
+    (16, 128, 20001, 4), (128, 512, 20001, 4), (48, 96, 40001, 2), (64, 32, 40001, 2), (128, 32, 190001, 2), (96, 96, 540001, 2),
+    (16, 32, 100001, 1), (32, 160, 100001, 1), (128, 512, 100001, 1), (64, 64, 250001, 1), (48, 32, 250001, 1), (112, 32, 600001, 1)])
+def test_conv1x1_wavefronts_of_a_window(c_in, c_out, pixels, parts, dtype):
+    pixels = EDGES + [pixels] + EDGES
+    assert _route(pixels, c_in, c_out) == (0, parts)
     _check(pixels, c_in, c_out, dtype)
