@@ -1839,14 +1839,15 @@ TORCH_LIBRARY_IMPL(nestedtensor, CUDA, m) {
   m.impl("packed_sequence_lowered", packed_sequence_lowered);
 }
 
-// Operators on plain tensors of any device: merge_tensor_mask is host logic over
-// torch reductions; nt_from_tensor_mask answers the trivial masks (empty, one
-// element) for any device and raises for host tensors otherwise.
 // These two pass no gradient on: their results require none, also where a weight does.
 TORCH_LIBRARY_IMPL(nestedtensor, AutogradCUDA, m) {
   m.impl("transpose_packed", torch::CppFunction::makeFallthrough());
   m.impl("conv1x1_packed", torch::CppFunction::makeFallthrough());
 }
+
+// Operators on plain tensors of any device: merge_tensor_mask is host logic over
+// torch reductions; nt_from_tensor_mask answers the trivial masks (empty, one
+// element) for any device and raises for host tensors otherwise.
 TORCH_LIBRARY_IMPL(nestedtensor, CompositeExplicitAutograd, m) {
   m.impl("merge_tensor_mask", merge_tensor_mask);
   m.impl("size_summary", size_summary);
