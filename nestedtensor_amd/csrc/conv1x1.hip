@@ -286,18 +286,18 @@ __global__ __launch_bounds__(64 * WAVES) void conv1x1_nchw_kernel(const T* __res
 // so the even and the odd accumulator of a channel are one dword of the result: 128 contiguous
 // bytes of a row per store and lane half.  Nothing is transposed, no window is
 // multiplied twice, and CG wavefronts share a window, a CG-th of the output channels each, so
-// that a small batch still spreads over the chip (us, in the cache / not; with CG 2 throughout):
-//   64 -> 256 on 2 600, 29 000, 127 000 pixels    27 -> 9, 30 -> 11, 41 / 42 -> 27 / 29
-//   64 -> 64  on 2 800, 32 000, 128 000           15 -> 9, 16 -> 9, 18 / 21 -> 14 / 17
-//   32 -> 128 on 3 400, 31 000, 122 000           14 -> 8, 16 -> 9, 16 / 17 -> 14 / 15
-//   128 -> 256 on 35 000, 110 000, 517 000        66 -> 20, 89 -> 27 / 32, 268 / 270 -> 138 / 145
-//   128 -> 64  on 95 000, 549 000                 36 -> 15 / 16, 93 / 99 -> 53 / 66
+// that a small batch still spreads over the chip (us, in the cache / not, whole-line kernel -> here):
+//   64 -> 256 on 2 600, 29 000, 127 000 pixels    28 / 31 -> 8 / 10, 28 / 33 -> 10 / 14, 36 / 44 -> 20 / 28
+//   64 -> 64  on 2 800, 32 000, 128 000           15 / 18 -> 6 / 7, 15 / 17 -> 6 / 8, 17 / 22 -> 10 / 15
+//   32 -> 128 on 3 400, 31 000, 122 000           14 / 16 -> 5 / 6, 14 / 16 -> 6 / 9, 15 / 19 -> 11 / 15
+//   128 -> 256 on 35 000, 110 000, 517 000        54 / 67 -> 17 / 21, 93 / 103 -> 25 / 32, 249 / 260 -> 141 / 148
+//   128 -> 64  on 95 000, 549 000                 37 / 43 -> 12 / 18, 92 / 113 -> 53 / 89
 // A row's 128 bytes are no whole line, and the parts of a line come from two wavefronts: they
 // meet in the L2 as long as the result is not much larger than that.  Beyond 64 MiB the
 // whole lines of conv1x1_nchw_kernel win (64 -> 256 on 552 000 pixels 84 / 93 against 127 / 168,
 // 64 -> 64 on 559 000 43 / 49 against 39 / 57, 96 -> 256 on 443 000 121 / 127 against 130 / 142), but not
-// where its tiles leave the LDS no room for enough wavefronts (96 -> 64 on 524 000 147 / 208
-// against 45 / 56, 128 channels above).
+// where its tiles leave the LDS no room for enough wavefronts (96 -> 64 on 524 000 137 / 227
+// against 40 / 63, 128 channels above).
 template <typename T, int KS, int CG>
 __global__ __launch_bounds__(512, 2) void conv1x1_direct_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                                 T* __restrict__ y, const int64_t* __restrict__ pix_offsets,
